@@ -264,6 +264,8 @@ int op_mat_mul_f32(htpops_context *ctx, float *dst, const float *act, const void
                    int weight_type);
 int op_mat_mul_permuted(htpops_context *ctx, float *dst, const float *act, const void *weight, int m, int k, int n,
                         int kind);
+// the same for matmuls of one row count and weight kind that the caller has validated and that nothing orders
+int op_mat_mul_permuted_group(htpops_context *ctx, const PermutedMatMul *members, int count, int m, int kind);
 int op_flash_attn(htpops_context *ctx, void *o, const void *q, const void *k, const void *v, const void *mask,
                   int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim, int qo_is_f32, int causal,
                   bool no_alloc = false);

@@ -140,6 +140,22 @@ hipError_t launch_permuted_weight_to_fragments(hipStream_t stream, void *dst, co
 hipError_t launch_mat_mul_fragments(hipStream_t stream, float *out, const float *act, const void *weight_fragments,
                                     int m, int k, int n, void *act_fragments);
 
+// The same formats read as they lie, nothing converted or kept, for up to kPermutedRowsMax rows: up to kPermutedGroupMax
+// matmuls of one row count and weight kind in one launch (plus one that puts the activations into operand order where
+// they do not fit LDS). The caller guarantees that no member reads what another writes. A member's result does not
+// depend on the others. `workspace`: permuted_rows_workspace_bytes.
+constexpr int kPermutedRowsMax  = 32;
+constexpr int kPermutedGroupMax = 8;
+struct PermutedMatMul {
+  float       *out;
+  const float *act;
+  const void  *weight;
+  int          k, n;
+};
+size_t     permuted_rows_workspace_bytes(const PermutedMatMul *members, int count, int m);
+hipError_t launch_permuted_rows_group(hipStream_t stream, const PermutedMatMul *members, int count, int m, int weight_kind,
+                                      void *workspace);
+
 // attention; see htpops_flash_attn_ptr. `workspace` holds split-KV partials (decode), size from
 // flash_attn_workspace_bytes. `q8_out` (or nullptr; used only where flash_attn_writes_q8_0 says so: decode with
 // head_dim 64 / 128 and fp32 output): the output row is also written there as Q8_0 blocks, bit for bit what

@@ -1,0 +1,466 @@
+// Up to 32 activation rows against the reference's own weight formats (its ops 1-4), read as they lie in memory.
+//
+// Replaces hmx_mat_mul_permuted_w16a32 and hmx_mat_mul_permuted_qk_0_d16a32 for decode-sized row counts (reference:
+// src/dsp/ops/mat_mul.c:758-855, :875-1153): fp16 activations times weights that are fp16(quant * scale), sums in fp32,
+// results rounded to fp16. The bound is the stream over the weight bytes (144 B per 256 Q4_0 or IQ4_NL weights, 272 B of
+// Q8_0, 512 B of fp16): a converted fp16 copy, which the many-row kernel wants, would be 3.6 times the bytes of the
+// 4-bit formats, so nothing is converted here and the weights are turned to fp16 in registers, on their way into the
+// matrix cores.
+//
+// The formats suit that: the 8 K rows of one column of a super-block are ONE dword of nibbles (two bytes per row pair
+// for Q8_0, a dword per row pair for fp16 tiles), and those are exactly the 8 values that a lane feeds to
+// v_mfma_f32_16x16x32_f16. A wave takes a 32 x 32 tile per step: lane (g = lane / 16, i = lane % 16) holds K rows
+// 8 g .. 8 g + 7 (super-block g of the tile) of columns 2 i and 2 i + 1, two matrix instructions per step and 16 rows.
+// A workgroup owns 32 columns over all of K, its waves take every eighth tile (the tiles of a column group are
+// contiguous, so a workgroup reads one stream), and their sums meet in LDS in wave order: a result does not depend on
+// the launch it is part of. Several steps of every wave are in flight before the first use.
+// Measured on MI355X, a message with the seven projections of a Llama-7B layer over Q4_0 super-blocks, one token
+// (114 MB): 28.1 us = 4.1 TB/s, against 374 us for a launch per matrix over fp16 copies in operand order (7 x 41 us on 64
+// to 172 workgroups, each behind a 5 us conversion of the row). Vector-ALU work is about 30 instructions per step and wave,
+// 10 us of it; depth 8 instead of 4 for the 4-bit formats 28.9 us, 4 or 16 waves per workgroup 30.3 and 31.0 us.
+// The activations, rounded to fp16, are read from LDS where they fit (one or a few rows: every workgroup converts them
+// for itself), else from a copy in operand order that one small launch makes.
+#include "device_utils.h"
+#include "kernels.h"
+
+#include <algorithm>
+
+namespace htpops {
+
+namespace {
+
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+typedef float    v4f __attribute__((ext_vector_type(4)));
+
+constexpr int kRowsWaves   = 8;
+constexpr int kRowsThreads = kRowsWaves * kWave;
+// Activations up to this many bytes are kept in LDS (two workgroups per compute unit at least; with 80 KiB allowed,
+// 8 rows of 4096 against IQ4_NL ran at 26.4 us per layer of seven 4096 x 4096 matrices, against 21.7 us in operand order).
+constexpr int kRowsActLds    = 64 * 1024;
+constexpr int kRowsWideTiles = 512;  // column groups of a launch from which a workgroup takes two (see the launcher)
+
+struct RowsMember {
+  float         *out;
+  const float   *act;   // fp32 rows
+  const uint4   *frag;  // the same in operand order (kernels that do not keep them in LDS)
+  const uint8_t *weight;
+  int            k, n, first;  // first: this member's first workgroup
+};
+struct RowsArgs {
+  RowsMember member[kPermutedGroupMax];
+  int        count, m;
+};
+
+template <int KIND>
+struct RawStep;  // what a lane loads of one 32 x 32 tile
+template <>
+struct RawStep<1> {
+  static constexpr int kTileBytes = 2048;
+  uint2                q[4];  // K row pair 4 g + v, columns 2 i and 2 i + 1
+};
+template <>
+struct RawStep<2> {
+  static constexpr int kTileBytes = 4 * 144;
+  uint4                s;  // 8 scales of super-block g
+  uint2                q;  // 8 nibbles of column 2 i, 8 of column 2 i + 1
+};
+template <>
+struct RawStep<4> : RawStep<2> {};
+template <>
+struct RawStep<3> {
+  static constexpr int kTileBytes = 4 * 272;
+  uint4                s;
+  uint32_t             q[4];  // row pair v: two bytes of column 2 i, two of column 2 i + 1
+};
+
+template <int KIND>
+__device__ __forceinline__ void load_step(RawStep<KIND> &r, const uint8_t *__restrict__ tile, int g, int i) {
+  if constexpr (KIND == 1) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      r.q[v] = *reinterpret_cast<const uint2 *>(tile + (uint32_t) (4 * g * 128 + 8 * i) + 128 * v);
+    }
+  } else if constexpr (KIND == 3) {
+    r.s = *reinterpret_cast<const uint4 *>(tile + (uint32_t) (g * 272));
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      r.q[v] = *reinterpret_cast<const uint32_t *>(tile + (uint32_t) (g * 272 + 4 * i) + 16 + 64 * v);
+    }
+  } else {
+    r.s = *reinterpret_cast<const uint4 *>(tile + (uint32_t) (g * 144));
+    r.q = *reinterpret_cast<const uint2 *>(tile + (uint32_t) (g * 144 + 8 * i) + 16);
+  }
+}
+
+__device__ __forceinline__ v2h as_v2h(uint32_t x) {
+  return __builtin_bit_cast(v2h, x);
+}
+// (a | b) of the masks below turns bytes into fp16 numbers 1024 + byte: 0x64xx
+__device__ __forceinline__ v2h biased_to_half(uint32_t x, _Float16 bias) {
+  return as_v2h(x) - (v2h){ bias, bias };  // exact: integers below 2048
+}
+
+// IQ4_NL code book (reference: src/dsp/ops/mat_mul.c:29-32), every value + 128: the four nibbles in the low halves of
+// x's bytes -> four bytes
+__device__ __forceinline__ uint32_t iq4_nl_bytes(uint32_t x) {
+  const uint32_t low3 = x & 0x07070707u;
+  const uint32_t a    = __builtin_amdgcn_perm(0x766a5d4fu, 0x3f2d1801u, low3);  // values 0 .. 7
+  const uint32_t b    = __builtin_amdgcn_perm(0xf1d9c5b5u, 0xa6998d81u, low3);  // values 8 .. 15
+  return __builtin_amdgcn_perm(b, a, 0x03020100u + ((x & 0x08080808u) >> 1));
+}
+
+// The B operand of column 2 i + J: K rows 8 g + 2 v, + 1 in dword v. Each weight is fp16(quant) * fp16(scale) rounded
+// once, as the reference's dequantizers make it (mat_mul.c:308-508). `sc` holds the four scales of the lane's columns,
+// each in both halves of a dword.
+struct VectorConstants {
+  uint32_t exponents = 0x64006400u;  // (in a vector register, so that masking and merging are one instruction)
+};
+template <int KIND, int J>
+__device__ __forceinline__ v8h dequant(const RawStep<KIND> &r, const v2h (&sc)[4], const VectorConstants &c) {
+  v2h h[4];
+  if constexpr (KIND == 1) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      h[v] = as_v2h(J ? r.q[v].y : r.q[v].x);
+    }
+  } else if constexpr (KIND == 2) {
+    // byte b holds row pair b & 1 (low nibble) and 2 + (b & 1) (high nibble), row b / 2 of the pair
+    const uint32_t q = J ? r.q.y : r.q.x;
+    const uint32_t q8 = q >> 8;
+    // low nibbles give 1024 + n, high ones 1024 + 16 n, which a fused multiply-add turns into n - 8 exactly as well
+    const v2h lo_bias = { (_Float16) 1032.0f, (_Float16) 1032.0f }, sixteenth = { (_Float16) 0.0625f, (_Float16) 0.0625f },
+              hi_bias = { (_Float16) -72.0f, (_Float16) -72.0f };
+    h[0] = (as_v2h((q & 0x000f000fu) | c.exponents) - lo_bias) * sc[0];
+    h[1] = (as_v2h((q8 & 0x000f000fu) | c.exponents) - lo_bias) * sc[1];
+    h[2] = __builtin_elementwise_fma(as_v2h((q & 0x00f000f0u) | c.exponents), sixteenth, hi_bias) * sc[2];
+    h[3] = __builtin_elementwise_fma(as_v2h((q8 & 0x00f000f0u) | c.exponents), sixteenth, hi_bias) * sc[3];
+  } else if constexpr (KIND == 4) {
+    const uint32_t q  = J ? r.q.y : r.q.x;
+    const uint32_t lo = iq4_nl_bytes(q), hi = iq4_nl_bytes(q >> 4);  // (the masks inside drop the other nibbles)
+    h[0] = biased_to_half(__builtin_amdgcn_perm(0x64646464u, lo, 0x04020400u), (_Float16) 1152.0f) * sc[0];
+    h[1] = biased_to_half(__builtin_amdgcn_perm(0x64646464u, lo, 0x04030401u), (_Float16) 1152.0f) * sc[1];
+    h[2] = biased_to_half(__builtin_amdgcn_perm(0x64646464u, hi, 0x04020400u), (_Float16) 1152.0f) * sc[2];
+    h[3] = biased_to_half(__builtin_amdgcn_perm(0x64646464u, hi, 0x04030401u), (_Float16) 1152.0f) * sc[3];
+  } else {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const uint32_t u = r.q[v] ^ 0x80808080u;
+      h[v] = biased_to_half(__builtin_amdgcn_perm(0x64646464u, u, J ? 0x04030402u : 0x04010400u), (_Float16) 1152.0f) * sc[v];
+    }
+  }
+  return __builtin_shufflevector(__builtin_shufflevector(h[0], h[1], 0, 1, 2, 3), __builtin_shufflevector(h[2], h[3], 0, 1, 2, 3),
+                                 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
+// MT row tiles of 16; NT column groups of 32 per workgroup (sharing the activations); ACT_LDS: the activations are
+// converted into LDS by every workgroup
+template <int KIND, int MT, int NT, bool ACT_LDS>
+__global__ __launch_bounds__(kRowsThreads) void permuted_rows_kernel(const RowsArgs args) {
+  extern __shared__ __align__(16) uint8_t rows_lds[];  // activations [m][k + 8] halfs, then the waves' sums
+  int idx = 0;
+  while (idx + 1 < args.count && (int) blockIdx.x >= args.member[idx + 1].first) {
+    ++idx;
+  }
+  const RowsMember &mb  = args.member[idx];
+  const int   m = args.m, k = mb.k, n = mb.n;
+  const int   lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int   g = lane >> 4, i = lane & 15;
+  const int   nt0 = ((int) blockIdx.x - mb.first) * NT, n_tiles = n / 32, k_tiles = k / 32;
+  constexpr int DEPTH = (KIND == 2 || KIND == 4 || NT == 2) ? 4 : 8;  // steps of a wave in flight
+  const uint8_t *w[NT];
+#pragma unroll
+  for (int c = 0; c < NT; ++c) {
+    w[c] = mb.weight + (size_t) min(nt0 + c, n_tiles - 1) * k_tiles * RawStep<KIND>::kTileBytes;
+  }
+
+  // the first rows' values are requested before the weights, so that waiting for them leaves the weights in flight
+  constexpr int kAhead = 6;
+  float4        pre[kAhead];
+  const int     quads = m * (k / 4);
+  if constexpr (ACT_LDS) {
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      pre[u] = reinterpret_cast<const float4 *>(mb.act)[min((int) threadIdx.x + u * kRowsThreads, quads - 1)];
+    }
+    asm volatile("" ::: "memory");
+  }
+  RawStep<KIND> raw[DEPTH][NT];
+  uint4         af[DEPTH][MT];
+  auto          load = [&](int d, int step) {
+    const int kt = min(wave + step * kRowsWaves, k_tiles - 1);  // (branch-free: steps past the end repeat the last tile)
+#pragma unroll
+    for (int c = 0; c < NT; ++c) {
+      load_step(raw[d][c], w[c] + (uint32_t) kt * (uint32_t) RawStep<KIND>::kTileBytes, g, i);
+    }
+    if constexpr (!ACT_LDS) {
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        af[d][t] = mb.frag[((size_t) t * k_tiles + kt) * kWave + lane];
+      }
+    }
+  };
+#pragma unroll
+  for (int d = 0; d < DEPTH; ++d) {
+    load(d, d);
+  }
+  const int pitch = k + 8;  // halfs
+  if constexpr (ACT_LDS) {
+    _Float16 *act = reinterpret_cast<_Float16 *>(rows_lds);
+    auto      put = [&](int q, const float4 &x) {
+      const int row = q / (k / 4), c = q - row * (k / 4);
+      *reinterpret_cast<v4h *>(act + (size_t) row * pitch + 4 * c) =
+        (v4h){ (_Float16) x.x, (_Float16) x.y, (_Float16) x.z, (_Float16) x.w };
+    };
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int q = (int) threadIdx.x + u * kRowsThreads;
+      if (q < quads) {
+        put(q, pre[u]);
+      }
+    }
+    for (int q = (int) threadIdx.x + kAhead * kRowsThreads; q < quads; q += kRowsThreads) {
+      put(q, reinterpret_cast<const float4 *>(mb.act)[q]);
+    }
+    // (not __syncthreads: its fence would wait for the weights as well)
+    asm volatile("s_waitcnt lgkmcnt(0)\n s_barrier" ::: "memory");
+  }
+
+  v4f acc[MT][NT][2];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+#pragma unroll
+    for (int c = 0; c < NT; ++c) {
+      acc[t][c][0] = acc[t][c][1] = (v4f){ 0.0f, 0.0f, 0.0f, 0.0f };
+    }
+  }
+  const uint32_t half_sel = (i >> 3) ? 0x03020302u : 0x01000100u;  // columns 16 .. 31 take the odd scales
+  const uint8_t *a_lds[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    // (rows past the last one repeat it: a result row depends on its own row only, and theirs are not stored)
+    a_lds[t] = rows_lds + ((size_t) min(16 * t + i, m - 1) * pitch + 8 * g) * 2;
+  }
+  VectorConstants vc;
+  asm("" : "+v"(vc.exponents));
+  auto use = [&](int d, int step) {
+    const int kt = wave + step * kRowsWaves;
+    if (kt < k_tiles) {
+      v8h a[MT];
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        if constexpr (ACT_LDS) {
+          a[t] = *reinterpret_cast<const v8h *>(a_lds[t] + (size_t) kt * 64);
+        } else {
+          a[t] = __builtin_bit_cast(v8h, af[d][t]);
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < NT; ++c) {
+        v2h sc[4];
+        if constexpr (KIND != 1) {
+          const uint4    s     = raw[d][c].s;
+          const uint32_t s4[4] = { s.x, s.y, s.z, s.w };
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            sc[v] = as_v2h(__builtin_amdgcn_perm(s4[v], s4[v], half_sel));
+          }
+        }
+        const v8h b0 = dequant<KIND, 0>(raw[d][c], sc, vc), b1 = dequant<KIND, 1>(raw[d][c], sc, vc);
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+          acc[t][c][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[t], b0, acc[t][c][0], 0, 0, 0);
+          acc[t][c][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[t], b1, acc[t][c][1], 0, 0, 0);
+        }
+      }
+    }
+  };
+  const int steps = (k_tiles + kRowsWaves - 1) / kRowsWaves;
+  int       s0    = 0;
+  for (; s0 + DEPTH < steps; s0 += DEPTH) {
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+      use(d, s0 + d);
+      load(d, s0 + d + DEPTH);
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < DEPTH; ++d) {
+    use(d, s0 + d);
+  }
+
+  // the waves' sums: D[4 g + r][i] of tile (t, c, j) is row 16 t + 4 g + r, column 2 i + j of column group c
+  __syncthreads();  // (everybody is done with the activations)
+  float    *red  = reinterpret_cast<float *>(rows_lds);  // [wave][row][32 NT]
+  const int rows = min(m, 16 * MT);
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = 16 * t + 4 * g + r;
+      if (row < rows) {
+#pragma unroll
+        for (int c = 0; c < NT; ++c) {
+          *reinterpret_cast<float2 *>(red + ((size_t) wave * rows + row) * (32 * NT) + 32 * c + 2 * i) =
+            make_float2(acc[t][c][0][r], acc[t][c][1][r]);
+        }
+      }
+    }
+  }
+  __syncthreads();
+  for (int o = threadIdx.x; o < rows * 32 * NT; o += kRowsThreads) {
+    float sum = 0.0f;
+#pragma unroll
+    for (int u = 0; u < kRowsWaves; ++u) {
+      sum += red[(size_t) u * rows * (32 * NT) + o];
+    }
+    const int col = nt0 * 32 + o % (32 * NT);
+    if (NT == 1 || col < n) {
+      mb.out[(size_t) (o / (32 * NT)) * n + col] = (float) (_Float16) sum;  // the reference stores fp16 results
+    }
+  }
+}
+
+// fp32 rows -> fp16 in A operand order: [row tile of 16][K step of 32][lane], lane (g, i) = row i, K 8 g .. 8 g + 7;
+// rows past the last one are zeros
+struct RowsActArgs {
+  const float *src[kPermutedGroupMax];
+  uint4       *dst[kPermutedGroupMax];
+  int          k[kPermutedGroupMax], first[kPermutedGroupMax];
+  int          count, m, tiles;
+};
+__global__ __launch_bounds__(256) void permuted_rows_act_kernel(const RowsActArgs args) {
+  int idx = 0;
+  while (idx + 1 < args.count && (int) blockIdx.x >= args.first[idx + 1]) {
+    ++idx;
+  }
+  const int k = args.k[idx], k_tiles = k / 32;
+  const int t = ((int) blockIdx.x - args.first[idx]) * 256 + (int) threadIdx.x;
+  const int lane = t & 63, f = t >> 6, step = f % k_tiles, tile = f / k_tiles;
+  if (tile >= args.tiles) {
+    return;
+  }
+  const int row = 16 * tile + (lane & 15);
+  uint4     o   = make_uint4(0, 0, 0, 0);
+  if (row < args.m) {
+    const float4 *s = reinterpret_cast<const float4 *>(args.src[idx] + (size_t) row * k + 32 * step + 8 * (lane >> 4));
+    const float4  a = s[0], b = s[1];
+    const v8h     h = { (_Float16) a.x, (_Float16) a.y, (_Float16) a.z, (_Float16) a.w,
+                        (_Float16) b.x, (_Float16) b.y, (_Float16) b.z, (_Float16) b.w };
+    o = __builtin_bit_cast(uint4, h);
+  }
+  args.dst[idx][t] = o;
+}
+
+bool act_in_lds(int m, int k) {
+  return (size_t) m * (k + 8) * 2 <= kRowsActLds;
+}
+
+template <int KIND>
+hipError_t launch_kind(hipStream_t stream, const RowsArgs &args, unsigned grid, size_t lds, bool act_lds, bool wide) {
+  void (*kernel)(RowsArgs) = nullptr;
+  if (args.m <= 16) {
+    kernel = act_lds ? permuted_rows_kernel<KIND, 1, 1, true> : permuted_rows_kernel<KIND, 1, 1, false>;
+  } else {
+    kernel = act_lds ? permuted_rows_kernel<KIND, 2, 1, true> : permuted_rows_kernel<KIND, 2, 1, false>;
+    if constexpr (KIND == 2 || KIND == 4) {
+      kernel = wide ? permuted_rows_kernel<KIND, 2, 2, false> : kernel;
+    }
+  }
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(kRowsThreads), lds, stream, args);
+  return hipGetLastError();
+}
+
+size_t act_bytes(int m, int k) {
+  return (size_t) ((m + 15) / 16) * 16 * (size_t) k * 2;
+}
+
+}  // namespace
+
+size_t permuted_rows_workspace_bytes(const PermutedMatMul *members, int count, int m) {
+  size_t bytes = 0;
+  for (int j = 0; j < count; ++j) {  // (members that read the same rows share a copy; counted once each, which is enough)
+    bytes += act_bytes(m, members[j].k);
+  }
+  return bytes;
+}
+
+hipError_t launch_permuted_rows_group(hipStream_t stream, const PermutedMatMul *members, int count, int m, int weight_kind,
+                                      void *workspace) {
+  if (count < 1 || count > kPermutedGroupMax || m < 1 || m > kPermutedRowsMax || weight_kind < 1 || weight_kind > 4) {
+    return hipErrorInvalidValue;
+  }
+  // the members with the longest columns first (a workgroup walks a column group's whole K), so that the launch does
+  // not end with them
+  int order[kPermutedGroupMax];
+  for (int j = 0; j < count; ++j) {
+    order[j] = j;
+  }
+  std::stable_sort(order, order + count, [&](int a, int b) { return members[a].k > members[b].k; });
+  bool act_lds = true;
+  int  k_max   = 0;
+  for (int j = 0; j < count; ++j) {
+    if (members[j].k % 32 != 0 || members[j].n % 32 != 0 || members[j].k <= 0 || members[j].n <= 0) {
+      return hipErrorInvalidValue;
+    }
+    act_lds = act_lds && act_in_lds(m, members[j].k);
+    k_max   = std::max(k_max, members[j].k);
+  }
+  // Activations in operand order come from L2, once per workgroup: with 17 .. 32 rows (2 KiB per step, against 576 B of
+  // 4-bit weights) and column groups enough, a workgroup takes two and halves that traffic (Llama-7B shapes, 32 rows of
+  // Q4_0: 48 -> 45 us). With up to 16 rows it changes nothing (39.0 against 38.4 us), and the wider formats lose
+  // (16 rows of fp16 tiles: 34.8 against 24.7 us).
+  int groups = 0;
+  for (int j = 0; j < count; ++j) {
+    groups += members[j].n / 32;
+  }
+  const bool wide = !act_lds && m > 16 && (weight_kind == 2 || weight_kind == 4) && groups >= kRowsWideTiles;
+  RowsArgs   args;
+  args.count = count, args.m = m;
+  unsigned     grid = 0;
+  RowsActArgs  conv;
+  unsigned     conv_grid = 0;
+  conv.count = 0, conv.m = m, conv.tiles = (m + 15) / 16;
+  uint8_t *ws = static_cast<uint8_t *>(workspace);
+  for (int j = 0; j < count; ++j) {
+    const PermutedMatMul &p = members[order[j]];
+    RowsMember           &a = args.member[j];
+    a.out = p.out, a.act = p.act, a.frag = nullptr, a.weight = static_cast<const uint8_t *>(p.weight), a.k = p.k, a.n = p.n;
+    a.first = (int) grid;
+    grid += (unsigned) (wide ? (p.n / 32 + 1) / 2 : p.n / 32);
+    if (!act_lds) {
+      int c = 0;
+      while (c < conv.count && !(conv.src[c] == p.act && conv.k[c] == p.k)) {
+        ++c;
+      }
+      if (c == conv.count) {
+        conv.src[c] = p.act, conv.k[c] = p.k, conv.dst[c] = reinterpret_cast<uint4 *>(ws), conv.first[c] = (int) conv_grid;
+        ws += act_bytes(m, p.k);
+        conv_grid += (unsigned) ((act_bytes(m, p.k) / 16 + 255) / 256);
+        ++conv.count;
+      }
+      a.frag = conv.dst[c];
+    }
+  }
+  if (!act_lds) {
+    hipLaunchKernelGGL(permuted_rows_act_kernel, dim3(conv_grid), dim3(256), 0, stream, conv);
+    if (hipError_t e = hipGetLastError(); e != hipSuccess) {
+      return e;
+    }
+  }
+  const size_t red = (size_t) kRowsWaves * m * 32 * (wide ? 2 : 1) * sizeof(float);
+  const size_t lds = std::max(red, act_lds ? (size_t) m * (k_max + 8) * 2 : 0);
+  switch (weight_kind) {
+    case 1:
+      return launch_kind<1>(stream, args, grid, lds, act_lds, wide);
+    case 2:
+      return launch_kind<2>(stream, args, grid, lds, act_lds, wide);
+    case 3:
+      return launch_kind<3>(stream, args, grid, lds, act_lds, wide);
+    default:
+      return launch_kind<4>(stream, args, grid, lds, act_lds, wide);
+  }
+}
+
+}  // namespace htpops

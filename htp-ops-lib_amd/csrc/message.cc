@@ -411,6 +411,62 @@ bool try_batch(htpops_context *ctx, const struct OpComputeRequest *req, struct R
   return true;
 }
 
+// The same for matmuls over the reference's own weight formats (ops 1-4): consecutive requests of one op and row count
+// that nothing orders run as one launch. They read fp32 rows and leave no state behind that other requests look at, so
+// they have a batch of their own; at most one of the two batches is open at a time.
+struct PermutedBatch {
+  int                   kind = 0, m = 0, count = 0;
+  struct RequestHeader *hdr[kPermutedGroupMax];
+  PermutedMatMul        member[kPermutedGroupMax];
+};
+
+void flush_permuted(htpops_context *ctx, PermutedBatch &b) {
+  if (b.count == 0) {
+    return;
+  }
+  ++ctx->message_submissions;
+  const int ret = op_mat_mul_permuted_group(ctx, b.member, b.count, b.m, b.kind);
+  for (int i = 0; i < b.count; ++i) {
+    b.hdr[i]->state = ret;
+  }
+  b.count = 0;
+}
+
+// true: the request is now part of the batch (its state is set when the batch runs); false: run it the ordinary way
+bool try_batch_permuted(htpops_context *ctx, const struct OpComputeRequest *req, struct RequestHeader *hdr, PermutedBatch &b) {
+  if (!ctx->has_device || req->op < HTP_OPS_MAT_MUL_PERMUTED_W16A32 || req->op > HTP_OPS_MAT_MUL_PERMUTED_W4D16A32_IQ4_NL) {
+    return false;
+  }
+  const auto *p    = reinterpret_cast<const MatMulParams *>(req->payload);
+  const int   kind = (int) req->op;
+  size_t      out_bytes, act_bytes;
+  if (p->m <= 0 || p->k <= 0 || p->n <= 0 || p->k % 32 != 0 || p->n % 32 != 0 ||
+      !mul3((size_t) p->m, (size_t) p->n, 4, &out_bytes) || !mul3((size_t) p->m, (size_t) p->k, 4, &act_bytes)) {
+    return false;
+  }
+  const size_t   w_bytes = permuted_weight_bytes((size_t) p->n, (size_t) p->k, kind);
+  PermutedMatMul one     = { (float *) resolve(ctx, p->output, out_bytes), (const float *) resolve(ctx, p->activation, act_bytes),
+                             resolve(ctx, p->weight, w_bytes), p->k, p->n };
+  if (!one.out || !one.act || !one.weight || !aligned(one.out, 128) || !aligned(one.act, 128) || !aligned(one.weight, 128) ||
+      ranges_overlap(one.out, out_bytes, one.act, act_bytes) || ranges_overlap(one.out, out_bytes, one.weight, w_bytes)) {
+    return false;  // the ordinary path reports what is wrong, or handles the aliasing in order
+  }
+  bool join = b.count > 0 && b.count < kPermutedGroupMax && b.kind == kind && b.m == p->m;
+  for (int i = 0; join && i < b.count; ++i) {
+    const PermutedMatMul &o = b.member[i];
+    const size_t oo = (size_t) b.m * o.n * 4, oa = (size_t) b.m * o.k * 4, ow = permuted_weight_bytes((size_t) o.n, (size_t) o.k, kind);
+    join = !ranges_overlap(one.out, out_bytes, o.out, oo) && !ranges_overlap(one.out, out_bytes, o.act, oa) &&
+           !ranges_overlap(one.out, out_bytes, o.weight, ow) && !ranges_overlap(o.out, oo, one.act, act_bytes) &&
+           !ranges_overlap(o.out, oo, one.weight, w_bytes);
+  }
+  if (!join) {
+    flush_permuted(ctx, b);
+    b.kind = kind, b.m = p->m;
+  }
+  b.hdr[b.count] = hdr, b.member[b.count++] = one;
+  return true;
+}
+
 // `next` behind a one-token fp32 attention request `req`: if it is the Q8_0 quantization of exactly that attention's
 // output row into a buffer that overlaps none of the attention's operands, notes where it wants the row
 // (ctx->attn_q8_out) and returns it; nullptr otherwise.
@@ -510,7 +566,8 @@ int enqueue_message(htpops_context *ctx, struct MessageHeader *msg, size_t msg_b
     return r;
   }
   const int n_reqs = msg->n_reqs;
-  GemvBatch batch;
+  GemvBatch     batch;
+  PermutedBatch permuted;
   ctx->act_fragments.src   = nullptr;
   ctx->in_message          = true;
   ctx->message_submissions = 0;
@@ -522,15 +579,24 @@ int enqueue_message(htpops_context *ctx, struct MessageHeader *msg, size_t msg_b
       case REQUEST_TYPE_OP_COMPUTE:
         if (size < sizeof(struct RequestHeader) + sizeof(struct OpComputeRequest)) {
           flush_batch(ctx, batch);
+          flush_permuted(ctx, permuted);
           hdr->state = HTPOPS_ERR_REJECTED;
         } else {
           const auto *req = reinterpret_cast<const struct OpComputeRequest *>(hdr->data);
           if (size < sizeof(struct RequestHeader) + sizeof(struct OpComputeRequest) + op_payload_bytes(req->op)) {
             flush_batch(ctx, batch);
+            flush_permuted(ctx, permuted);
             hdr->state = fail(ctx, HTPOPS_ERR_REJECTED, "message: request %d is shorter than the parameters of op %u", i,
                               req->op);
             break;
           }
+          if (req->op >= HTP_OPS_MAT_MUL_PERMUTED_W16A32 && req->op <= HTP_OPS_MAT_MUL_PERMUTED_W4D16A32_IQ4_NL) {
+            flush_batch(ctx, batch);
+            if (try_batch_permuted(ctx, req, hdr, permuted)) {
+              break;
+            }
+          }
+          flush_permuted(ctx, permuted);
           const bool  matmul_payload =
             size >= sizeof(struct RequestHeader) + sizeof(struct OpComputeRequest) + sizeof(MatMulParams);
           const bool  norm_payload =
@@ -566,6 +632,7 @@ int enqueue_message(htpops_context *ctx, struct MessageHeader *msg, size_t msg_b
       case REQUEST_TYPE_RPCMEM_MAP:
         {
           flush_batch(ctx, batch);
+          flush_permuted(ctx, permuted);
           // reference: commu.c:102-110 -- only the puts are acted on
           const auto *map = reinterpret_cast<const struct RpcmemMapRequest *>(hdr->data);
           int         ret = 0;
@@ -585,6 +652,7 @@ int enqueue_message(htpops_context *ctx, struct MessageHeader *msg, size_t msg_b
     }
   }
   flush_batch(ctx, batch);
+  flush_permuted(ctx, permuted);
   ctx->in_message        = false;
   ctx->act_fragments.src = nullptr;
   return HTPOPS_OK;

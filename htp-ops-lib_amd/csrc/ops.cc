@@ -318,6 +318,37 @@ int op_mat_mul_f32(htpops_context *ctx, float *dst, const float *act, const void
   return run_mat_mul(ctx, plan, dst, ws, weight, m, k, n, weight_type, ws + q_bytes);
 }
 
+namespace {
+
+// decode-sized row counts: the weights are streamed in their own format, which is a fraction of the bytes of a converted
+// copy (and costs a host with caller-registered weights no conversion per call)
+int run_permuted_rows(htpops_context *ctx, const PermutedMatMul *members, int count, int m, int kind) {
+  if (int r = ensure_workspace(ctx, permuted_rows_workspace_bytes(members, count, m))) {
+    return r;
+  }
+  HTPOPS_HIP(ctx, launch_permuted_rows_group(ctx->stream, members, count, m, kind, ctx->workspace));
+  return HTPOPS_OK;
+}
+
+}  // namespace
+
+int op_mat_mul_permuted_group(htpops_context *ctx, const PermutedMatMul *members, int count, int m, int kind) {
+  if (count > 1 && m <= kPermutedRowsMax) {
+    for (int i = 0; i < count; ++i) {
+      note_device_write(ctx, members[i].out, (size_t) m * members[i].n * 4);
+    }
+    return run_permuted_rows(ctx, members, count, m, kind);
+  }
+  int ret = HTPOPS_OK;
+  for (int i = 0; i < count; ++i) {
+    const PermutedMatMul &p = members[i];
+    if (int r = op_mat_mul_permuted(ctx, p.out, p.act, p.weight, m, p.k, p.n, kind)) {
+      ret = r;
+    }
+  }
+  return ret;
+}
+
 // hmx_mat_mul_permuted_w16a32 / hmx_mat_mul_permuted_qk_0_d16a32 (reference: src/dsp/ops/mat_mul.c:758-855, :875-1153)
 int op_mat_mul_permuted(htpops_context *ctx, float *dst, const float *act, const void *weight, int m, int k, int n,
                         int kind) {
@@ -335,6 +366,10 @@ int op_mat_mul_permuted(htpops_context *ctx, float *dst, const float *act, const
     return r;
   }
   note_device_write(ctx, dst, (size_t) m * n * 4);
+  if (m <= kPermutedRowsMax) {
+    const PermutedMatMul one = { dst, act, weight, k, n };
+    return run_permuted_rows(ctx, &one, 1, m, kind);
+  }
   const void *frag = find_copy(ctx, weight, kind, k, n);
   // Converted copies are kept only for weights in buffers the context allocated (their contents change only through
   // htpops_buffer_write or as an op's output, both of which drop the copy). Caller-registered memory may be rewritten

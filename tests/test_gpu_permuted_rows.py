@@ -1,0 +1,65 @@
+"""GPU parity of the few-row matmuls over the reference's own weight formats (ops 1-4 with up to 32 rows, the weights read
+as they lie): sizes at the edges of its tiles, and grouping inside a message."""
+import numpy as np
+import pytest
+
+from pyhtpops import api
+from pyhtpops import workloads as wl
+from test_gpu_parity_permuted import OPS, check, make_weights
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = api.Context(device=0)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("kind", [1, 2, 3, 4])
+@pytest.mark.parametrize("m,k,n", [
+    (1, 32, 32), (2, 256, 32),       # one tile; one tile per wave
+    (1, 32 * 33, 96), (3, 32 * 65, 64),  # a step of one wave only, behind 4 and 8 whole ones
+    (16, 2016, 64), (17, 96, 32),    # the last single row tile, activations at the edge of LDS; the first double one
+    (16, 2080, 64), (32, 1056, 160), # activations in operand order, one and two row tiles
+    (1, 12320, 32), (5, 6560, 32),   # long rows: more activations than are requested ahead; just past LDS
+])
+def test_few_rows_at_the_edges(ctx, oracle, kind, m, k, n):
+    # the tolerance is `check`'s: fp32 accumulation plus one fp16 spacing
+    check(ctx, oracle, kind, m, k, n, m * 7 + k + n)
+
+
+@pytest.mark.parametrize("kind", [2, 4])
+def test_two_column_groups_per_workgroup(ctx, oracle, kind):
+    # 17 .. 32 rows, activations past LDS, at least 512 column groups of 32 (an odd number: the last workgroup has one)
+    check(ctx, oracle, kind, 19, 1760, 513 * 32, 3)
+
+
+@pytest.mark.parametrize("kind,m", [(1, 1), (2, 1), (3, 7), (4, 32), (2, 40)])
+def test_grouped_requests_equal_their_own_launches(ctx, kind, m):
+    # Requests of a message that nothing orders share a launch; the last two depend on earlier ones (one reads an output,
+    # one overwrites an output). Every output must hold, byte for byte, what one message per request gives.
+    rng = wl.rng_for(87, kind * 100 + m)
+    shapes = [(128, 96), (64, 256), (96, 96), (128, 1056)]  # (n, k)
+    acts = {k: ctx.upload(wl.make_activations(rng, m, k)) for k in (96, 256, 1056)}
+    ws = [ctx.upload(np.ascontiguousarray(make_weights(rng, n, k, kind)[0]).view(np.uint8)) for n, k in shapes]
+    w_last = ctx.upload(np.ascontiguousarray(make_weights(rng, 64, 96, kind)[0]).view(np.uint8))
+    results = []
+    for grouped in (True, False):
+        outs = [ctx.upload(np.zeros(m * n, np.float32)) for n, _ in shapes] + [ctx.upload(np.zeros(m * 64, np.float32))]
+        reqs = [api.mat_mul_params((outs[j], 0), (acts[k], 0), (ws[j], 0), m, k, n) for j, (n, k) in enumerate(shapes)]
+        reqs.append(api.mat_mul_params((outs[4], 0), (outs[2], 0), (w_last, 0), m, 96, 64))     # reads output 2
+        reqs.append(api.mat_mul_params((outs[1], 0), (acts[96], 0), (w_last, 0), m, 96, 64))    # overwrites output 1
+        reqs = [(api.REQUEST_TYPE_OP_COMPUTE, api.op_compute_request(OPS[kind], r)) for r in reqs]
+        for msg in ([api.build_message(reqs)] if grouped else [api.build_message([r]) for r in reqs]):
+            assert ctx.process_message(msg) == 0 and not any(api.message_request_states(msg)), ctx.last_error()
+        if grouped:
+            assert ctx.last_message_submissions() == 2
+        results.append([ctx.read(h, np.uint8, ctx.size(h)) for h in outs])
+        for h in outs:
+            ctx.release(h)
+    for a, b in zip(*results):
+        assert np.array_equal(a, b) and a.any()
+    for h in list(acts.values()) + ws + [w_last]:
+        ctx.release(h)
