@@ -161,6 +161,10 @@ extern "C" int htpops_init_backend(htpops_context **out_ctx, int device) {
       delete ctx;
       return HTPOPS_ERR_HIP;
     }
+    if (hipMalloc(&ctx->attn_shares, kAttnSharesBytes) != hipSuccess) {
+      (void) hipGetLastError();
+      ctx->attn_shares = nullptr;
+    }
     ctx->device     = device;
     ctx->has_device = true;
   }
@@ -199,6 +203,9 @@ extern "C" int htpops_close(htpops_context *ctx) {
   if (ctx->has_device) {
     if (ctx->tickets) {
       (void) hipFree(ctx->tickets);
+    }
+    if (ctx->attn_shares) {
+      (void) hipFree(ctx->attn_shares);
     }
     for (const auto &e : ctx->frag_cache) {
       (void) hipFree(e.frag);

@@ -6,8 +6,8 @@
 // [kv_len][n_kv_heads][D]; the optional fp16 mask [qo_len][align_up(kv_len, 64)] is ADDED to the scaled scores (the
 // scalar routine's convention, reference :1505-1512); `causal` hides key j from query i when j > i + kv_len - qo_len.
 //
-// Three kernels:
-//  * prefill (any qo_len, head_dim 64 or 128): one workgroup = 32 query rows x up to 4 query heads of one KV head (one
+// The kernels:
+//  * prefill (several query rows, head_dim 64 or 128): one workgroup = 32 query rows x up to 4 query heads of one KV head (one
 //    wave per head, so a K/V tile staged in LDS serves the whole GQA group). Scores are computed transposed,
 //    S^T = K Q^T with v_mfma_f32_32x32x16_f16, which puts one query per lane: row max / row sum are register
 //    reductions plus one exchange between the two lane halves. K and V blocks come into LDS as they lie in memory, by
@@ -23,7 +23,11 @@
 //  * decode (qo_len == 1, head_dim 64 or 128): bandwidth bound. The KV range is split across workgroups (n_kv_heads
 //    alone would leave the GPU idle); both products run on the matrix cores with the heads of the GQA group as one
 //    operand, and a second tiny kernel merges the per-split (max, sum, O) partials in one trip to memory.
-//  * any other even head_dim up to 256 (the reference's flash_attn_sp_hdim.c domain): a plain kernel without MFMA.
+//  * head dims that are other multiples of 16 up to 256 (the reference's flash_attn_sp_hdim.c domain): the prefill kernel
+//    with rows padded to a multiple of 32, for one query row too (its keys split over workgroups, like every grid that
+//    would leave CUs idle); the probabilities as fp16 pairs. 500 causal rows by mask, 16 / 4 heads of 96: 364 us in the
+//    plain kernel, 18.8 us here.
+//  * any other even head_dim up to 256: a plain kernel without MFMA.
 #include "device_utils.h"
 #include "kernels.h"
 
@@ -58,36 +62,52 @@ constexpr int kPfThreads = 256;  // threads of one key group: 4 waves, one per q
 constexpr int kBQ        = 32;  // query rows per wave tile
 constexpr int kBK        = 64;  // keys per KV block
 
-template <int D>
+// One key group's share of LDS. K and V tiles of a block of keys, two buffers each: the next block arrives by DMA while
+// one is used (the DMA chooses what each lane fetches, not where it lands: a lane lands 16 bytes behind its neighbour).
+// Head dims up to DP are kept in rows of DP halfs; a row's 16-byte pieces are arranged so that the 16-byte fragment
+// reads of 8 neighbouring K rows and the transposing reads of 4 neighbouring V rows fall into different banks: where
+// DP % 64 == 0 the pieces are exclusive-or'ed with low bits of the row number (K: key % 8; V: 2 (key % 4), which keeps
+// 32-byte pieces whole for the transposing reads), else K rows are one piece longer (an odd number of them) and V rows,
+// an odd multiple of 64 bytes, lie right as they are.
+template <int DP>
 struct PrefillSmem {
-  // K and V tiles of a block of keys, rows as they lie in memory ([key][D] halfs), two buffers each: the next block
-  // arrives by DMA while one is used. The 16-byte pieces of a row are stored exclusive-or'ed with low bits of the row
-  // number (the DMA chooses what each lane fetches, not where it lands): K rows with key % 8, so that the 16-byte
-  // fragment reads of 8 neighbouring keys fall into different banks; V rows with 2 (key % 4), which keeps 32-byte
-  // pieces whole for the transposing reads and puts the four rows of such a read into different banks.
-  uint8_t k[2][kBK * D * 2];
-  uint8_t v[2][kBK * D * 2];
+  static constexpr bool kXor     = DP % 64 == 0;
+  static constexpr int  kKPieces = kXor ? DP / 8 : DP / 8 + 1;  // 16-byte pieces of a K row, of a V row
+  static constexpr int  kVPieces = DP / 8;
+  uint8_t k[2][kBK * kKPieces * 16];
+  uint8_t v[2][kBK * kVPieces * 16];
+  // each wave's mask values of the next block ([query][64 keys] halfs, the pieces of a row exclusive-or'ed with query % 8)
+  uint8_t mask[kPfThreads / kWave][kBQ * kBK * 2];
 };
 
-// GROUPS = 1 or 2 key groups per workgroup (4 waves each); with 2 they take alternate KV blocks of the same queries
-template <int D, bool QO_F32, int GROUPS>
-__global__ __launch_bounds__(kPfThreads *GROUPS, 2) void flash_attn_prefill_kernel(void *__restrict__ o_ptr,
-                                                                        const void *__restrict__ q_ptr,
-                                                                        const _Float16 *__restrict__ k_ptr,
-                                                                        const _Float16 *__restrict__ v_ptr,
-                                                                        const _Float16 *__restrict__ mask, int qo_len,
-                                                                        int kv_len, int n_heads, int n_kv_heads,
-                                                                        int flags) {
+// Floats of one 32-query tile of one head in the split-KV partials, for `units` = 4 * 32-column tiles of O^T: the
+// (max, sum) pair of each lane, then unit for unit the lanes' four values.
+__host__ __device__ constexpr size_t prefill_partial_floats(int units) {
+  return (size_t) units * 4 * kWave + 2 * kWave;
+}
+
+// FULL: head_dim == DP (64 or 128); else head_dim is any multiple of 16 in (DP - 32, DP], and the probabilities keep
+// 22 bits (an fp16 pair, two matrix instructions per fragment of V): the plain kernel that these head dims took before
+// held them in fp32. GROUPS = 1 or 2 key groups per workgroup (4 waves each); with 2 they take alternate KV blocks of the
+// same queries. With gridDim.z > 1 the blocks of a workgroup's queries are dealt to gridDim.z workgroups, each of which
+// leaves its (max, sum, O) in `part` for flash_attn_prefill_merge_kernel.
+template <int DP, bool FULL, bool QO_F32, int GROUPS>
+__global__ __launch_bounds__(kPfThreads *GROUPS, DP <= 128 ? 2 : 1) void flash_attn_prefill_kernel(
+  void *__restrict__ o_ptr, const void *__restrict__ q_ptr, const _Float16 *__restrict__ k_ptr,
+  const _Float16 *__restrict__ v_ptr, const _Float16 *__restrict__ mask, int qo_len, int kv_len, int n_heads,
+  int n_kv_heads, int head_dim, int flags, float *__restrict__ part) {
+  using Smem = PrefillSmem<DP>;
   const bool causal = (flags & 1) != 0, mask_threshold = (flags & 2) != 0;
-  __shared__ __align__(1024) PrefillSmem<D> sm_all[GROUPS];
-  constexpr int KSTEPS = D / 16;  // MFMA k-steps over the head dimension
-  constexpr int DT     = D / 32;  // 32-row tiles of O^T
+  __shared__ __align__(1024) Smem sm_all[GROUPS];
+  constexpr int KSTEPS = DP / 16;  // MFMA k-steps over the head dimension
+  constexpr int DT     = DP / 32;  // 32-row tiles of O^T
+  const int     D      = FULL ? DP : head_dim;
   // With GROUPS = 2, two groups of 4 waves work on the same queries and heads: group g takes KV blocks g, g + 2, ...
   // with its own K/V tiles in LDS and its own running (max, sum, O); the two states are merged through LDS at the
   // end. The longest workgroup then walks half as many iterations, which pays when the grid is too small to keep two
   // independent workgroups on every CU busy to the end (few query blocks, or the uneven lengths under `causal`).
-  const int           grp = __builtin_amdgcn_readfirstlane((int) threadIdx.x / kPfThreads);  // (the same for a wave)
-  PrefillSmem<D>     &sm  = sm_all[grp];
+  const int grp = __builtin_amdgcn_readfirstlane((int) threadIdx.x / kPfThreads);  // (the same for a wave)
+  Smem     &sm  = sm_all[grp];
 
   const int group = n_heads / n_kv_heads;
   const int gc    = group < 4 ? group : 4;  // heads handled by one workgroup
@@ -96,7 +116,7 @@ __global__ __launch_bounds__(kPfThreads *GROUPS, 2) void flash_attn_prefill_kern
 
   const int tid  = threadIdx.x % kPfThreads;  // within the key group
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5;
   const int col  = lane & 31;
 
@@ -107,9 +127,10 @@ __global__ __launch_bounds__(kPfThreads *GROUPS, 2) void flash_attn_prefill_kern
   const int q_block  = (int) (gridDim.y - 1 - blockIdx.y);
   const int h_kv     = blockIdx.x / sub_groups;
   const int h_in_grp = (blockIdx.x % sub_groups) * gc + wave % gc;
-  const bool wave_on = h_in_grp < group && wave / gc < qsub;
   const int  head    = h_kv * group + (h_in_grp < group ? h_in_grp : 0);
   const int  q_base  = (q_block * qsub + (wave / gc < qsub ? wave / gc : 0)) * kBQ;
+  // waves without a head or without a query only help to bring the tiles
+  const bool wave_on = h_in_grp < group && wave / gc < qsub && q_base < qo_len;
   const int  q_row   = q_base + col;                  // this lane's query
   const bool q_ok    = wave_on && q_row < qo_len;
   const int  q_clamp = q_row < qo_len ? q_row : qo_len - 1;
@@ -126,6 +147,10 @@ __global__ __launch_bounds__(kPfThreads *GROUPS, 2) void flash_attn_prefill_kern
 #pragma unroll
     for (int s = 0; s < KSTEPS; ++s) {
       const int d0 = 16 * s + 8 * half;
+      if (!FULL && s == KSTEPS - 1 && 16 * s >= D) {  // (this step is left out below)
+        qf[s] = (v8h){ 0, 0, 0, 0, 0, 0, 0, 0 };
+        continue;
+      }
       if (QO_F32) {
         const float4 *p  = reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(q_ptr) + base + d0);
         const float4  a  = p[0], b = p[1];
@@ -156,120 +181,177 @@ __global__ __launch_bounds__(kPfThreads *GROUPS, 2) void flash_attn_prefill_kern
 
   // keys visible to the LAST query row of the workgroup bound the KV loop under `causal`
   const int q_hi     = min(qo_len, (q_block + 1) * qsub * kBQ) - 1;
-  const int kv_limit = causal ? min(kv_len, q_hi + (kv_len - qo_len) + 1) : kv_len;
+  const int kv_limit = causal ? max(0, min(kv_len, q_hi + (kv_len - qo_len) + 1)) : kv_len;
   const int q_shift  = kv_len - qo_len;
   // last key this lane's query may see, relative to the first key this lane holds in a block (key0 = 4 * half)
   const int vis_last = (causal ? min(kv_len - 1, q_row + q_shift) : kv_len - 1) - 4 * half;
+  // this workgroup's share of the blocks
+  const int per  = ((kv_limit + kBK - 1) / kBK + (int) gridDim.z - 1) / (int) gridDim.z * kBK;
+  const int k_lo = (int) blockIdx.z * per, k_hi = min(kv_limit, k_lo + per);
 
   // The next K/V block travels global memory -> LDS by DMA (global_load_lds, 1 KiB per instruction: no registers, no
-  // stores) while the current one is being used. A tile is TILE_B / 1024 instructions, the four waves take every
-  // fourth; lane L of an instruction lands at byte 16 L of its KiB = row L / CHUNKS, piece L % CHUNKS, and fetches the
-  // piece that belongs there. Per lane the source offsets inside a block never change (kept in registers); what
-  // changes per block is a base address the same for all lanes.
-  constexpr int ROWB     = D * 2;          // bytes of a K or V row
-  constexpr int CHUNKS   = ROWB / 16;      // 16-byte pieces of a row
-  constexpr int DMA_ROWS = 1024 / ROWB;    // rows per DMA instruction
-  constexpr int TILE_B   = kBK * ROWB;
-  constexpr int NDMA     = TILE_B / 1024 / 4;  // instructions per wave and tile
-  const int     wave_u   = __builtin_amdgcn_readfirstlane(wave);
-  uint32_t      src_off[2][NDMA];  // [K, V]: byte offset of this lane's piece from the block's first row of this KV head
+  // stores) while the current one is being used. A tile of 64 rows is as many instructions as a row has pieces, the four
+  // waves take every fourth; lane L of instruction i lands at piece 64 i + L of the tile and fetches what belongs there
+  // (a row's last piece again where that lies behind the head dim). Per lane the source offsets inside a block never
+  // change (kept in registers); what changes per block is a base address the same for all lanes.
+  constexpr int KP = Smem::kKPieces, VP = Smem::kVPieces;
+  constexpr int KROWB = KP * 16, VROWB = VP * 16;          // bytes of a row in LDS
+  constexpr int KDMA = (KP + 3) / 4, VDMA = (VP + 3) / 4;  // instructions per wave and tile, at most
+  auto k_piece = [&](int j, int &row) {
+    const int p = (wave + 4 * j) * kWave + lane;
+    row = p / KP;
+    return min((p % KP) ^ (Smem::kXor ? row & 7 : 0), D / 8 - 1);
+  };
+  auto v_piece = [&](int j, int &row) {
+    const int p = (wave + 4 * j) * kWave + lane;
+    row = p / VP;
+    return min((p % VP) ^ (Smem::kXor ? 2 * (row & 3) : 0), D / 8 - 1);
+  };
+  uint32_t k_src[KDMA], v_src[VDMA];  // byte offset of this lane's piece from the block's first row of this KV head
 #pragma unroll
-  for (int j = 0; j < NDMA; ++j) {
-    const int row = (wave_u + 4 * j) * DMA_ROWS + lane / CHUNKS, piece = lane % CHUNKS;
-    src_off[0][j] = (uint32_t) row * (uint32_t) (kv_stride * 2) + 16u * (uint32_t) (piece ^ (row & 7));
-    src_off[1][j] = (uint32_t) row * (uint32_t) (kv_stride * 2) + 16u * (uint32_t) (piece ^ (2 * (row & 3)));
+  for (int j = 0; j < KDMA; ++j) {
+    int       row;
+    const int piece = k_piece(j, row);
+    k_src[j] = (uint32_t) row * (uint32_t) (kv_stride * 2) + 16u * (uint32_t) piece;
+  }
+#pragma unroll
+  for (int j = 0; j < VDMA; ++j) {
+    int       row;
+    const int piece = v_piece(j, row);
+    v_src[j] = (uint32_t) row * (uint32_t) (kv_stride * 2) + 16u * (uint32_t) piece;
   }
   auto fetch = [&](int k0, int buf) {
     const uint32_t to_k = (uint32_t) (uintptr_t) sm.k[buf], to_v = (uint32_t) (uintptr_t) sm.v[buf];
-    const uint8_t *kb = reinterpret_cast<const uint8_t *>(k_ptr + (size_t) h_kv * D + (size_t) k0 * kv_stride);
-    const uint8_t *vb = reinterpret_cast<const uint8_t *>(v_ptr + (size_t) h_kv * D + (size_t) k0 * kv_stride);
     if (k0 + kBK <= kv_len) {
+      const uint8_t *kb = reinterpret_cast<const uint8_t *>(k_ptr + (size_t) h_kv * D + (size_t) k0 * kv_stride);
+      const uint8_t *vb = reinterpret_cast<const uint8_t *>(v_ptr + (size_t) h_kv * D + (size_t) k0 * kv_stride);
 #pragma unroll
-      for (int j = 0; j < NDMA; ++j) {
-        asm volatile("s_mov_b32 m0, %2\n s_nop 0\n global_load_lds_dwordx4 %0, %1" ::"v"(src_off[0][j]), "s"(kb),
-                     "s"(to_k + (uint32_t) ((wave_u + 4 * j) * 1024))
-                     : "memory");
+      for (int j = 0; j < KDMA; ++j) {
+        if (KP % 4 == 0 || wave + 4 * j < KP) {
+          asm volatile("s_mov_b32 m0, %2\n s_nop 0\n global_load_lds_dwordx4 %0, %1" ::"v"(k_src[j]), "s"(kb),
+                       "s"(to_k + (uint32_t) ((wave + 4 * j) * 1024))
+                       : "memory");
+        }
       }
 #pragma unroll
-      for (int j = 0; j < NDMA; ++j) {
-        asm volatile("s_mov_b32 m0, %2\n s_nop 0\n global_load_lds_dwordx4 %0, %1" ::"v"(src_off[1][j]), "s"(vb),
-                     "s"(to_v + (uint32_t) ((wave_u + 4 * j) * 1024))
-                     : "memory");
+      for (int j = 0; j < VDMA; ++j) {
+        if (VP % 4 == 0 || wave + 4 * j < VP) {
+          asm volatile("s_mov_b32 m0, %2\n s_nop 0\n global_load_lds_dwordx4 %0, %1" ::"v"(v_src[j]), "s"(vb),
+                       "s"(to_v + (uint32_t) ((wave + 4 * j) * 1024))
+                       : "memory");
+        }
       }
       return;
     }
     // last, partial block: rows past the end repeat the last key (their scores are hidden below)
 #pragma unroll
-    for (int j = 0; j < 2 * NDMA; ++j) {
-      const int  jj  = j % NDMA;
-      const bool isv = j >= NDMA;
-      const int  row = (wave_u + 4 * jj) * DMA_ROWS + lane / CHUNKS, piece = lane % CHUNKS;
-      const int  key = min(k0 + row, kv_len - 1);
-      const int  log = isv ? piece ^ (2 * (row & 3)) : piece ^ (row & 7);
-      const _Float16 *src = (isv ? v_ptr : k_ptr) + (size_t) key * kv_stride + (size_t) h_kv * D + 8 * log;
+    for (int j = 0; j < KDMA + VDMA; ++j) {
+      const bool isv = j >= KDMA;
+      const int  jj  = isv ? j - KDMA : j;
+      if (wave + 4 * jj >= (isv ? VP : KP)) {
+        continue;
+      }
+      int       row;
+      const int piece = isv ? v_piece(jj, row) : k_piece(jj, row);
+      const int key   = min(k0 + row, kv_len - 1);
+      const _Float16 *src = (isv ? v_ptr : k_ptr) + (size_t) key * kv_stride + (size_t) h_kv * D + 8 * piece;
       asm volatile("s_mov_b32 m0, %1\n s_nop 0\n global_load_lds_dwordx4 %0, off" ::"v"(src),
-                   "s"((isv ? to_v : to_k) + (uint32_t) ((wave_u + 4 * jj) * 1024))
+                   "s"((isv ? to_v : to_k) + (uint32_t) ((wave + 4 * jj) * 1024))
                    : "memory");
     }
   };
-  // additive mask values of this lane's 2 x 16 keys of a block: requested a block ahead, like the tiles
-  auto fetch_mask = [&](v4h (&m)[2][4], int k0) {
+  // The wave's mask values of a block travel the same way, each wave its own (no barrier needed): 32 rows of 128 bytes,
+  // 16 bytes a lane, or 4 bytes a lane where the mask is not 16-byte aligned. (Loads into registers, 8 bytes a lane from
+  // 32 rows at once, cost the address path 512 cycles per wave and block, as much as half the matrix instructions.)
+  const bool mask_wide = (reinterpret_cast<uintptr_t>(mask) & 15) == 0 && mask_ld < ((size_t) 1 << 25);  // (32-bit offsets)
+  const int  mask_rows = min(kBQ, qo_len - q_base);  // rows past the last query repeat it
+  uint32_t   mask_src[4];  // byte offset of this lane's piece of rows 8 i .. 8 i + 7
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
+  for (int i = 0; i < 4; ++i) {
+    const int row = 8 * i + (lane >> 3);
+    mask_src[i]   = (uint32_t) min(row, mask_rows - 1) * (uint32_t) (mask_ld * 2) + 16u * (uint32_t) ((lane & 7) ^ (row & 7));
+  }
+  auto fetch_mask = [&](int k0) {
+    const _Float16 *base = mask + (size_t) q_base * mask_ld + k0;
+    const uint32_t  to   = (uint32_t) (uintptr_t) sm.mask[wave];
+    if (mask_wide) {
 #pragma unroll
-      for (int rg = 0; rg < 4; ++rg) {
-        // four consecutive keys: one 8-byte load (rows are padded to a multiple of 64 keys)
-        m[kt][rg] = *reinterpret_cast<const v4h *>(mask + (size_t) q_clamp * mask_ld + k0 + 32 * kt + 8 * rg + 4 * half);
+      for (int i = 0; i < 4; ++i) {
+        asm volatile("s_mov_b32 m0, %2\n s_nop 0\n global_load_lds_dwordx4 %0, %1" ::"v"(mask_src[i]), "s"(base),
+                     "s"(to + (uint32_t) (i * 1024))
+                     : "memory");
+      }
+    } else {
+#pragma unroll 1
+      for (int i = 0; i < 16; ++i) {
+        const int       row = 2 * i + (lane >> 5), d = lane & 31;
+        const _Float16 *src = base + (size_t) min(row, mask_rows - 1) * mask_ld + 8 * ((d >> 2) ^ (row & 7)) + 2 * (d & 3);
+        asm volatile("s_mov_b32 m0, %1\n s_nop 0\n global_load_lds_dword %0, off" ::"v"(src), "s"(to + (uint32_t) (i * 256)) : "memory");
       }
     }
   };
   // where this lane's fragments lie in a tile (bytes): K row `col` (+ 32 per tile), piece 2 s + half; V: the lane
   // (16-lane group g = lane / 16, i = lane % 16 = 4 j + q) points at row 4 half + j (+ 16 u + 8 per read), the 8-byte
-  // piece q of columns 32 t + 16 (g & 1) .. + 15, and receives column 32 t + 16 (g & 1) + i of four rows
+  // piece q of columns 32 t + 16 (g & 1) .. + 15, and receives column 32 t + 16 (g & 1) + i of four rows (columns behind
+  // the head dim repeat its last 16 and are not stored)
   uint32_t k_at[KSTEPS], v_at[DT];
   {
 #pragma unroll
     for (int s = 0; s < KSTEPS; ++s) {
-      k_at[s] = (uint32_t) (col * ROWB + 16 * ((2 * s + half) ^ (col & 7)));
+      k_at[s] = (uint32_t) (col * KROWB + 16 * ((2 * s + half) ^ (Smem::kXor ? col & 7 : 0)));
     }
     const int g = lane >> 4, j = (lane >> 2) & 3, q = lane & 3;
 #pragma unroll
     for (int t = 0; t < DT; ++t) {
-      v_at[t] = (uint32_t) ((4 * half + j) * ROWB + 16 * ((4 * t + 2 * (g & 1) + (q >> 1)) ^ (2 * j)) + 8 * (q & 1));
+      const int c0 = FULL ? 32 * t + 16 * (g & 1) : min(32 * t + 16 * (g & 1), D - 16);
+      v_at[t] = (uint32_t) ((4 * half + j) * VROWB + 16 * ((c0 / 8 + (q >> 1)) ^ (Smem::kXor ? 2 * j : 0)) + 8 * (q & 1));
     }
   }
   typedef short v4s __attribute__((ext_vector_type(4)));
 
-  v4h mreg[2][4], mnext[2][4];
-  if (grp * kBK < kv_limit) {
-    fetch(grp * kBK, 0);
-    if (mask) {
-      fetch_mask(mnext, grp * kBK);
+  const bool use_mask = mask != nullptr && wave_on;
+  uint2      mreg[2][4];  // this lane's 2 x 16 mask values: keys 32 kt + 8 rg + 4 half + 0 .. 3
+  if (k_lo + grp * kBK < k_hi) {
+    fetch(k_lo + grp * kBK, 0);
+    if (use_mask) {
+      fetch_mask(k_lo + grp * kBK);
     }
   }
 
   int it = 0;
-  for (int kk = 0; kk < kv_limit; kk += GROUPS * kBK, ++it) {
+  for (int kk = k_lo; kk < k_hi; kk += GROUPS * kBK, ++it) {
     const int  k0   = kk + grp * kBK;  // this key group's block of the iteration
-    const bool live = k0 < kv_limit;   // (the last iteration may have a block for the first group only)
     const int  buf  = it & 1;
     // this wave's share of the block has landed; behind the barrier everybody's has, and nobody reads the other
     // buffer (the previous block) any more
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (mask) {
+    bool live = wave_on && k0 < k_hi;  // (the last iteration may have a block for the first group only)
+    bool plain = true;                 // no mask value of the wave's block is anything but zero
+    if (use_mask && k0 < k_hi) {
+      uint32_t all = 0xffffffffu, any = 0;
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt) {
 #pragma unroll
         for (int rg = 0; rg < 4; ++rg) {
-          mreg[kt][rg] = mnext[kt][rg];
+          mreg[kt][rg] = *reinterpret_cast<const uint2 *>(sm.mask[wave] + col * 128 + 16 * ((4 * kt + rg) ^ (col & 7)) + 8 * half);
+          all &= mreg[kt][rg].x & mreg[kt][rg].y;
+          any |= mreg[kt][rg].x | mreg[kt][rg].y;
         }
       }
+      // (the values are in registers before the next block's overwrite them)
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      plain = __builtin_amdgcn_ballot_w64((any & 0x7fff7fffu) != 0) == 0;
+      // A block that the mask hides from all 32 queries (-inf throughout; a causal mask hides half of a prompt's blocks)
+      // is passed over, as under `causal`.
+      if (__builtin_amdgcn_ballot_w64(!(all == 0xfc00fc00u && any == 0xfc00fc00u)) == 0) {
+        live = false;
+      }
     }
-    if (k0 + GROUPS * kBK < kv_limit) {
+    if (k0 + GROUPS * kBK < k_hi) {
       fetch(k0 + GROUPS * kBK, buf ^ 1);
-      if (mask) {
-        fetch_mask(mnext, k0 + GROUPS * kBK);
+      if (use_mask) {
+        fetch_mask(k0 + GROUPS * kBK);
       }
     }
     if (!live) {
@@ -299,7 +381,7 @@ __global__ __launch_bounds__(kPfThreads *GROUPS, 2) void flash_attn_prefill_kern
       for (int s = 0; s < PF && s < KSTEPS; ++s) {
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt) {
-          kf[s][kt] = *reinterpret_cast<const v8h *>(k_tile + k_at[s] + 32 * kt * ROWB);
+          kf[s][kt] = *reinterpret_cast<const v8h *>(k_tile + k_at[s] + 32 * kt * KROWB);
         }
       }
 #pragma unroll
@@ -307,8 +389,11 @@ __global__ __launch_bounds__(kPfThreads *GROUPS, 2) void flash_attn_prefill_kern
         if (s + PF < KSTEPS) {
 #pragma unroll
           for (int kt = 0; kt < 2; ++kt) {
-            kf[(s + PF) % (PF + 1)][kt] = *reinterpret_cast<const v8h *>(k_tile + k_at[s + PF] + 32 * kt * ROWB);
+            kf[(s + PF) % (PF + 1)][kt] = *reinterpret_cast<const v8h *>(k_tile + k_at[s + PF] + 32 * kt * KROWB);
           }
+        }
+        if (!FULL && s == KSTEPS - 1 && 16 * s >= D) {
+          continue;  // (behind the head dim, the same for all waves)
         }
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt) {
@@ -318,17 +403,17 @@ __global__ __launch_bounds__(kPfThreads *GROUPS, 2) void flash_attn_prefill_kern
     }
 
     // ---- mask (lane = query; register r of tile kt is key k0 + 32 kt + 8 (r / 4) + 4 half + r % 4) ----
-    // Only blocks that a mask, the causal diagonal or the end of the keys touches pay for it (the same for the
-    // whole wave).
-    if (mask != nullptr || k0 + kBK > kv_len || (causal && k0 + kBK - 1 > q_base + q_shift)) {
+    // Only blocks that mask values other than zero, the causal diagonal or the end of the keys touch pay for it (the same
+    // for the whole wave).
+    if (!plain || k0 + kBK > kv_len || (causal && k0 + kBK - 1 > q_base + q_shift)) {
       const int last = vis_last - k0;  // registers whose key offset 32 kt + 8 (r / 4) + r % 4 exceeds it are hidden
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt) {
 #pragma unroll
         for (int rg = 0; rg < 4; ++rg) {
           float add[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
-          if (mask) {
-            const v4h mv = mreg[kt][rg];
+          if (!plain) {
+            const v4h mv = __builtin_bit_cast(v4h, mreg[kt][rg]);
             add[0] = mask_term(mv[0], mask_threshold), add[1] = mask_term(mv[1], mask_threshold);
             add[2] = mask_term(mv[2], mask_threshold), add[3] = mask_term(mv[3], mask_threshold);
           }
@@ -380,9 +465,10 @@ __global__ __launch_bounds__(kPfThreads *GROUPS, 2) void flash_attn_prefill_kern
       l_run *= alpha;
       m_run = move ? m_ref + mx : m_run;
     }
-    // the probabilities, rounded to fp16 in pairs as the matrix instruction takes them; the row sum adds up the
-    // rounded values (v_dot2_f32_f16 with ones: two per instruction, fp32 sums), so O and l see the same numbers
-    uint32_t pk[2][8];
+    // the probabilities, rounded to fp16 in pairs as the matrix instruction takes them. FULL: the row sum adds up the
+    // rounded values (v_dot2_f32_f16 with ones: two per instruction, fp32 sums), so O and l see the same numbers; else
+    // what the rounding left out goes into a second fp16 pair and the row sum adds up the fp32 values.
+    uint32_t pk[2][8], pk_lo[FULL ? 1 : 2][FULL ? 1 : 8];
     float    psum[4] = { 0.0f, 0.0f, 0.0f, 0.0f };  // (four chains: an addition waits for the one before it in its chain)
     {
       const v2h ones = { (_Float16) 1.0f, (_Float16) 1.0f };
@@ -390,9 +476,16 @@ __global__ __launch_bounds__(kPfThreads *GROUPS, 2) void flash_attn_prefill_kern
       for (int kt = 0; kt < 2; ++kt) {
 #pragma unroll
         for (int r = 0; r < 16; r += 2) {
-          const v2h p2  = { (_Float16) fast_exp2(st[kt][r]), (_Float16) fast_exp2(st[kt][r + 1]) };
-          pk[kt][r / 2] = __builtin_bit_cast(uint32_t, p2);
-          psum[(r / 2) & 3] = __builtin_amdgcn_fdot2(p2, ones, psum[(r / 2) & 3], false);
+          const float p0 = fast_exp2(st[kt][r]), p1 = fast_exp2(st[kt][r + 1]);
+          const v2h   p2 = { (_Float16) p0, (_Float16) p1 };
+          pk[kt][r / 2]  = __builtin_bit_cast(uint32_t, p2);
+          if constexpr (FULL) {
+            psum[(r / 2) & 3] = __builtin_amdgcn_fdot2(p2, ones, psum[(r / 2) & 3], false);
+          } else {
+            const v2h lo      = { (_Float16) (p0 - (float) p2[0]), (_Float16) (p1 - (float) p2[1]) };
+            pk_lo[kt][r / 2]  = __builtin_bit_cast(uint32_t, lo);
+            psum[(r / 2) & 3] += p0 + p1;
+          }
         }
       }
     }
@@ -408,12 +501,17 @@ __global__ __launch_bounds__(kPfThreads *GROUPS, 2) void flash_attn_prefill_kern
 #pragma unroll
         for (int t = 0; t < DT; ++t) {
           // (V^T fragment: column 32 t + lane % 32 of keys 32 kt + 16 u + 4 half + 0 .. 3 and + 8 .. 11)
-          const uint8_t *at = v_tile + v_at[t] + (32 * kt + 16 * u) * ROWB;
+          const uint8_t *at = v_tile + v_at[t] + (32 * kt + 16 * u) * VROWB;
           const v4s a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((v4s __attribute__((address_space(3))) *) at);
-          const v4s a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((v4s __attribute__((address_space(3))) *) (at + 8 * ROWB));
+          const v4s a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((v4s __attribute__((address_space(3))) *) (at + 8 * VROWB));
           const v8h vf = __builtin_bit_cast(v8h, (short __attribute__((ext_vector_type(8)))){ a0[0], a0[1], a0[2], a0[3],
                                                                                              a1[0], a1[1], a1[2], a1[3] });
           oacc[t]      = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pf, oacc[t], 0, 0, 0);
+          if constexpr (!FULL) {
+            const v8h pl = __builtin_bit_cast(v8h, make_uint4(pk_lo[kt][4 * u], pk_lo[kt][4 * u + 1], pk_lo[kt][4 * u + 2],
+                                                              pk_lo[kt][4 * u + 3]));
+            oacc[t]      = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pl, oacc[t], 0, 0, 0);
+          }
         }
       }
     }
@@ -446,6 +544,7 @@ __global__ __launch_bounds__(kPfThreads *GROUPS, 2) void flash_attn_prefill_kern
     const float m_safe = (m_all == -INFINITY) ? 0.0f : m_all;  // nothing visible at all: keep the exponents finite
     const float a0 = fast_exp2(m_run - m_safe), a1 = fast_exp2(m1 - m_safe);
     l_tot          = a0 * l_tot + a1 * l1;
+    m_run          = m_all;
 #pragma unroll
     for (int t = 0; t < DT; ++t) {
 #pragma unroll
@@ -453,6 +552,25 @@ __global__ __launch_bounds__(kPfThreads *GROUPS, 2) void flash_attn_prefill_kern
         oacc[t][r] = a0 * oacc[t][r] + a1 * xch[(2 + 16 * t + r) * kWave];
       }
     }
+  }
+
+  // ---- a share of the keys only: leave (max, sum, O) as they are, lane for lane ----
+  if (gridDim.z > 1) {
+    if (wave_on) {
+      const size_t n_tiles = (size_t) ((qo_len + kBQ - 1) / kBQ) * n_heads;
+      const size_t tile    = (size_t) (q_base / kBQ) * n_heads + head;
+      float *rec = part + ((size_t) blockIdx.z * n_tiles + tile) * prefill_partial_floats(4 * DT);
+      reinterpret_cast<float2 *>(rec)[lane] = make_float2(m_run, l_tot);
+      float4 *out = reinterpret_cast<float4 *>(rec + 2 * kWave) + lane;
+#pragma unroll
+      for (int t = 0; t < DT; ++t) {
+#pragma unroll
+        for (int rg = 0; rg < 4; ++rg) {
+          out[(4 * t + rg) * kWave] = make_float4(oacc[t][4 * rg], oacc[t][4 * rg + 1], oacc[t][4 * rg + 2], oacc[t][4 * rg + 3]);
+        }
+      }
+    }
+    return;
   }
 
   // ---- finish: O = O^T / l, one query per lane; register r of tile t is d = 32 t + 8 (r / 4) + 4 half + r % 4 ----
@@ -464,6 +582,9 @@ __global__ __launch_bounds__(kPfThreads *GROUPS, 2) void flash_attn_prefill_kern
 #pragma unroll
       for (int rg = 0; rg < 4; ++rg) {
         const int d0 = 32 * t + 8 * rg + 4 * half;
+        if (!FULL && d0 >= D) {
+          continue;
+        }
         float     v[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -476,6 +597,69 @@ __global__ __launch_bounds__(kPfThreads *GROUPS, 2) void flash_attn_prefill_kern
           *reinterpret_cast<v4h *>(reinterpret_cast<_Float16 *>(o_ptr) + base + d0) = hv;
         }
       }
+    }
+  }
+}
+
+// Puts the shares of a split prefill together: a wave per 32-query tile, head and unit of four output columns per half
+// (`units` of them), lane for lane as the prefill kernel left them. All loads of kPfMergeChunk shares are requested
+// before the first use; chunks are folded into a running (max, sum, O) like KV blocks are.
+constexpr int kPfMergeChunk = 8;
+
+template <bool QO_F32>
+__global__ __launch_bounds__(256) void flash_attn_prefill_merge_kernel(void *__restrict__ o_ptr,
+                                                                       const float *__restrict__ part, int n_splits,
+                                                                       int n_tiles, int units, int qo_len, int n_heads,
+                                                                       int D) {
+  const int lane = threadIdx.x & 63;
+  const int id   = (int) blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6);
+  const int tile = id / units, unit = id % units;
+  if (tile >= n_tiles) {
+    return;
+  }
+  const size_t stride = (size_t) n_tiles * prefill_partial_floats(units);
+  const float *rec    = part + (size_t) tile * prefill_partial_floats(units);
+  float        m_run = -INFINITY, l_run = 0.0f;
+  float        v[4]  = { 0.0f, 0.0f, 0.0f, 0.0f };
+  for (int s0 = 0; s0 < n_splits; s0 += kPfMergeChunk) {
+    float2 ml[kPfMergeChunk];
+    float4 x[kPfMergeChunk];
+#pragma unroll
+    for (int u = 0; u < kPfMergeChunk; ++u) {
+      ml[u] = make_float2(-INFINITY, 0.0f);
+      x[u]  = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      if (s0 + u < n_splits) {
+        const float *at = rec + (size_t) (s0 + u) * stride;
+        ml[u] = reinterpret_cast<const float2 *>(at)[lane];
+        x[u]  = reinterpret_cast<const float4 *>(at + 2 * kWave)[(size_t) unit * kWave + lane];
+      }
+    }
+    float m_new = m_run;
+#pragma unroll
+    for (int u = 0; u < kPfMergeChunk; ++u) {
+      m_new = fmaxf(m_new, ml[u].x);
+    }
+    const float m_safe = (m_new == -INFINITY) ? 0.0f : m_new;
+    const float keep   = fast_exp2(m_run - m_safe);
+    l_run *= keep, v[0] *= keep, v[1] *= keep, v[2] *= keep, v[3] *= keep;
+#pragma unroll
+    for (int u = 0; u < kPfMergeChunk; ++u) {
+      const float f = fast_exp2(ml[u].x - m_safe);
+      l_run += f * ml[u].y;
+      v[0] += f * x[u].x, v[1] += f * x[u].y, v[2] += f * x[u].z, v[3] += f * x[u].w;
+    }
+    m_run = m_new;
+  }
+  const int   head = tile % n_heads, q_row = tile / n_heads * kBQ + (lane & 31);
+  const int   d0   = 8 * unit + 4 * (lane >> 5);
+  const float inv  = 1.0f / l_run;
+  if (q_row < qo_len && d0 < D) {
+    const size_t at = ((size_t) q_row * n_heads + head) * D + d0;
+    if (QO_F32) {
+      *reinterpret_cast<float4 *>(reinterpret_cast<float *>(o_ptr) + at) = make_float4(v[0] * inv, v[1] * inv, v[2] * inv, v[3] * inv);
+    } else {
+      v4h hv = { (_Float16) (v[0] * inv), (_Float16) (v[1] * inv), (_Float16) (v[2] * inv), (_Float16) (v[3] * inv) };
+      *reinterpret_cast<v4h *>(reinterpret_cast<_Float16 *>(o_ptr) + at) = hv;
     }
   }
 }
@@ -815,7 +999,7 @@ __global__ __launch_bounds__(D *MG) void flash_attn_decode_merge_kernel(void *__
 
 // ------------------------------------------------------------------------------------------------ any even head_dim
 
-// Head dims the MFMA kernels above are not built for (anything but 64 and 128; the reference routes head_dim % 64 != 0
+// Head dims the MFMA kernels above are not built for (even, but no multiple of 16; the reference routes head_dim % 64 != 0
 // to its own variant, src/dsp/ops/flash_attn_sp_hdim.c:782-832, which only asks for an even head_dim). One workgroup
 // per (query row, head); its four waves take every fourth 64-key block, with one key per lane for the scores (dot
 // products of fp16 pairs, v_dot2_f32_f16) and one output column per lane (d = lane + 64 i) for O += p V, then merge their
@@ -957,9 +1141,10 @@ __global__ __launch_bounds__(kGenThreads) void flash_attn_any_dim_kernel(void *_
   }
 }
 
-template <int D, bool QO_F32>
+template <int DP, bool FULL, bool QO_F32>
 hipError_t launch_prefill(hipStream_t stream, void *o, const void *q, const void *k, const void *v, const void *mask,
-                          int qo_len, int kv_len, int n_heads, int n_kv_heads, bool causal, int forced, bool mask_threshold) {
+                          int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim, bool causal, int forced,
+                          bool mask_threshold, float *scratch, size_t scratch_bytes) {
   const int group      = n_heads / n_kv_heads;
   const int gc         = group < 4 ? group : 4;
   const int qsub       = 4 / gc;
@@ -968,23 +1153,44 @@ hipError_t launch_prefill(hipStream_t stream, void *o, const void *q, const void
   if (q_blocks > 65535u) {
     return hipErrorInvalidValue;
   }
-  const dim3 grid((unsigned) (n_kv_heads * sub_groups), q_blocks);
+  constexpr unsigned kCus       = 256;
+  constexpr int      kMaxGroups = DP <= 128 ? 2 : 1;  // (what LDS and registers of a CU hold)
+  const unsigned     x = (unsigned) (n_kv_heads * sub_groups), wgs = x * q_blocks;
+  // Split the keys while that gives CUs without a workgroup one, down to two blocks per key group and workgroup (the merge
+  // is a second launch of about 4 us). Whole decoder layers on the 256-CU device, unsplit (with the mask loaded straight into
+  // registers) and split: 5 rows over 1029 keys, 12 / 2 heads of 128 (4 workgroups) 65.3 and 47.8 us; 128 rows over 1152
+  // (16 workgroups) 118.0 and 94.5 us; 512 rows over 2048 keys, 32 / 8 heads (128 workgroups) 372 and 338 us.
+  unsigned     splits = 1;
+  const size_t tiles  = (size_t) ((qo_len + kBQ - 1) / kBQ) * n_heads;
+  if (!forced && scratch != nullptr && wgs <= kCus / 2) {
+    const size_t share  = tiles * prefill_partial_floats(DP / 8) * sizeof(float);
+    const size_t blocks = ((size_t) kv_len + kBK - 1) / kBK;
+    const size_t most   = std::min({ (size_t) (kCus / wgs), blocks / (2 * kMaxGroups), scratch_bytes / share });
+    splits              = most < 2 ? 1u : (unsigned) most;
+  }
+  const dim3 grid(x, q_blocks, splits);
   // Two key groups per workgroup when the grid leaves CUs without a second workgroup, or (causal) when the workgroups
   // all fit at once and their uneven lengths would leave the long ones running alone. Measured on the 256-CU device,
   // 32 query / 8 KV heads of 128: 2048 x 2048 causal 59 us against 65 us, 1024 x 1024 without `causal` 30 against
   // 33 us; but 2048 x 2048 without `causal` 101 against 92 us.
-  constexpr unsigned kCus = 256;
-  const unsigned     wgs  = grid.x * grid.y;
-  const bool         two  = forced ? forced == 2 : (wgs <= kCus || (causal && wgs <= 2 * kCus));
+  const unsigned all = wgs * splits;
+  const bool     two = kMaxGroups == 2 && (forced ? forced == 2 : (all <= kCus || (causal && all <= 2 * kCus)));
+  const int      flags = (causal ? 1 : 0) | (mask_threshold ? 2 : 0);
   if (two) {
-    hipLaunchKernelGGL((flash_attn_prefill_kernel<D, QO_F32, 2>), grid, dim3(kPfThreads * 2), 0, stream, o, q,
-                       (const _Float16 *) k, (const _Float16 *) v, (const _Float16 *) mask, qo_len, kv_len, n_heads,
-                       n_kv_heads, (causal ? 1 : 0) | (mask_threshold ? 2 : 0));
+    hipLaunchKernelGGL((flash_attn_prefill_kernel<DP, FULL, QO_F32, kMaxGroups>), grid, dim3(kPfThreads * kMaxGroups), 0, stream,
+                       o, q, (const _Float16 *) k, (const _Float16 *) v, (const _Float16 *) mask, qo_len, kv_len, n_heads,
+                       n_kv_heads, head_dim, flags, scratch);
   } else {
-    hipLaunchKernelGGL((flash_attn_prefill_kernel<D, QO_F32, 1>), grid, dim3(kPfThreads), 0, stream, o, q,
+    hipLaunchKernelGGL((flash_attn_prefill_kernel<DP, FULL, QO_F32, 1>), grid, dim3(kPfThreads), 0, stream, o, q,
                        (const _Float16 *) k, (const _Float16 *) v, (const _Float16 *) mask, qo_len, kv_len, n_heads,
-                       n_kv_heads, (causal ? 1 : 0) | (mask_threshold ? 2 : 0));
+                       n_kv_heads, head_dim, flags, scratch);
   }
+  if (hipError_t e = hipGetLastError(); e != hipSuccess || splits == 1) {
+    return e;
+  }
+  constexpr int kUnits = DP / 8;
+  hipLaunchKernelGGL(flash_attn_prefill_merge_kernel<QO_F32>, dim3((unsigned) ((tiles * kUnits + 3) / 4)), dim3(256), 0, stream, o,
+                     scratch, (int) splits, (int) tiles, kUnits, qo_len, n_heads, head_dim);
   return hipGetLastError();
 }
 
@@ -1082,25 +1288,9 @@ hipError_t launch_flash_attn_decode_part(hipStream_t stream, int part, void *o, 
 hipError_t launch_flash_attn(hipStream_t stream, void *o, const void *q, const void *k, const void *v,
                              const void *mask, int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim,
                              bool qo_is_f32, bool causal, void *workspace, void *q8_out, int forced_key_groups,
-                             bool mask_threshold) {
-  if (head_dim != 64 && head_dim != 128) {
-    if (head_dim <= 0 || head_dim % 2 != 0 || head_dim > kGenMaxD || qo_len > 0x7fffffff || n_heads > 65535) {
-      return hipErrorNotSupported;
-    }
-    const dim3 grid((unsigned) qo_len, (unsigned) n_heads);
-    if (qo_is_f32) {
-      hipLaunchKernelGGL(flash_attn_any_dim_kernel<true>, grid, dim3(kGenThreads), 0, stream, o, q,
-                         (const _Float16 *) k, (const _Float16 *) v, (const _Float16 *) mask, qo_len, kv_len, n_heads,
-                         n_kv_heads, head_dim, (causal ? 1 : 0) | (mask_threshold ? 2 : 0));
-    } else {
-      hipLaunchKernelGGL(flash_attn_any_dim_kernel<false>, grid, dim3(kGenThreads), 0, stream, o, q,
-                         (const _Float16 *) k, (const _Float16 *) v, (const _Float16 *) mask, qo_len, kv_len, n_heads,
-                         n_kv_heads, head_dim, (causal ? 1 : 0) | (mask_threshold ? 2 : 0));
-    }
-    return hipGetLastError();
-  }
+                             bool mask_threshold, void *shares, size_t shares_bytes) {
   // with a single query row the causal rule (key j visible iff j <= kv_len - 1) hides nothing
-  if (qo_len == 1) {
+  if (qo_len == 1 && (head_dim == 64 || head_dim == 128)) {
     float *ws = static_cast<float *>(workspace);
     if (head_dim == 128) {
       return qo_is_f32 ? launch_decode<128, true>(stream, o, q, k, v, mask, kv_len, n_heads, n_kv_heads, ws, q8_out, mask_threshold) :
@@ -1109,17 +1299,49 @@ hipError_t launch_flash_attn(hipStream_t stream, void *o, const void *q, const v
     return qo_is_f32 ? launch_decode<64, true>(stream, o, q, k, v, mask, kv_len, n_heads, n_kv_heads, ws, q8_out, mask_threshold) :
                        launch_decode<64, false>(stream, o, q, k, v, mask, kv_len, n_heads, n_kv_heads, ws, q8_out, mask_threshold);
   }
+#define HTPOPS_PREFILL(DP, FULL)                                                                                     \
+  qo_is_f32 ? launch_prefill<DP, FULL, true>(stream, o, q, k, v, mask, qo_len, kv_len, n_heads, n_kv_heads, head_dim, \
+                                             causal, forced_key_groups, mask_threshold, static_cast<float *>(shares), \
+                                             shares_bytes) :                                                         \
+              launch_prefill<DP, FULL, false>(stream, o, q, k, v, mask, qo_len, kv_len, n_heads, n_kv_heads, head_dim, \
+                                              causal, forced_key_groups, mask_threshold, static_cast<float *>(shares), \
+                                              shares_bytes)
   if (head_dim == 128) {
-    return qo_is_f32 ?
-             launch_prefill<128, true>(stream, o, q, k, v, mask, qo_len, kv_len, n_heads, n_kv_heads, causal,
-                                        forced_key_groups, mask_threshold) :
-             launch_prefill<128, false>(stream, o, q, k, v, mask, qo_len, kv_len, n_heads, n_kv_heads, causal,
-                                        forced_key_groups, mask_threshold);
+    return HTPOPS_PREFILL(128, true);
   }
-  return qo_is_f32 ? launch_prefill<64, true>(stream, o, q, k, v, mask, qo_len, kv_len, n_heads, n_kv_heads, causal,
-                                        forced_key_groups, mask_threshold) :
-                     launch_prefill<64, false>(stream, o, q, k, v, mask, qo_len, kv_len, n_heads, n_kv_heads, causal,
-                                        forced_key_groups, mask_threshold);
+  if (head_dim == 64) {
+    return HTPOPS_PREFILL(64, true);
+  }
+  if (head_dim <= 0 || head_dim % 2 != 0 || head_dim > kGenMaxD || n_heads > 65535) {
+    return hipErrorNotSupported;
+  }
+  // Multiples of 16 fill the matrix instructions' k steps, and their rows (multiples of 32 bytes behind 16-byte aligned
+  // buffers) can be fetched 16 bytes at a time; every other even head dim, and more query blocks than a grid has rows,
+  // take the plain kernel.
+  if (head_dim % 16 == 0 && qo_len <= 65535 * kBQ) {
+    switch ((head_dim + 31) / 32) {
+      case 1: return HTPOPS_PREFILL(32, false);
+      case 2: return HTPOPS_PREFILL(64, false);
+      case 3: return HTPOPS_PREFILL(96, false);
+      case 4: return HTPOPS_PREFILL(128, false);
+      case 5: return HTPOPS_PREFILL(160, false);
+      case 6: return HTPOPS_PREFILL(192, false);
+      case 7: return HTPOPS_PREFILL(224, false);
+      default: return HTPOPS_PREFILL(256, false);
+    }
+  }
+#undef HTPOPS_PREFILL
+  const dim3 grid((unsigned) qo_len, (unsigned) n_heads);
+  if (qo_is_f32) {
+    hipLaunchKernelGGL(flash_attn_any_dim_kernel<true>, grid, dim3(kGenThreads), 0, stream, o, q,
+                       (const _Float16 *) k, (const _Float16 *) v, (const _Float16 *) mask, qo_len, kv_len, n_heads,
+                       n_kv_heads, head_dim, (causal ? 1 : 0) | (mask_threshold ? 2 : 0));
+  } else {
+    hipLaunchKernelGGL(flash_attn_any_dim_kernel<false>, grid, dim3(kGenThreads), 0, stream, o, q,
+                       (const _Float16 *) k, (const _Float16 *) v, (const _Float16 *) mask, qo_len, kv_len, n_heads,
+                       n_kv_heads, head_dim, (causal ? 1 : 0) | (mask_threshold ? 2 : 0));
+  }
+  return hipGetLastError();
 }
 
 }  // namespace htpops

@@ -411,8 +411,7 @@ int op_flash_attn(htpops_context *ctx, void *o, const void *q, const void *k, co
     return fail(ctx, HTPOPS_ERR_REJECTED, "flash_attn: n_heads=%d is not a multiple of n_kv_heads=%d", n_heads,
                 n_kv_heads);
   }
-  // reference: flash_attn_sp_hdim.c:785-788 (an odd head_dim is refused); 64 and 128 take the MFMA kernels, every
-  // other even head_dim up to 256 the general one
+  // reference: flash_attn_sp_hdim.c:785-788 (an odd head_dim is refused)
   if (head_dim % 2 != 0 || head_dim > 256) {
     return fail(ctx, HTPOPS_ERR_REJECTED, "flash_attn: head_dim=%d (even values up to 256 are built)", head_dim);
   }
@@ -461,7 +460,7 @@ int op_flash_attn(htpops_context *ctx, void *o, const void *q, const void *k, co
   }
   HTPOPS_HIP(ctx, launch_flash_attn(ctx->stream, o, q, k, v, mask, qo_len, kv_len, n_heads, n_kv_heads, head_dim,
                                     qo_is_f32 != 0, causal != 0, ws, q8_out, ctx->opt.attn_key_groups,
-                                    ctx->opt.attn_mask_threshold != 0));
+                                    ctx->opt.attn_mask_threshold != 0, ctx->attn_shares, ctx->attn_shares ? kAttnSharesBytes : 0));
   ctx->attn_q8_done = q8_out != nullptr;
   return HTPOPS_OK;
 }
