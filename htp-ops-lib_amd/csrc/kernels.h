@@ -130,21 +130,7 @@ size_t     mat_mul_workspace_bytes(int m, int k, int n);
 hipError_t launch_mat_mul_q8_0_act(hipStream_t stream, float *out, const void *act, const void *weight, int m, int k,
                                    int n, WeightType wt, void *workspace, unsigned *tickets, int ticket_slots);
 
-// The reference's native weight formats (ops 1-4): a weight buffer (weight_kind 1 fp16 tiles, 2 Q4_0, 3 Q8_0,
-// 4 IQ4_NL super-blocks) is converted once into MFMA fragment order (permuted_weight_fragment_bytes), then
-// out fp32 [m][n] = fp16(act fp16 x W fp16); `act_fragments` is scratch of permuted_act_fragment_bytes.
-size_t     permuted_weight_fragment_bytes(int k, int n);
-size_t     permuted_act_fragment_bytes(int m, int k);
-hipError_t launch_permuted_weight_to_fragments(hipStream_t stream, void *dst, const void *src, int k, int n,
-                                               int weight_kind);
-hipError_t launch_mat_mul_fragments(hipStream_t stream, float *out, const float *act, const void *weight_fragments,
-                                    int m, int k, int n, void *act_fragments);
-
-// The same formats read as they lie, nothing converted or kept, for up to kPermutedRowsMax rows: up to kPermutedGroupMax
-// matmuls of one row count and weight kind in one launch (plus one that puts the activations into operand order where
-// they do not fit LDS). The caller guarantees that no member reads what another writes. A member's result does not
-// depend on the others. `workspace`: permuted_rows_workspace_bytes.
-constexpr int kPermutedRowsMax  = 32;
+// The reference's native weight formats (ops 1-4; weight_kind 1 fp16 tiles, 2 Q4_0, 3 Q8_0, 4 IQ4_NL super-blocks).
 constexpr int kPermutedGroupMax = 8;
 struct PermutedMatMul {
   float       *out;
@@ -152,6 +138,21 @@ struct PermutedMatMul {
   const void  *weight;
   int          k, n;
 };
+// Many rows: a weight buffer is converted once into MFMA fragment order (permuted_weight_fragment_bytes), then
+// out fp32 [m][n] = fp16(act fp16 x W fp16): up to kPermutedGroupMax matmuls of one row count in one launch, plus one that
+// converts the distinct activations into `workspace` (permuted_gemm_workspace_bytes). The caller guarantees that no
+// member reads what another writes. A member's result does not depend on the others.
+size_t     permuted_weight_fragment_bytes(int k, int n);
+hipError_t launch_permuted_weight_to_fragments(hipStream_t stream, void *dst, const void *src, int k, int n,
+                                               int weight_kind);
+size_t     permuted_gemm_workspace_bytes(const PermutedMatMul *members, int count, int m);
+hipError_t launch_permuted_gemm_group(hipStream_t stream, const PermutedMatMul *members, const void *const *weight_fragments,
+                                      int count, int m, void *workspace);
+
+// The same formats read as they lie, nothing converted or kept, for up to kPermutedRowsMax rows: up to kPermutedGroupMax
+// matmuls of one row count and weight kind in one launch (plus one that puts the activations into operand order where
+// they do not fit LDS), under the same rules. `workspace`: permuted_rows_workspace_bytes.
+constexpr int kPermutedRowsMax = 32;
 size_t     permuted_rows_workspace_bytes(const PermutedMatMul *members, int count, int m);
 hipError_t launch_permuted_rows_group(hipStream_t stream, const PermutedMatMul *members, int count, int m, int weight_kind,
                                       void *workspace);

@@ -330,14 +330,53 @@ int run_permuted_rows(htpops_context *ctx, const PermutedMatMul *members, int co
   return HTPOPS_OK;
 }
 
+// more rows: one launch over converted copies of the weights, which are kept (kept already, or in a buffer of which copies
+// may be kept; see op_mat_mul_permuted)
+int run_permuted_gemm(htpops_context *ctx, const PermutedMatMul *members, int count, int m, int kind) {
+  const void *frag[kPermutedGroupMax];
+  for (int i = 0; i < count; ++i) {
+    const PermutedMatMul &p = members[i];
+    frag[i]                 = find_copy(ctx, p.weight, kind, p.k, p.n);
+    if (frag[i]) {
+      continue;
+    }
+    void *fresh = nullptr;
+    if (int r = new_copy(ctx, p.weight, permuted_weight_bytes((size_t) p.n, (size_t) p.k, kind), kind, p.k, p.n,
+                         permuted_weight_fragment_bytes(p.k, p.n), &fresh)) {
+      return r;
+    }
+    const hipError_t e = launch_permuted_weight_to_fragments(ctx->stream, fresh, p.weight, p.k, p.n, kind);
+    if (e != hipSuccess) {
+      forget_copy(ctx, fresh);
+      return fail(ctx, HTPOPS_ERR_HIP, "weight conversion: %s", hipGetErrorString(e));
+    }
+    frag[i] = fresh;
+  }
+  if (int r = ensure_workspace(ctx, permuted_gemm_workspace_bytes(members, count, m))) {
+    return r;
+  }
+  HTPOPS_HIP(ctx, launch_permuted_gemm_group(ctx->stream, members, frag, count, m, ctx->workspace));
+  return HTPOPS_OK;
+}
+
+bool keeps_copy(htpops_context *ctx, const PermutedMatMul &p, int kind) {
+  return find_copy(ctx, p.weight, kind, p.k, p.n) != nullptr ||
+         may_keep_copies(ctx, p.weight, permuted_weight_bytes((size_t) p.n, (size_t) p.k, kind));
+}
+
 }  // namespace
 
 int op_mat_mul_permuted_group(htpops_context *ctx, const PermutedMatMul *members, int count, int m, int kind) {
-  if (count > 1 && m <= kPermutedRowsMax) {
+  bool together = count > 1;
+  for (int i = 0; together && i < count; ++i) {
+    together = m <= kPermutedRowsMax || keeps_copy(ctx, members[i], kind);
+  }
+  if (together) {
     for (int i = 0; i < count; ++i) {
       note_device_write(ctx, members[i].out, (size_t) m * members[i].n * 4);
     }
-    return run_permuted_rows(ctx, members, count, m, kind);
+    return m <= kPermutedRowsMax ? run_permuted_rows(ctx, members, count, m, kind) :
+                                   run_permuted_gemm(ctx, members, count, m, kind);
   }
   int ret = HTPOPS_OK;
   for (int i = 0; i < count; ++i) {
@@ -366,37 +405,23 @@ int op_mat_mul_permuted(htpops_context *ctx, float *dst, const float *act, const
     return r;
   }
   note_device_write(ctx, dst, (size_t) m * n * 4);
+  const PermutedMatMul one = { dst, act, weight, k, n };
   if (m <= kPermutedRowsMax) {
-    const PermutedMatMul one = { dst, act, weight, k, n };
     return run_permuted_rows(ctx, &one, 1, m, kind);
   }
-  const void *frag = find_copy(ctx, weight, kind, k, n);
   // Converted copies are kept only for weights in buffers the context allocated (their contents change only through
   // htpops_buffer_write or as an op's output, both of which drop the copy). Caller-registered memory may be rewritten
   // behind the context's back: it is converted into the workspace on every call.
-  const size_t act_bytes  = (permuted_act_fragment_bytes(m, k) + 255) & ~(size_t) 255;
-  const size_t frag_bytes = permuted_weight_fragment_bytes(k, n);
-  const bool   cacheable  = !frag && may_keep_copies(ctx, weight, permuted_weight_bytes((size_t) n, (size_t) k, kind));
-  if (int r = ensure_workspace(ctx, act_bytes + ((frag || cacheable) ? 0 : frag_bytes))) {
+  if (keeps_copy(ctx, one, kind)) {
+    return run_permuted_gemm(ctx, &one, 1, m, kind);
+  }
+  const size_t act_bytes = permuted_gemm_workspace_bytes(&one, 1, m);  // (a multiple of 1 KiB)
+  if (int r = ensure_workspace(ctx, act_bytes + permuted_weight_fragment_bytes(k, n))) {
     return r;
   }
-  if (!frag) {
-    void *fresh = static_cast<uint8_t *>(ctx->workspace) + act_bytes;
-    if (cacheable) {
-      if (int r = new_copy(ctx, weight, permuted_weight_bytes((size_t) n, (size_t) k, kind), kind, k, n, frag_bytes, &fresh)) {
-        return r;
-      }
-    }
-    const hipError_t e = launch_permuted_weight_to_fragments(ctx->stream, fresh, weight, k, n, kind);
-    if (e != hipSuccess) {
-      if (cacheable) {
-        forget_copy(ctx, fresh);
-      }
-      return fail(ctx, HTPOPS_ERR_HIP, "weight conversion: %s", hipGetErrorString(e));
-    }
-    frag = fresh;
-  }
-  HTPOPS_HIP(ctx, launch_mat_mul_fragments(ctx->stream, dst, act, frag, m, k, n, ctx->workspace));
+  const void *frag = static_cast<uint8_t *>(ctx->workspace) + act_bytes;
+  HTPOPS_HIP(ctx, launch_permuted_weight_to_fragments(ctx->stream, const_cast<void *>(frag), weight, k, n, kind));
+  HTPOPS_HIP(ctx, launch_permuted_gemm_group(ctx->stream, &one, &frag, 1, m, ctx->workspace));
   return HTPOPS_OK;
 }
 

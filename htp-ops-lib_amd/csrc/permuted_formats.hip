@@ -112,11 +112,16 @@ __global__ __launch_bounds__(256) void dequant_permuted_q8_kernel(uint4 *__restr
   dst[t] = make_uint4(out[0], out[1], out[2], out[3]);
 }
 
-// activations fp32 [m][k] -> fragment order with rows on lanes; rows >= m are zero
-__global__ __launch_bounds__(256) void act_to_fragments_kernel(uint4 *__restrict__ dst, const float *__restrict__ act,
-                                                               int m, int k, int m_tiles) {
+// activations fp32 [m][k] -> fragment order with rows on lanes; rows >= m are zero. One grid row per activation matrix.
+struct ActMembers {
+  const float *src[kPermutedGroupMax];
+  uint4       *dst[kPermutedGroupMax];
+  int          k[kPermutedGroupMax];
+};
+
+__global__ __launch_bounds__(256) void act_to_fragments_kernel(ActMembers members, int m, int m_tiles) {
   const size_t t = (size_t) blockIdx.x * 256 + threadIdx.x;
-  const int    k_steps = k / 16;
+  const int    k = members.k[blockIdx.y], k_steps = k / 16;
   const int    lane = (int) (t & 63);
   const size_t f    = t >> 6;
   const int    step = (int) (f % (size_t) k_steps), tile = (int) (f / (size_t) k_steps);
@@ -126,91 +131,169 @@ __global__ __launch_bounds__(256) void act_to_fragments_kernel(uint4 *__restrict
   const int row = tile * 32 + (lane & 31);
   uint4     o   = make_uint4(0, 0, 0, 0);
   if (row < m) {
-    const float4 *s = reinterpret_cast<const float4 *>(act + (size_t) row * k + 16 * step + 8 * (lane >> 5));
+    const float4 *s = reinterpret_cast<const float4 *>(members.src[blockIdx.y] + (size_t) row * k + 16 * step + 8 * (lane >> 5));
     const float4  a = s[0], b = s[1];
     o = make_uint4(pack_halfs(a.x, a.y), pack_halfs(a.z, a.w), pack_halfs(b.x, b.y), pack_halfs(b.z, b.w));
   }
-  dst[t] = o;
+  members.dst[blockIdx.y][t] = o;
 }
 
-// out[m][n] = fp16(sum_k A[m][k] * W[k][n]) widened to fp32; both operands in fragment order.
-// A workgroup is WM x WN waves, a wave owns MT x NT tiles of 32 x 32 and walks K with DEPTH fragment sets in flight.
-template <int MT, int NT, int WM, int WN>
-__global__ __launch_bounds__(WM *WN * 64) void gemm_f16_fragments_kernel(float *__restrict__ out,
-                                                                         const uint4 *__restrict__ a_frag,
-                                                                         const uint4 *__restrict__ b_frag, int m, int n,
-                                                                         int k_steps, int m_tiles, int n_tiles) {
-  constexpr int DEPTH = 4;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave / WN, wn = wave % WN;
-  const int mt0 = (blockIdx.y * WM + wm) * MT, nt0 = (blockIdx.x * WN + wn) * NT;
-  if (mt0 >= m_tiles || nt0 >= n_tiles) {
-    return;  // no barriers in this kernel
+// out[m][n] = fp16(sum_k A[m][k] * W[k][n]) widened to fp32; both operands in fragment order; the matmuls of a message
+// that nothing orders in one launch.
+// A workgroup owns MT row tiles x 4 column tiles of 32 x 32. Its four waves are two column halves times two halves of K;
+// a wave holds MT x 2 tiles, and the halves of K are added through LDS at the end. The operand pieces of a step (16 of K: MT KiB of rows that two
+// waves share, 2 KiB of columns per wave) come into LDS by DMA as they lie in memory, in a ring of four slots, requested
+// three steps ahead; the fragments of step s + 1 are read while the products of step s run, so a step costs one barrier.
+// A wave reads (MT + 2) KiB of LDS for 2 MT matrix instructions: from MT = 3 on less than the LDS delivers while
+// they run. Straight into registers (each wave its own 4 KiB of a step for four instructions, a launch per matrix)
+// the path from L2 into a CU was the limit: 300 rows, seven
+// projections of hidden 2048 / ffn 5632 took 264.8 us, now 94.6 (72 of them here = 430 TFLOP/s; the copies are 59 MB).
+// A sum's order depends on k alone (never on MT or on the other members of a launch).
+struct GemmMembers {
+  float       *out[kPermutedGroupMax];
+  const uint8_t *a[kPermutedGroupMax], *w[kPermutedGroupMax];
+  int          n_tiles[kPermutedGroupMax], k_steps[kPermutedGroupMax];
+  int          col_begin[kPermutedGroupMax + 1];  // in units of 4 column tiles
+  int          count;
+};
+
+template <int MT>
+__global__ __launch_bounds__(256, 2) void gemm_f16_fragments_kernel(GemmMembers members, int m, int m_tiles, int row_blocks) {
+  constexpr int RING  = 4;
+  constexpr int STEP  = 2 * MT + 8;            // KiB of a step: the rows of both K halves, the columns of four waves
+  constexpr int APART = (MT + 1) / 2;          // row pieces that a wave brings (a shared odd one is brought twice)
+  constexpr int PIECES = APART + 2;            // DMA instructions of a wave and step
+  __shared__ __align__(1024) uint8_t lds[RING][STEP * 1024];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kh = wave >> 1, wn = wave & 1;
+  // Workgroup ids go round the 8 XCDs: the row blocks of a column block follow each other on one XCD, so its weights come
+  // from that L2 for all but the first, and the column blocks (longest K first) are dealt out evenly.
+  const int turn = (int) blockIdx.x >> 3;
+  const int col  = turn / row_blocks * 8 + ((int) blockIdx.x & 7), rb = turn % row_blocks;
+  if (col >= members.col_begin[members.count]) {
+    return;
   }
-  const uint4 *ap[MT], *bp[NT];
+  int id = 0;
+  while (id + 1 < members.count && col >= members.col_begin[id + 1]) {
+    ++id;
+  }
+  const int n_tiles = members.n_tiles[id], k_steps = members.k_steps[id], steps = k_steps / 2;
+  const int mt0 = rb * MT, nt0 = (col - members.col_begin[id]) * 4 + 2 * wn;
+
+  // what this wave brings of every step: pieces of 1 KiB, the steps of a tile behind each other
+  const uint8_t *src[PIECES];
+  uint32_t       to[PIECES];
+#pragma unroll
+  for (int p = 0; p < PIECES; ++p) {
+    if (p < APART) {
+      const int i = min(p * 2 + wn, MT - 1);
+      src[p] = members.a[id] + (size_t) min(mt0 + i, m_tiles - 1) * k_steps * 1024;
+      to[p]  = (uint32_t) (kh * MT + i) * 1024;
+    } else {
+      const int j = p - APART;
+      src[p] = members.w[id] + (size_t) min(nt0 + j, n_tiles - 1) * k_steps * 1024;
+      to[p]  = (uint32_t) (2 * MT + 2 * wave + j) * 1024;
+    }
+    src[p] += (size_t) kh * steps * 1024;
+  }
+  const uint32_t lds0 = (uint32_t) (uintptr_t) &lds[0][0];
+  auto fetch = [&](int step) {  // (past the end: the last step again, so that the count of requests in flight stays)
+    const size_t   off  = (size_t) min(step, steps - 1) * 1024;
+    const uint32_t slot = lds0 + (uint32_t) (step & (RING - 1)) * (STEP * 1024);
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p) {
+      asm volatile("s_mov_b32 m0, %2\n s_nop 0\n global_load_lds_dwordx4 %0, %1" ::"v"(lane * 16), "s"(src[p] + off), "s"(slot + to[p]) : "memory");
+    }
+  };
+  struct Frags {
+    uint4 a[MT], b[2];
+  };
+  auto read = [&](Frags &f, int step) {
+    const uint8_t *slot = lds[step & (RING - 1)];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      f.a[i] = *reinterpret_cast<const uint4 *>(slot + (kh * MT + i) * 1024 + lane * 16);
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      f.b[j] = *reinterpret_cast<const uint4 *>(slot + (2 * MT + 2 * wave + j) * 1024 + lane * 16);
+    }
+  };
+  v16f acc[MT][2];
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
-    ap[i] = a_frag + (size_t) min(mt0 + i, m_tiles - 1) * k_steps * 64 + lane;
-  }
 #pragma unroll
-  for (int j = 0; j < NT; ++j) {
-    bp[j] = b_frag + (size_t) min(nt0 + j, n_tiles - 1) * k_steps * 64 + lane;
-  }
-  v16f acc[MT][NT];
-#pragma unroll
-  for (int i = 0; i < MT; ++i) {
-#pragma unroll
-    for (int j = 0; j < NT; ++j) {
+    for (int j = 0; j < 2; ++j) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         acc[i][j][r] = 0.0f;
       }
     }
   }
-  uint4 ar[DEPTH][MT], br[DEPTH][NT];
-  auto  load = [&](int d, int step) {
-    const size_t off = (size_t) min(step, k_steps - 1) * 64;  // branch-free: steps past the end repeat the last one
+  // Behind the barrier of step s everybody's pieces of step s + 1 have landed (all but the youngest two steps' requests
+  // have returned) and the fragments of step s are in everybody's registers, so its slot takes step s + 4.
+  auto turn_over = [&](int s, Frags &now, Frags &next) {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * PIECES) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    fetch(s + RING);
+    read(next, s + 1);
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
-      ar[d][i] = ap[i][off];
-    }
 #pragma unroll
-    for (int j = 0; j < NT; ++j) {
-      br[d][j] = bp[j][off];
+      for (int j = 0; j < 2; ++j) {
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, now.a[i]), __builtin_bit_cast(v8h, now.b[j]),
+                                                           acc[i][j], 0, 0, 0);
+      }
     }
   };
 #pragma unroll
-  for (int d = 0; d < DEPTH; ++d) {
-    load(d, d);
+  for (int s = 0; s < RING; ++s) {
+    fetch(s);
   }
-  for (int s0 = 0; s0 < k_steps; s0 += DEPTH) {
-#pragma unroll
-    for (int d = 0; d < DEPTH; ++d) {
-      if (s0 + d < k_steps) {
-#pragma unroll
-        for (int i = 0; i < MT; ++i) {
-#pragma unroll
-          for (int j = 0; j < NT; ++j) {
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, ar[d][i]),
-                                                               __builtin_bit_cast(v8h, br[d][j]), acc[i][j], 0, 0, 0);
-          }
-        }
-      }
-      load(d, s0 + d + DEPTH);
-    }
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * PIECES) : "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  Frags f0, f1;
+  read(f0, 0);
+  int s = 0;
+  for (; s + 1 < steps; s += 2) {
+    turn_over(s, f0, f1);
+    turn_over(s + 1, f1, f0);
   }
+  if (s < steps) {
+    turn_over(s, f0, f1);
+  }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+
   // D[i][j]: j = lane % 32 (column), i = 8 (r / 4) + 4 (lane / 32) + r % 4 (row)
+  float *xch = reinterpret_cast<float *>(&lds[0][0]) + (size_t) wn * 2 * 16 * 64 + lane;
+  static_assert(2 * 2 * 16 * 64 * sizeof(float) <= sizeof(lds), "a row tile of both column halves fits");
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
+    __syncthreads();  // nobody reads the ring, or the row tile before, any more
+    if (kh == 1) {
 #pragma unroll
-    for (int j = 0; j < NT; ++j) {
-      if (mt0 + i < m_tiles && nt0 + j < n_tiles) {
-        const int col = (nt0 + j) * 32 + (lane & 31);
+      for (int j = 0; j < 2; ++j) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const int row = (mt0 + i) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-          if (row < m) {
-            out[(size_t) row * n + col] = (float) (_Float16) acc[i][j][r];  // the reference stores fp16 results
+          xch[(16 * j + r) * 64] = acc[i][j][r];
+        }
+      }
+    }
+    __syncthreads();
+    if (kh == 0 && mt0 + i < m_tiles) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        if (nt0 + j < n_tiles) {
+          const int c = (nt0 + j) * 32 + (lane & 31);
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int row = (mt0 + i) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+            const float sum = acc[i][j][r] + xch[(16 * j + r) * 64];
+            if (row < m) {
+              members.out[id][(size_t) row * (n_tiles * 32) + c] = (float) (_Float16) sum;  // the reference stores fp16 results
+            }
           }
         }
       }
@@ -258,32 +341,89 @@ hipError_t launch_permuted_weight_to_fragments(hipStream_t stream, void *dst, co
   return hipGetLastError();
 }
 
-hipError_t launch_mat_mul_fragments(hipStream_t stream, float *out, const float *act, const void *weight_fragments,
-                                    int m, int k, int n, void *act_fragments) {
-  if (k % 32 != 0 || n % 32 != 0 || m <= 0) {
+size_t permuted_gemm_workspace_bytes(const PermutedMatMul *members, int count, int m) {
+  size_t total = 0;
+  for (int i = 0; i < count; ++i) {
+    bool seen = false;
+    for (int j = 0; j < i; ++j) {
+      seen = seen || (members[j].act == members[i].act && members[j].k == members[i].k);
+    }
+    total += seen ? 0 : permuted_act_fragment_bytes(m, members[i].k);
+  }
+  return total;
+}
+
+hipError_t launch_permuted_gemm_group(hipStream_t stream, const PermutedMatMul *members, const void *const *weight_fragments,
+                                      int count, int m, void *workspace) {
+  if (count <= 0 || count > kPermutedGroupMax || m <= 0) {
     return hipErrorInvalidValue;
   }
-  const int    k_steps = k / 16, n_tiles = n / 32, m_tiles = (m + 31) / 32;
-  const size_t a_pieces = (size_t) m_tiles * k_steps * 64;
-  hipLaunchKernelGGL(act_to_fragments_kernel, dim3((unsigned) ((a_pieces + 255) / 256)), dim3(256), 0, stream,
-                     static_cast<uint4 *>(act_fragments), act, m, k, m_tiles);
+  const int   m_tiles = (m + 31) / 32;
+  ActMembers  acts    = {};
+  GemmMembers g       = {};
+  int         n_acts = 0, order[kPermutedGroupMax], act_of[kPermutedGroupMax], k_max = 0;
+  uint8_t    *ws     = static_cast<uint8_t *>(workspace);
+  for (int i = 0; i < count; ++i) {
+    const PermutedMatMul &p = members[i];
+    if (p.k % 32 != 0 || p.n % 32 != 0) {
+      return hipErrorInvalidValue;
+    }
+    int j = 0;
+    while (j < n_acts && !(acts.src[j] == p.act && acts.k[j] == p.k)) {
+      ++j;
+    }
+    if (j == n_acts) {
+      acts.src[j] = p.act, acts.k[j] = p.k, acts.dst[j] = reinterpret_cast<uint4 *>(ws);
+      ws += permuted_act_fragment_bytes(m, p.k);
+      ++n_acts;
+      k_max = p.k > k_max ? p.k : k_max;
+    }
+    act_of[i] = j;
+    int at = i;  // longest K first: the launch ends with short workgroups
+    while (at > 0 && members[order[at - 1]].k < p.k) {
+      order[at] = order[at - 1];
+      --at;
+    }
+    order[at] = i;
+  }
+  const size_t a_pieces = (size_t) m_tiles * (k_max / 16) * 64;
+  hipLaunchKernelGGL(act_to_fragments_kernel, dim3((unsigned) ((a_pieces + 255) / 256), (unsigned) n_acts), dim3(256), 0, stream,
+                     acts, m, m_tiles);
   if (hipError_t e = hipGetLastError(); e != hipSuccess) {
     return e;
   }
-  const uint4 *a = static_cast<const uint4 *>(act_fragments), *b = static_cast<const uint4 *>(weight_fragments);
-  if (m_tiles == 1) {
-    // weight streaming: one 32-column tile per wave, as many workgroups as possible
-    hipLaunchKernelGGL((gemm_f16_fragments_kernel<1, 1, 1, 2>), dim3((unsigned) ((n_tiles + 1) / 2), 1), dim3(128), 0,
-                       stream, out, a, b, m, n, k_steps, m_tiles, n_tiles);
-  } else if (m_tiles <= 4) {
-    hipLaunchKernelGGL((gemm_f16_fragments_kernel<1, 2, 2, 2>), dim3((unsigned) ((n_tiles + 3) / 4),
-                                                                      (unsigned) ((m_tiles + 1) / 2)),
-                       dim3(256), 0, stream, out, a, b, m, n, k_steps, m_tiles, n_tiles);
-  } else {
-    hipLaunchKernelGGL((gemm_f16_fragments_kernel<2, 2, 2, 2>), dim3((unsigned) ((n_tiles + 3) / 4),
-                                                                      (unsigned) ((m_tiles + 3) / 4)),
-                       dim3(256), 0, stream, out, a, b, m, n, k_steps, m_tiles, n_tiles);
+  int cols = 0;
+  g.count  = count;
+  for (int i = 0; i < count; ++i) {
+    const PermutedMatMul &p = members[order[i]];
+    g.out[i] = p.out, g.a[i] = reinterpret_cast<const uint8_t *>(acts.dst[act_of[order[i]]]);
+    g.w[i]       = static_cast<const uint8_t *>(weight_fragments[order[i]]);
+    g.n_tiles[i] = p.n / 32, g.k_steps[i] = p.k / 16;
+    g.col_begin[i] = cols;
+    cols += (p.n / 32 + 3) / 4;
   }
+  g.col_begin[count] = cols;
+  // The most row tiles per workgroup that still give every CU one workgroup (two fit), spread evenly over the row blocks.
+  int mt = m_tiles < 5 ? m_tiles : 5;
+  while (mt > 1 && (long) cols * ((m_tiles + mt - 1) / mt) < 256) {
+    --mt;
+  }
+  const int row_blocks = (m_tiles + mt - 1) / mt;
+  mt = (m_tiles + row_blocks - 1) / row_blocks;
+  const long long grid = (long long) ((cols + 7) / 8) * 8 * row_blocks;
+  if (grid > 0x7fffffffLL) {
+    return hipErrorInvalidValue;
+  }
+#define HTPOPS_GEMM(MT)                                                                                               \
+  hipLaunchKernelGGL(gemm_f16_fragments_kernel<MT>, dim3((unsigned) grid), dim3(256), 0, stream, g, m, m_tiles, row_blocks)
+  switch (mt) {
+    case 1: HTPOPS_GEMM(1); break;
+    case 2: HTPOPS_GEMM(2); break;
+    case 3: HTPOPS_GEMM(3); break;
+    case 4: HTPOPS_GEMM(4); break;
+    default: HTPOPS_GEMM(5); break;
+  }
+#undef HTPOPS_GEMM
   return hipGetLastError();
 }
 

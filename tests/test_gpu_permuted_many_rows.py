@@ -1,0 +1,55 @@
+"""GPU parity of the many-row matmuls over the reference's own weight formats (ops 1-4 with more than 32 rows): row counts
+and column counts at the edges of a workgroup's tiles, one K step per half, and grouping inside a message."""
+import numpy as np
+import pytest
+
+from pyhtpops import api
+from pyhtpops import workloads as wl
+from test_gpu_parity_permuted import OPS, check, make_weights
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = api.Context(device=0)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("kind,m,k,n", [
+    (1, 33, 32, 32), (2, 65, 64, 128), (3, 64, 96, 160), (4, 97, 160, 64),     # one, two, three, five steps per half of K
+    (1, 100, 512, 4096 + 32), (2, 130, 256, 8192), (3, 160, 128, 32768 + 96),  # 1, 3 and 5 row tiles per workgroup
+    (4, 290, 2048, 96), (2, 350, 64, 16384 + 32), (1, 128, 96, 32768)])        # (the last: 4 row tiles)
+def test_many_rows_at_the_edges(ctx, oracle, kind, m, k, n):
+    check(ctx, oracle, kind, m, k, n, m * 3 + k + n)
+
+
+def test_many_rows_grouped_with_caller_owned_weights(ctx):
+    # one message: shared rows, different k (a long one last), and a member whose weights may not be kept converted: every
+    # output byte for byte what one message per request gives
+    rng = wl.rng_for(88, 0)
+    m, kind = 70, 4
+    shapes = [(128, 96), (64, 1056), (416, 96), (128, 2080)]  # (n, k)
+    acts = {k: ctx.upload(wl.make_activations(rng, m, k)) for k in (96, 1056, 2080)}
+    ws = [ctx.upload(np.ascontiguousarray(make_weights(rng, n, k, kind)[0]).view(np.uint8)) for n, k in shapes]
+    for foreign in (False, True):
+        seen = list(ws)
+        if foreign:
+            seen[1] = ctx.register(ctx.device_ptr(ws[1]), ctx.size(ws[1]))
+        results = []
+        for grouped in (True, False):
+            outs = [ctx.upload(np.zeros(m * n, np.float32)) for n, _ in shapes]
+            reqs = [(api.REQUEST_TYPE_OP_COMPUTE, api.op_compute_request(OPS[kind], api.mat_mul_params(
+                (outs[j], 0), (acts[k], 0), (seen[j], 0), m, k, n))) for j, (n, k) in enumerate(shapes)]
+            for msg in ([api.build_message(reqs)] if grouped else [api.build_message([r]) for r in reqs]):
+                assert ctx.process_message(msg) == 0 and not any(api.message_request_states(msg)), ctx.last_error()
+            results.append([ctx.read(h, np.uint8, ctx.size(h)) for h in outs])
+            for h in outs:
+                ctx.release(h)
+        for a, b in zip(*results):
+            assert np.array_equal(a, b) and a.any()
+        if foreign:
+            ctx.release(seen[1])
+    for h in list(acts.values()) + ws:
+        ctx.release(h)
