@@ -127,6 +127,10 @@ struct htpops_context {
     int         m = 0, k = 0;
     int         kind = 0;  // which kernel family's layout (PlanKind)
   } act_fragments;
+  // Workspace that the next request of the message needs for the matmul it makes of the rows the current one quantizes, when
+  // that takes the int8 fragment kernels (0: it is something else): the quantizer then leaves the rows there in operand order
+  // too, and notes them in `act_fragments`.
+  size_t next_fragments_ws = 0;
   bool in_message = false;
   // how many separately launched units (grouped launches and single ops) the most recent message walk issued
   int  message_submissions = 0;
@@ -221,7 +225,8 @@ void forget_copy(htpops_context *ctx, void *frag);
 // ---- ops (ops.cc) ----
 constexpr int kSkinnyGroupMaxM = 8;   // rows of the K-sliced kernel's grouped launch
 constexpr int kBatchMaxM       = 16;  // rows up to which same-activation requests of a message are grouped
-constexpr int kManyRowsMinM    = 33;  // rows from which a matmul takes the matrix-core kernels
+constexpr int kManyRowsMinM    = 17;  // rows from which a matmul may take the many-row kernels (see plan_mat_mul)
+constexpr int kFp6MinM         = 33;  // ... and from which the FP6 kernel is one of them
 
 constexpr int kFragKindRowLayout = 100;  // + ggml type: int8 fragments (kinds 1..4 are the tile-permuted formats of ops 1-4)
 constexpr int kFragKindLaneOrder = 300;  // + ggml type: weights in matrix-core operand order (2..16 activation rows)

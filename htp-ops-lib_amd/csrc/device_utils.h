@@ -78,4 +78,36 @@ __device__ __forceinline__ float quad_max(float v) {
 }
 #undef HTPOPS_DPP_STEP
 
+// Activations in the operand order of the int8 matmul, [32-row tile][block][64 lanes] of 16 bytes: lane (c = row % 32, h)
+// holds elements 16 h .. 16 h + 15 of its row's block. The scale array behind them holds a dword (fp16 scale, 0) per row and
+// block, [tile][block][64] with zeros in the upper 32, and ends in one row of 64 zeros.
+struct ActFragments {
+  uint2    *frag   = nullptr;
+  uint32_t *scales = nullptr;
+  int       m_tiles = 0, nblk = 0;
+};
+inline ActFragments act_fragments_at(void *base, int m, int k) {
+  ActFragments f;
+  if (base) {
+    f.m_tiles = (m + 31) / 32, f.nblk = k / kQK;
+    f.frag   = static_cast<uint2 *>(base);
+    f.scales = reinterpret_cast<uint32_t *>(static_cast<uint8_t *>(base) + (((size_t) f.m_tiles * f.nblk * 1024 + 255) & ~(size_t) 255));
+  }
+  return f;
+}
+// eight quants of a block (those of lane `part` of the quad that holds it) and, from lanes 0 and 1, its scale
+__device__ __forceinline__ void store_act_fragment(const ActFragments &f, int row, int kb, int part, uint2 quants, uint16_t scale) {
+  const size_t at = ((size_t) (row >> 5) * f.nblk + kb) * 64 + (row & 31);
+  f.frag[(at + 32 * (part >> 1)) * 2 + (part & 1)] = quants;
+  if (part < 2) {
+    f.scales[at + 32 * part] = part == 0 ? scale : 0u;
+  }
+}
+// the row of zeros, from 64 threads of the grid
+__device__ __forceinline__ void end_act_fragments(const ActFragments &f, int thread) {
+  if (thread < 64) {
+    f.scales[(size_t) f.m_tiles * f.nblk * 64 + thread] = 0u;
+  }
+}
+
 }  // namespace htpops

@@ -126,8 +126,9 @@ __global__ __launch_bounds__(256) void act_to_i8_fragments_kernel(ActMembers grp
   mem.frag[t] = make_uint4(o[0], o[1], o[2], o[3]);
   // scale rows of 64 dwords: lanes 32..63 of the scale-product instruction hold K slots that must contribute nothing
   mem.scales[((size_t) tile * nblk + kb) * 64 + lane] = h == 0 ? sc : 0u;
-  if (t < 64) {
-    mem.scales[(size_t) m_tiles * nblk * 64 + t] = 0u;  // the row that blocks past the end of K are pointed at
+  if (t < 32) {  // (the row that blocks past the end of K are pointed at; one row tile and one pair are 32 threads)
+    mem.scales[(size_t) m_tiles * nblk * 64 + t]      = 0u;
+    mem.scales[(size_t) m_tiles * nblk * 64 + 32 + t] = 0u;
   }
 }
 
@@ -184,8 +185,9 @@ __global__ __launch_bounds__(256) void act_pairs_to_i8_fragments_kernel(ActMembe
   mem.scales[base0 + 32 + c] = 0u;
   mem.scales[base1 + c]      = a[8] >> 16;
   mem.scales[base1 + 32 + c] = 0u;
-  if (t < 64) {
-    mem.scales[(size_t) m_tiles * nblk * 64 + t] = 0u;  // the row that blocks past the end of K are pointed at
+  if (t < 32) {  // (the row that blocks past the end of K are pointed at; one row tile and one pair are 32 threads)
+    mem.scales[(size_t) m_tiles * nblk * 64 + t]      = 0u;
+    mem.scales[(size_t) m_tiles * nblk * 64 + 32 + t] = 0u;
   }
 }
 
@@ -193,6 +195,7 @@ __global__ __launch_bounds__(256) void act_pairs_to_i8_fragments_kernel(ActMembe
 
 constexpr int kGiThreads = 256;
 constexpr int kGiWaves   = 4;
+constexpr int kMaxParts  = 8;  // workgroups that may share a tile's K
 #ifndef GI_DEPTH_U1
 #define GI_DEPTH_U1 4
 #endif
@@ -220,9 +223,9 @@ struct FragMember {
   int             n, nblk, n_tiles;
   int             ksplit;  // waves that share a tile's K (used by the instantiation that takes it at run time)
   int             share;   // small tiles: which operand the workgroup shares through LDS (kShare*)
-  int             kparts;  // kShareWeights: workgroups that share a tile's K (partial tiles meet in `exchange`)
+  int             kparts;  // workgroups that share a tile's K (partial tiles meet in `exchange`)
   float          *exchange;
-  unsigned       *tickets;  // one zeroed counter per (tile, wave) of this member, left zeroed
+  unsigned       *tickets;  // one zeroed counter per tile of this member, left zeroed
   unsigned        wg_begin;
 };
 struct FragMembers {
@@ -245,6 +248,7 @@ __device__ __forceinline__ const FragMember &member_of_workgroup(const FragMembe
 }
 
 // one workgroup's share of a member; `red`: RedSlots x (UM UN) x 16 x 64 floats of LDS
+// (kGiWaves slots where the member's kparts > 1)
 template <int KSPLIT_T, int UM, int UN>
 __device__ __forceinline__ void fragments_workgroup(const FragMember &mem, int m, int m_tiles, float *red_lds) {
   // fragment sets in flight per wave: small tiles run one wave per SIMD and must cover the memory latency alone
@@ -267,13 +271,16 @@ __device__ __forceinline__ void fragments_workgroup(const FragMember &mem, int m
   // Workgroup ids go round-robin over the 8 XCDs (each with its own L2). All row blocks of one column group are
   // given consecutive slots of ONE XCD, so the weight fragments they share are fetched into that L2 once.
   const int gy = (m_tiles + UM - 1) / UM, gx = (n_tiles + UN * TILES - 1) / (UN * TILES);
-  const int xcd = wg & 7, slot = wg >> 3;
+  const int kparts = UM * UN == 1 && KSPLIT_T == 0 ? mem.kparts : 1;
+  const int xcd = wg & 7, slot = __builtin_amdgcn_readfirstlane((int) (wg >> 3) / kparts), kpart = __builtin_amdgcn_readfirstlane((int) (wg >> 3) % kparts);
   const int by = slot % gy, bx = (slot / gy) * 8 + xcd;
   if (bx >= gx) {
     return;  // whole workgroup (the grid is padded to a multiple of 8 column groups)
   }
   const int mt0 = by * UM, nt0 = (bx * TILES + tw) * UN;
   const bool tile_ok = nt0 < n_tiles;  // mt0 < m_tiles by construction
+  // blocks of this workgroup's part of K: [blk0, blk1)
+  const int  blk0 = __builtin_amdgcn_readfirstlane((int) ((unsigned) (kpart * nblk) / (unsigned) kparts)), blk1 = __builtin_amdgcn_readfirstlane((int) ((unsigned) ((kpart + 1) * nblk) / (unsigned) kparts));
 
   // Operand streams as buffer resources: a load is then resource (scalar) + per-lane offset (a register that never
   // changes) + scalar offset of the block, and costs no vector-ALU instruction.
@@ -298,7 +305,7 @@ __device__ __forceinline__ void fragments_workgroup(const FragMember &mem, int m
   const int lane16 = lane * 16, lane4 = lane * 4, c4 = c * 4;
   auto load = [&](FragSet<UM, UN> &s, int kb_raw) {
     const int  kb   = min(kb_raw, nblk - 1);  // branch-free: blocks past the end repeat the last one ...
-    const bool live = kb_raw < nblk;          // ... with activation scales of zero: they add nothing
+    const bool live = kb_raw < blk1;          // ... with activation scales of zero: they add nothing
 #pragma unroll
     for (int i = 0; i < UM; ++i) {
       s.a[i]  = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ra[i], lane16, kb * 1024, 0));
@@ -326,7 +333,7 @@ __device__ __forceinline__ void fragments_workgroup(const FragMember &mem, int m
   FragSet<UM, UN> ring[kGiDepth];
 #pragma unroll
   for (int d = 0; d < kGiDepth; ++d) {
-    load(ring[d], ks + d * KSPLIT);
+    load(ring[d], blk0 + ks + d * KSPLIT);
   }
   const v16f zf = { 0 };
   const v16i zi = { 0 };
@@ -349,7 +356,7 @@ __device__ __forceinline__ void fragments_workgroup(const FragMember &mem, int m
   // 16 converts and the 16 fmas of the CURRENT one, so neither pipe waits for the other.
   v16i sum_next = mfma_sum(ring[0], 0, 0);
   v16f scl_next = mfma_scale(ring[0], 0, 0);
-  const int steps = (nblk - ks + KSPLIT - 1) / KSPLIT;  // blocks of this wave
+  const int steps = (blk1 - blk0 - ks + KSPLIT - 1) / KSPLIT;  // blocks of this wave
   for (int s0 = 0; s0 < steps; s0 += kGiDepth) {
 #pragma unroll
     for (int d = 0; d < kGiDepth; ++d) {
@@ -380,7 +387,64 @@ __device__ __forceinline__ void fragments_workgroup(const FragMember &mem, int m
         asm volatile("" : "+v"(acc[i][j]));
       }
       // every matrix instruction that reads ring[d] has been issued: fetch the set DEPTH steps ahead
-      load(ring[d], ks + (s0 + d + kGiDepth) * KSPLIT);
+      load(ring[d], blk0 + ks + (s0 + d + kGiDepth) * KSPLIT);
+    }
+  }
+
+  if constexpr (UM * UN == 1 && KSPLIT_T == 0) {
+    if (kparts > 1) {
+      // ---- several workgroups share the tile (KSPLIT = 4: one tile per workgroup): all waves park their sums in LDS, each
+      // adds up (in wave order) and leaves a quarter of this part in `exchange`; the workgroup that comes last adds all
+      // parts in part order and stores. (Order between the parts and the ticket: see shared_operand_workgroup; the barrier
+      // stands between the waves' waits and the ticket.) ----
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        red[wave][0][r][lane] = acc[0][0][r];
+      }
+      __syncthreads();
+      const size_t tile_slot = (size_t) nt0 * m_tiles + mt0;
+      float       *parts     = mem.exchange + tile_slot * kparts * 1024;
+      for (int r = 4 * wave; r < 4 * wave + 4; ++r) {
+        const float v = red[0][0][r][lane] + red[1][0][r][lane] + red[2][0][r][lane] + red[3][0][r][lane];
+        __hip_atomic_store(&parts[kpart * 1024 + r * 64 + lane], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      unsigned *said = reinterpret_cast<unsigned *>(red_lds);
+      if (threadIdx.x == 0) {
+        *said = __hip_atomic_fetch_add(&mem.tickets[tile_slot], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      __syncthreads();
+      if (*said != (unsigned) (kparts - 1)) {
+        return;
+      }
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      const int col = nt0 * 32 + c;
+      float     part[kMaxParts][4];  // (every load requested before the first use: one trip to memory, not one per part)
+#pragma unroll
+      for (int p = 0; p < kMaxParts; ++p) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          part[p][q] = p < kparts ? __hip_atomic_load(&parts[p * 1024 + (4 * wave + q) * 64 + lane], __ATOMIC_RELAXED,
+                                                      __HIP_MEMORY_SCOPE_AGENT) : 0.0f;
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        float v = 0.0f;
+#pragma unroll
+        for (int p = 0; p < kMaxParts; ++p) {
+          v += part[p][q];
+        }
+        const int r = 4 * wave + q, row = mt0 * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
+        if (row < m && col < n) {
+          out[(size_t) row * n + col] = v;
+        }
+      }
+      if (threadIdx.x == 0) {
+        __hip_atomic_store(&mem.tickets[tile_slot], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // ready for the next launch
+      }
+      return;
     }
   }
 
@@ -447,8 +511,7 @@ __global__ __launch_bounds__(kGiThreads) void gemm_i8_fragments_kernel(FragMembe
 constexpr int kShBlocks = 4;                              // blocks per stage
 constexpr int kShStages = 3;
 constexpr int kShStage  = kShBlocks * (1024 + 256);       // fragments, then the scale rows (256 or 128 bytes a block)
-constexpr int kShLds    = kShStages * kShStage > RedSlots<0, 1, 1>::kValue * 16 * 64 * 4 ?
-                              kShStages * kShStage : RedSlots<0, 1, 1>::kValue * 16 * 64 * 4;
+constexpr int kShLds    = kShStages * kShStage > kGiWaves * 16 * 64 * 4 ? kShStages * kShStage : kGiWaves * 16 * 64 * 4;
 enum { kSharePlain = 0, kShareActivations = 1, kShareWeights = 2 };
 
 template <bool SHARE_W>
@@ -619,10 +682,22 @@ __device__ __forceinline__ void shared_operand_workgroup(const FragMember &mem, 
     for (int r = 0; r < 16; ++r) {
       acc[r] = 0.0f;
     }
-    for (int p = 0; p < kparts; ++p) {  // all parts, this wave's own included, in part order
+    for (int p = 0; p < kparts; p += 2) {  // all parts, this wave's own included, in part order; two per trip to memory
+      float x[2][16];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        acc[r] += __hip_atomic_load(&parts[p * 1024 + r * 64 + lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      for (int u = 0; u < 2; ++u) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          x[u][r] = p + u < kparts ? __hip_atomic_load(&parts[(p + u) * 1024 + r * 64 + lane], __ATOMIC_RELAXED,
+                                                       __HIP_MEMORY_SCOPE_AGENT) : 0.0f;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          acc[r] += x[u][r];
+        }
       }
     }
     if (lane == 0) {
@@ -704,7 +779,7 @@ struct TileConfig {
 TileConfig tile_config(int m, int n, int k, int forced_unit) {
   const int m_tiles = (m + 31) / 32, n_tiles = (n + 31) / 32, nblk = k / 32;
   const int wave_tiles  = ((m_tiles + 1) / 2) * ((n_tiles + 1) / 2);
-  const int unit        = forced_unit == 1 || forced_unit == 2 ? forced_unit : (wave_tiles < 512 ? 1 : 2);
+  const int unit        = forced_unit == 1 || forced_unit == 2 ? forced_unit : (m_tiles == 1 || wave_tiles < 512 ? 1 : 2);
   if (unit == 1) {
     return { 1, nblk >= 192 ? 4 : nblk >= 96 ? 2 : 1 };
   }
@@ -716,34 +791,52 @@ TileConfig tile_config(int m, int n, int k, int forced_unit) {
 // the Qwen2-like block at m = 128: these launches want waves more than they want bytes saved.
 constexpr int kSmallUN = 1;
 
-// small tiles: which operand the four waves of a workgroup share (see shared_operand_workgroup) and, with the weights
-// shared, over how many workgroups K is split (`split_k`: the caller has scratch for the partial tiles)
+// small tiles: which operand the four waves of a workgroup share (see shared_operand_workgroup), else how many of them share
+// a tile's K, and over how many workgroups K is split (`split_k`: the caller has scratch for the partial tiles). All of it
+// follows the matrix alone, so that a member of a launch is computed as on its own.
 struct SmallTilePlan {
-  int share, kparts;
+  int share, ksplit, kparts;
 };
-SmallTilePlan small_tile_plan(int m_tiles, int nblk, TileConfig cfg, bool split_k) {
-  if (cfg.unit != 1 || nblk % kShBlocks != 0 || nblk < 2 * kShBlocks) {
-    return { kSharePlain, 1 };
+constexpr int kSmallWgs = 256;  // a launch of fewer workgroups leaves CUs without one
+SmallTilePlan small_tile_plan(int m_tiles, int n_tiles, int nblk, TileConfig cfg, bool split_k) {
+  if (cfg.unit != 1) {
+    return { kSharePlain, cfg.ksplit, 1 };
   }
-  const bool row_groups = m_tiles % kGiWaves == 0;
-  if (cfg.ksplit != 1) {
-    // a wave should walk some 48 blocks (as the plain body's split of K aims at)
-    // (measured on the Qwen2 block at 128 rows, k = 8960: 24 / 32 / 40 / 48 / 64 blocks per part 38.7 / 38.6 / 35.3 / 35.8 / 37.0 us)
-    return row_groups && split_k ? SmallTilePlan{ kShareWeights, std::min(8, nblk / 48) } : SmallTilePlan{ kSharePlain, 1 };
+  const bool staged     = nblk % kShBlocks == 0 && nblk >= 2 * kShBlocks;
+  const bool row_groups = staged && m_tiles % kGiWaves == 0;
+  if (row_groups && (cfg.ksplit == 1 || split_k)) {
+    // Long K: a wave should walk some 48 blocks (as the plain body's split of K aims at; measured on the Qwen2 block at 128
+    // rows, k = 8960: 24 / 32 / 40 / 48 / 64 blocks per part 38.7 / 38.6 / 35.3 / 35.8 / 37.0 us). Where the matrix alone
+    // would leave half of the CUs idle, down to 24 (128 rows, a decoder layer of Qwen2 size: 92.6 -> 90.0 us; down to 12
+    // blocks the same, but 28.9 -> 32.0 us for its seven projections in one launch; at 256 rows, q and o on 96
+    // workgroups, those take 82.5 us unsplit and 85.6 split).
+    int kparts = cfg.ksplit != 1 ? std::min(kMaxParts, nblk / 48) : 1;
+    if (split_k) {
+      kparts = std::max(kparts, std::min({ kMaxParts, kSmallWgs / 2 / (n_tiles * (m_tiles / kGiWaves)), nblk / 24 }));
+    }
+    return { kShareWeights, 1, kparts };
+  }
+  // Other row counts: a matrix that would leave CUs idle gets all four waves of a workgroup, and as many workgroups as
+  // there are CUs for, on a tile's K, down to 12 blocks per wave. fp32 rows (quantized on the way), unsplit with 12 blocks
+  // a wave at least / split: k = 8960, n = 1537, 33 rows 23.7 / 14.3 us; k = n = 4096, 33 rows 20.5 / 14.5. (16 waves of
+  // one workgroup on a tile's K instead, no exchange: 27 rows, k = 8960, n = 1537 14.2 against 11.9 us.)
+  const int wgs = m_tiles * ((n_tiles + kGiWaves / cfg.ksplit - 1) / (kGiWaves / cfg.ksplit));
+  if (split_k && wgs < kSmallWgs && nblk >= 2 * kGiWaves) {
+    return { kSharePlain, kGiWaves, std::max(1, std::min({ kMaxParts, kSmallWgs / (m_tiles * n_tiles), nblk / (kGiWaves * 12) })) };
   }
   // (measured on the Qwen2 block at 128 rows: weights shared 39.6 us, activations shared 40.2 us, neither 43.9 us)
-  return { row_groups ? kShareWeights : kShareActivations, 1 };
+  return { staged && cfg.ksplit == 1 ? kShareActivations : kSharePlain, cfg.ksplit, 1 };
 }
 
 unsigned member_workgroups(int m_tiles, int n_tiles, TileConfig cfg, SmallTilePlan plan) {
   if (plan.share == kShareWeights) {
     return (unsigned) ((n_tiles + 7) / 8 * 8 * (m_tiles / kGiWaves) * plan.kparts);
   }
-  const unsigned tiles_per_wg = kGiWaves / cfg.ksplit;
+  const unsigned tiles_per_wg = kGiWaves / plan.ksplit;
   const unsigned un = cfg.unit == 1 ? kSmallUN : cfg.unit;
   const unsigned gy = (unsigned) ((m_tiles + cfg.unit - 1) / cfg.unit);
   const unsigned gx = (unsigned) ((n_tiles + un * tiles_per_wg - 1) / (un * tiles_per_wg));
-  return (gx + 7) / 8 * 8 * gy;
+  return (gx + 7) / 8 * 8 * gy * plan.kparts;
 }
 
 const uint32_t *scales_of(const void *fragments, size_t tiles, size_t nblk) {
@@ -795,7 +888,7 @@ hipError_t launch_act_to_i8_fragments_group(hipStream_t stream, int count, void 
 
 size_t gemm_i8_fragments_exchange_bytes(int m, int n, int k, int forced_unit) {
   const int           m_tiles = (m + 31) / 32, n_tiles = (n + 31) / 32, nblk = k / 32;
-  const SmallTilePlan plan    = small_tile_plan(m_tiles, nblk, tile_config(m, n, k, forced_unit), true);
+  const SmallTilePlan plan    = small_tile_plan(m_tiles, n_tiles, nblk, tile_config(m, n, k, forced_unit), true);
   return plan.kparts > 1 ? (size_t) ((n_tiles + 7) / 8 * 8) * m_tiles * plan.kparts * 1024 * sizeof(float) : 0;
 }
 
@@ -811,7 +904,7 @@ hipError_t launch_gemm_i8_fragments_group(hipStream_t stream, int count, float *
   const int   m_tiles = (m + 31) / 32;
   FragMembers grp;
   unsigned    total = 0;
-  TileConfig  cfg   = { 0, 0 };
+  TileConfig  cfg   = {};
   // Workgroups start in block order: the members whose waves have the most blocks to walk go first, so that the launch
   // ends on short waves (members are independent of each other, their order is free).
   int order[kGemmGroupMax];
@@ -839,15 +932,15 @@ hipError_t launch_gemm_i8_fragments_group(hipStream_t stream, int count, float *
     grp.m[slot].n        = ns[i];
     grp.m[slot].nblk     = nblk;
     grp.m[slot].n_tiles  = n_tiles;
-    grp.m[slot].ksplit   = c.ksplit;
     grp.m[slot].wg_begin = total;
     // K split over workgroups while the caller's scratch for partial tiles and its ticket counters last
     const size_t  xbytes  = gemm_i8_fragments_exchange_bytes(m, ns[i], ks[i], forced_unit);
     const int     xslots  = (n_tiles + 7) / 8 * 8 * m_tiles;
-    const bool    split_k = exchange && tickets && xbytes > 0 && exchange_used + xbytes <= exchange_bytes &&
-                         tickets_used + xslots <= ticket_slots;
-    SmallTilePlan plan    = small_tile_plan(m_tiles, nblk, c, split_k);
+    const bool    split_k = xbytes == 0 || (exchange && tickets && exchange_used + xbytes <= exchange_bytes &&
+                                            tickets_used + xslots <= ticket_slots);
+    SmallTilePlan plan    = small_tile_plan(m_tiles, n_tiles, nblk, c, split_k);
     grp.m[slot].share    = plan.share;
+    grp.m[slot].ksplit   = plan.ksplit;
     grp.m[slot].kparts   = plan.kparts;
     grp.m[slot].exchange = nullptr;
     grp.m[slot].tickets  = nullptr;

@@ -103,9 +103,12 @@ int run_fragment_group(htpops_context *ctx, GemvBatch &b) {
   for (int i = 0; i < b.count; ++i) {
     xbytes += gemm_i8_fragments_exchange_bytes(b.m, b.n[i], b.k[i], ctx->opt.gemm_tile_units);
   }
-  if (int r = ensure_workspace(ctx, total + xbytes)) {
+  if (int r = ensure_workspace(ctx, total + xbytes, true)) {
     return r;
   }
+  // (the first matrix may lie there already, left by its quantizer or by an earlier matmul over the same rows)
+  const auto &noted = ctx->act_fragments;
+  const int   ready = noted.src == acts[0] && noted.m == b.m && noted.k == act_k[0] && noted.kind == (int) kPlanFragments ? 1 : 0;
   ctx->act_fragments.src = nullptr;
   uint8_t    *ws = static_cast<uint8_t *>(ctx->workspace);
   void       *act_dst[kGemmGroupMax];
@@ -116,7 +119,9 @@ int run_fragment_group(htpops_context *ctx, GemvBatch &b) {
   for (int i = 0; i < b.count; ++i) {
     af[i] = act_dst[act_of[i]];
   }
-  HTPOPS_HIP(ctx, launch_act_to_i8_fragments_group(ctx->stream, n_acts, act_dst, acts, act_k, b.m));
+  if (n_acts > ready) {
+    HTPOPS_HIP(ctx, launch_act_to_i8_fragments_group(ctx->stream, n_acts - ready, act_dst + ready, acts + ready, act_k + ready, b.m));
+  }
   HTPOPS_HIP(ctx, launch_gemm_i8_fragments_group(ctx->stream, b.count, b.out, af, wf, b.n, b.k, b.m, ws + total, xbytes,
                                                  ctx->tickets, kTicketSlots, ctx->opt.gemm_tile_units));
   return HTPOPS_OK;
@@ -467,6 +472,36 @@ bool try_batch_permuted(htpops_context *ctx, const struct OpComputeRequest *req,
   return true;
 }
 
+// What `next` behind a quantizing request `req` (op 13 or 14) needs of the workspace if it is a matmul over exactly the rows
+// that one writes and takes the int8 fragment kernels (see htpops_context::next_fragments_ws); else 0.
+size_t fragments_of_next(htpops_context *ctx, const struct OpComputeRequest *req, const struct RequestHeader *next, size_t size) {
+  if (next->type != REQUEST_TYPE_OP_COMPUTE ||
+      size < sizeof(struct RequestHeader) + sizeof(struct OpComputeRequest) + sizeof(MatMulParams)) {
+    return 0;
+  }
+  const auto *mm = reinterpret_cast<const struct OpComputeRequest *>(next->data);
+  if (!ctx->has_device || (mm->op != HTP_OPS_MAT_MUL_Q4_0_Q8_0 && mm->op != HTP_OPS_MAT_MUL_Q8_0_Q8_0)) {
+    return 0;
+  }
+  const bool  normalize = req->op == HTP_OPS_RMS_NORM_QUANTIZE_Q8_0;
+  const auto *pn = reinterpret_cast<const RmsNormExParams *>(req->payload);
+  const auto *pq = reinterpret_cast<const RmsNormF32Params *>(req->payload);
+  const auto *p  = reinterpret_cast<const MatMulParams *>(mm->payload);
+  const int   wt = mm->op == HTP_OPS_MAT_MUL_Q4_0_Q8_0 ? kQ4_0 : kQ8_0;
+  if (p->m < kManyRowsMinM || p->n <= 0 || p->k <= 0 || p->k % 32 != 0 || p->k != (normalize ? pn->ne0 : pq->ne0) ||
+      p->m != (normalize ? pn->ne1 : pq->ne1)) {
+    return 0;
+  }
+  const size_t bytes = q8_0_bytes((size_t) p->m, (size_t) p->k);
+  const void  *act   = resolve(ctx, p->activation, bytes);
+  const void  *w     = resolve(ctx, p->weight, weight_bytes((size_t) p->n, (size_t) p->k, wt));
+  if (!act || !w || act != resolve(ctx, normalize ? pn->dst : pq->dst, bytes)) {
+    return 0;
+  }
+  const MatMulPlan plan = plan_mat_mul(ctx, w, aligned(act, 4), p->m, p->k, p->n, wt);
+  return plan.kind == kPlanFragments ? plan.ws_bytes : 0;
+}
+
 // `next` behind a one-token fp32 attention request `req`: if it is the Q8_0 quantization of exactly that attention's
 // output row into a buffer that overlaps none of the attention's operands, notes where it wants the row
 // (ctx->attn_q8_out) and returns it; nullptr otherwise.
@@ -619,9 +654,14 @@ int enqueue_message(htpops_context *ctx, struct MessageHeader *msg, size_t msg_b
               next = attention_output_quantizer(ctx, req, message_header_get_request_ptr(msg, i + 1),
                                                 message_header_get_request_size(msg, i + 1));
             }
+            if (norm_payload && i + 1 < n_reqs) {
+              ctx->next_fragments_ws = fragments_of_next(ctx, req, message_header_get_request_ptr(msg, i + 1),
+                                                         message_header_get_request_size(msg, i + 1));
+            }
             ctx->attn_q8_done = false;
             hdr->state        = htpops_execute_op(ctx, req);
             ctx->attn_q8_out  = nullptr;
+            ctx->next_fragments_ws = 0;
             if (next && ctx->attn_q8_done && hdr->state == HTPOPS_OK) {
               next->state = HTPOPS_OK;
               ++i;  // (the row is written: that request needs no launch)

@@ -26,6 +26,30 @@ int op_rms_norm(htpops_context *ctx, float *dst, const float *src, const float *
   return HTPOPS_OK;
 }
 
+namespace {
+
+// where a quantizer of m rows of k leaves them in operand order as well (nullptr: nobody asked)
+int wanted_fragments(htpops_context *ctx, int m, int k, void **where) {
+  *where = nullptr;
+  if (ctx->next_fragments_ws == 0 || (long long) m * (k / 32) > 0x7fffffffLL) {
+    return HTPOPS_OK;
+  }
+  if (int r = ensure_workspace(ctx, ctx->next_fragments_ws)) {
+    return r;
+  }
+  *where = ctx->workspace;
+  return HTPOPS_OK;
+}
+
+void note_fragments(htpops_context *ctx, const void *where, const void *rows, int m, int k) {
+  if (where) {
+    auto &af = ctx->act_fragments;
+    af.src = rows, af.src_bytes = q8_0_bytes((size_t) m, (size_t) k), af.m = m, af.k = k, af.kind = (int) kPlanFragments;
+  }
+}
+
+}  // namespace
+
 int op_quantize(htpops_context *ctx, void *dst, const float *src, int k, int m) {
   if (!dst || !src || k <= 0 || m <= 0 || k % 32 != 0) {
     return fail(ctx, HTPOPS_ERR_REJECTED, "quantize_q8_0: null buffer or bad size (k=%d m=%d, k %% 32 must be 0)", k, m);
@@ -36,8 +60,13 @@ int op_quantize(htpops_context *ctx, void *dst, const float *src, int k, int m) 
   if (int r = need_device(ctx)) {
     return r;
   }
+  void *frags = nullptr;
+  if (int r = wanted_fragments(ctx, m, k, &frags)) {
+    return r;
+  }
   note_device_write(ctx, dst, q8_0_bytes((size_t) m, (size_t) k));
-  HTPOPS_HIP(ctx, launch_quantize_q8_0(ctx->stream, dst, src, k, m));
+  HTPOPS_HIP(ctx, launch_quantize_q8_0(ctx->stream, dst, src, k, m, frags));
+  note_fragments(ctx, frags, dst, m, k);
   return HTPOPS_OK;
 }
 
@@ -53,8 +82,13 @@ int op_rms_norm_quantize(htpops_context *ctx, void *dst, const float *src, const
     return r;
   }
   if (ne0 <= 16384) {
+    void *frags = nullptr;
+    if (int r = wanted_fragments(ctx, ne1, ne0, &frags)) {
+      return r;
+    }
     note_device_write(ctx, dst, q8_0_bytes((size_t) ne1, (size_t) ne0));
-    HTPOPS_HIP(ctx, launch_rms_norm_quantize_q8_0(ctx->stream, dst, src, weight, eps, ne0, ne1));
+    HTPOPS_HIP(ctx, launch_rms_norm_quantize_q8_0(ctx->stream, dst, src, weight, eps, ne0, ne1, frags));
+    note_fragments(ctx, frags, dst, ne1, ne0);
     return HTPOPS_OK;
   }
   // very long rows: normalize into the workspace, then quantize
@@ -148,7 +182,7 @@ MatMulPlan plan_mat_mul(htpops_context *ctx, const void *weight, bool act_aligne
   // (htpops_buffer_prepare_weights) may change behind the context's back, so nothing converted from it is kept, and
   // the FP6 conversion is too slow to redo per call.
   const int use_fp6 = ctx->opt.gemm_fp6;
-  if (wt == kQ4_0 && use_fp6 != 0 && gemm_fp6_lds_fits(m, k, n) && aligned(weight, 4) && act_aligned &&
+  if (m >= kFp6MinM && wt == kQ4_0 && use_fp6 != 0 && gemm_fp6_lds_fits(m, k, n) && aligned(weight, 4) && act_aligned &&
       (use_fp6 > 0 || gemm_fp6_lds_fills_device(m, n))) {
     lookup_copy(kFragKindFp6Tiles + wt);
     if (p.cached || p.cacheable) {
@@ -156,6 +190,17 @@ MatMulPlan plan_mat_mul(htpops_context *ctx, const void *weight, bool act_aligne
       p.act_bytes    = (gemm_fp6_lds_act_tile_bytes(m, k) + 255) & ~(size_t) 255;
       p.weight_bytes = gemm_fp6_lds_weight_tile_bytes(k, n);
       p.ws_bytes     = p.act_bytes;
+      return p;
+    }
+  }
+  // Up to 32 rows only over a copy that is kept: the kernels that read the weights as they are beat a conversion per call.
+  // 17 to 32 rows, K-sliced kernel / here: seven projections of a Llama-7B / Qwen2-1.5B layer, Q8_0, 117 and 65 us in seven
+  // launches / 47 and 19 us; one matrix over fp32 rows, k = 8960, n = 1537 13.2 / 11.9, k = 4096, n = 11008 27.5 / 17.0,
+  // but k = 1024, n = 700 8.4 / 9.6.
+  if (m < kFp6MinM) {
+    lookup_copy(kFragKindRowLayout + wt);
+    if (!p.cached && !p.cacheable) {
+      p.ws_bytes = mat_mul_workspace_bytes(m, k, n);
       return p;
     }
   }
@@ -234,7 +279,8 @@ int run_few_rows(htpops_context *ctx, float *dst, const void *act, const void *w
   return HTPOPS_OK;
 }
 
-// `ws` is this matmul's share of the workspace (plan.ws_bytes, already ensured by the caller)
+// `ws` is this matmul's share of the workspace (plan.ws_bytes, already ensured by the caller). act = nullptr (int8 fragments
+// only): the activations lie at its start in operand order already.
 int run_mat_mul(htpops_context *ctx, MatMulPlan &plan, float *dst, const void *act, const void *weight, int m, int k,
                 int n, int wt, uint8_t *ws) {
   note_device_write(ctx, dst, (size_t) m * n * 4);
@@ -260,9 +306,9 @@ int run_mat_mul(htpops_context *ctx, MatMulPlan &plan, float *dst, const void *a
   // rows with the same kernel family (note_device_write above has already cleared the record if this matmul writes
   // into its own activations).
   auto      &af    = ctx->act_fragments;
-  const bool ready = af.src == act && af.m == m && af.k == k && af.kind == (int) plan.kind && ws == ctx->workspace;
-  const bool keep  = ready || (ctx->in_message && ws == ctx->workspace &&
-                               !ranges_overlap(dst, (size_t) m * n * 4, act, q8_0_bytes((size_t) m, (size_t) k)));
+  const bool ready = !act || (af.src == act && af.m == m && af.k == k && af.kind == (int) plan.kind && ws == ctx->workspace);
+  const bool keep  = act && (ready || (ctx->in_message && ws == ctx->workspace &&
+                               !ranges_overlap(dst, (size_t) m * n * 4, act, q8_0_bytes((size_t) m, (size_t) k))));
   af.src = nullptr;
   if (plan.kind == kPlanLdsFp6) {
     HTPOPS_HIP(ctx, launch_gemm_fp6_lds(ctx->stream, dst, act, frags, m, k, n, ws, ready));
@@ -307,9 +353,18 @@ int op_mat_mul_f32(htpops_context *ctx, float *dst, const float *act, const void
   if (int r = need_device(ctx)) {
     return r;
   }
+  MatMulPlan plan = plan_mat_mul(ctx, weight, true, m, k, n, weight_type);
+  if (plan.kind == kPlanFragments && (long long) m * (k / 32) <= 0x7fffffffLL) {
+    // the quantizer writes the operand order the matmul wants: the rows in block_q8_0 form would have one reader, another
+    // launch that puts them into that order (33 rows, k = 8960, n = 1537: 3 of 18 us)
+    if (int r = ensure_workspace(ctx, plan.ws_bytes)) {
+      return r;
+    }
+    HTPOPS_HIP(ctx, launch_quantize_q8_0(ctx->stream, nullptr, act, k, m, ctx->workspace));
+    return run_mat_mul(ctx, plan, dst, nullptr, weight, m, k, n, weight_type, static_cast<uint8_t *>(ctx->workspace));
+  }
   // workspace: [quantized activations][what the matmul itself needs]
   const size_t q_bytes = (q8_0_bytes((size_t) m, (size_t) k) + 255) & ~(size_t) 255;
-  MatMulPlan   plan    = plan_mat_mul(ctx, weight, true, m, k, n, weight_type);
   if (int r = ensure_workspace(ctx, q_bytes + plan.ws_bytes)) {
     return r;
   }

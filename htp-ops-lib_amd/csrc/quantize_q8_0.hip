@@ -21,9 +21,11 @@ constexpr int kWaveOutBytes   = kBlocksPerWave * 34;       // 544
 constexpr int kWaveOutDwords  = kWaveOutBytes / 4;         // 136
 
 // total_blocks = m * k / 32; blocks are contiguous in both src (128 B each) and dst (34 B each).
+// FRAGMENTS: the quants also go to `fragments` (see ActFragments), and dst may be nullptr.
+template <bool FRAGMENTS>
 __global__ __launch_bounds__(kThreads) void quantize_q8_0_kernel(uint8_t *__restrict__ dst,
                                                                   const float *__restrict__ src,
-                                                                  long long total_blocks) {
+                                                                  long long total_blocks, ActFragments fragments) {
   __shared__ __attribute__((aligned(16))) uint16_t stage[kThreads / kWave][kWaveOutBytes / 2];
 
   const int       lane       = threadIdx.x & (kWave - 1);
@@ -66,6 +68,21 @@ __global__ __launch_bounds__(kThreads) void quantize_q8_0_kernel(uint8_t *__rest
     q[i] = (int) roundf(x[i] * id);
   }
 
+  if constexpr (FRAGMENTS) {
+    if (live) {
+      const unsigned b = (unsigned) block, nblk = (unsigned) fragments.nblk;  // (the launcher sees to the range)
+      const uint2    packed = { (uint32_t) ((q[0] & 0xff) | ((q[1] & 0xff) << 8) | ((q[2] & 0xff) << 16) | ((uint32_t) q[3] << 24)),
+                                (uint32_t) ((q[4] & 0xff) | ((q[5] & 0xff) << 8) | ((q[6] & 0xff) << 16) | ((uint32_t) q[7] << 24)) };
+      store_act_fragment(fragments, (int) (b / nblk), (int) (b % nblk), part, packed, __half_as_ushort(__float2half_rn(d)));
+    }
+    if (blockIdx.x == 0 && threadIdx.x < kWave) {
+      end_act_fragments(fragments, threadIdx.x);
+    }
+    if (dst == nullptr) {
+      return;
+    }
+  }
+
   // LDS image of this wave's 16 blocks: block b at byte 34 b; its quants start at 34 b + 2 + 8 part.
   uint16_t *img  = stage[wave];
   const int base = ((lane >> 2) * 34 + 2 + part * 8) / 2;  // in uint16 units
@@ -98,11 +115,19 @@ __global__ __launch_bounds__(kThreads) void quantize_q8_0_kernel(uint8_t *__rest
 
 }  // namespace
 
-hipError_t launch_quantize_q8_0(hipStream_t stream, void *dst, const float *src, int k, int m) {
+hipError_t launch_quantize_q8_0(hipStream_t stream, void *dst, const float *src, int k, int m, void *act_fragments) {
   const long long total_blocks = (long long) m * (k / kQK);
   const long long groups       = (total_blocks + kBlocksPerGroup - 1) / kBlocksPerGroup;
-  hipLaunchKernelGGL(quantize_q8_0_kernel, dim3((unsigned) groups), dim3(kThreads), 0, stream, (uint8_t *) dst, src,
-                     total_blocks);
+  if (act_fragments) {
+    if (total_blocks > 0x7fffffffLL) {
+      return hipErrorInvalidValue;
+    }
+    hipLaunchKernelGGL(quantize_q8_0_kernel<true>, dim3((unsigned) groups), dim3(kThreads), 0, stream, (uint8_t *) dst, src,
+                       total_blocks, act_fragments_at(act_fragments, m, k));
+  } else {
+    hipLaunchKernelGGL(quantize_q8_0_kernel<false>, dim3((unsigned) groups), dim3(kThreads), 0, stream, (uint8_t *) dst, src,
+                       total_blocks, ActFragments());
+  }
   return hipGetLastError();
 }
 

@@ -130,11 +130,12 @@ __global__ __launch_bounds__(kThreads) void rms_norm_generic_kernel(float *__res
 
 // Fused RMSNorm -> Q8_0. Four neighbouring lanes hold one quant block (8 floats each) and exchange amax inside the
 // quad; BPT slices per thread in registers (rows up to kThreads * 8 * BPT floats). Needs ne0 % 32 == 0.
-template <int BPT>
+// FRAGMENTS: the quants also go to `fragments` (see ActFragments).
+template <int BPT, bool FRAGMENTS>
 __global__ __launch_bounds__(kThreads) void rms_norm_quantize_kernel(uint8_t *__restrict__ dst,
                                                                      const float *__restrict__ src,
                                                                      const float *__restrict__ weight, float eps,
-                                                                     int ne0) {
+                                                                     int ne0, ActFragments fragments) {
   __shared__ float lds[kWaves];
   const size_t row = blockIdx.x;
   const int    nb  = ne0 / kQK;
@@ -203,15 +204,27 @@ __global__ __launch_bounds__(kThreads) void rms_norm_quantize_kernel(uint8_t *__
     const float d  = amax / 127.0f;
     const float id = (d != 0.0f) ? 1.0f / d : 0.0f;
     if (blk < nb) {
-      uint16_t *o16 = reinterpret_cast<uint16_t *>(out + (size_t) blk * 34);
+      uint16_t      *o16  = reinterpret_cast<uint16_t *>(out + (size_t) blk * 34);
+      const uint16_t bits = __half_as_ushort(__float2half_rn(d));
       if (part == 0) {
-        o16[0] = __half_as_ushort(__float2half_rn(d));
+        o16[0] = bits;
       }
+      uint32_t packed[2];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int q0 = (int) roundf(y[2 * i] * id), q1 = (int) roundf(y[2 * i + 1] * id);
-        o16[1 + part * 4 + i] = (uint16_t) ((q0 & 0xff) | ((q1 & 0xff) << 8));
+        const uint32_t two = (uint32_t) ((q0 & 0xff) | ((q1 & 0xff) << 8));
+        o16[1 + part * 4 + i] = (uint16_t) two;
+        packed[i / 2]         = i % 2 == 0 ? two : packed[i / 2] | (two << 16);
       }
+      if constexpr (FRAGMENTS) {
+        store_act_fragment(fragments, (int) row, blk, part, make_uint2(packed[0], packed[1]), bits);
+      }
+    }
+  }
+  if constexpr (FRAGMENTS) {
+    if (blockIdx.x == 0) {
+      end_act_fragments(fragments, threadIdx.x);
     }
   }
 }
@@ -242,21 +255,29 @@ hipError_t launch_rms_norm_f32(hipStream_t stream, float *dst, const float *src,
 }
 
 hipError_t launch_rms_norm_quantize_q8_0(hipStream_t stream, void *dst, const float *src, const float *weight,
-                                         float eps, int ne0, int ne1) {
-  const int nb = ne0 / kQK;
-  dim3      grid((unsigned) ne1), block(kThreads);
-  uint8_t  *out = (uint8_t *) dst;
+                                         float eps, int ne0, int ne1, void *act_fragments) {
+  const int          nb = ne0 / kQK;
+  const dim3         grid((unsigned) ne1), block(kThreads);
+  uint8_t           *out = (uint8_t *) dst;
+  const ActFragments fr  = act_fragments_at(act_fragments, ne1, ne0);
+#define HTPOPS_RMSQ(BPT)                                                                                              \
+  if (act_fragments) {                                                                                                \
+    hipLaunchKernelGGL((rms_norm_quantize_kernel<BPT, true>), grid, block, 0, stream, out, src, weight, eps, ne0, fr); \
+  } else {                                                                                                            \
+    hipLaunchKernelGGL((rms_norm_quantize_kernel<BPT, false>), grid, block, 0, stream, out, src, weight, eps, ne0, fr); \
+  }
   if (nb <= (kThreads / 4) * 1) {
-    hipLaunchKernelGGL(rms_norm_quantize_kernel<1>, grid, block, 0, stream, out, src, weight, eps, ne0);
+    HTPOPS_RMSQ(1);
   } else if (nb <= (kThreads / 4) * 2) {
-    hipLaunchKernelGGL(rms_norm_quantize_kernel<2>, grid, block, 0, stream, out, src, weight, eps, ne0);
+    HTPOPS_RMSQ(2);
   } else if (nb <= (kThreads / 4) * 4) {
-    hipLaunchKernelGGL(rms_norm_quantize_kernel<4>, grid, block, 0, stream, out, src, weight, eps, ne0);
+    HTPOPS_RMSQ(4);
   } else if (nb <= (kThreads / 4) * 8) {
-    hipLaunchKernelGGL(rms_norm_quantize_kernel<8>, grid, block, 0, stream, out, src, weight, eps, ne0);
+    HTPOPS_RMSQ(8);
   } else {
     return hipErrorInvalidValue;  // rows longer than 16384: the C-ABI layer runs the two ops separately
   }
+#undef HTPOPS_RMSQ
   return hipGetLastError();
 }
 

@@ -103,7 +103,7 @@ int htpops_buffer_invalidate(htpops_context *ctx, int handle);
 
 /* Makes, now, the converted copy of the weight matrix [n][k/32] (weight_type GGML_TYPE_Q4_0 or GGML_TYPE_Q8_0) at
  * `offset` of the buffer that matmuls over `m_hint` activation rows will use (none at m_hint = 1; operand-order nibbles
- * for 2..16 rows; FP6 tiles or int8 fragments from 33 rows), so that the first matmul does not pay for the conversion
+ * for 2..16 rows; int8 fragments from 17 rows, or FP6 tiles from 33), so that the first matmul does not pay for the conversion
  * and its hipMalloc. The reference maps weights once and treats them as immutable (src/dsp/op_executor.cc:124-130);
  * this call states the same for the buffer: it is the opt-in that puts CALLER-REGISTERED memory under the contract of
  * the context's own buffers -- converted copies of its weights are kept from now on (also those that later matmuls at

@@ -1,0 +1,56 @@
+"""GPU parity of the int8 fragment matmuls whose K is dealt to several waves and workgroups (17 rows and more, matrices too
+small to fill the chip): against the oracle at the edges of the split, and grouped in a message against one request each."""
+import numpy as np
+import pytest
+
+from pyhtpops import api
+from pyhtpops import workloads as wl
+from test_gpu_parity_core import check_mat_mul
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = api.Context(device=0)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("wt", [wl.GGML_TYPE_Q4_0, wl.GGML_TYPE_Q8_0])
+@pytest.mark.parametrize("m,k,n", [
+    (17, 64, 32), (20, 224, 40), (32, 256, 33),        # below, just below and at eight blocks; one pair of blocks
+    (18, 1536, 100), (33, 1568, 70), (31, 3104, 17),   # 12 blocks a wave and one more; an odd number of blocks
+    (65, 8960, 65), (40, 12320, 32),                   # five and eight workgroups per tile
+    (128, 768, 64), (128, 1600, 96), (256, 8960, 33)]) # whole groups of four row tiles: one, two and five parts
+def test_split_k_at_the_edges(ctx, oracle, wt, m, k, n):
+    # the tolerance is `check_mat_mul`'s: exact block sums, fp32 over the blocks in another order
+    rng = wl.rng_for(59, m * 131 + k + n + wt)
+    first, x, w = check_mat_mul(ctx, oracle, rng, m, k, n, wt)
+    again = ctx.run_mat_mul(oracle.quantize_q8_0(x), w, m, k, n, wt)
+    assert np.array_equal(first, again)
+
+
+@pytest.mark.parametrize("m", [17, 50, 128])
+def test_grouped_split_k_equals_single_requests(ctx, oracle, m):
+    rng = wl.rng_for(60, m)
+    wt, op = wl.GGML_TYPE_Q8_0, api.HTP_OPS_MAT_MUL_Q8_0_Q8_0
+    shapes = [(96, 1536), (256, 1536), (64, 8960), (40, 256), (1000, 1536)]
+    acts = {k: ctx.upload(oracle.quantize_q8_0(wl.make_activations(rng, m, k))) for k in (1536, 8960, 256)}
+    ws = [ctx.upload(wl.make_weights(rng, n, k, wt)) for n, k in shapes]
+    results = []
+    for grouped in (True, False):
+        outs = [ctx.upload(np.zeros(m * n, np.float32)) for n, _ in shapes]
+        reqs = [(api.REQUEST_TYPE_OP_COMPUTE, api.op_compute_request(op, api.mat_mul_params((outs[j], 0), (acts[k], 0), (ws[j], 0), m, k, n)))
+                for j, (n, k) in enumerate(shapes)]
+        for msg in ([api.build_message(reqs)] if grouped else [api.build_message([r]) for r in reqs]):
+            assert ctx.process_message(msg) == 0 and not any(api.message_request_states(msg)), ctx.last_error()
+        if grouped:
+            assert ctx.last_message_submissions() == 1
+        results.append([ctx.read(h, np.uint8, ctx.size(h)) for h in outs])
+        for h in outs:
+            ctx.release(h)
+    for a, b in zip(*results):
+        assert np.array_equal(a, b) and a.any()
+    for h in list(acts.values()) + ws:
+        ctx.release(h)
