@@ -69,7 +69,7 @@ constexpr int kBK        = 64;  // keys per KV block
 // DP % 64 == 0 the pieces are exclusive-or'ed with low bits of the row number (K: key % 8; V: 2 (key % 4), which keeps
 // 32-byte pieces whole for the transposing reads), else K rows are one piece longer (an odd number of them) and V rows,
 // an odd multiple of 64 bytes, lie right as they are.
-template <int DP>
+template <int DP, bool MASK>
 struct PrefillSmem {
   static constexpr bool kXor     = DP % 64 == 0;
   static constexpr int  kKPieces = kXor ? DP / 8 : DP / 8 + 1;  // 16-byte pieces of a K row, of a V row
@@ -77,7 +77,7 @@ struct PrefillSmem {
   uint8_t k[2][kBK * kKPieces * 16];
   uint8_t v[2][kBK * kVPieces * 16];
   // each wave's mask values of the next block ([query][64 keys] halfs, the pieces of a row exclusive-or'ed with query % 8)
-  uint8_t mask[kPfThreads / kWave][kBQ * kBK * 2];
+  uint8_t mask[MASK ? kPfThreads / kWave : 1][MASK ? kBQ * kBK * 2 : 16];
 };
 
 // Floats of one 32-query tile of one head in the split-KV partials, for `units` = 4 * 32-column tiles of O^T: the
@@ -89,14 +89,15 @@ __host__ __device__ constexpr size_t prefill_partial_floats(int units) {
 // FULL: head_dim == DP (64 or 128); else head_dim is any multiple of 16 in (DP - 32, DP], and the probabilities keep
 // 22 bits (an fp16 pair, two matrix instructions per fragment of V): the plain kernel that these head dims took before
 // held them in fp32. GROUPS = 1 or 2 key groups per workgroup (4 waves each); with 2 they take alternate KV blocks of the
-// same queries. With gridDim.z > 1 the blocks of a workgroup's queries are dealt to gridDim.z workgroups, each of which
-// leaves its (max, sum, O) in `part` for flash_attn_prefill_merge_kernel.
-template <int DP, bool FULL, bool QO_F32, int GROUPS>
+// same queries. MASK: there is one (a kernel of its own: the tests for it cost 2048 x 2048 without one 1 to 2 %). With
+// gridDim.z > 1 the blocks of a workgroup's queries are dealt to gridDim.z workgroups, each of which leaves its
+// (max, sum, O) in `part` for flash_attn_prefill_merge_kernel.
+template <int DP, bool FULL, bool QO_F32, int GROUPS, bool MASK>
 __global__ __launch_bounds__(kPfThreads *GROUPS, DP <= 128 ? 2 : 1) void flash_attn_prefill_kernel(
   void *__restrict__ o_ptr, const void *__restrict__ q_ptr, const _Float16 *__restrict__ k_ptr,
   const _Float16 *__restrict__ v_ptr, const _Float16 *__restrict__ mask, int qo_len, int kv_len, int n_heads,
   int n_kv_heads, int head_dim, int flags, float *__restrict__ part) {
-  using Smem = PrefillSmem<DP>;
+  using Smem = PrefillSmem<DP, MASK>;
   const bool causal = (flags & 1) != 0, mask_threshold = (flags & 2) != 0;
   __shared__ __align__(1024) Smem sm_all[GROUPS];
   constexpr int KSTEPS = DP / 16;  // MFMA k-steps over the head dimension
@@ -309,7 +310,7 @@ __global__ __launch_bounds__(kPfThreads *GROUPS, DP <= 128 ? 2 : 1) void flash_a
   }
   typedef short v4s __attribute__((ext_vector_type(4)));
 
-  const bool use_mask = mask != nullptr && wave_on;
+  const bool use_mask = MASK && wave_on;
   uint2      mreg[2][4];  // this lane's 2 x 16 mask values: keys 32 kt + 8 rg + 4 half + 0 .. 3
   if (k_lo + grp * kBK < k_hi) {
     fetch(k_lo + grp * kBK, 0);
@@ -1176,15 +1177,20 @@ hipError_t launch_prefill(hipStream_t stream, void *o, const void *q, const void
   const unsigned all = wgs * splits;
   const bool     two = kMaxGroups == 2 && (forced ? forced == 2 : (all <= kCus || (causal && all <= 2 * kCus)));
   const int      flags = (causal ? 1 : 0) | (mask_threshold ? 2 : 0);
-  if (two) {
-    hipLaunchKernelGGL((flash_attn_prefill_kernel<DP, FULL, QO_F32, kMaxGroups>), grid, dim3(kPfThreads * kMaxGroups), 0, stream,
-                       o, q, (const _Float16 *) k, (const _Float16 *) v, (const _Float16 *) mask, qo_len, kv_len, n_heads,
-                       n_kv_heads, head_dim, flags, scratch);
+#define HTPOPS_LAUNCH(GROUPS, MASK)                                                                                   \
+  hipLaunchKernelGGL((flash_attn_prefill_kernel<DP, FULL, QO_F32, GROUPS, MASK>), grid, dim3(kPfThreads * GROUPS), 0, stream, o, \
+                     q, (const _Float16 *) k, (const _Float16 *) v, (const _Float16 *) mask, qo_len, kv_len, n_heads, \
+                     n_kv_heads, head_dim, flags, scratch)
+  if (two && mask) {
+    HTPOPS_LAUNCH(kMaxGroups, true);
+  } else if (two) {
+    HTPOPS_LAUNCH(kMaxGroups, false);
+  } else if (mask) {
+    HTPOPS_LAUNCH(1, true);
   } else {
-    hipLaunchKernelGGL((flash_attn_prefill_kernel<DP, FULL, QO_F32, 1>), grid, dim3(kPfThreads), 0, stream, o, q,
-                       (const _Float16 *) k, (const _Float16 *) v, (const _Float16 *) mask, qo_len, kv_len, n_heads,
-                       n_kv_heads, head_dim, flags, scratch);
+    HTPOPS_LAUNCH(1, false);
   }
+#undef HTPOPS_LAUNCH
   if (hipError_t e = hipGetLastError(); e != hipSuccess || splits == 1) {
     return e;
   }
