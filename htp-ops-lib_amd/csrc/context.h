@@ -103,7 +103,7 @@ struct htpops_context {
   // zeroed ticket counters of the K-sliced matmul (each launch leaves them zeroed)
   unsigned *tickets = nullptr;
 
-  // Converted copies of weights (MFMA fragment order for ops 1-4, int8 fragments, FP6 tiles, operand-order nibbles),
+  // Converted copies of weights (int8 fragments, FP6 tiles, operand-order nibbles),
   // keyed by the source range and the kind; dropped when the source is written through the registry, released or
   // invalidated.
   struct FragEntry {
@@ -228,7 +228,7 @@ constexpr int kBatchMaxM       = 16;  // rows up to which same-activation reques
 constexpr int kManyRowsMinM    = 17;  // rows from which a matmul may take the many-row kernels (see plan_mat_mul)
 constexpr int kFp6MinM         = 33;  // ... and from which the FP6 kernel is one of them
 
-constexpr int kFragKindRowLayout = 100;  // + ggml type: int8 fragments (kinds 1..4 are the tile-permuted formats of ops 1-4)
+constexpr int kFragKindRowLayout = 100;  // + ggml type: int8 fragments
 constexpr int kFragKindLaneOrder = 300;  // + ggml type: weights in matrix-core operand order (2..16 activation rows)
 constexpr int kFragKindBlockPairs = 350; // + ggml type: the same for the two-blocks-per-instruction kernel (2..8 rows)
 constexpr int kFragKindFp6Tiles  = 400;  // + ggml type: FP6 operand tiles of the many-row Q4_0 matmul (LDS kernel)

@@ -140,23 +140,16 @@ struct PermutedMatMul {
   const void  *weight;
   int          k, n;
 };
-// Many rows: a weight buffer is converted once into MFMA fragment order (permuted_weight_fragment_bytes), then
-// out fp32 [m][n] = fp16(act fp16 x W fp16): up to kPermutedGroupMax matmuls of one row count in one launch, plus one that
-// converts the distinct activations into `workspace` (permuted_gemm_workspace_bytes). The caller guarantees that no
-// member reads what another writes. A member's result does not depend on the others.
-size_t     permuted_weight_fragment_bytes(int k, int n);
-hipError_t launch_permuted_weight_to_fragments(hipStream_t stream, void *dst, const void *src, int k, int n,
-                                               int weight_kind);
-size_t     permuted_gemm_workspace_bytes(const PermutedMatMul *members, int count, int m);
-hipError_t launch_permuted_gemm_group(hipStream_t stream, const PermutedMatMul *members, const void *const *weight_fragments,
-                                      int count, int m, void *workspace);
-
-// The same formats read as they lie, nothing converted or kept, for up to kPermutedRowsMax rows: up to kPermutedGroupMax
-// matmuls of one row count and weight kind in one launch (plus one that puts the activations into operand order where
-// they do not fit LDS), under the same rules. `workspace`: permuted_rows_workspace_bytes.
+// out fp32 [m][n] = fp16(act fp16 x W fp16), the weights read as they lie, nothing converted or kept: up to kPermutedGroupMax
+// matmuls of one row count and weight kind in one launch (plus one that puts the distinct activations into operand order
+// where they do not fit LDS). The caller guarantees that no member reads what another writes. A member's result does not
+// depend on the others. The first for up to kPermutedRowsMax rows, the second for more; `workspace`: theirs.
 constexpr int kPermutedRowsMax = 32;
 size_t     permuted_rows_workspace_bytes(const PermutedMatMul *members, int count, int m);
 hipError_t launch_permuted_rows_group(hipStream_t stream, const PermutedMatMul *members, int count, int m, int weight_kind,
+                                      void *workspace);
+size_t     permuted_gemm_workspace_bytes(const PermutedMatMul *members, int count, int m);
+hipError_t launch_permuted_gemm_group(hipStream_t stream, const PermutedMatMul *members, int count, int m, int weight_kind,
                                       void *workspace);
 
 // attention; see htpops_flash_attn_ptr. `workspace` holds split-KV partials (decode), size from

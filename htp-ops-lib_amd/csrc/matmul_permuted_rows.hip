@@ -1,11 +1,12 @@
-// Up to 32 activation rows against the reference's own weight formats (its ops 1-4), read as they lie in memory.
+// Activation rows against the reference's own weight formats (its ops 1-4), read as they lie in memory.
 //
-// Replaces hmx_mat_mul_permuted_w16a32 and hmx_mat_mul_permuted_qk_0_d16a32 for decode-sized row counts (reference:
-// src/dsp/ops/mat_mul.c:758-855, :875-1153): fp16 activations times weights that are fp16(quant * scale), sums in fp32,
-// results rounded to fp16. The bound is the stream over the weight bytes (144 B per 256 Q4_0 or IQ4_NL weights, 272 B of
-// Q8_0, 512 B of fp16): a converted fp16 copy, which the many-row kernel wants, would be 3.6 times the bytes of the
-// 4-bit formats, so nothing is converted here and the weights are turned to fp16 in registers, on their way into the
-// matrix cores.
+// Replaces hmx_mat_mul_permuted_w16a32 and hmx_mat_mul_permuted_qk_0_d16a32 (reference: src/dsp/ops/mat_mul.c:758-855,
+// :875-1153; fp16 tiles of src/host/test.c:300-312, super-blocks of 8 K rows x 32 columns with one fp16 scale per 2 x 16
+// patch, dequantizers mat_mul.c:308-508): fp16 activations times weights that are fp16(quant * scale), sums in fp32,
+// results rounded to fp16. With few rows the bound is the stream over the weight bytes (144 B per 256 Q4_0 or IQ4_NL
+// weights, 272 B of Q8_0, 512 B of fp16): a converted fp16 copy would be 3.6 times the bytes of the 4-bit formats, so
+// nothing is converted and the weights are turned to fp16 in registers, on their way into the matrix cores. The first
+// kernel below takes up to 32 rows, the second more.
 //
 // The formats suit that: the 8 K rows of one column of a super-block are ONE dword of nibbles (two bytes per row pair
 // for Q8_0, a dword per row pair for fp16 tiles), and those are exactly the 8 values that a lane feeds to
@@ -353,6 +354,232 @@ __global__ __launch_bounds__(256) void permuted_rows_act_kernel(const RowsActArg
   args.dst[idx][t] = o;
 }
 
+// ---- more than 32 rows ----------------------------------------------------------------------------------------------
+// The same weights, turned to fp16 in registers by every wave that multiplies with them; what has to be saved here is the path
+// from L2 into a CU (with both operands as fp16 in memory it was the limit: 16 KiB per K step of 16 and workgroup of
+// 128 x 128 outputs at 30 bytes a nanosecond). A workgroup owns R row tiles of 16 x 4 column groups of 32; its four waves
+// are two column halves times two halves of K, added through LDS at the end. A wave holds R x 64 outputs: the two column
+// groups' weights come straight into registers, kDepth K steps of 32 ahead (4-bit formats: 1.1 KiB a step), each turned to
+// fp16 once for R matrix instructions per operand; the rows, fp16 in operand order, come into LDS by DMA in a ring of four
+// slots, three steps ahead, and are read as they are used. One barrier a step; two workgroups on a CU fill each
+// other's gaps. The matmuls of a message that nothing orders share a launch, longest K first.
+// Seven projections, 300 rows (hidden 2048, ffn 5632, IQ4_NL), weights not in a cache: 76.2 us (400 TFLOP/s), against 94.7
+// with fp16 copies of the weights staged through LDS like the rows and 264.8 with a launch per matrix over such copies; the
+// first pass over new weights 100 against 413 us. With the weights cached the fp16 copies were as fast (75.9) and, for
+// fp16 tiles and for few small matrices, up to 15 % faster; hidden 4096, ffn 8960, 33 rows: 115 us there, 73 here.
+struct GemmMember {
+  float         *out;
+  const uint8_t *frag, *weight;
+  int            n_tiles, k_tiles, col_begin;  // col_begin: in units of 4 column groups
+};
+struct GemmArgs {
+  GemmMember member[kPermutedGroupMax];
+  int        count, cols, m, row_tiles, row_blocks;
+};
+
+template <int KIND>
+struct RawLoads {  // load instructions of a step and column group
+  static constexpr int kCount = KIND == 1 ? 4 : KIND == 3 ? 5 : 2;
+};
+
+// load_step through a buffer resource: one instruction per field, whatever surrounds it (they are counted below)
+template <int KIND>
+__device__ __forceinline__ void load_step_counted(RawStep<KIND> &r, __amdgpu_buffer_rsrc_t tiles, int at, int g, int i) {
+  if constexpr (KIND == 1) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      r.q[v] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(tiles, 4 * g * 128 + 8 * i + 128 * v, at, 0));
+    }
+  } else if constexpr (KIND == 3) {
+    r.s = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(tiles, g * 272, at, 0));
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      r.q[v] = __builtin_amdgcn_raw_buffer_load_b32(tiles, g * 272 + 4 * i + 16 + 64 * v, at, 0);
+    }
+  } else {
+    r.s = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(tiles, g * 144, at, 0));
+    r.q = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(tiles, g * 144 + 8 * i + 16, at, 0));
+  }
+}
+
+template <int KIND, int R>
+__global__ __launch_bounds__(256, 2) void permuted_gemm_kernel(const GemmArgs args) {
+  constexpr int RING = 4, kDepth = 4;
+  constexpr int APART = (R + 1) / 2;                      // row pieces of 1 KiB that a wave brings per step (an odd one is brought twice)
+  constexpr int BLOADS = 2 * RawLoads<KIND>::kCount;      // weight loads of a wave per step
+  __shared__ __align__(1024) uint8_t lds[RING][2 * R * 1024];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kh = wave >> 1, wn = wave & 1;
+  const int g = lane >> 4, i = lane & 15;
+  // Workgroup ids go round the 8 XCDs: the row blocks of a column block follow each other on one XCD, so its weights come
+  // from that L2 for all but the first, and the column blocks (longest K first) are dealt out evenly.
+  const int turn = (int) blockIdx.x >> 3;
+  const int col  = turn / args.row_blocks * 8 + ((int) blockIdx.x & 7), rb = turn % args.row_blocks;
+  if (col >= args.cols) {
+    return;
+  }
+  int id = 0;
+  while (id + 1 < args.count && col >= args.member[id + 1].col_begin) {
+    ++id;
+  }
+  const GemmMember &mb = args.member[id];
+  const int n_tiles = mb.n_tiles, k_tiles = mb.k_tiles;
+  const int mt0 = rb * R, nt0 = (col - mb.col_begin) * 4 + 2 * wn;
+  // this wave's half of K: steps kt0 .. kt0 + mine - 1 (both halves run `steps` turns)
+  const int steps = (k_tiles + 1) / 2;
+  const int kt0 = kh * steps, mine = kh == 0 ? steps : k_tiles - steps;
+  auto      step_at = [&](int s) { return min(kt0 + s, k_tiles - 1); };  // (past the end: the last step again)
+
+  __amdgpu_buffer_rsrc_t tiles[2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const uint8_t *base = mb.weight + (size_t) min(nt0 + c, n_tiles - 1) * k_tiles * RawStep<KIND>::kTileBytes;
+    tiles[c] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(base), 0, (int) 0xffffffffu, 0x00020000);
+  }
+  RawStep<KIND> raw[kDepth][2];
+  auto load = [&](int d, int s) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      load_step_counted<KIND>(raw[d][c], tiles[c], step_at(s) * RawStep<KIND>::kTileBytes, g, i);
+    }
+  };
+  const uint8_t *src[APART];
+  uint32_t       to[APART];
+#pragma unroll
+  for (int p = 0; p < APART; ++p) {
+    const int t = min(2 * p + wn, R - 1);
+    src[p] = mb.frag + (size_t) min(mt0 + t, args.row_tiles - 1) * k_tiles * 1024;
+    to[p]  = (uint32_t) (uintptr_t) &lds[0][0] + (uint32_t) (kh * R + t) * 1024;
+  }
+  auto fetch = [&](int s) {
+    const size_t   off  = (size_t) step_at(s) * 1024;
+    const uint32_t slot = (uint32_t) (s & (RING - 1)) * (2 * R * 1024);
+#pragma unroll
+    for (int p = 0; p < APART; ++p) {
+      asm volatile("s_mov_b32 m0, %2\n s_nop 0\n global_load_lds_dwordx4 %0, %1" ::"v"(lane * 16), "s"(src[p] + off), "s"(slot + to[p]) : "memory");
+    }
+  };
+
+  v4f acc[R][2][2];
+#pragma unroll
+  for (int t = 0; t < R; ++t) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      acc[t][c][0] = acc[t][c][1] = (v4f){ 0.0f, 0.0f, 0.0f, 0.0f };
+    }
+  }
+  const uint32_t  half_sel = (i >> 3) ? 0x03020302u : 0x01000100u;  // columns 16 .. 31 take the odd scales
+  VectorConstants vc;
+  asm("" : "+v"(vc.exponents));
+
+  // Requests in order: weights of step 0, then rows of step s and weights of step s + 1 in turn; from turn s on, rows of step
+  // s + 3 and weights of step s + kDepth.
+#pragma unroll
+  for (int s = 0; s < kDepth; ++s) {
+    load(s, s);
+    asm volatile("" ::: "memory");
+    if (s < RING - 1) {
+      fetch(s);
+    }
+  }
+  for (int s0 = 0; s0 < steps; s0 += kDepth) {
+#pragma unroll
+    for (int d = 0; d < kDepth; ++d) {
+      const int s = s0 + d;
+      if (s >= steps) {
+        break;
+      }
+      // This wave's rows of step s have landed: behind them it has asked for the rows of two steps and the weights of three.
+      // Behind the barrier everybody's have, and nobody reads the slot of step s - 1 any more.
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * APART + 3 * BLOADS) : "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      fetch(s + RING - 1);
+      v8h b[2][2];
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        v2h sc[4];
+        if constexpr (KIND != 1) {
+          const uint4    q     = raw[d][c].s;
+          const uint32_t q4[4] = { q.x, q.y, q.z, q.w };
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            sc[v] = as_v2h(__builtin_amdgcn_perm(q4[v], q4[v], half_sel));
+          }
+        }
+        b[c][0] = dequant<KIND, 0>(raw[d][c], sc, vc), b[c][1] = dequant<KIND, 1>(raw[d][c], sc, vc);
+      }
+      load(d, s + kDepth);
+      asm volatile("" ::: "memory");
+      if (s < mine) {
+        const uint8_t *rows = &lds[s & (RING - 1)][kh * R * 1024] + lane * 16;
+#pragma unroll
+        for (int t = 0; t < R; ++t) {
+          const v8h a = *reinterpret_cast<const v8h *>(rows + t * 1024);
+#pragma unroll
+          for (int c = 0; c < 2; ++c) {
+            acc[t][c][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[c][0], acc[t][c][0], 0, 0, 0);
+            acc[t][c][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[c][1], acc[t][c][1], 0, 0, 0);
+          }
+        }
+      }
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (rows past the end have landed before the ring is used again)
+
+  // the second half of K hands its sums over; D[4 g + r][i] of tile (t, c, j) is row 16 t + 4 g + r, column 2 i + j of group c
+  static_assert(2 * R * 4 * kWave * sizeof(v4f) <= sizeof(lds), "the sums of both column halves fit");
+  v4f *xch = reinterpret_cast<v4f *>(&lds[0][0]) + (size_t) wn * R * 4 * kWave + lane;
+  __syncthreads();
+  if (kh == 1) {
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        xch[(4 * t + 2 * c) * kWave] = acc[t][c][0], xch[(4 * t + 2 * c + 1) * kWave] = acc[t][c][1];
+      }
+    }
+  }
+  __syncthreads();
+  if (kh == 1) {
+    return;
+  }
+  const int n = n_tiles * 32;
+#pragma unroll
+  for (int t = 0; t < R; ++t) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      if (mt0 + t < args.row_tiles && nt0 + c < n_tiles) {
+        const v4f even = acc[t][c][0] + xch[(4 * t + 2 * c) * kWave], odd = acc[t][c][1] + xch[(4 * t + 2 * c + 1) * kWave];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int row = 16 * (mt0 + t) + 4 * g + r;
+          if (row < args.m) {  // (the reference stores fp16 results)
+            *reinterpret_cast<float2 *>(mb.out + (size_t) row * n + 32 * (nt0 + c) + 2 * i) =
+              make_float2((float) (_Float16) even[r], (float) (_Float16) odd[r]);
+          }
+        }
+      }
+    }
+  }
+}
+
+template <int KIND>
+hipError_t launch_gemm_kind(hipStream_t stream, const GemmArgs &args, unsigned grid, int r) {
+  void (*kernel)(GemmArgs) = nullptr;
+  switch (r) {
+    case 2: kernel = permuted_gemm_kernel<KIND, 2>; break;
+    case 3: kernel = permuted_gemm_kernel<KIND, 3>; break;
+    case 4: kernel = permuted_gemm_kernel<KIND, 4>; break;
+    case 5: kernel = permuted_gemm_kernel<KIND, 5>; break;
+    case 6: kernel = permuted_gemm_kernel<KIND, 6>; break;
+    case 7: kernel = permuted_gemm_kernel<KIND, 7>; break;
+    default: kernel = permuted_gemm_kernel<KIND, 8>; break;
+  }
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, stream, args);
+  return hipGetLastError();
+}
+
 bool act_in_lds(int m, int k) {
   return (size_t) m * (k + 8) * 2 <= kRowsActLds;
 }
@@ -460,6 +687,71 @@ hipError_t launch_permuted_rows_group(hipStream_t stream, const PermutedMatMul *
       return launch_kind<3>(stream, args, grid, lds, act_lds, wide);
     default:
       return launch_kind<4>(stream, args, grid, lds, act_lds, wide);
+  }
+}
+
+size_t permuted_gemm_workspace_bytes(const PermutedMatMul *members, int count, int m) {
+  return permuted_rows_workspace_bytes(members, count, m);
+}
+
+hipError_t launch_permuted_gemm_group(hipStream_t stream, const PermutedMatMul *members, int count, int m, int weight_kind,
+                                      void *workspace) {
+  if (count < 1 || count > kPermutedGroupMax || m < 1 || weight_kind < 1 || weight_kind > 4) {
+    return hipErrorInvalidValue;
+  }
+  int order[kPermutedGroupMax];
+  for (int j = 0; j < count; ++j) {
+    if (members[j].k % 32 != 0 || members[j].n % 32 != 0 || members[j].k <= 0 || members[j].n <= 0) {
+      return hipErrorInvalidValue;
+    }
+    order[j] = j;
+  }
+  std::stable_sort(order, order + count, [&](int a, int b) { return members[a].k > members[b].k; });
+  GemmArgs    args = {};
+  RowsActArgs conv = {};
+  unsigned    conv_grid = 0;
+  uint8_t    *ws = static_cast<uint8_t *>(workspace);
+  args.count = count, args.m = m, args.row_tiles = conv.tiles = (m + 15) / 16, conv.m = m;
+  for (int j = 0; j < count; ++j) {
+    const PermutedMatMul &p = members[order[j]];
+    int                   c = 0;
+    while (c < conv.count && !(conv.src[c] == p.act && conv.k[c] == p.k)) {
+      ++c;
+    }
+    if (c == conv.count) {
+      conv.src[c] = p.act, conv.k[c] = p.k, conv.dst[c] = reinterpret_cast<uint4 *>(ws), conv.first[c] = (int) conv_grid;
+      ws += act_bytes(m, p.k);
+      conv_grid += (unsigned) ((act_bytes(m, p.k) / 16 + 255) / 256);
+      ++conv.count;
+    }
+    args.member[j] = { p.out, reinterpret_cast<const uint8_t *>(conv.dst[c]), static_cast<const uint8_t *>(p.weight), p.n / 32,
+                       p.k / 32, args.cols };
+    args.cols += (p.n / 32 + 3) / 4;
+  }
+  hipLaunchKernelGGL(permuted_rows_act_kernel, dim3(conv_grid), dim3(256), 0, stream, conv);
+  if (hipError_t e = hipGetLastError(); e != hipSuccess) {
+    return e;
+  }
+  // The most row tiles per workgroup that still give every CU one workgroup (two fit), spread evenly over the row blocks.
+  int r = std::min(8, args.row_tiles);
+  while (r > 2 && (long) args.cols * ((args.row_tiles + r - 1) / r) < 256) {
+    --r;
+  }
+  args.row_blocks = (args.row_tiles + r - 1) / r;
+  r = std::max(2, (args.row_tiles + args.row_blocks - 1) / args.row_blocks);
+  const long long grid = (long long) ((args.cols + 7) / 8) * 8 * args.row_blocks;
+  if (grid > 0x7fffffffLL) {
+    return hipErrorInvalidValue;
+  }
+  switch (weight_kind) {
+    case 1:
+      return launch_gemm_kind<1>(stream, args, (unsigned) grid, r);
+    case 2:
+      return launch_gemm_kind<2>(stream, args, (unsigned) grid, r);
+    case 3:
+      return launch_gemm_kind<3>(stream, args, (unsigned) grid, r);
+    default:
+      return launch_gemm_kind<4>(stream, args, (unsigned) grid, r);
   }
 }
 

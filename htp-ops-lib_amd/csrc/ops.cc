@@ -373,74 +373,19 @@ int op_mat_mul_f32(htpops_context *ctx, float *dst, const float *act, const void
   return run_mat_mul(ctx, plan, dst, ws, weight, m, k, n, weight_type, ws + q_bytes);
 }
 
-namespace {
-
-// decode-sized row counts: the weights are streamed in their own format, which is a fraction of the bytes of a converted
-// copy (and costs a host with caller-registered weights no conversion per call)
-int run_permuted_rows(htpops_context *ctx, const PermutedMatMul *members, int count, int m, int kind) {
-  if (int r = ensure_workspace(ctx, permuted_rows_workspace_bytes(members, count, m))) {
-    return r;
-  }
-  HTPOPS_HIP(ctx, launch_permuted_rows_group(ctx->stream, members, count, m, kind, ctx->workspace));
-  return HTPOPS_OK;
-}
-
-// more rows: one launch over converted copies of the weights, which are kept (kept already, or in a buffer of which copies
-// may be kept; see op_mat_mul_permuted)
-int run_permuted_gemm(htpops_context *ctx, const PermutedMatMul *members, int count, int m, int kind) {
-  const void *frag[kPermutedGroupMax];
-  for (int i = 0; i < count; ++i) {
-    const PermutedMatMul &p = members[i];
-    frag[i]                 = find_copy(ctx, p.weight, kind, p.k, p.n);
-    if (frag[i]) {
-      continue;
-    }
-    void *fresh = nullptr;
-    if (int r = new_copy(ctx, p.weight, permuted_weight_bytes((size_t) p.n, (size_t) p.k, kind), kind, p.k, p.n,
-                         permuted_weight_fragment_bytes(p.k, p.n), &fresh)) {
-      return r;
-    }
-    const hipError_t e = launch_permuted_weight_to_fragments(ctx->stream, fresh, p.weight, p.k, p.n, kind);
-    if (e != hipSuccess) {
-      forget_copy(ctx, fresh);
-      return fail(ctx, HTPOPS_ERR_HIP, "weight conversion: %s", hipGetErrorString(e));
-    }
-    frag[i] = fresh;
-  }
-  if (int r = ensure_workspace(ctx, permuted_gemm_workspace_bytes(members, count, m))) {
-    return r;
-  }
-  HTPOPS_HIP(ctx, launch_permuted_gemm_group(ctx->stream, members, frag, count, m, ctx->workspace));
-  return HTPOPS_OK;
-}
-
-bool keeps_copy(htpops_context *ctx, const PermutedMatMul &p, int kind) {
-  return find_copy(ctx, p.weight, kind, p.k, p.n) != nullptr ||
-         may_keep_copies(ctx, p.weight, permuted_weight_bytes((size_t) p.n, (size_t) p.k, kind));
-}
-
-}  // namespace
-
+// The weights are read in their own formats at every row count: a converted copy would be up to 3.6 times the bytes.
 int op_mat_mul_permuted_group(htpops_context *ctx, const PermutedMatMul *members, int count, int m, int kind) {
-  bool together = count > 1;
-  for (int i = 0; together && i < count; ++i) {
-    together = m <= kPermutedRowsMax || keeps_copy(ctx, members[i], kind);
-  }
-  if (together) {
-    for (int i = 0; i < count; ++i) {
-      note_device_write(ctx, members[i].out, (size_t) m * members[i].n * 4);
-    }
-    return m <= kPermutedRowsMax ? run_permuted_rows(ctx, members, count, m, kind) :
-                                   run_permuted_gemm(ctx, members, count, m, kind);
-  }
-  int ret = HTPOPS_OK;
   for (int i = 0; i < count; ++i) {
-    const PermutedMatMul &p = members[i];
-    if (int r = op_mat_mul_permuted(ctx, p.out, p.act, p.weight, m, p.k, p.n, kind)) {
-      ret = r;
-    }
+    note_device_write(ctx, members[i].out, (size_t) m * members[i].n * 4);
   }
-  return ret;
+  const bool few = m <= kPermutedRowsMax;
+  if (int r = ensure_workspace(ctx, few ? permuted_rows_workspace_bytes(members, count, m) :
+                                          permuted_gemm_workspace_bytes(members, count, m))) {
+    return r;
+  }
+  HTPOPS_HIP(ctx, few ? launch_permuted_rows_group(ctx->stream, members, count, m, kind, ctx->workspace) :
+                        launch_permuted_gemm_group(ctx->stream, members, count, m, kind, ctx->workspace));
+  return HTPOPS_OK;
 }
 
 // hmx_mat_mul_permuted_w16a32 / hmx_mat_mul_permuted_qk_0_d16a32 (reference: src/dsp/ops/mat_mul.c:758-855, :875-1153)
@@ -459,25 +404,8 @@ int op_mat_mul_permuted(htpops_context *ctx, float *dst, const float *act, const
   if (int r = need_device(ctx)) {
     return r;
   }
-  note_device_write(ctx, dst, (size_t) m * n * 4);
   const PermutedMatMul one = { dst, act, weight, k, n };
-  if (m <= kPermutedRowsMax) {
-    return run_permuted_rows(ctx, &one, 1, m, kind);
-  }
-  // Converted copies are kept only for weights in buffers the context allocated (their contents change only through
-  // htpops_buffer_write or as an op's output, both of which drop the copy). Caller-registered memory may be rewritten
-  // behind the context's back: it is converted into the workspace on every call.
-  if (keeps_copy(ctx, one, kind)) {
-    return run_permuted_gemm(ctx, &one, 1, m, kind);
-  }
-  const size_t act_bytes = permuted_gemm_workspace_bytes(&one, 1, m);  // (a multiple of 1 KiB)
-  if (int r = ensure_workspace(ctx, act_bytes + permuted_weight_fragment_bytes(k, n))) {
-    return r;
-  }
-  const void *frag = static_cast<uint8_t *>(ctx->workspace) + act_bytes;
-  HTPOPS_HIP(ctx, launch_permuted_weight_to_fragments(ctx->stream, const_cast<void *>(frag), weight, k, n, kind));
-  HTPOPS_HIP(ctx, launch_permuted_gemm_group(ctx->stream, &one, &frag, 1, m, ctx->workspace));
-  return HTPOPS_OK;
+  return op_mat_mul_permuted_group(ctx, &one, 1, m, kind);
 }
 
 int op_flash_attn(htpops_context *ctx, void *o, const void *q, const void *k, const void *v, const void *mask,

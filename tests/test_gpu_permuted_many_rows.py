@@ -18,15 +18,16 @@ def ctx():
 
 
 @pytest.mark.parametrize("kind,m,k,n", [
-    (1, 33, 32, 32), (2, 65, 64, 128), (3, 64, 96, 160), (4, 97, 160, 64),     # one, two, three, five steps per half of K
-    (1, 100, 512, 4096 + 32), (2, 130, 256, 8192), (3, 160, 128, 32768 + 96),  # 1, 3 and 5 row tiles per workgroup
-    (4, 290, 2048, 96), (2, 350, 64, 16384 + 32), (1, 128, 96, 32768)])        # (the last: 4 row tiles)
+    (1, 33, 32, 32), (2, 65, 64, 128), (3, 64, 96, 160), (4, 97, 160, 64),     # one step of K in all; one, two, three per half
+    (1, 100, 512, 4096 + 32), (2, 130, 256, 8192), (4, 290, 2048, 96),         # two row tiles of 16 per workgroup
+    (4, 33, 64, 32768), (2, 64, 96, 32768), (3, 160, 128, 32768 + 96),         # three, four, five of them
+    (3, 96, 32, 32768), (4, 300, 64, 16384), (1, 128, 96, 32768), (2, 350, 64, 16384 + 32)])  # six, seven, eight, eight
 def test_many_rows_at_the_edges(ctx, oracle, kind, m, k, n):
     check(ctx, oracle, kind, m, k, n, m * 3 + k + n)
 
 
 def test_many_rows_grouped_with_caller_owned_weights(ctx):
-    # one message: shared rows, different k (a long one last), and a member whose weights may not be kept converted: every
+    # one message: shared rows, different k (a long one last), and a member whose weights lie in registered memory: every
     # output byte for byte what one message per request gives
     rng = wl.rng_for(88, 0)
     m, kind = 70, 4
