@@ -602,27 +602,29 @@ __global__ __launch_bounds__(kPfThreads *GROUPS, DP <= 128 ? 2 : 1) void flash_a
   }
 }
 
-// Puts the shares of a split prefill together: a wave per 32-query tile, head and unit of four output columns per half
-// (`units` of them), lane for lane as the prefill kernel left them. All loads of kPfMergeChunk shares are requested
-// before the first use; chunks are folded into a running (max, sum, O) like KV blocks are.
+// Puts the shares of a split prefill together: G waves per 32-query tile, head and unit of four output columns per half
+// (`units` of them), lane for lane as the prefill kernel left them. Each takes every G-th run of kPfMergeChunk shares, all
+// loads of a run requested before the first use, folded into a running (max, sum, O) like KV blocks are; with G = 4 (more
+// shares than a run holds) the four states meet in LDS (one row, 16384 keys, 16 / 4 heads of 96, 64 shares: 23.0 -> 19.2 us).
 constexpr int kPfMergeChunk = 8;
 
-template <bool QO_F32>
+template <bool QO_F32, int G>
 __global__ __launch_bounds__(256) void flash_attn_prefill_merge_kernel(void *__restrict__ o_ptr,
                                                                        const float *__restrict__ part, int n_splits,
                                                                        int n_tiles, int units, int qo_len, int n_heads,
                                                                        int D) {
-  const int lane = threadIdx.x & 63;
-  const int id   = (int) blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6);
+  __shared__ float states[G == 1 ? 1 : G][6][G == 1 ? 1 : kWave];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6);
+  const int id   = G == 1 ? (int) blockIdx.x * 4 + wave : (int) blockIdx.x;
   const int tile = id / units, unit = id % units;
-  if (tile >= n_tiles) {
+  if (tile >= n_tiles) {  // (G = 4: the whole workgroup or none of it)
     return;
   }
   const size_t stride = (size_t) n_tiles * prefill_partial_floats(units);
   const float *rec    = part + (size_t) tile * prefill_partial_floats(units);
   float        m_run = -INFINITY, l_run = 0.0f;
   float        v[4]  = { 0.0f, 0.0f, 0.0f, 0.0f };
-  for (int s0 = 0; s0 < n_splits; s0 += kPfMergeChunk) {
+  for (int s0 = G == 1 ? 0 : wave * kPfMergeChunk; s0 < n_splits; s0 += G * kPfMergeChunk) {
     float2 ml[kPfMergeChunk];
     float4 x[kPfMergeChunk];
 #pragma unroll
@@ -650,6 +652,32 @@ __global__ __launch_bounds__(256) void flash_attn_prefill_merge_kernel(void *__r
       v[0] += f * x[u].x, v[1] += f * x[u].y, v[2] += f * x[u].z, v[3] += f * x[u].w;
     }
     m_run = m_new;
+  }
+  if constexpr (G > 1) {
+    states[wave][0][lane] = m_run, states[wave][1][lane] = l_run;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      states[wave][2 + e][lane] = v[e];
+    }
+    __syncthreads();
+    if (wave != 0) {
+      return;
+    }
+#pragma unroll
+    for (int w = 1; w < G; ++w) {
+      m_run = fmaxf(m_run, states[w][0][lane]);
+    }
+    const float m_safe = (m_run == -INFINITY) ? 0.0f : m_run;
+    l_run = 0.0f, v[0] = v[1] = v[2] = v[3] = 0.0f;
+#pragma unroll
+    for (int w = 0; w < G; ++w) {  // (a wave without shares has m = -inf, l = v = 0)
+      const float f = fast_exp2(states[w][0][lane] - m_safe);
+      l_run += f * states[w][1][lane];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[e] += f * states[w][2 + e][lane];
+      }
+    }
   }
   const int   head = tile % n_heads, q_row = tile / n_heads * kBQ + (lane & 31);
   const int   d0   = 8 * unit + 4 * (lane >> 5);
@@ -1167,7 +1195,10 @@ hipError_t launch_prefill(hipStream_t stream, void *o, const void *q, const void
     const size_t share  = tiles * prefill_partial_floats(DP / 8) * sizeof(float);
     const size_t blocks = ((size_t) kv_len + kBK - 1) / kBK;
     const size_t most   = std::min({ (size_t) (kCus / wgs), blocks / (2 * kMaxGroups), scratch_bytes / share });
-    splits              = most < 2 ? 1u : (unsigned) most;
+    // (for few tiles down to one block, while one trip of the merge takes all shares: 5 rows over 1029 keys, 12 tiles, 14.4 ->
+    // 12.6 us; but 128 rows over 1152, 48 tiles, 17.5 -> 17.8, and 500 rows over 500, 256 tiles, 18.7 -> 20.2)
+    const size_t finer  = std::min({ (size_t) (kCus / wgs), blocks / kMaxGroups, scratch_bytes / share, (size_t) kPfMergeChunk });
+    splits              = most < 2 ? 1u : (unsigned) (tiles <= 32 ? std::max(most, finer) : most);
   }
   const dim3 grid(x, q_blocks, splits);
   // Two key groups per workgroup when the grid leaves CUs without a second workgroup, or (causal) when the workgroups
@@ -1195,8 +1226,13 @@ hipError_t launch_prefill(hipStream_t stream, void *o, const void *q, const void
     return e;
   }
   constexpr int kUnits = DP / 8;
-  hipLaunchKernelGGL(flash_attn_prefill_merge_kernel<QO_F32>, dim3((unsigned) ((tiles * kUnits + 3) / 4)), dim3(256), 0, stream, o,
-                     scratch, (int) splits, (int) tiles, kUnits, qo_len, n_heads, head_dim);
+  if (splits > (unsigned) kPfMergeChunk) {
+    hipLaunchKernelGGL((flash_attn_prefill_merge_kernel<QO_F32, 4>), dim3((unsigned) (tiles * kUnits)), dim3(256), 0, stream, o,
+                       scratch, (int) splits, (int) tiles, kUnits, qo_len, n_heads, head_dim);
+  } else {
+    hipLaunchKernelGGL((flash_attn_prefill_merge_kernel<QO_F32, 1>), dim3((unsigned) ((tiles * kUnits + 3) / 4)), dim3(256), 0,
+                       stream, o, scratch, (int) splits, (int) tiles, kUnits, qo_len, n_heads, head_dim);
+  }
   return hipGetLastError();
 }
 
