@@ -728,6 +728,129 @@ __global__ __launch_bounds__(kGiThreads, 4) void gemm_i8_fragments_small_kernel(
   }
 }
 
+// ---- 128 x 64 tiles with both operands staged through LDS -----------------------------------------------------------
+// Straight into registers a 64 x 64 wave tile pulls 1.2 KB per unit through the path from L2 into its CU, whose 10 TB/s (all
+// CUs) end at about 500 TFLOP/s. Here a workgroup owns 4 row tiles x 2 column tiles; its eight waves are two halves of K
+// times 2 x 2 waves of two row tiles and one column tile, and what a half needs of a block (four row and two column
+// fragments and their scales, 7.25 KiB for eight units) comes into LDS once, by DMA, two instructions per wave and block, in a
+// ring of four slots three blocks ahead. One barrier a block; two workgroups on a CU fill each other's gaps. The halves
+// are added through LDS. What bounds it then is the vector ALU (32 instructions a unit)
+// and the scale product. Times: see tile_config.
+constexpr int kStRing  = 4;
+constexpr int kStSlot  = 4 * 1024 + 1024 + 2 * 1024 + 256;  // row fragments, their scales, column fragments, their scales
+constexpr int kStWaves = 8;
+
+__global__ __launch_bounds__(kStWaves *kWave, 4) void gemm_i8_fragments_staged_kernel(FragMembers grp, int m, int m_tiles) {
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[2][kStRing][kStSlot];
+  const FragMember &mem = member_of_workgroup(grp);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kh = wave >> 2, w4 = wave & 3, wm = w4 >> 1, wn = w4 & 1;
+  const int c = lane & 31, h = lane >> 5;
+  const int n = mem.n, nblk = mem.nblk, n_tiles = mem.n_tiles;
+  // all row blocks of a column block on one XCD, behind each other (as in fragments_workgroup)
+  const unsigned wg = blockIdx.x - mem.wg_begin;
+  const int gy = (m_tiles + 3) / 4, gx = (n_tiles + 1) / 2;
+  const int xcd = wg & 7, slot_ = (int) (wg >> 3), by = slot_ % gy, bx = (slot_ / gy) * 8 + xcd;
+  if (bx >= gx) {
+    return;
+  }
+  const int mt0 = 4 * by, nt0 = 2 * bx;
+  // this half's blocks: kb0 .. kb0 + mine - 1 (both halves run `steps` turns)
+  const int steps = (nblk + 1) / 2, kb0 = kh * steps, mine = kh == 0 ? steps : nblk - steps;
+
+  // wave w brings row fragment w and one more piece: row scales, column scales, column fragment 0, column fragment 1
+  const uint8_t *a_src = reinterpret_cast<const uint8_t *>(mem.a_frag) + (size_t) min(mt0 + w4, m_tiles - 1) * nblk * 1024;
+  const uint8_t *b_src = reinterpret_cast<const uint8_t *>(mem.b_frag) + (size_t) min(nt0 + (w4 & 1), n_tiles - 1) * nblk * 1024;
+  // (per lane: 16 lanes per row tile, 16 bytes each; 32 lanes per column tile, 4 bytes each)
+  const uint8_t *as_src = reinterpret_cast<const uint8_t *>(mem.a_scale) + (size_t) min(mt0 + (lane >> 4), m_tiles - 1) * nblk * 256 + (lane & 15) * 16;
+  const uint8_t *bs_src = reinterpret_cast<const uint8_t *>(mem.b_scale) + (size_t) min(nt0 + h, n_tiles - 1) * nblk * 128 + c * 4;
+  const uint32_t to0 = (uint32_t) (uintptr_t) &lds[kh][0][0];
+  auto fetch = [&](int s) {  // (past the end: the last block again, so that the count of requests in flight stays)
+    const size_t   kb = (size_t) min(kb0 + s, nblk - 1);
+    const uint32_t to = to0 + (uint32_t) (s & (kStRing - 1)) * kStSlot;
+    asm volatile("s_mov_b32 m0, %2\n s_nop 0\n global_load_lds_dwordx4 %0, %1" ::"v"(lane * 16), "s"(a_src + kb * 1024), "s"(to + w4 * 1024) : "memory");
+    if (w4 >= 2) {
+      asm volatile("s_mov_b32 m0, %2\n s_nop 0\n global_load_lds_dwordx4 %0, %1" ::"v"(lane * 16), "s"(b_src + kb * 1024), "s"(to + 5120 + (w4 - 2) * 1024) : "memory");
+    } else if (w4 == 0) {
+      asm volatile("s_mov_b32 m0, %1\n s_nop 0\n global_load_lds_dwordx4 %0, off" ::"v"(as_src + kb * 256), "s"(to + 4096) : "memory");
+    } else {
+      asm volatile("s_mov_b32 m0, %1\n s_nop 0\n global_load_lds_dword %0, off" ::"v"(bs_src + kb * 128), "s"(to + 7168) : "memory");
+    }
+  };
+  v16f acc[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      acc[u][r] = 0.0f;
+    }
+  }
+  const v16f zf = { 0 };
+  const v16i zi = { 0 };
+#pragma unroll
+  for (int s = 0; s < kStRing - 1; ++s) {
+    fetch(s);
+  }
+  for (int s = 0; s < steps; ++s) {
+    // this wave's pieces of block s have landed (those of two more blocks may be on their way); behind the barrier everybody's
+    // have, and nobody reads the slot of block s - 1 any more
+    asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    fetch(s + kStRing - 1);
+    if (s < mine) {
+      const uint8_t *at = &lds[kh][s & (kStRing - 1)][0];
+      const v4i      b  = *reinterpret_cast<const v4i *>(at + 5120 + wn * 1024 + lane * 16);
+      const uint2    db = make_uint2(*reinterpret_cast<const uint32_t *>(at + 7168 + wn * 128 + c * 4), 0u);
+      v4i            a[2];
+      uint2          da[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        a[u]  = *reinterpret_cast<const v4i *>(at + (2 * wm + u) * 1024 + lane * 16);
+        da[u] = make_uint2(*reinterpret_cast<const uint32_t *>(at + 4096 + (2 * wm + u) * 256 + lane * 4), 0u);
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const v16i sum = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[u], b, zi, 0, 0, 0);
+        const v16f scl = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(v4h, da[u]), __builtin_bit_cast(v4h, db), zf, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          acc[u][r] = __builtin_fmaf((float) sum[r], scl[r], acc[u][r]);
+        }
+      }
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (pieces past the end have landed before the ring is used again)
+  float *xch = reinterpret_cast<float *>(&lds[0][0][0]) + (size_t) w4 * 2 * 16 * kWave + lane;
+  static_assert(4 * 2 * 16 * kWave * sizeof(float) <= sizeof(lds), "the sums of a half fit");
+  __syncthreads();
+  if (kh == 1) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        xch[(16 * u + r) * kWave] = acc[u][r];
+      }
+    }
+  }
+  __syncthreads();
+  if (kh == 1) {
+    return;
+  }
+  const int col = (nt0 + wn) * 32 + c;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int   row = (mt0 + 2 * wm + u) * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
+      const float v   = acc[u][r] + xch[(16 * u + r) * kWave];
+      if (row < m && col < n) {
+        mem.out[(size_t) row * n + col] = v;
+      }
+    }
+  }
+}
+
 size_t round256(size_t x) {
   return (x + 255) & ~(size_t) 255;
 }
@@ -767,6 +890,8 @@ hipError_t launch_weights_to_i8_fragments(hipStream_t stream, void *dst, const v
 
 namespace {
 
+constexpr int kStagedUnit = 3;  // gemm_i8_fragments_staged_kernel
+
 struct TileConfig {
   int unit, ksplit;
 };
@@ -779,6 +904,14 @@ struct TileConfig {
 TileConfig tile_config(int m, int n, int k, int forced_unit) {
   const int m_tiles = (m + 31) / 32, n_tiles = (n + 31) / 32, nblk = k / 32;
   const int wave_tiles  = ((m_tiles + 1) / 2) * ((n_tiles + 1) / 2);
+  // Both operands through LDS where that gives every CU a workgroup of 128 x 64 and pads the rows by less than a seventh.
+  // Before / with it, Q8_0: seven projections at 256 rows, Llama-7B / Qwen2-1.5B, 238 / 82.7 and 197 / 61.8 us; layers of 512 rows 441 /
+  // 165 and 393 / 147. (From 128 workgroups on: the projections 161, but a layer of 200 rows, whose o has a launch of
+  // its own, 283 against 247; 300 rows, padded by a fifth, 315 and 325; one matrix of 344 workgroups 47.5 and 50.4.)
+  const int row_blocks = (m_tiles + 3) / 4;
+  if (forced_unit != 1 && forced_unit != 2 && 28 * row_blocks <= 8 * m_tiles && row_blocks * ((n_tiles + 1) / 2) >= 256) {
+    return { kStagedUnit, 2 };
+  }
   const int unit        = forced_unit == 1 || forced_unit == 2 ? forced_unit : (m_tiles == 1 || wave_tiles < 512 ? 1 : 2);
   if (unit == 1) {
     return { 1, nblk >= 192 ? 4 : nblk >= 96 ? 2 : 1 };
@@ -820,8 +953,10 @@ SmallTilePlan small_tile_plan(int m_tiles, int n_tiles, int nblk, TileConfig cfg
   // there are CUs for, on a tile's K, down to 12 blocks per wave. fp32 rows (quantized on the way), unsplit with 12 blocks
   // a wave at least / split: k = 8960, n = 1537, 33 rows 23.7 / 14.3 us; k = n = 4096, 33 rows 20.5 / 14.5. (16 waves of
   // one workgroup on a tile's K instead, no exchange: 27 rows, k = 8960, n = 1537 14.2 against 11.9 us.)
+  // (short K with 128 tiles and more keeps the shared activations: seven projections of Qwen2 size at 70 rows 26.6 against
+  // 28.5 us)
   const int wgs = m_tiles * ((n_tiles + kGiWaves / cfg.ksplit - 1) / (kGiWaves / cfg.ksplit));
-  if (split_k && wgs < kSmallWgs && nblk >= 2 * kGiWaves) {
+  if (split_k && wgs < kSmallWgs && nblk >= 2 * kGiWaves && (cfg.ksplit > 1 || m_tiles * n_tiles < kSmallWgs / 2)) {
     return { kSharePlain, kGiWaves, std::max(1, std::min({ kMaxParts, kSmallWgs / (m_tiles * n_tiles), nblk / (kGiWaves * 12) })) };
   }
   // (measured on the Qwen2 block at 128 rows: weights shared 39.6 us, activations shared 40.2 us, neither 43.9 us)
@@ -829,6 +964,9 @@ SmallTilePlan small_tile_plan(int m_tiles, int n_tiles, int nblk, TileConfig cfg
 }
 
 unsigned member_workgroups(int m_tiles, int n_tiles, TileConfig cfg, SmallTilePlan plan) {
+  if (cfg.unit == kStagedUnit) {
+    return (unsigned) (((n_tiles + 1) / 2 + 7) / 8 * 8 * ((m_tiles + 3) / 4));
+  }
   if (plan.share == kShareWeights) {
     return (unsigned) ((n_tiles + 7) / 8 * 8 * (m_tiles / kGiWaves) * plan.kparts);
   }
@@ -846,7 +984,7 @@ const uint32_t *scales_of(const void *fragments, size_t tiles, size_t nblk) {
 }  // namespace
 
 bool gemm_i8_fragments_groupable(int m, int n, int forced_unit) {
-  return tile_config(m, n, 32, forced_unit).unit == 1;
+  return tile_config(m, n, 32, forced_unit).unit != 2;
 }
 
 hipError_t launch_act_to_i8_fragments_group(hipStream_t stream, int count, void *const *act_fragments,
@@ -892,13 +1030,12 @@ size_t gemm_i8_fragments_exchange_bytes(int m, int n, int k, int forced_unit) {
   return plan.kparts > 1 ? (size_t) ((n_tiles + 7) / 8 * 8) * m_tiles * plan.kparts * 1024 * sizeof(float) : 0;
 }
 
-hipError_t launch_gemm_i8_fragments_group(hipStream_t stream, int count, float *const *outs,
-                                          const void *const *act_fragments, const void *const *weight_fragments,
-                                          const int *ns, const int *ks, int m, void *exchange, size_t exchange_bytes,
-                                          unsigned *tickets, int ticket_slots, int forced_unit) {
-  if (count < 1 || count > kGemmGroupMax || m <= 0) {
-    return hipErrorInvalidValue;
-  }
+namespace {
+
+// the members of one tile configuration
+hipError_t launch_members(hipStream_t stream, int count, float *const *outs, const void *const *act_fragments,
+                          const void *const *weight_fragments, const int *ns, const int *ks, int m, void *exchange,
+                          size_t exchange_bytes, unsigned *tickets, int ticket_slots, int forced_unit) {
   size_t exchange_used = 0;
   int    tickets_used  = 0;
   const int   m_tiles = (m + 31) / 32;
@@ -919,7 +1056,7 @@ hipError_t launch_gemm_i8_fragments_group(hipStream_t stream, int count, float *
       return hipErrorInvalidValue;
     }
     const TileConfig c = tile_config(m, ns[i], ks[i], forced_unit);
-    if (slot > 0 && (c.unit != cfg.unit || (c.unit != 1 && c.ksplit != cfg.ksplit))) {
+    if (slot > 0 && (c.unit != cfg.unit || (c.unit == 2 && c.ksplit != cfg.ksplit))) {
       return hipErrorNotSupported;  // every member runs in the configuration it would get alone
     }
     cfg               = c;
@@ -952,7 +1089,9 @@ hipError_t launch_gemm_i8_fragments_group(hipStream_t stream, int count, float *
     total += member_workgroups(m_tiles, n_tiles, cfg, plan);
   }
   grp.count = count;
-  if (cfg.unit == 1) {
+  if (cfg.unit == kStagedUnit) {
+    hipLaunchKernelGGL(gemm_i8_fragments_staged_kernel, dim3(total), dim3(kStWaves * kWave), 0, stream, grp, m, m_tiles);
+  } else if (cfg.unit == 1) {
     hipLaunchKernelGGL(gemm_i8_fragments_small_kernel, dim3(total), dim3(kGiThreads), 0, stream, grp, m, m_tiles);
   } else if (cfg.ksplit == 4) {
     hipLaunchKernelGGL((gemm_i8_fragments_kernel<4, 2, 2>), dim3(total), dim3(kGiThreads), 0, stream, grp, m, m_tiles);
@@ -960,6 +1099,38 @@ hipError_t launch_gemm_i8_fragments_group(hipStream_t stream, int count, float *
     hipLaunchKernelGGL((gemm_i8_fragments_kernel<2, 2, 2>), dim3(total), dim3(kGiThreads), 0, stream, grp, m, m_tiles);
   }
   return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_gemm_i8_fragments_group(hipStream_t stream, int count, float *const *outs,
+                                          const void *const *act_fragments, const void *const *weight_fragments,
+                                          const int *ns, const int *ks, int m, void *exchange, size_t exchange_bytes,
+                                          unsigned *tickets, int ticket_slots, int forced_unit) {
+  if (count < 1 || count > kGemmGroupMax || m <= 0) {
+    return hipErrorInvalidValue;
+  }
+  for (int staged = 1; staged >= 0; --staged) {
+    float      *out[kGemmGroupMax];
+    const void *act[kGemmGroupMax], *weight[kGemmGroupMax];
+    int         n[kGemmGroupMax], k[kGemmGroupMax], members = 0;
+    for (int i = 0; i < count; ++i) {
+      if (ks[i] <= 0 || ks[i] % 32 != 0 || ns[i] <= 0) {
+        return hipErrorInvalidValue;
+      }
+      if ((tile_config(m, ns[i], ks[i], forced_unit).unit == kStagedUnit) == (staged != 0)) {
+        out[members] = outs[i], act[members] = act_fragments[i], weight[members] = weight_fragments[i];
+        n[members] = ns[i], k[members++] = ks[i];
+      }
+    }
+    if (members > 0) {
+      if (hipError_t e = launch_members(stream, members, out, act, weight, n, k, m, exchange, exchange_bytes, tickets,
+                                        ticket_slots, forced_unit); e != hipSuccess) {
+        return e;
+      }
+    }
+  }
+  return hipSuccess;
 }
 
 hipError_t launch_gemm_i8_fragments(hipStream_t stream, float *out, const void *act_q8_0, const void *weight_fragments,

@@ -31,11 +31,23 @@ def test_split_k_at_the_edges(ctx, oracle, wt, m, k, n):
     assert np.array_equal(first, again)
 
 
+@pytest.mark.parametrize("wt", [wl.GGML_TYPE_Q4_0, wl.GGML_TYPE_Q8_0])
+@pytest.mark.parametrize("m,k,n", [
+    (97, 32, 16384), (128, 96, 16383), (110, 320, 16400),  # one, three and ten blocks; ragged columns
+    (225, 64, 8161), (256, 1120, 8192)])                   # two row blocks, the last row tile ragged or whole
+def test_staged_operands_at_the_edges(ctx, oracle, wt, m, k, n):
+    ctx.set_option("gemm_fp6", 0)
+    rng = wl.rng_for(59, m * 131 + k + n + wt)
+    first, x, w = check_mat_mul(ctx, oracle, rng, m, k, n, wt)
+    assert np.array_equal(first, ctx.run_mat_mul(oracle.quantize_q8_0(x), w, m, k, n, wt))
+    ctx.set_option("gemm_fp6", api.DEFAULT_OPTIONS["gemm_fp6"])
+
+
 @pytest.mark.parametrize("m", [17, 50, 128])
 def test_grouped_split_k_equals_single_requests(ctx, oracle, m):
     rng = wl.rng_for(60, m)
     wt, op = wl.GGML_TYPE_Q8_0, api.HTP_OPS_MAT_MUL_Q8_0_Q8_0
-    shapes = [(96, 1536), (256, 1536), (64, 8960), (40, 256), (1000, 1536)]
+    shapes = [(96, 1536), (256, 1536), (64, 8960), (40, 256), (1000, 1536)] + ([(16384, 256)] if m == 128 else [])  # (the last: staged)
     acts = {k: ctx.upload(oracle.quantize_q8_0(wl.make_activations(rng, m, k))) for k in (1536, 8960, 256)}
     ws = [ctx.upload(wl.make_weights(rng, n, k, wt)) for n, k in shapes]
     results = []
