@@ -17,7 +17,8 @@
 //   act       converted per call from block_q8_0 rows (a pure re-ordering)
 // A wave owns 64 x 64 outputs (2 x 2 units per block) and a share of K; the KSPLIT waves of one tile are summed
 // through LDS in a fixed order. Launches with too few such tiles to fill the chip use 32 x 32 tiles (one unit per
-// block) instead: four times the workgroups, each with a quarter of the vector-ALU work.
+// block) instead: four times the workgroups, each with a quarter of the vector-ALU work; matrices that leave CUs idle
+// even so have K split over workgroups too. From 256 tiles of 128 x 64 on both operands are staged through LDS.
 #include "device_utils.h"
 #include "kernels.h"
 

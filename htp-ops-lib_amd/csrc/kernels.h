@@ -109,9 +109,9 @@ hipError_t launch_gemm_i8_fragments(hipStream_t stream, float *out, const void *
                                     size_t exchange_bytes, unsigned *tickets, int ticket_slots, int forced_unit);
 // The same for up to kGemmGroupMax matmuls of one row count m in one launch each for the conversions and the products:
 // member i multiplies the converted activations act_fragments[i] (gemm_i8_act_fragment_bytes(m, ks[i]) each; members
-// that read the same rows may share one) by weight_fragments[i]. Every member must be `groupable` (the tile
-// configuration it gets depends on (m, n) alone, and a launch has one), else hipErrorNotSupported; a member's result
-// is bit for bit what its own launch gives, provided `exchange` holds the sum of the members' exchange bytes.
+// that read the same rows may share one) by weight_fragments[i]. Every member must be `groupable` (one of
+// the tile configurations that take members of any k, each of them a launch of its own), else hipErrorNotSupported; a
+// member's result is bit for bit what its own launch gives, provided `exchange` holds the sum of the members' exchange bytes.
 constexpr int kGemmGroupMax = 8;
 bool       gemm_i8_fragments_groupable(int m, int n, int forced_unit);
 // launch_gemm_fp6_lds for up to kGemmGroupMax matmuls over the SAME activation rows (one conversion, act_tiles): the

@@ -42,7 +42,8 @@ namespace {
 //    launch; where a real data dependency exists (o after attention after q/k/v) the run is split there;
 //  * 2..16 rows: members of the same k; those that take the repacked-weight kernel share its launch whatever rows
 //    they read, the others only with members that read the same rows (q/k/v or gate/up);
-//  * many rows on small output tiles: one launch for the products, one for the activation conversions.
+//  * many rows (17 and more over converted weights): one launch per tile configuration for the products, one for the
+//    conversions of activations that their quantizers have not left in operand order already.
 struct GemvBatch {
   int                   wt = 0, m = 0, count = 0;
   struct RequestHeader *hdr[kGemvGroupMax];
