@@ -142,7 +142,7 @@ struct PermutedMatMul {
 };
 // out fp32 [m][n] = fp16(act fp16 x W fp16), the weights read as they lie, nothing converted or kept: up to kPermutedGroupMax
 // matmuls of one row count and weight kind in one launch (plus one that puts the distinct activations into operand order
-// where they do not fit LDS). The caller guarantees that no member reads what another writes. A member's result does not
+// where they do not fit LDS). The caller guarantees that no member reads what one of them writes. A member's result does not
 // depend on the others. The first for up to kPermutedRowsMax rows, the second for more; `workspace`: theirs.
 constexpr int kPermutedRowsMax = 32;
 size_t     permuted_rows_workspace_bytes(const PermutedMatMul *members, int count, int m);
@@ -151,6 +151,8 @@ hipError_t launch_permuted_rows_group(hipStream_t stream, const PermutedMatMul *
 size_t     permuted_gemm_workspace_bytes(const PermutedMatMul *members, int count, int m);
 hipError_t launch_permuted_gemm_group(hipStream_t stream, const PermutedMatMul *members, int count, int m, int weight_kind,
                                       void *workspace);
+// Results made aside to where they belong; 16-byte aligned, a multiple of 16 bytes, no overlap.
+hipError_t launch_copy_results(hipStream_t stream, float *dst, const float *src, size_t bytes);
 
 // attention; see htpops_flash_attn_ptr. `workspace` holds split-KV partials (decode), size from
 // flash_attn_workspace_bytes. `q8_out` (or nullptr; used only where flash_attn_writes_q8_0 says so: decode with

@@ -564,6 +564,12 @@ __global__ __launch_bounds__(256, 2) void permuted_gemm_kernel(const GemmArgs ar
   }
 }
 
+__global__ __launch_bounds__(256) void copy_results_kernel(uint4 *__restrict__ dst, const uint4 *__restrict__ src, size_t count) {
+  for (size_t i = (size_t) blockIdx.x * 256 + threadIdx.x; i < count; i += (size_t) gridDim.x * 256) {
+    dst[i] = src[i];
+  }
+}
+
 template <int KIND>
 hipError_t launch_gemm_kind(hipStream_t stream, const GemmArgs &args, unsigned grid, int r) {
   void (*kernel)(GemmArgs) = nullptr;
@@ -753,6 +759,13 @@ hipError_t launch_permuted_gemm_group(hipStream_t stream, const PermutedMatMul *
     default:
       return launch_gemm_kind<4>(stream, args, (unsigned) grid, r);
   }
+}
+
+hipError_t launch_copy_results(hipStream_t stream, float *dst, const float *src, size_t bytes) {
+  const size_t count = bytes / 16;
+  hipLaunchKernelGGL(copy_results_kernel, dim3((unsigned) std::min<size_t>((count + 255) / 256, 4096)), dim3(256), 0, stream,
+                     reinterpret_cast<uint4 *>(dst), reinterpret_cast<const uint4 *>(src), count);
+  return hipGetLastError();
 }
 
 }  // namespace htpops

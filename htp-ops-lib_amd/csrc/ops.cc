@@ -378,13 +378,27 @@ int op_mat_mul_permuted_group(htpops_context *ctx, const PermutedMatMul *members
   for (int i = 0; i < count; ++i) {
     note_device_write(ctx, members[i].out, (size_t) m * members[i].n * 4);
   }
-  const bool few = m <= kPermutedRowsMax;
-  if (int r = ensure_workspace(ctx, few ? permuted_rows_workspace_bytes(members, count, m) :
-                                          permuted_gemm_workspace_bytes(members, count, m))) {
+  const bool   few   = m <= kPermutedRowsMax;
+  const size_t bytes = few ? permuted_rows_workspace_bytes(members, count, m) : permuted_gemm_workspace_bytes(members, count, m);
+  // The kernels read rows and weights while other workgroups of the launch store results. A result that lies over either (only
+  // a request by itself: the members of a batch leave each other's buffers alone) is made behind the workspace and copied.
+  PermutedMatMul aside     = members[0];
+  float *const   where     = aside.out;
+  const size_t   out_bytes = (size_t) m * aside.n * 4, w_bytes = permuted_weight_bytes((size_t) aside.n, (size_t) aside.k, kind);
+  const bool     overlaps  = count == 1 && (ranges_overlap(where, out_bytes, aside.act, (size_t) m * aside.k * 4) ||
+                                        ranges_overlap(where, out_bytes, aside.weight, w_bytes));
+  if (int r = ensure_workspace(ctx, bytes + (overlaps ? out_bytes : 0))) {
     return r;
+  }
+  if (overlaps) {
+    aside.out = reinterpret_cast<float *>(static_cast<uint8_t *>(ctx->workspace) + bytes);
+    members   = &aside;
   }
   HTPOPS_HIP(ctx, few ? launch_permuted_rows_group(ctx->stream, members, count, m, kind, ctx->workspace) :
                         launch_permuted_gemm_group(ctx->stream, members, count, m, kind, ctx->workspace));
+  if (overlaps) {
+    HTPOPS_HIP(ctx, launch_copy_results(ctx->stream, where, aside.out, out_bytes));
+  }
   return HTPOPS_OK;
 }
 
