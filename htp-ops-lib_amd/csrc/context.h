@@ -250,7 +250,8 @@ struct MatMulPlan {
 };
 
 // `act_aligned`: the Q8_0 activations start on a 4-byte boundary (the re-tiling pass of the FP6 kernel reads dwords)
-MatMulPlan plan_mat_mul(htpops_context *ctx, const void *weight, bool act_aligned, int m, int k, int n, int wt);
+MatMulPlan plan_mat_mul(htpops_context *ctx, const void *weight, bool act_aligned, int m, int k, int n, int wt,
+                        bool overwrites = false);
 // The converted copy a plan wants, from the cache or made now and cached (plan.cacheable); *out stays nullptr for a
 // plan whose weights may not be cached (the caller converts into its workspace).
 int plan_weight_copy(htpops_context *ctx, MatMulPlan &plan, const void *weight, int k, int n, int wt, const void **out);

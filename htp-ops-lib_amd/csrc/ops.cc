@@ -166,7 +166,8 @@ int lane_order_weights(htpops_context *ctx, const void *weight, const void *act,
 }
 
 // `act_aligned`: the Q8_0 activations start on a 4-byte boundary (the re-tiling pass of the FP6 kernel reads dwords)
-MatMulPlan plan_mat_mul(htpops_context *ctx, const void *weight, bool act_aligned, int m, int k, int n, int wt) {
+// `overwrites`: the output lies over the weights, so no copy of them is used or kept (one is made in the workspace, in order)
+MatMulPlan plan_mat_mul(htpops_context *ctx, const void *weight, bool act_aligned, int m, int k, int n, int wt, bool overwrites) {
   MatMulPlan p;
   if (m < kManyRowsMinM || k % 32 != 0) {
     p.ws_bytes = mat_mul_workspace_bytes(m, k, n);
@@ -174,8 +175,8 @@ MatMulPlan plan_mat_mul(htpops_context *ctx, const void *weight, bool act_aligne
   }
   auto lookup_copy = [&](int frag_kind) {
     p.frag_kind = frag_kind;
-    p.cached    = find_copy(ctx, weight, frag_kind, k, n);
-    p.cacheable = !p.cached && may_keep_copies(ctx, weight, weight_bytes((size_t) n, (size_t) k, wt));
+    p.cached    = overwrites ? nullptr : find_copy(ctx, weight, frag_kind, k, n);
+    p.cacheable = !overwrites && !p.cached && may_keep_copies(ctx, weight, weight_bytes((size_t) n, (size_t) k, wt));
   };
   // Q4_0 weights whose converted copy may be kept, on a shape whose output tiles fill the device: the FP6 kernel over
   // that copy (half the vector-ALU work per block sum of the int8 path). Registered memory that was never prepared
@@ -197,7 +198,7 @@ MatMulPlan plan_mat_mul(htpops_context *ctx, const void *weight, bool act_aligne
   // 17 to 32 rows, K-sliced kernel / here: seven projections of a Llama-7B / Qwen2-1.5B layer, Q8_0, 117 and 65 us in seven
   // launches / 47 and 19 us; one matrix over fp32 rows, k = 8960, n = 1537 13.2 / 11.9, k = 4096, n = 11008 27.5 / 17.0,
   // but k = 1024, n = 700 8.4 / 9.6.
-  if (m < kFp6MinM) {
+  if (m < kFp6MinM && !overwrites) {
     lookup_copy(kFragKindRowLayout + wt);
     if (!p.cached && !p.cacheable) {
       p.ws_bytes = mat_mul_workspace_bytes(m, k, n);
@@ -279,11 +280,11 @@ int run_few_rows(htpops_context *ctx, float *dst, const void *act, const void *w
   return HTPOPS_OK;
 }
 
-// `ws` is this matmul's share of the workspace (plan.ws_bytes, already ensured by the caller). act = nullptr (int8 fragments
-// only): the activations lie at its start in operand order already.
+// `ws` is this matmul's share of the workspace (plan.ws_bytes, already ensured by the caller, who has noted the write to `dst`
+// before planning: it drops copies). act = nullptr (int8 fragments only): the activations lie at its start in operand order
+// already.
 int run_mat_mul(htpops_context *ctx, MatMulPlan &plan, float *dst, const void *act, const void *weight, int m, int k,
                 int n, int wt, uint8_t *ws) {
-  note_device_write(ctx, dst, (size_t) m * n * 4);
   if (plan.kind == kPlanFewRows) {
     ctx->act_fragments.src = nullptr;  // these kernels put something else at the start of the workspace
     return run_few_rows(ctx, dst, act, weight, m, k, n, wt, ws);
@@ -303,8 +304,8 @@ int run_mat_mul(htpops_context *ctx, MatMulPlan &plan, float *dst, const void *a
     frags = fresh;
   }
   // The converted activations at the start of the workspace are shared by the requests of a message that read the same
-  // rows with the same kernel family (note_device_write above has already cleared the record if this matmul writes
-  // into its own activations).
+  // rows with the same kernel family (note_device_write has already cleared the record if this matmul writes into its own
+  // activations).
   auto      &af    = ctx->act_fragments;
   const bool ready = !act || (af.src == act && af.m == m && af.k == k && af.kind == (int) plan.kind && ws == ctx->workspace);
   const bool keep  = act && (ready || (ctx->in_message && ws == ctx->workspace &&
@@ -325,6 +326,10 @@ int run_mat_mul(htpops_context *ctx, MatMulPlan &plan, float *dst, const void *a
   return HTPOPS_OK;
 }
 
+bool writes_weights(const void *dst, const void *weight, int m, int k, int n, int wt) {
+  return ranges_overlap(dst, (size_t) m * n * 4, weight, weight_bytes((size_t) n, (size_t) k, wt));
+}
+
 }  // namespace
 
 int op_mat_mul_q8(htpops_context *ctx, float *dst, const void *act, const void *weight, int m, int k, int n,
@@ -335,7 +340,8 @@ int op_mat_mul_q8(htpops_context *ctx, float *dst, const void *act, const void *
   if (int r = need_device(ctx)) {
     return r;
   }
-  MatMulPlan plan = plan_mat_mul(ctx, weight, aligned(act, 4), m, k, n, weight_type);
+  note_device_write(ctx, dst, (size_t) m * n * 4);
+  MatMulPlan plan = plan_mat_mul(ctx, weight, aligned(act, 4), m, k, n, weight_type, writes_weights(dst, weight, m, k, n, weight_type));
   if (int r = ensure_workspace(ctx, plan.ws_bytes, /*keep_act_fragments=*/true)) {
     return r;
   }
@@ -353,7 +359,8 @@ int op_mat_mul_f32(htpops_context *ctx, float *dst, const float *act, const void
   if (int r = need_device(ctx)) {
     return r;
   }
-  MatMulPlan plan = plan_mat_mul(ctx, weight, true, m, k, n, weight_type);
+  note_device_write(ctx, dst, (size_t) m * n * 4);
+  MatMulPlan plan = plan_mat_mul(ctx, weight, true, m, k, n, weight_type, writes_weights(dst, weight, m, k, n, weight_type));
   if (plan.kind == kPlanFragments && (long long) m * (k / 32) <= 0x7fffffffLL) {
     // the quantizer writes the operand order the matmul wants: the rows in block_q8_0 form would have one reader, another
     // launch that puts them into that order (33 rows, k = 8960, n = 1537: 3 of 18 us)

@@ -1,0 +1,47 @@
+"""GPU: a many-row matmul whose output lies over its own weights, of which the context holds (or would keep) a converted
+copy: the result is that of an output elsewhere, and no copy of the overwritten weights answers a later request."""
+import numpy as np
+import pytest
+
+from pyhtpops import api
+from pyhtpops import workloads as wl
+
+pytestmark = pytest.mark.gpu
+
+OPS = {(wl.GGML_TYPE_Q4_0, False): api.HTP_OPS_MAT_MUL_Q4_0_Q8_0, (wl.GGML_TYPE_Q8_0, False): api.HTP_OPS_MAT_MUL_Q8_0_Q8_0,
+       (wl.GGML_TYPE_Q4_0, True): api.HTP_OPS_MAT_MUL_Q4_0_A32, (wl.GGML_TYPE_Q8_0, True): api.HTP_OPS_MAT_MUL_Q8_0_A32}
+
+
+@pytest.mark.parametrize("wt", [wl.GGML_TYPE_Q4_0, wl.GGML_TYPE_Q8_0])
+@pytest.mark.parametrize("m,k,n", [(20, 1024, 2048), (32, 8960, 64), (40, 512, 700), (512, 1024, 8192)])  # (the last: FP6 for Q4_0)
+@pytest.mark.parametrize("fp32_rows", [False, True])
+def test_output_over_the_weights(oracle, wt, m, k, n, fp32_rows):
+    rng = wl.rng_for(95, m + k + n + wt)
+    w, x = np.ascontiguousarray(wl.make_weights(rng, n, k, wt)).view(np.uint8).reshape(-1), wl.make_activations(rng, m, k)
+    x = x if fp32_rows else oracle.quantize_q8_0(x)
+    out_bytes = m * n * 4
+    at = w.size // 2 // 256 * 256  # the output covers the weights' second half and what lies behind
+    image = np.zeros(max(w.size, at + out_bytes), np.uint8)
+    image[:w.size] = w
+    print("matmul over its weights", wt, m, k, n, fp32_rows, flush=True)
+    with api.Context(device=0) as ctx:
+        op = OPS[wt, fp32_rows]
+        hx, hw, hb, ho = ctx.upload(x), ctx.upload(w), ctx.upload(image), ctx.alloc(out_bytes)
+
+        def run(out, weights, rows=m):
+            assert ctx.execute(op, api.mat_mul_params(out, (hx, 0), (weights, 0), rows, k, n)) == 0, ctx.last_error()
+            ctx.synchronize()
+            return ctx.read(out[0], np.float32, rows * n, out[1]).reshape(rows, n)
+
+        want = run((ho, 0), hw)
+        assert np.array_equal(want, run((ho, 0), hb)) and want.any()  # (a copy of the second buffer's weights is there now)
+        got = run((hb, at), hb)
+        if m <= 40:
+            assert np.array_equal(want, got)
+        else:  # (without a copy that may be kept Q4_0 takes the int8 kernels: other fp32 sums over the same exact block sums)
+            assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max()
+        # what lies there now, read as weights: the columns whose blocks were left alone are what they were
+        left = at // (w.size // n)
+        assert np.array_equal(run((ho, 0), hb)[:, :left], want[:, :left])
+        ctx.write(hb, image)
+        assert np.array_equal(run((ho, 0), hb), want)
