@@ -161,7 +161,7 @@ extern "C" int htpops_init_backend(htpops_context **out_ctx, int device) {
       delete ctx;
       return HTPOPS_ERR_HIP;
     }
-    if (hipMalloc(&ctx->attn_shares, kAttnSharesBytes) != hipSuccess) {
+    if (hipMalloc(&ctx->attn_shares, htpops::kAttnSharesBytes) != hipSuccess) {
       (void) hipGetLastError();
       ctx->attn_shares = nullptr;
     }

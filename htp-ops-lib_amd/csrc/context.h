@@ -47,8 +47,6 @@ constexpr int kTicketSlots = 1 << 16;
 
 // size of the static device array behind htpops_flash_attn_noalloc_ptr (context.cc)
 constexpr size_t kNoAllocScratchBytes = (size_t) 8 << 20;
-// size of htpops_context::attn_shares: two shares of 512 queries of 32 heads of 128 take 17 MB
-constexpr size_t kAttnSharesBytes = (size_t) 32 << 20;
 
 // The switches of a context: kernel choices that tests and A/B measurements override. Read once from the environment
 // when the context is created (HTPOPS_<NAME> in upper case), changed afterwards only through htpops_set_option; no
@@ -97,8 +95,9 @@ struct htpops_context {
   void  *workspace       = nullptr;
   size_t workspace_bytes = 0;
   // What the workgroups that share a query block's keys leave for their merge (attention of several query rows, or of a
-  // head dim that one-row attention has no kernel for): one block for the context's life, so the entry point that may not
-  // allocate splits its keys as the ordinary one does. nullptr (no memory when the context was made): keys are not split.
+  // head dim that one-row attention has no kernel for): kAttnSharesBytes for the context's life (recordings hold the
+  // address), there from the start so that the entry point that may not allocate has it too. nullptr (no memory when the
+  // context was made): one workgroup walks all shares, with the same results.
   void *attn_shares = nullptr;
   // zeroed ticket counters of the K-sliced matmul (each launch leaves them zeroed)
   unsigned *tickets = nullptr;

@@ -58,9 +58,28 @@ __device__ __forceinline__ float fast_exp2(float x) {
 
 // ------------------------------------------------------------------------------------------------ prefill
 
+// Two states (max, sum, O) of one query become one: m takes the larger maximum; the factors of the state that m belonged to
+// (`keep`) and of the other (returned). Written once, and with the fused operations spelled out, so that the same states
+// give the same bits wherever they meet.
+__device__ __forceinline__ float fold_factors(float &m, float other, float &keep) {
+  const float m_new  = fmaxf(m, other);
+  const float m_safe = (m_new == -INFINITY) ? 0.0f : m_new;  // nothing visible at all: keep the exponents finite
+  keep = fast_exp2(m - m_safe);
+  m    = m_new;
+  return fast_exp2(other - m_safe);
+}
+__device__ __forceinline__ float fold(float fa, float a, float fb, float b) {
+  return __builtin_fmaf(fa, a, fb * b);
+}
+template <int N>
+struct Const {
+  static constexpr int value = N;
+};
+
 constexpr int kPfThreads = 256;  // threads of one key group: 4 waves, one per query head
 constexpr int kBQ        = 32;  // query rows per wave tile
 constexpr int kBK        = 64;  // keys per KV block
+constexpr int kPfMergeChunk = 8;  // shares whose parts the merge kernel has under way at a time
 
 // One key group's share of LDS. K and V tiles of a block of keys, two buffers each: the next block arrives by DMA while
 // one is used (the DMA chooses what each lane fetches, not where it lands: a lane lands 16 bytes behind its neighbour).
@@ -90,13 +109,17 @@ __host__ __device__ constexpr size_t prefill_partial_floats(int units) {
 // 22 bits (an fp16 pair, two matrix instructions per fragment of V): the plain kernel that these head dims took before
 // held them in fp32. GROUPS = 1 or 2 key groups per workgroup (4 waves each); with 2 they take alternate KV blocks of the
 // same queries. MASK: there is one (a kernel of its own: the tests for it cost 2048 x 2048 without one 1 to 2 %). With
-// gridDim.z > 1 the blocks of a workgroup's queries are dealt to gridDim.z workgroups, each of which leaves its
-// (max, sum, O) in `part` for flash_attn_prefill_merge_kernel.
-template <int DP, bool FULL, bool QO_F32, int GROUPS, bool MASK>
+// `shares` > 1 the blocks of a workgroup's queries are dealt to that many workgroups (gridDim.z), each of which leaves its
+// (max, sum, O) in `part` for flash_attn_prefill_merge_kernel. ALL: one workgroup walks all shares itself and folds them in
+// registers in the order and with the arithmetic of that kernel: the same bits without any memory between workgroups, for
+// launches that must not hold an address of the context's (the mask may be absent then). It is bound by latency, like the
+// unsplit walk, and pays for every share a handing-over through LDS: 5 rows over 1029 keys, 12 / 2 heads of 128, 8 shares 45 us
+// against 20 us unsplit and 12 us on 32 workgroups; 500 rows over 500, 16 / 4 heads of 96, 22 us against 19.
+template <int DP, bool FULL, bool QO_F32, int GROUPS, bool MASK, bool ALL>
 __global__ __launch_bounds__(kPfThreads *GROUPS, DP <= 128 ? 2 : 1) void flash_attn_prefill_kernel(
   void *__restrict__ o_ptr, const void *__restrict__ q_ptr, const _Float16 *__restrict__ k_ptr,
   const _Float16 *__restrict__ v_ptr, const _Float16 *__restrict__ mask, int qo_len, int kv_len, int n_heads,
-  int n_kv_heads, int head_dim, int flags, float *__restrict__ part) {
+  int n_kv_heads, int head_dim, int flags, float *__restrict__ part, int shares) {
   using Smem = PrefillSmem<DP, MASK>;
   const bool causal = (flags & 1) != 0, mask_threshold = (flags & 2) != 0;
   __shared__ __align__(1024) Smem sm_all[GROUPS];
@@ -186,9 +209,7 @@ __global__ __launch_bounds__(kPfThreads *GROUPS, DP <= 128 ? 2 : 1) void flash_a
   const int q_shift  = kv_len - qo_len;
   // last key this lane's query may see, relative to the first key this lane holds in a block (key0 = 4 * half)
   const int vis_last = (causal ? min(kv_len - 1, q_row + q_shift) : kv_len - 1) - 4 * half;
-  // this workgroup's share of the blocks
-  const int per  = ((kv_limit + kBK - 1) / kBK + (int) gridDim.z - 1) / (int) gridDim.z * kBK;
-  const int k_lo = (int) blockIdx.z * per, k_hi = min(kv_limit, k_lo + per);
+  const int per = ((kv_limit + kBK - 1) / kBK + shares - 1) / shares * kBK;  // keys of a share
 
   // The next K/V block travels global memory -> LDS by DMA (global_load_lds, 1 KiB per instruction: no registers, no
   // stores) while the current one is being used. A tile of 64 rows is as many instructions as a row has pieces, the four
@@ -221,7 +242,7 @@ __global__ __launch_bounds__(kPfThreads *GROUPS, DP <= 128 ? 2 : 1) void flash_a
     const int piece = v_piece(j, row);
     v_src[j] = (uint32_t) row * (uint32_t) (kv_stride * 2) + 16u * (uint32_t) piece;
   }
-  auto fetch = [&](int k0, int buf) {
+  auto fetch = [&](int k0, int buf) __attribute__((always_inline)) {  // (in registers: the DMA takes scalar bases)
     const uint32_t to_k = (uint32_t) (uintptr_t) sm.k[buf], to_v = (uint32_t) (uintptr_t) sm.v[buf];
     if (k0 + kBK <= kv_len) {
       const uint8_t *kb = reinterpret_cast<const uint8_t *>(k_ptr + (size_t) h_kv * D + (size_t) k0 * kv_stride);
@@ -272,7 +293,7 @@ __global__ __launch_bounds__(kPfThreads *GROUPS, DP <= 128 ? 2 : 1) void flash_a
     const int row = 8 * i + (lane >> 3);
     mask_src[i]   = (uint32_t) min(row, mask_rows - 1) * (uint32_t) (mask_ld * 2) + 16u * (uint32_t) ((lane & 7) ^ (row & 7));
   }
-  auto fetch_mask = [&](int k0) {
+  auto fetch_mask = [&](int k0) __attribute__((always_inline)) {
     const _Float16 *base = mask + (size_t) q_base * mask_ld + k0;
     const uint32_t  to   = (uint32_t) (uintptr_t) sm.mask[wave];
     if (mask_wide) {
@@ -310,213 +331,361 @@ __global__ __launch_bounds__(kPfThreads *GROUPS, DP <= 128 ? 2 : 1) void flash_a
   }
   typedef short v4s __attribute__((ext_vector_type(4)));
 
-  const bool use_mask = MASK && wave_on;
+  const bool use_mask = MASK && wave_on && (!ALL || mask != nullptr);
   uint2      mreg[2][4];  // this lane's 2 x 16 mask values: keys 32 kt + 8 rg + 4 half + 0 .. 3
-  if (k_lo + grp * kBK < k_hi) {
-    fetch(k_lo + grp * kBK, 0);
-    if (use_mask) {
-      fetch_mask(k_lo + grp * kBK);
-    }
-  }
 
-  int it = 0;
-  for (int kk = k_lo; kk < k_hi; kk += GROUPS * kBK, ++it) {
-    const int  k0   = kk + grp * kBK;  // this key group's block of the iteration
-    const int  buf  = it & 1;
-    // this wave's share of the block has landed; behind the barrier everybody's has, and nobody reads the other
-    // buffer (the previous block) any more
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    bool live = wave_on && k0 < k_hi;  // (the last iteration may have a block for the first group only)
-    bool plain = true;                 // no mask value of the wave's block is anything but zero
-    if (use_mask && k0 < k_hi) {
-      uint32_t all = 0xffffffffu, any = 0;
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt) {
-#pragma unroll
-        for (int rg = 0; rg < 4; ++rg) {
-          mreg[kt][rg] = *reinterpret_cast<const uint2 *>(sm.mask[wave] + col * 128 + 16 * ((4 * kt + rg) ^ (col & 7)) + 8 * half);
-          all &= mreg[kt][rg].x & mreg[kt][rg].y;
-          any |= mreg[kt][rg].x | mreg[kt][rg].y;
-        }
-      }
-      // (the values are in registers before the next block's overwrite them)
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      plain = __builtin_amdgcn_ballot_w64((any & 0x7fff7fffu) != 0) == 0;
-      // A block that the mask hides from all 32 queries (-inf throughout; a causal mask hides half of a prompt's blocks)
-      // is passed over, as under `causal`.
-      if (__builtin_amdgcn_ballot_w64(!(all == 0xfc00fc00u && any == 0xfc00fc00u)) == 0) {
-        live = false;
-      }
-    }
-    if (k0 + GROUPS * kBK < k_hi) {
-      fetch(k0 + GROUPS * kBK, buf ^ 1);
-      if (use_mask) {
-        fetch_mask(k0 + GROUPS * kBK);
-      }
-    }
-    if (!live) {
-      continue;
-    }
-    const uint8_t *k_tile = sm.k[buf], *v_tile = sm.v[buf];
-
-    // ---- S^T - m = K Q^T - m: two 32-key tiles, accumulated on top of minus the running maximum ----
-    // Scores come out of the MFMA already relative to the maximum seen so far, so a block that brings no new maximum
-    // to any query of the wave (the usual case after the first few blocks) needs no subtraction and no rescaling.
-    const bool  fresh = m_run == -INFINITY;  // nothing visible yet for this query
-    const float m_ref = fresh ? 0.0f : m_run;
-    v16f st[2];
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        st[kt][r] = -m_ref;
-      }
-    }
-    // the two key tiles advance side by side (independent accumulators), and the fragments of step s + PF are
-    // requested before the products of step s
-    {
-      constexpr int PF = 3;  // steps ahead (an LDS read takes longer to return than two steps' products to issue)
-      v8h kf[PF + 1][2];
-#pragma unroll
-      for (int s = 0; s < PF && s < KSTEPS; ++s) {
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt) {
-          kf[s][kt] = *reinterpret_cast<const v8h *>(k_tile + k_at[s] + 32 * kt * KROWB);
-        }
-      }
-#pragma unroll
-      for (int s = 0; s < KSTEPS; ++s) {
-        if (s + PF < KSTEPS) {
-#pragma unroll
-          for (int kt = 0; kt < 2; ++kt) {
-            kf[(s + PF) % (PF + 1)][kt] = *reinterpret_cast<const v8h *>(k_tile + k_at[s + PF] + 32 * kt * KROWB);
-          }
-        }
-        if (!FULL && s == KSTEPS - 1 && 16 * s >= D) {
-          continue;  // (behind the head dim, the same for all waves)
-        }
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt) {
-          st[kt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[s % (PF + 1)][kt], qf[s], st[kt], 0, 0, 0);
-        }
-      }
-    }
-
-    // ---- mask (lane = query; register r of tile kt is key k0 + 32 kt + 8 (r / 4) + 4 half + r % 4) ----
-    // Only blocks that mask values other than zero, the causal diagonal or the end of the keys touch pay for it (the same
-    // for the whole wave).
-    if (!plain || k0 + kBK > kv_len || (causal && k0 + kBK - 1 > q_base + q_shift)) {
-      const int last = vis_last - k0;  // registers whose key offset 32 kt + 8 (r / 4) + r % 4 exceeds it are hidden
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt) {
-#pragma unroll
-        for (int rg = 0; rg < 4; ++rg) {
-          float add[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
-          if (!plain) {
-            const v4h mv = __builtin_bit_cast(v4h, mreg[kt][rg]);
-            add[0] = mask_term(mv[0], mask_threshold), add[1] = mask_term(mv[1], mask_threshold);
-            add[2] = mask_term(mv[2], mask_threshold), add[3] = mask_term(mv[3], mask_threshold);
-          }
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int r = 4 * rg + e;
-            st[kt][r]   = (32 * kt + 8 * rg + e > last) ? -INFINITY : st[kt][r] + add[e];
-          }
-        }
-      }
-    }
-
-    // ---- online softmax on scores relative to m_ref ----
-    float mx = -INFINITY;
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        mx = fmaxf(mx, st[kt][r]);
-      }
-    }
-    {
-      // both 32-lane halves of the wave hold the same queries: v_permlane32_swap hands each the other's maximum
-      const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
-      mx            = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
-    }
-    // the first visible block of a query sets its maximum (either sign), later blocks only raise it
-    const bool move = fresh ? (mx != -INFINITY) : (mx > 0.0f);
-    if (__builtin_amdgcn_ballot_w64(move) != 0) {
-      // (a statement the compiler cannot run ahead of the test: without it the 97 instructions below are turned into
-      // selects and run for every block)
-      asm volatile("" ::: "memory");
-      const float delta = move ? mx : 0.0f;
-      const float alpha = fresh ? 0.0f : fast_exp2(-delta);  // O and l of a fresh query are still zero
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          st[kt][r] -= delta;
-        }
-      }
+  // the keys of share `z`, from an empty state
+  auto walk = [&](int z) __attribute__((always_inline)) {
+    const int k_lo = z * per, k_hi = min(kv_limit, k_lo + per);
+    if constexpr (ALL) {
+      __syncthreads();  // (nobody uses LDS for the share before any more)
+      m_run = -INFINITY, l_run = 0.0f;
 #pragma unroll
       for (int t = 0; t < DT; ++t) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          oacc[t][r] *= alpha;
+          oacc[t][r] = 0.0f;
         }
       }
-      l_run *= alpha;
-      m_run = move ? m_ref + mx : m_run;
     }
-    // the probabilities, rounded to fp16 in pairs as the matrix instruction takes them. FULL: the row sum adds up the
-    // rounded values (v_dot2_f32_f16 with ones: two per instruction, fp32 sums), so O and l see the same numbers; else
-    // what the rounding left out goes into a second fp16 pair and the row sum adds up the fp32 values.
-    uint32_t pk[2][8], pk_lo[FULL ? 1 : 2][FULL ? 1 : 8];
-    float    psum[4] = { 0.0f, 0.0f, 0.0f, 0.0f };  // (four chains: an addition waits for the one before it in its chain)
-    {
-      const v2h ones = { (_Float16) 1.0f, (_Float16) 1.0f };
+    if (k_lo + grp * kBK < k_hi) {
+      fetch(k_lo + grp * kBK, 0);
+      if (use_mask) {
+        fetch_mask(k_lo + grp * kBK);
+      }
+    }
+
+    int it = 0;
+    for (int kk = k_lo; kk < k_hi; kk += GROUPS * kBK, ++it) {
+      const int  k0   = kk + grp * kBK;  // this key group's block of the iteration
+      const int  buf  = it & 1;
+      // this wave's share of the block has landed; behind the barrier everybody's has, and nobody reads the other
+      // buffer (the previous block) any more
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      bool live = wave_on && k0 < k_hi;  // (the last iteration may have a block for the first group only)
+      bool plain = true;                 // no mask value of the wave's block is anything but zero
+      if (use_mask && k0 < k_hi) {
+        uint32_t all = 0xffffffffu, any = 0;
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt) {
+#pragma unroll
+          for (int rg = 0; rg < 4; ++rg) {
+            mreg[kt][rg] = *reinterpret_cast<const uint2 *>(sm.mask[wave] + col * 128 + 16 * ((4 * kt + rg) ^ (col & 7)) + 8 * half);
+            all &= mreg[kt][rg].x & mreg[kt][rg].y;
+            any |= mreg[kt][rg].x | mreg[kt][rg].y;
+          }
+        }
+        // (the values are in registers before the next block's overwrite them)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        plain = __builtin_amdgcn_ballot_w64((any & 0x7fff7fffu) != 0) == 0;
+        // A block that the mask hides from all 32 queries (-inf throughout; a causal mask hides half of a prompt's blocks)
+        // is passed over, as under `causal`.
+        if (__builtin_amdgcn_ballot_w64(!(all == 0xfc00fc00u && any == 0xfc00fc00u)) == 0) {
+          live = false;
+        }
+      }
+      if (k0 + GROUPS * kBK < k_hi) {
+        fetch(k0 + GROUPS * kBK, buf ^ 1);
+        if (use_mask) {
+          fetch_mask(k0 + GROUPS * kBK);
+        }
+      }
+      if (!live) {
+        continue;
+      }
+      const uint8_t *k_tile = sm.k[buf], *v_tile = sm.v[buf];
+
+      // ---- S^T - m = K Q^T - m: two 32-key tiles, accumulated on top of minus the running maximum ----
+      // Scores come out of the MFMA already relative to the maximum seen so far, so a block that brings no new maximum
+      // to any query of the wave (the usual case after the first few blocks) needs no subtraction and no rescaling.
+      const bool  fresh = m_run == -INFINITY;  // nothing visible yet for this query
+      const float m_ref = fresh ? 0.0f : m_run;
+      v16f st[2];
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt) {
 #pragma unroll
-        for (int r = 0; r < 16; r += 2) {
-          const float p0 = fast_exp2(st[kt][r]), p1 = fast_exp2(st[kt][r + 1]);
-          const v2h   p2 = { (_Float16) p0, (_Float16) p1 };
-          pk[kt][r / 2]  = __builtin_bit_cast(uint32_t, p2);
-          if constexpr (FULL) {
-            psum[(r / 2) & 3] = __builtin_amdgcn_fdot2(p2, ones, psum[(r / 2) & 3], false);
-          } else {
-            const v2h lo      = { (_Float16) (p0 - (float) p2[0]), (_Float16) (p1 - (float) p2[1]) };
-            pk_lo[kt][r / 2]  = __builtin_bit_cast(uint32_t, lo);
-            psum[(r / 2) & 3] += p0 + p1;
+        for (int r = 0; r < 16; ++r) {
+          st[kt][r] = -m_ref;
+        }
+      }
+      // the two key tiles advance side by side (independent accumulators), and the fragments of step s + PF are
+      // requested before the products of step s
+      {
+        constexpr int PF = 3;  // steps ahead (an LDS read takes longer to return than two steps' products to issue)
+        v8h kf[PF + 1][2];
+#pragma unroll
+        for (int s = 0; s < PF && s < KSTEPS; ++s) {
+#pragma unroll
+          for (int kt = 0; kt < 2; ++kt) {
+            kf[s][kt] = *reinterpret_cast<const v8h *>(k_tile + k_at[s] + 32 * kt * KROWB);
+          }
+        }
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s) {
+          if (s + PF < KSTEPS) {
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) {
+              kf[(s + PF) % (PF + 1)][kt] = *reinterpret_cast<const v8h *>(k_tile + k_at[s + PF] + 32 * kt * KROWB);
+            }
+          }
+          if (!FULL && s == KSTEPS - 1 && 16 * s >= D) {
+            continue;  // (behind the head dim, the same for all waves)
+          }
+#pragma unroll
+          for (int kt = 0; kt < 2; ++kt) {
+            st[kt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[s % (PF + 1)][kt], qf[s], st[kt], 0, 0, 0);
           }
         }
       }
-    }
-    l_run += (psum[0] + psum[1]) + (psum[2] + psum[3]);
 
-    // ---- O^T += V^T P^T ----
-    // MFMA (kt, u) covers keys 32 kt + 16 u + {4 half + 0..3, 8 + 4 half + 0..3}: exactly registers 8 u .. 8 u + 7
+      // ---- mask (lane = query; register r of tile kt is key k0 + 32 kt + 8 (r / 4) + 4 half + r % 4) ----
+      // Only blocks that mask values other than zero, the causal diagonal or the end of the keys touch pay for it (the same
+      // for the whole wave).
+      if (!plain || k0 + kBK > kv_len || (causal && k0 + kBK - 1 > q_base + q_shift)) {
+        const int last = vis_last - k0;  // registers whose key offset 32 kt + 8 (r / 4) + r % 4 exceeds it are hidden
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
+        for (int kt = 0; kt < 2; ++kt) {
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const v8h pf = __builtin_bit_cast(v8h, make_uint4(pk[kt][4 * u], pk[kt][4 * u + 1], pk[kt][4 * u + 2], pk[kt][4 * u + 3]));
+          for (int rg = 0; rg < 4; ++rg) {
+            float add[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
+            if (!plain) {
+              const v4h mv = __builtin_bit_cast(v4h, mreg[kt][rg]);
+              add[0] = mask_term(mv[0], mask_threshold), add[1] = mask_term(mv[1], mask_threshold);
+              add[2] = mask_term(mv[2], mask_threshold), add[3] = mask_term(mv[3], mask_threshold);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const int r = 4 * rg + e;
+              st[kt][r]   = (32 * kt + 8 * rg + e > last) ? -INFINITY : st[kt][r] + add[e];
+            }
+          }
+        }
+      }
+
+      // ---- online softmax on scores relative to m_ref ----
+      float mx = -INFINITY;
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          mx = fmaxf(mx, st[kt][r]);
+        }
+      }
+      {
+        // both 32-lane halves of the wave hold the same queries: v_permlane32_swap hands each the other's maximum
+        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+        mx            = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+      }
+      // the first visible block of a query sets its maximum (either sign), later blocks only raise it
+      const bool move = fresh ? (mx != -INFINITY) : (mx > 0.0f);
+      if (__builtin_amdgcn_ballot_w64(move) != 0) {
+        // (a statement the compiler cannot run ahead of the test: without it the 97 instructions below are turned into
+        // selects and run for every block)
+        asm volatile("" ::: "memory");
+        const float delta = move ? mx : 0.0f;
+        const float alpha = fresh ? 0.0f : fast_exp2(-delta);  // O and l of a fresh query are still zero
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            st[kt][r] -= delta;
+          }
+        }
 #pragma unroll
         for (int t = 0; t < DT; ++t) {
-          // (V^T fragment: column 32 t + lane % 32 of keys 32 kt + 16 u + 4 half + 0 .. 3 and + 8 .. 11)
-          const uint8_t *at = v_tile + v_at[t] + (32 * kt + 16 * u) * VROWB;
-          const v4s a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((v4s __attribute__((address_space(3))) *) at);
-          const v4s a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((v4s __attribute__((address_space(3))) *) (at + 8 * VROWB));
-          const v8h vf = __builtin_bit_cast(v8h, (short __attribute__((ext_vector_type(8)))){ a0[0], a0[1], a0[2], a0[3],
-                                                                                             a1[0], a1[1], a1[2], a1[3] });
-          oacc[t]      = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pf, oacc[t], 0, 0, 0);
-          if constexpr (!FULL) {
-            const v8h pl = __builtin_bit_cast(v8h, make_uint4(pk_lo[kt][4 * u], pk_lo[kt][4 * u + 1], pk_lo[kt][4 * u + 2],
-                                                              pk_lo[kt][4 * u + 3]));
-            oacc[t]      = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pl, oacc[t], 0, 0, 0);
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            oacc[t][r] *= alpha;
+          }
+        }
+        l_run *= alpha;
+        m_run = move ? m_ref + mx : m_run;
+      }
+      // the probabilities, rounded to fp16 in pairs as the matrix instruction takes them. FULL: the row sum adds up the
+      // rounded values (v_dot2_f32_f16 with ones: two per instruction, fp32 sums), so O and l see the same numbers; else
+      // what the rounding left out goes into a second fp16 pair and the row sum adds up the fp32 values.
+      uint32_t pk[2][8], pk_lo[FULL ? 1 : 2][FULL ? 1 : 8];
+      float    psum[4] = { 0.0f, 0.0f, 0.0f, 0.0f };  // (four chains: an addition waits for the one before it in its chain)
+      {
+        const v2h ones = { (_Float16) 1.0f, (_Float16) 1.0f };
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt) {
+#pragma unroll
+          for (int r = 0; r < 16; r += 2) {
+            const float p0 = fast_exp2(st[kt][r]), p1 = fast_exp2(st[kt][r + 1]);
+            const v2h   p2 = { (_Float16) p0, (_Float16) p1 };
+            pk[kt][r / 2]  = __builtin_bit_cast(uint32_t, p2);
+            if constexpr (FULL) {
+              psum[(r / 2) & 3] = __builtin_amdgcn_fdot2(p2, ones, psum[(r / 2) & 3], false);
+            } else {
+              const v2h lo      = { (_Float16) (p0 - (float) p2[0]), (_Float16) (p1 - (float) p2[1]) };
+              pk_lo[kt][r / 2]  = __builtin_bit_cast(uint32_t, lo);
+              psum[(r / 2) & 3] += p0 + p1;
+            }
+          }
+        }
+      }
+      l_run += (psum[0] + psum[1]) + (psum[2] + psum[3]);
+
+      // ---- O^T += V^T P^T ----
+      // MFMA (kt, u) covers keys 32 kt + 16 u + {4 half + 0..3, 8 + 4 half + 0..3}: exactly registers 8 u .. 8 u + 7
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const v8h pf = __builtin_bit_cast(v8h, make_uint4(pk[kt][4 * u], pk[kt][4 * u + 1], pk[kt][4 * u + 2], pk[kt][4 * u + 3]));
+#pragma unroll
+          for (int t = 0; t < DT; ++t) {
+            // (V^T fragment: column 32 t + lane % 32 of keys 32 kt + 16 u + 4 half + 0 .. 3 and + 8 .. 11)
+            const uint8_t *at = v_tile + v_at[t] + (32 * kt + 16 * u) * VROWB;
+            const v4s a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((v4s __attribute__((address_space(3))) *) at);
+            const v4s a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((v4s __attribute__((address_space(3))) *) (at + 8 * VROWB));
+            const v8h vf = __builtin_bit_cast(v8h, (short __attribute__((ext_vector_type(8)))){ a0[0], a0[1], a0[2], a0[3],
+                                                                                               a1[0], a1[1], a1[2], a1[3] });
+            oacc[t]      = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pf, oacc[t], 0, 0, 0);
+            if constexpr (!FULL) {
+              const v8h pl = __builtin_bit_cast(v8h, make_uint4(pk_lo[kt][4 * u], pk_lo[kt][4 * u + 1], pk_lo[kt][4 * u + 2],
+                                                                pk_lo[kt][4 * u + 3]));
+              oacc[t]      = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pl, oacc[t], 0, 0, 0);
+            }
           }
         }
       }
     }
+
+  };
+
+  // O = O^T / l, one query per lane; register r of tile t is d = 32 t + 8 (r / 4) + 4 half + r % 4
+  auto store = [&](int t, const v16f &o, float inv) {
+    if (!q_ok) {
+      return;
+    }
+    const size_t base = (size_t) q_row * qo_stride + (size_t) head * D;
+#pragma unroll
+    for (int rg = 0; rg < 4; ++rg) {
+      const int d0 = 32 * t + 8 * rg + 4 * half;
+      if (!FULL && d0 >= D) {
+        continue;
+      }
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[e] = o[4 * rg + e] * inv;
+      }
+      if (QO_F32) {
+        *reinterpret_cast<float4 *>(reinterpret_cast<float *>(o_ptr) + base + d0) = make_float4(v[0], v[1], v[2], v[3]);
+      } else {
+        v4h hv = { (_Float16) v[0], (_Float16) v[1], (_Float16) v[2], (_Float16) v[3] };
+        *reinterpret_cast<v4h *>(reinterpret_cast<_Float16 *>(o_ptr) + base + d0) = hv;
+      }
+    }
+  };
+
+  // ---- all shares in this workgroup. With two key groups, each folds its half of the columns (the first KEEP tiles of O,
+  // and the others), so that the totals of a group are half the registers. ----
+  if constexpr (ALL) {
+    constexpr int KEEP  = GROUPS == 2 ? (DT + 1) / 2 : DT;
+    constexpr int STATE = 16 * KEEP + 2;  // floats per lane that a group hands to the other
+    static_assert(GROUPS == 1 || (size_t) 2 * (kPfThreads / kWave) * STATE * kWave * sizeof(float) <= sizeof(sm_all),
+                  "the handed-over states fit the K/V tiles");
+    float *to = reinterpret_cast<float *>(&sm_all[0]) + (size_t) ((1 - grp) * 4 + wave) * STATE * kWave + lane;
+    const float *from = reinterpret_cast<const float *>(&sm_all[0]) + (size_t) (grp * 4 + wave) * STATE * kWave + lane;
+    float m_tot = -INFINITY, l_tot = 0.0f;
+    v16f  total[KEEP];
+#pragma unroll
+    for (int t = 0; t < KEEP; ++t) {
+      total[t] = (v16f){ 0 };
+    }
+    // the runs of shares in the order in which the merge kernel's waves take them
+    const int waves = shares > kPfMergeChunk ? 4 : 1;
+    for (int w = 0; w < waves; ++w) {
+      float m_wave = -INFINITY, l_wave = 0.0f;
+      v16f  sum[KEEP];
+#pragma unroll
+      for (int t = 0; t < KEEP; ++t) {
+        sum[t] = (v16f){ 0 };
+      }
+      for (int s0 = w * kPfMergeChunk; s0 < shares; s0 += waves * kPfMergeChunk) {
+        for (int z = s0; z < min(s0 + kPfMergeChunk, shares); ++z) {
+          walk(z);
+          float m_own = m_run, l_own = l_run + __shfl_xor(l_run, 32, kWave);
+          if constexpr (GROUPS == 2) {
+            __syncthreads();  // everybody is done with the tiles
+            to[0] = m_own, to[kWave] = l_own;
+            auto give = [&](auto first, auto count) {
+#pragma unroll
+              for (int t = 0; t < decltype(count)::value; ++t) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                  to[(2 + 16 * t + r) * kWave] = oacc[decltype(first)::value + t][r];
+                }
+              }
+            };
+            if (grp == 0) {
+              give(Const<KEEP>(), Const<DT - KEEP>());
+            } else {
+              give(Const<0>(), Const<KEEP>());
+            }
+            __syncthreads();
+            const float m_other = from[0], l_other = from[kWave];
+            float       own;
+            const float other = fold_factors(m_own, m_other, own);
+            l_own = grp == 0 ? fold(own, l_own, other, l_other) : fold(other, l_other, own, l_own);
+            if (grp == 0) {
+#pragma unroll
+              for (int t = 0; t < KEEP; ++t) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                  oacc[t][r] = fold(own, oacc[t][r], other, from[(2 + 16 * t + r) * kWave]);
+                }
+              }
+            } else {
+#pragma unroll
+              for (int t = 0; t < DT - KEEP; ++t) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                  oacc[t][r] = fold(other, from[(2 + 16 * t + r) * kWave], own, oacc[KEEP + t][r]);
+                }
+              }
+            }
+          }
+          float       keep;
+          const float add = fold_factors(m_wave, m_own, keep);
+          l_wave          = fold(add, l_own, keep, l_wave);
+#pragma unroll
+          for (int t = 0; t < KEEP; ++t) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+              sum[t][r] = fold(add, oacc[t][r], keep, sum[t][r]);
+            }
+          }
+        }
+      }
+      float       keep;
+      const float add = fold_factors(m_tot, m_wave, keep);
+      l_tot           = fold(add, l_wave, keep, l_tot);
+#pragma unroll
+      for (int t = 0; t < KEEP; ++t) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          total[t][r] = fold(add, sum[t][r], keep, total[t][r]);
+        }
+      }
+    }
+    const float inv = 1.0f / l_tot;
+#pragma unroll
+    for (int t = 0; t < KEEP; ++t) {
+      if (grp == 0) {
+        store(t, total[t], inv);
+      } else if (KEEP + t < DT) {
+        store(KEEP + t, total[t], inv);
+      }
+    }
+    return;
   }
+
+  walk((int) blockIdx.z);
 
   // ---- the second key group hands its state over: m, l and O of the same query, lane for lane ----
   float l_tot = l_run + __shfl_xor(l_run, 32, kWave);
@@ -541,22 +710,20 @@ __global__ __launch_bounds__(kPfThreads *GROUPS, DP <= 128 ? 2 : 1) void flash_a
       return;
     }
     const float m1 = xch[0], l1 = xch[kWave];
-    const float m_all  = fmaxf(m_run, m1);
-    const float m_safe = (m_all == -INFINITY) ? 0.0f : m_all;  // nothing visible at all: keep the exponents finite
-    const float a0 = fast_exp2(m_run - m_safe), a1 = fast_exp2(m1 - m_safe);
-    l_tot          = a0 * l_tot + a1 * l1;
-    m_run          = m_all;
+    float       a0;
+    const float a1 = fold_factors(m_run, m1, a0);
+    l_tot = fold(a0, l_tot, a1, l1);
 #pragma unroll
     for (int t = 0; t < DT; ++t) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        oacc[t][r] = a0 * oacc[t][r] + a1 * xch[(2 + 16 * t + r) * kWave];
+        oacc[t][r] = fold(a0, oacc[t][r], a1, xch[(2 + 16 * t + r) * kWave]);
       }
     }
   }
 
   // ---- a share of the keys only: leave (max, sum, O) as they are, lane for lane ----
-  if (gridDim.z > 1) {
+  if (shares > 1) {
     if (wave_on) {
       const size_t n_tiles = (size_t) ((qo_len + kBQ - 1) / kBQ) * n_heads;
       const size_t tile    = (size_t) (q_base / kBQ) * n_heads + head;
@@ -574,40 +741,17 @@ __global__ __launch_bounds__(kPfThreads *GROUPS, DP <= 128 ? 2 : 1) void flash_a
     return;
   }
 
-  // ---- finish: O = O^T / l, one query per lane; register r of tile t is d = 32 t + 8 (r / 4) + 4 half + r % 4 ----
-  const float inv   = 1.0f / l_tot;
-  if (q_ok) {
-    const size_t base = (size_t) q_row * qo_stride + (size_t) head * D;
+  const float inv = 1.0f / l_tot;
 #pragma unroll
-    for (int t = 0; t < DT; ++t) {
-#pragma unroll
-      for (int rg = 0; rg < 4; ++rg) {
-        const int d0 = 32 * t + 8 * rg + 4 * half;
-        if (!FULL && d0 >= D) {
-          continue;
-        }
-        float     v[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          v[e] = oacc[t][4 * rg + e] * inv;
-        }
-        if (QO_F32) {
-          *reinterpret_cast<float4 *>(reinterpret_cast<float *>(o_ptr) + base + d0) = make_float4(v[0], v[1], v[2], v[3]);
-        } else {
-          v4h hv = { (_Float16) v[0], (_Float16) v[1], (_Float16) v[2], (_Float16) v[3] };
-          *reinterpret_cast<v4h *>(reinterpret_cast<_Float16 *>(o_ptr) + base + d0) = hv;
-        }
-      }
-    }
+  for (int t = 0; t < DT; ++t) {
+    store(t, oacc[t], inv);
   }
 }
 
 // Puts the shares of a split prefill together: G waves per 32-query tile, head and unit of four output columns per half
 // (`units` of them), lane for lane as the prefill kernel left them. Each takes every G-th run of kPfMergeChunk shares, all
-// loads of a run requested before the first use, folded into a running (max, sum, O) like KV blocks are; with G = 4 (more
+// loads of a run requested before the first use, folded one by one into a running (max, sum, O); with G = 4 (more
 // shares than a run holds) the four states meet in LDS (one row, 16384 keys, 16 / 4 heads of 96, 64 shares: 23.0 -> 19.2 us).
-constexpr int kPfMergeChunk = 8;
-
 template <bool QO_F32, int G>
 __global__ __launch_bounds__(256) void flash_attn_prefill_merge_kernel(void *__restrict__ o_ptr,
                                                                        const float *__restrict__ part, int n_splits,
@@ -637,21 +781,14 @@ __global__ __launch_bounds__(256) void flash_attn_prefill_merge_kernel(void *__r
         x[u]  = reinterpret_cast<const float4 *>(at + 2 * kWave)[(size_t) unit * kWave + lane];
       }
     }
-    float m_new = m_run;
 #pragma unroll
     for (int u = 0; u < kPfMergeChunk; ++u) {
-      m_new = fmaxf(m_new, ml[u].x);
+      float       keep;
+      const float f = fold_factors(m_run, ml[u].x, keep);
+      l_run = fold(f, ml[u].y, keep, l_run);
+      v[0] = fold(f, x[u].x, keep, v[0]), v[1] = fold(f, x[u].y, keep, v[1]);
+      v[2] = fold(f, x[u].z, keep, v[2]), v[3] = fold(f, x[u].w, keep, v[3]);
     }
-    const float m_safe = (m_new == -INFINITY) ? 0.0f : m_new;
-    const float keep   = fast_exp2(m_run - m_safe);
-    l_run *= keep, v[0] *= keep, v[1] *= keep, v[2] *= keep, v[3] *= keep;
-#pragma unroll
-    for (int u = 0; u < kPfMergeChunk; ++u) {
-      const float f = fast_exp2(ml[u].x - m_safe);
-      l_run += f * ml[u].y;
-      v[0] += f * x[u].x, v[1] += f * x[u].y, v[2] += f * x[u].z, v[3] += f * x[u].w;
-    }
-    m_run = m_new;
   }
   if constexpr (G > 1) {
     states[wave][0][lane] = m_run, states[wave][1][lane] = l_run;
@@ -664,18 +801,13 @@ __global__ __launch_bounds__(256) void flash_attn_prefill_merge_kernel(void *__r
       return;
     }
 #pragma unroll
-    for (int w = 1; w < G; ++w) {
-      m_run = fmaxf(m_run, states[w][0][lane]);
-    }
-    const float m_safe = (m_run == -INFINITY) ? 0.0f : m_run;
-    l_run = 0.0f, v[0] = v[1] = v[2] = v[3] = 0.0f;
-#pragma unroll
-    for (int w = 0; w < G; ++w) {  // (a wave without shares has m = -inf, l = v = 0)
-      const float f = fast_exp2(states[w][0][lane] - m_safe);
-      l_run += f * states[w][1][lane];
+    for (int w = 1; w < G; ++w) {  // (a wave without shares has m = -inf, l = v = 0)
+      float       keep;
+      const float f = fold_factors(m_run, states[w][0][lane], keep);
+      l_run = fold(f, states[w][1][lane], keep, l_run);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        v[e] += f * states[w][2 + e][lane];
+        v[e] = fold(f, states[w][2 + e][lane], keep, v[e]);
       }
     }
   }
@@ -1170,59 +1302,80 @@ __global__ __launch_bounds__(kGenThreads) void flash_attn_any_dim_kernel(void *_
   }
 }
 
-template <int DP, bool FULL, bool QO_F32>
-hipError_t launch_prefill(hipStream_t stream, void *o, const void *q, const void *k, const void *v, const void *mask,
-                          int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim, bool causal, int forced,
-                          bool mask_threshold, float *scratch, size_t scratch_bytes) {
+// The launch of a prefill: grid (x, q_blocks, splits). It follows the sizes alone, so that every entry point splits the keys
+// of a request alike.
+constexpr unsigned kCus = 256;
+constexpr int prefill_key_groups(int dp) {  // the most that LDS and registers of a CU hold
+  return dp <= 128 ? 2 : 1;
+}
+struct PrefillPlan {
+  unsigned x, q_blocks, splits;
+  size_t   tiles;  // of 32 queries of one head
+};
+PrefillPlan prefill_plan(int dp, int qo_len, int kv_len, int n_heads, int n_kv_heads, int forced) {
   const int group      = n_heads / n_kv_heads;
   const int gc         = group < 4 ? group : 4;
   const int qsub       = 4 / gc;
   const int sub_groups = (group + gc - 1) / gc;
-  const unsigned q_blocks = (unsigned) ((qo_len + qsub * kBQ - 1) / (qsub * kBQ));
-  if (q_blocks > 65535u) {
-    return hipErrorInvalidValue;
-  }
-  constexpr unsigned kCus       = 256;
-  constexpr int      kMaxGroups = DP <= 128 ? 2 : 1;  // (what LDS and registers of a CU hold)
-  const unsigned     x = (unsigned) (n_kv_heads * sub_groups), wgs = x * q_blocks;
+  PrefillPlan p;
+  p.x        = (unsigned) (n_kv_heads * sub_groups);
+  p.q_blocks = (unsigned) ((qo_len + qsub * kBQ - 1) / (qsub * kBQ));
+  p.tiles    = (size_t) ((qo_len + kBQ - 1) / kBQ) * n_heads;
+  p.splits   = 1;
   // Split the keys while that gives CUs without a workgroup one, down to two blocks per key group and workgroup (the merge
   // is a second launch of about 4 us). Whole decoder layers on the 256-CU device, unsplit (with the mask loaded straight into
   // registers) and split: 5 rows over 1029 keys, 12 / 2 heads of 128 (4 workgroups) 65.3 and 47.8 us; 128 rows over 1152
   // (16 workgroups) 118.0 and 94.5 us; 512 rows over 2048 keys, 32 / 8 heads (128 workgroups) 372 and 338 us.
-  unsigned     splits = 1;
-  const size_t tiles  = (size_t) ((qo_len + kBQ - 1) / kBQ) * n_heads;
-  if (!forced && scratch != nullptr && wgs <= kCus / 2) {
-    const size_t share  = tiles * prefill_partial_floats(DP / 8) * sizeof(float);
-    const size_t blocks = ((size_t) kv_len + kBK - 1) / kBK;
-    const size_t most   = std::min({ (size_t) (kCus / wgs), blocks / (2 * kMaxGroups), scratch_bytes / share });
+  const unsigned wgs = p.x * p.q_blocks;
+  if (!forced && wgs <= kCus / 2) {
+    const size_t share  = p.tiles * prefill_partial_floats(dp / 8) * sizeof(float);
+    const size_t blocks = ((size_t) kv_len + kBK - 1) / kBK, groups = (size_t) prefill_key_groups(dp);
+    const size_t most   = std::min({ (size_t) (kCus / wgs), blocks / (2 * groups), kAttnSharesBytes / share });
     // (for few tiles down to one block, while one trip of the merge takes all shares: 5 rows over 1029 keys, 12 tiles, 14.4 ->
     // 12.6 us; but 128 rows over 1152, 48 tiles, 17.5 -> 17.8, and 500 rows over 500, 256 tiles, 18.7 -> 20.2)
-    const size_t finer  = std::min({ (size_t) (kCus / wgs), blocks / kMaxGroups, scratch_bytes / share, (size_t) kPfMergeChunk });
-    splits              = most < 2 ? 1u : (unsigned) (tiles <= 32 ? std::max(most, finer) : most);
+    const size_t finer  = std::min({ (size_t) (kCus / wgs), blocks / groups, kAttnSharesBytes / share, (size_t) kPfMergeChunk });
+    p.splits            = most < 2 ? 1u : (unsigned) (p.tiles <= 32 ? std::max(most, finer) : most);
   }
-  const dim3 grid(x, q_blocks, splits);
+  return p;
+}
+
+template <int DP, bool FULL, bool QO_F32>
+hipError_t launch_prefill(hipStream_t stream, void *o, const void *q, const void *k, const void *v, const void *mask,
+                          int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim, bool causal, int forced,
+                          bool mask_threshold, float *scratch) {
+  const PrefillPlan plan = prefill_plan(DP, qo_len, kv_len, n_heads, n_kv_heads, forced);
+  if (plan.q_blocks > 65535u) {
+    return hipErrorInvalidValue;
+  }
+  constexpr int  kMaxGroups = prefill_key_groups(DP);
+  const unsigned splits = plan.splits;
+  const size_t   tiles  = plan.tiles;
+  const bool     alone  = splits > 1 && scratch == nullptr;  // (a workgroup walks all shares)
+  const dim3     grid(plan.x, plan.q_blocks, alone ? 1 : splits);
   // Two key groups per workgroup when the grid leaves CUs without a second workgroup, or (causal) when the workgroups
   // all fit at once and their uneven lengths would leave the long ones running alone. Measured on the 256-CU device,
   // 32 query / 8 KV heads of 128: 2048 x 2048 causal 59 us against 65 us, 1024 x 1024 without `causal` 30 against
-  // 33 us; but 2048 x 2048 without `causal` 101 against 92 us.
-  const unsigned all = wgs * splits;
+  // 33 us; but 2048 x 2048 without `causal` 101 against 92 us. (A split grid never has more workgroups than CUs.)
+  const unsigned all = plan.x * plan.q_blocks * splits;
   const bool     two = kMaxGroups == 2 && (forced ? forced == 2 : (all <= kCus || (causal && all <= 2 * kCus)));
   const int      flags = (causal ? 1 : 0) | (mask_threshold ? 2 : 0);
-#define HTPOPS_LAUNCH(GROUPS, MASK)                                                                                   \
-  hipLaunchKernelGGL((flash_attn_prefill_kernel<DP, FULL, QO_F32, GROUPS, MASK>), grid, dim3(kPfThreads * GROUPS), 0, stream, o, \
-                     q, (const _Float16 *) k, (const _Float16 *) v, (const _Float16 *) mask, qo_len, kv_len, n_heads, \
-                     n_kv_heads, head_dim, flags, scratch)
-  if (two && mask) {
-    HTPOPS_LAUNCH(kMaxGroups, true);
+#define HTPOPS_LAUNCH(GROUPS, MASK, ALL)                                                                              \
+  hipLaunchKernelGGL((flash_attn_prefill_kernel<DP, FULL, QO_F32, GROUPS, MASK, ALL>), grid, dim3(kPfThreads * GROUPS), 0, stream, \
+                     o, q, (const _Float16 *) k, (const _Float16 *) v, (const _Float16 *) mask, qo_len, kv_len, n_heads, \
+                     n_kv_heads, head_dim, flags, scratch, (int) splits)
+  if (alone) {
+    HTPOPS_LAUNCH(kMaxGroups, true, true);
+  } else if (two && mask) {
+    HTPOPS_LAUNCH(kMaxGroups, true, false);
   } else if (two) {
-    HTPOPS_LAUNCH(kMaxGroups, false);
+    HTPOPS_LAUNCH(kMaxGroups, false, false);
   } else if (mask) {
-    HTPOPS_LAUNCH(1, true);
+    HTPOPS_LAUNCH(1, true, false);
   } else {
-    HTPOPS_LAUNCH(1, false);
+    HTPOPS_LAUNCH(1, false, false);
   }
 #undef HTPOPS_LAUNCH
-  if (hipError_t e = hipGetLastError(); e != hipSuccess || splits == 1) {
+  if (hipError_t e = hipGetLastError(); e != hipSuccess || splits == 1 || alone) {
     return e;
   }
   constexpr int kUnits = DP / 8;
@@ -1312,6 +1465,22 @@ size_t flash_attn_workspace_bytes(int qo_len, int kv_len, int n_heads, int head_
   return (size_t) n_heads * n_splits * ((size_t) head_dim + 2) * sizeof(float);
 }
 
+namespace {
+
+// Multiples of 16 fill the matrix instructions' k steps, and their rows (multiples of 32 bytes behind 16-byte aligned
+// buffers) can be fetched 16 bytes at a time; every other even head dim, and more query blocks than a grid has rows, take
+// the plain kernel. Head dims 64 and 128 have prefill (several rows) and decode (one row) kernels of their own.
+bool takes_prefill(int qo_len, int head_dim) {
+  return head_dim == 64 || head_dim == 128 ? qo_len > 1 : head_dim % 16 == 0 && qo_len <= 65535 * kBQ;
+}
+
+}  // namespace
+
+bool flash_attn_splits_keys(int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim, int forced_key_groups) {
+  return takes_prefill(qo_len, head_dim) &&
+         prefill_plan((head_dim + 31) / 32 * 32, qo_len, kv_len, n_heads, n_kv_heads, forced_key_groups).splits > 1;
+}
+
 hipError_t launch_flash_attn_decode_part(hipStream_t stream, int part, void *o, const void *q, const void *k,
                                          const void *v, int kv_len, int n_heads, int n_kv_heads, int head_dim,
                                          bool qo_is_f32, void *workspace) {
@@ -1330,7 +1499,7 @@ hipError_t launch_flash_attn_decode_part(hipStream_t stream, int part, void *o, 
 hipError_t launch_flash_attn(hipStream_t stream, void *o, const void *q, const void *k, const void *v,
                              const void *mask, int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim,
                              bool qo_is_f32, bool causal, void *workspace, void *q8_out, int forced_key_groups,
-                             bool mask_threshold, void *shares, size_t shares_bytes) {
+                             bool mask_threshold, void *shares) {
   // with a single query row the causal rule (key j visible iff j <= kv_len - 1) hides nothing
   if (qo_len == 1 && (head_dim == 64 || head_dim == 128)) {
     float *ws = static_cast<float *>(workspace);
@@ -1343,11 +1512,9 @@ hipError_t launch_flash_attn(hipStream_t stream, void *o, const void *q, const v
   }
 #define HTPOPS_PREFILL(DP, FULL)                                                                                     \
   qo_is_f32 ? launch_prefill<DP, FULL, true>(stream, o, q, k, v, mask, qo_len, kv_len, n_heads, n_kv_heads, head_dim, \
-                                             causal, forced_key_groups, mask_threshold, static_cast<float *>(shares), \
-                                             shares_bytes) :                                                         \
+                                             causal, forced_key_groups, mask_threshold, static_cast<float *>(shares)) : \
               launch_prefill<DP, FULL, false>(stream, o, q, k, v, mask, qo_len, kv_len, n_heads, n_kv_heads, head_dim, \
-                                              causal, forced_key_groups, mask_threshold, static_cast<float *>(shares), \
-                                              shares_bytes)
+                                              causal, forced_key_groups, mask_threshold, static_cast<float *>(shares))
   if (head_dim == 128) {
     return HTPOPS_PREFILL(128, true);
   }
@@ -1357,10 +1524,7 @@ hipError_t launch_flash_attn(hipStream_t stream, void *o, const void *q, const v
   if (head_dim <= 0 || head_dim % 2 != 0 || head_dim > kGenMaxD || n_heads > 65535) {
     return hipErrorNotSupported;
   }
-  // Multiples of 16 fill the matrix instructions' k steps, and their rows (multiples of 32 bytes behind 16-byte aligned
-  // buffers) can be fetched 16 bytes at a time; every other even head dim, and more query blocks than a grid has rows,
-  // take the plain kernel.
-  if (head_dim % 16 == 0 && qo_len <= 65535 * kBQ) {
+  if (takes_prefill(qo_len, head_dim)) {
     switch ((head_dim + 31) / 32) {
       case 1: return HTPOPS_PREFILL(32, false);
       case 2: return HTPOPS_PREFILL(64, false);

@@ -159,13 +159,16 @@ hipError_t launch_copy_results(hipStream_t stream, float *dst, const float *src,
 // head_dim 64 / 128 and fp32 output): the output row is also written there as Q8_0 blocks, bit for bit what
 // launch_quantize_q8_0 makes of it. `forced_key_groups` 1 / 2 forces how many key groups a prefill workgroup holds
 // (0: by grid size). `mask_threshold`: the mask selects keys (keep iff mask > -16, reference:
-// src/dsp/ops/flash_attn.c:448-460) instead of being added to the scores (:1505-1512). `shares` (or nullptr): where the
-// workgroups that share a query block's keys leave their parts; the prefill kernel splits as far as `shares_bytes` holds.
+// src/dsp/ops/flash_attn.c:448-460) instead of being added to the scores (:1505-1512). `shares`: kAttnSharesBytes, where the
+// workgroups that share a query block's keys leave their parts (used where flash_attn_splits_keys says so); nullptr: one
+// workgroup walks all of them, with the same results bit for bit.
+constexpr size_t kAttnSharesBytes = (size_t) 32 << 20;  // two shares of 512 queries of 32 heads of 128 take 17 MB
+bool       flash_attn_splits_keys(int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim, int forced_key_groups);
 size_t     flash_attn_workspace_bytes(int qo_len, int kv_len, int n_heads, int head_dim);
 hipError_t launch_flash_attn(hipStream_t stream, void *o, const void *q, const void *k, const void *v,
                              const void *mask, int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim,
                              bool qo_is_f32, bool causal, void *workspace, void *q8_out, int forced_key_groups,
-                             bool mask_threshold, void *shares, size_t shares_bytes);
+                             bool mask_threshold, void *shares);
 // One of the two launches of one-token attention by itself, for timing: part 1 = the split-KV launch (writes the
 // partial records into `workspace`), part 2 = the merge launch (reads them). Same arguments as above otherwise.
 hipError_t launch_flash_attn_decode_part(hipStream_t stream, int part, void *o, const void *q, const void *k,

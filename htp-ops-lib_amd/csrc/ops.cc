@@ -429,6 +429,23 @@ int op_mat_mul_permuted(htpops_context *ctx, float *dst, const float *act, const
   return op_mat_mul_permuted_group(ctx, &one, 1, m, kind);
 }
 
+namespace {
+
+// Where shared keys meet, or nullptr: a caller is capturing the stream (or there was no memory). A graph of theirs may be
+// launched beside the context's own work, or after the context is closed, so it must not hold an address of the context's.
+// A recording of the context's own is launched on its stream only.
+void *attention_shares(htpops_context *ctx) {
+  const bool             recording = ctx->collect_ranges != nullptr;
+  hipStreamCaptureStatus status    = hipStreamCaptureStatusNone;
+  if (!recording && hipStreamIsCapturing(ctx->stream, &status) != hipSuccess) {
+    (void) hipGetLastError();
+    return nullptr;
+  }
+  return recording || status == hipStreamCaptureStatusNone ? ctx->attn_shares : nullptr;
+}
+
+}  // namespace
+
 int op_flash_attn(htpops_context *ctx, void *o, const void *q, const void *k, const void *v, const void *mask,
                   int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim, int qo_is_f32, int causal,
                   bool no_alloc) {
@@ -487,9 +504,13 @@ int op_flash_attn(htpops_context *ctx, void *o, const void *q, const void *k, co
     q8_out = ctx->attn_q8_out;
     note_device_write(ctx, q8_out, q8_0_bytes(1, (size_t) n_heads * head_dim));
   }
+  void *shares = nullptr;
+  if (flash_attn_splits_keys(qo_len, kv_len, n_heads, n_kv_heads, head_dim, ctx->opt.attn_key_groups)) {
+    shares = attention_shares(ctx);
+  }
   HTPOPS_HIP(ctx, launch_flash_attn(ctx->stream, o, q, k, v, mask, qo_len, kv_len, n_heads, n_kv_heads, head_dim,
                                     qo_is_f32 != 0, causal != 0, ws, q8_out, ctx->opt.attn_key_groups,
-                                    ctx->opt.attn_mask_threshold != 0, ctx->attn_shares, ctx->attn_shares ? kAttnSharesBytes : 0));
+                                    ctx->opt.attn_mask_threshold != 0, shares));
   ctx->attn_q8_done = q8_out != nullptr;
   return HTPOPS_OK;
 }

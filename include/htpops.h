@@ -225,11 +225,14 @@ int htpops_flash_attn_ptr(htpops_context *ctx, void *o, const void *q, const voi
 /* htpops_flash_attn_ptr for callers that cannot allocate device memory: code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc. It has no counterpart in the reference. Same arguments, same kernels, same
  * results bit for bit; the split-KV partials of decode attention (qo_len == 1, head_dim 64 or 128) go to a static 8 MiB
- * device array inside the library instead of the context's grown-on-demand workspace (those of every other shape go to a
- * block that the context holds from the start, from both entry points), and the call performs no hipMalloc / hipFree
- * of any kind. Limit (that decode only): n_heads * ceil(kv_len / 64) * (head_dim + 2) * 4 bytes <= 8 MiB (e.g. 32 heads of 128 up to
- * kv_len 32256); larger requests, and outputs that overlap weights the context holds a converted copy of, return -1
- * with a message. All contexts on one GPU share the array, and it keeps the last call's contents: calls on one
+ * device array inside the library instead of the context's grown-on-demand workspace, and the call performs no
+ * hipMalloc / hipFree of any kind. Where several workgroups share the keys of other shapes, their parts go to a block that
+ * the context holds from the start (32 MiB), from both entry points; calls that are being captured into a caller's graph
+ * use no memory of the context's instead (one workgroup then takes all parts in turn: the same bits, in up to twice the
+ * time that not sharing would take), so such a graph may be launched on any stream, and after htpops_close.
+ * Limit (decode with head_dim 64 or 128 only): n_heads * ceil(kv_len / 64) * (head_dim + 2) * 4 bytes <= 8 MiB (e.g. 32
+ * heads of 128 up to kv_len 32256); larger requests, and outputs that overlap weights the context holds a converted copy
+ * of, return -1 with a message. All contexts on one GPU share the array, and it keeps the last call's contents: calls on one
  * context are ordered by its stream; a context that calls this while ANOTHER context's calls may still be running
  * (that context has not been through htpops_synchronize, htpops_finish_message or htpops_close since its last such
  * call) gets HTPOPS_ERR_BUSY instead of a race. */

@@ -65,3 +65,91 @@ def test_mask_at_eight_bytes_and_the_call_that_allocates_nothing(ctx, oracle, qo
         ctx.release(h)
     assert np.array_equal(outs[0].view(np.uint16), outs[1].view(np.uint16))
     assert np.abs(outs[0].astype(np.float32) - want.astype(np.float32)).max() <= ATOL
+
+
+def _entry(ctx, name, o, q, k, v, mask, sizes, f32, causal):
+    fn = getattr(ctx.lib, "htpops_flash_attn_%sptr" % name)
+    p = [ctypes.c_void_p(ctx.device_ptr(h)) if h is not None else None for h in (o, q, k, v, mask)]
+    assert fn(ctx._ctx, *p, *sizes, int(f32), int(causal)) == 0, ctx.last_error()
+
+
+@pytest.mark.parametrize("qo,kv,nh,nkv,d", [
+    (5, 1029, 12, 2, 128), (33, 513, 7, 1, 64), (512, 2048, 32, 8, 128), (1, 9000, 2, 1, 96), (3, 20000, 4, 4, 128), (2, 5000, 2, 2, 64),
+    (1, 6000, 1, 1, 16), (31, 640, 3, 1, 160), (4, 9000, 2, 1, 192), (65, 700, 4, 1, 208), (40, 1100, 8, 4, 240), (1, 9000, 5, 1, 256),
+    (100, 90, 4, 2, 96), (200, 700, 2, 1, 48)])  # (9000 keys and more: more shares than one run of the merge)
+@pytest.mark.parametrize("f32", [False, True])
+def test_entry_points_and_captured_calls_give_the_same_bits(ctx, oracle, qo, kv, nh, nkv, d, f32):
+    # Keys on several workgroups (both entry points), and all shares in one (a call that a caller captures).
+    rng = wl.rng_for(66, qo * 1000 + kv + d)
+    q, k, v = wl.make_attention_inputs(rng, qo, kv, nh, nkv, d)
+    q = q.astype(np.float32) if f32 else q
+    mask = wl.make_causal_mask(qo, kv) if qo <= kv else np.zeros((qo, (kv + 63) // 64 * 64), np.float16)
+    mask[:, 64:70] = 1.5
+    mask[qo // 2, :] = -np.inf  # (a query that sees nothing: not a number from both)
+    hs = [ctx.upload(x) for x in (q, k, v, mask)] + [ctx.alloc(q.nbytes) for _ in range(3)]
+    hip, stream = ctx.lib, ctx.lib.htpops_get_stream(ctx._ctx)
+    for hm, causal in ((None, False), (None, True), (hs[3], False)):
+        print("attention entries", qo, kv, nh, nkv, d, f32, hm is not None, causal, flush=True)
+        for name, ho in (("", hs[4]), ("noalloc_", hs[5])):
+            _entry(ctx, name, ho, hs[0], hs[1], hs[2], hm, (qo, kv, nh, nkv, d), f32, causal)
+        graph, executable = ctypes.c_void_p(), ctypes.c_void_p()
+        assert hip.hipStreamBeginCapture(ctypes.c_void_p(stream), 2) == 0
+        _entry(ctx, "noalloc_", hs[6], hs[0], hs[1], hs[2], hm, (qo, kv, nh, nkv, d), f32, causal)
+        assert hip.hipStreamEndCapture(ctypes.c_void_p(stream), ctypes.byref(graph)) == 0
+        assert hip.hipGraphInstantiate(ctypes.byref(executable), graph, None, None, ctypes.c_size_t(0)) == 0
+        assert hip.hipGraphLaunch(executable, ctypes.c_void_p(stream)) == 0
+        ctx.synchronize()
+        hip.hipGraphExecDestroy(executable), hip.hipGraphDestroy(graph)
+        a, b, c = (ctx.read(h, q.dtype, q.size).reshape(q.shape) for h in hs[4:])
+        assert np.array_equal(a.view(np.uint8), b.view(np.uint8)) and np.array_equal(a.view(np.uint8), c.view(np.uint8))
+        if hm is None and (not causal or qo <= kv) and qo * kv < 300000:
+            want = oracle.flash_attn(q, k, v, None, nh, nkv, d, causal)
+            assert np.abs(b.astype(np.float32) - want.astype(np.float32)).max() <= ATOL
+    for h in hs:
+        ctx.release(h)
+
+
+@pytest.mark.parametrize("name", ["noalloc_", ""])
+def test_a_callers_graph_holds_nothing_of_the_context(ctx, name):
+    # Attention over shared keys, captured by the caller from the context's stream: launched on a stream of the caller's beside
+    # the context's own attention, and again once the context is gone, it gives what it gave. (The buffers are another
+    # context's; the HIP calls are those of the runtime that the library is linked to.)
+    rng = wl.rng_for(67, 0)
+    sizes = qo, kv, nh, nkv, d = 5, 1029, 12, 2, 128
+    q, k, v = wl.make_attention_inputs(rng, qo, kv, nh, nkv, d)
+    q2 = wl.make_attention_inputs(rng, qo, kv, nh, nkv, d)[0]
+    hq, hk, hv, hq2, ho, ho2 = hs = [ctx.upload(x) for x in (q, k, v, q2, np.zeros_like(q), np.zeros_like(q))]
+    first = api.Context(device=0)
+    hip = first.lib
+
+    def call(entry, out, query):
+        p = [ctypes.c_void_p(ctx.device_ptr(h)) for h in (out, query, hk, hv)]
+        assert getattr(first.lib, "htpops_flash_attn_%sptr" % entry)(first._ctx, *p, None, *sizes, 0, 1) == 0, first.last_error()
+
+    call("", ho, hq)  # (the context has its block for shares now)
+    call("", ho2, hq2)
+    first.synchronize()
+    want, want2 = (ctx.read(h, np.uint16, q.size) for h in (ho, ho2))
+    stream = ctypes.c_void_p(first.lib.htpops_get_stream(first._ctx))
+    graph, executable, nodes, other = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_size_t(), ctypes.c_void_p()
+    assert hip.hipStreamCreate(ctypes.byref(other)) == 0
+    assert hip.hipStreamBeginCapture(stream, 2) == 0
+    call(name, ho, hq)
+    assert hip.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+    assert hip.hipGraphGetNodes(graph, None, ctypes.byref(nodes)) == 0 and nodes.value == 1  # (no parts, no merge)
+    assert hip.hipGraphInstantiate(ctypes.byref(executable), graph, None, None, ctypes.c_size_t(0)) == 0
+    for i in range(20):
+        for h in (ho, ho2):
+            ctx.write(h, np.zeros_like(q))
+        assert hip.hipGraphLaunch(executable, other) == 0
+        call("", ho2, hq2)
+        first.synchronize()
+        assert hip.hipStreamSynchronize(other) == 0
+        assert np.array_equal(ctx.read(ho, np.uint16, q.size), want) and np.array_equal(ctx.read(ho2, np.uint16, q.size), want2), i
+    first.close()
+    ctx.write(ho, np.zeros_like(q))
+    assert hip.hipGraphLaunch(executable, other) == 0 and hip.hipStreamSynchronize(other) == 0
+    assert np.array_equal(ctx.read(ho, np.uint16, q.size), want)
+    assert hip.hipGraphExecDestroy(executable) == 0 and hip.hipGraphDestroy(graph) == 0 and hip.hipStreamDestroy(other) == 0
+    for h in hs:
+        ctx.release(h)
