@@ -285,8 +285,8 @@ __device__ __forceinline__ void fragments_workgroup(const FragMember &mem, int m
 
   // Operand streams as buffer resources: a load is then resource (scalar) + per-lane offset (a register that never
   // changes) + scalar offset of the block, and costs no vector-ALU instruction.
-  auto resource = [](const void *base) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int) 0xffffffffu, 0x00020000);
+  auto resource = [](const void *base, uint32_t bytes = 0xffffffffu) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int) bytes, 0x00020000);
   };
   __amdgpu_buffer_rsrc_t ra[UM], rb[UN], rsa[UM], rsb[UN];
   int                    zero_row[UM];  // byte offset of the row of zero scales from this tile's scale rows
@@ -301,12 +301,13 @@ __device__ __forceinline__ void fragments_workgroup(const FragMember &mem, int m
   for (int j = 0; j < UN; ++j) {
     const size_t nt = (size_t) min(nt0 + j, n_tiles - 1);
     rb[j]  = resource(b_frag + nt * nblk * 64);
-    rsb[j] = resource(b_scale + nt * nblk * 32);
+    rsb[j] = resource(b_scale + nt * nblk * 32, (uint32_t) nblk * 128);
   }
-  const int lane16 = lane * 16, lane4 = lane * 4, c4 = c * 4;
+  // (weight scales are bounded by their tile: lanes 32 .. 63 and blocks past the end point behind it and get zeros)
+  const int lane16 = lane * 16, lane4 = lane * 4, c4 = h == 0 ? c * 4 : nblk * 128;
   auto load = [&](FragSet<UM, UN> &s, int kb_raw) {
     const int  kb   = min(kb_raw, nblk - 1);  // branch-free: blocks past the end repeat the last one ...
-    const bool live = kb_raw < blk1;          // ... with activation scales of zero: they add nothing
+    const bool live = kb_raw < blk1;          // ... with scales of zero on both sides: they add nothing
 #pragma unroll
     for (int i = 0; i < UM; ++i) {
       s.a[i]  = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ra[i], lane16, kb * 1024, 0));
@@ -315,7 +316,7 @@ __device__ __forceinline__ void fragments_workgroup(const FragMember &mem, int m
 #pragma unroll
     for (int j = 0; j < UN; ++j) {
       s.b[j]  = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rb[j], lane16, kb * 1024, 0));
-      s.dw[j] = __builtin_amdgcn_raw_buffer_load_b32(rsb[j], c4, kb * 128, 0);
+      s.dw[j] = __builtin_amdgcn_raw_buffer_load_b32(rsb[j], c4, live ? kb * 128 : nblk * 128, 0);
     }
   };
 
@@ -338,8 +339,8 @@ __device__ __forceinline__ void fragments_workgroup(const FragMember &mem, int m
   }
   const v16f zf = { 0 };
   const v16i zi = { 0 };
-  // scale operands of a unit: (scale, 0, 0, 0) in K slot 0; the activation side holds zeros in the lanes of K slots
-  // 4..7, so whatever the weight side holds there contributes nothing
+  // scale operands of a unit: (scale, 0, 0, 0) in K slot 0; both sides hold zeros in the lanes of K slots 4..7 (the weight
+  // side too: zero times an infinite scale is not a number)
   auto scale_operand = [&](uint32_t packed) {
     const uint2 u = make_uint2(packed, 0u);
     return __builtin_bit_cast(v4h, u);
@@ -564,12 +565,12 @@ __device__ __forceinline__ void shared_operand_workgroup(const FragMember &mem, 
   const int mine = wave == 0 ? 2 : 1;  // transfers of this wave per stage
 
   // -- the wave's own operand: eight blocks in registers (two stages), block q of stage s in slot (s % 2) * 4 + q --
-  auto resource = [](const void *base) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int) 0xffffffffu, 0x00020000);
+  auto resource = [](const void *base, uint32_t bytes = 0xffffffffu) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int) bytes, 0x00020000);
   };
   __amdgpu_buffer_rsrc_t ro  = SHARE_W ? resource(mem.a_frag + (size_t) mt * nblk * 64) : resource(mem.b_frag + ntc * nblk * 64);
-  __amdgpu_buffer_rsrc_t rso = SHARE_W ? resource(mem.a_scale + (size_t) mt * nblk * 64) : resource(mem.b_scale + ntc * nblk * 32);
-  const int own_scale_off = SHARE_W ? lane * 4 : c * 4;
+  __amdgpu_buffer_rsrc_t rso = SHARE_W ? resource(mem.a_scale + (size_t) mt * nblk * 64) : resource(mem.b_scale + ntc * nblk * 32, (uint32_t) nblk * 128);
+  const int own_scale_off = SHARE_W ? lane * 4 : h == 0 ? c * 4 : nblk * 128;  // (weight scales: zeros in lanes 32 .. 63)
   uint4     oq[2 * kShBlocks];
   uint32_t  dq[2 * kShBlocks];
   auto load_own = [&](int slot_, int kb_raw) {
@@ -599,7 +600,15 @@ __device__ __forceinline__ void shared_operand_workgroup(const FragMember &mem, 
   const v16f zf = { 0 };
   const v16i zi = { 0 };
   typedef __attribute__((address_space(3))) const uint8_t *lds_ptr;
-  const uint32_t sh_rd = ring0 + lane16, sc_rd = ring0 + kShBlocks * 1024 + (SHARE_W ? c * 4 : lane * 4);
+  // (weight scales take half of a stage's scale rows; lanes 32 .. 63 read zeros from the other half, written here once)
+  const uint32_t sh_rd = ring0 + lane16, sc_rd = ring0 + kShBlocks * 1024 + (SHARE_W ? h * (kShBlocks * kScaleRow) + c * 4 : lane * 4);
+  if (SHARE_W) {
+    for (int i = threadIdx.x; i < kShStages * kShBlocks * kScaleRow / 4; i += kGiThreads) {
+      const int in_stage = i % (kShBlocks * kScaleRow / 4), s = i / (kShBlocks * kScaleRow / 4);
+      *reinterpret_cast<uint32_t *>(lds + s * kShStage + kShBlocks * (1024 + kScaleRow) + in_stage * 4) = 0u;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (the barrier of the first stage makes them everybody's)
+  }
 
   auto stage = [&](auto parity_tag, int s) {
     constexpr int P = decltype(parity_tag)::value;  // s % 2: which half of the own registers
@@ -788,6 +797,8 @@ __global__ __launch_bounds__(kStWaves *kWave, 4) void gemm_i8_fragments_staged_k
   }
   const v16f zf = { 0 };
   const v16i zi = { 0 };
+  // the column's scale; lanes 32 .. 63 read a zero, the upper half of the first row's activation scale
+  const uint32_t db_at = h == 0 ? 7168 + wn * 128 + c * 4 : 4096 + 128;
 #pragma unroll
   for (int s = 0; s < kStRing - 1; ++s) {
     fetch(s);
@@ -802,7 +813,7 @@ __global__ __launch_bounds__(kStWaves *kWave, 4) void gemm_i8_fragments_staged_k
     if (s < mine) {
       const uint8_t *at = &lds[kh][s & (kStRing - 1)][0];
       const v4i      b  = *reinterpret_cast<const v4i *>(at + 5120 + wn * 1024 + lane * 16);
-      const uint2    db = make_uint2(*reinterpret_cast<const uint32_t *>(at + 7168 + wn * 128 + c * 4), 0u);
+      const uint2    db = make_uint2(*reinterpret_cast<const uint32_t *>(at + db_at), 0u);
       v4i            a[2];
       uint2          da[2];
 #pragma unroll
