@@ -18,7 +18,7 @@
 // A wave owns 64 x 64 outputs (2 x 2 units per block) and a share of K; the KSPLIT waves of one tile are summed
 // through LDS in a fixed order. Launches with too few such tiles to fill the chip use 32 x 32 tiles (one unit per
 // block) instead: four times the workgroups, each with a quarter of the vector-ALU work; matrices that leave CUs idle
-// even so have K split over workgroups too. From 256 tiles of 128 x 64 on both operands are staged through LDS.
+// even so have K split over workgroups too. From 280 tiles of 128 x 64 on both operands are staged through LDS.
 #include "device_utils.h"
 #include "kernels.h"
 
@@ -746,12 +746,16 @@ __global__ __launch_bounds__(kGiThreads, 4) void gemm_i8_fragments_small_kernel(
 // ring of four slots three blocks ahead. One barrier a block; two workgroups on a CU fill each other's gaps. The halves
 // are added through LDS. What bounds it then is the vector ALU (32 instructions a unit)
 // and the scale product. Times: see tile_config.
+// RT = 2: 64 x 64 tiles, one row tile a wave, for launches with too few of the larger ones (see launch_members); the same sums.
 constexpr int kStRing  = 4;
-constexpr int kStSlot  = 4 * 1024 + 1024 + 2 * 1024 + 256;  // row fragments, their scales, column fragments, their scales
 constexpr int kStWaves = 8;
 
+template <int RT>
 __global__ __launch_bounds__(kStWaves *kWave, 4) void gemm_i8_fragments_staged_kernel(FragMembers grp, int m, int m_tiles) {
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[2][kStRing][kStSlot];
+  constexpr int WT = RT / 2;  // row tiles of a wave
+  // a slot: row fragments, their scales, column fragments, their scales
+  constexpr int kScales = RT * 1024, kCols = kScales + 1024, kColScales = kCols + 2 * 1024, kSlot = kColScales + 256;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[2][kStRing][kSlot];
   const FragMember &mem = member_of_workgroup(grp);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int kh = wave >> 2, w4 = wave & 3, wm = w4 >> 1, wn = w4 & 1;
@@ -759,37 +763,40 @@ __global__ __launch_bounds__(kStWaves *kWave, 4) void gemm_i8_fragments_staged_k
   const int n = mem.n, nblk = mem.nblk, n_tiles = mem.n_tiles;
   // all row blocks of a column block on one XCD, behind each other (as in fragments_workgroup)
   const unsigned wg = blockIdx.x - mem.wg_begin;
-  const int gy = (m_tiles + 3) / 4, gx = (n_tiles + 1) / 2;
+  const int gy = (m_tiles + RT - 1) / RT, gx = (n_tiles + 1) / 2;
   const int xcd = wg & 7, slot_ = (int) (wg >> 3), by = slot_ % gy, bx = (slot_ / gy) * 8 + xcd;
   if (bx >= gx) {
     return;
   }
-  const int mt0 = 4 * by, nt0 = 2 * bx;
+  const int mt0 = RT * by, nt0 = 2 * bx;
   // this half's blocks: kb0 .. kb0 + mine - 1 (both halves run `steps` turns)
   const int steps = (nblk + 1) / 2, kb0 = kh * steps, mine = kh == 0 ? steps : nblk - steps;
 
-  // wave w brings row fragment w and one more piece: row scales, column scales, column fragment 0, column fragment 1
+  // wave w brings row fragment w (if there is one: RT) and one more piece: row scales, column scales, column fragment 0,
+  // column fragment 1
   const uint8_t *a_src = reinterpret_cast<const uint8_t *>(mem.a_frag) + (size_t) min(mt0 + w4, m_tiles - 1) * nblk * 1024;
   const uint8_t *b_src = reinterpret_cast<const uint8_t *>(mem.b_frag) + (size_t) min(nt0 + (w4 & 1), n_tiles - 1) * nblk * 1024;
   // (per lane: 16 lanes per row tile, 16 bytes each; 32 lanes per column tile, 4 bytes each)
-  const uint8_t *as_src = reinterpret_cast<const uint8_t *>(mem.a_scale) + (size_t) min(mt0 + (lane >> 4), m_tiles - 1) * nblk * 256 + (lane & 15) * 16;
+  const uint8_t *as_src = reinterpret_cast<const uint8_t *>(mem.a_scale) + (size_t) min(mt0 + min(lane >> 4, RT - 1), m_tiles - 1) * nblk * 256 + (lane & 15) * 16;
   const uint8_t *bs_src = reinterpret_cast<const uint8_t *>(mem.b_scale) + (size_t) min(nt0 + h, n_tiles - 1) * nblk * 128 + c * 4;
   const uint32_t to0 = (uint32_t) (uintptr_t) &lds[kh][0][0];
   auto fetch = [&](int s) {  // (past the end: the last block again, so that the count of requests in flight stays)
     const size_t   kb = (size_t) min(kb0 + s, nblk - 1);
-    const uint32_t to = to0 + (uint32_t) (s & (kStRing - 1)) * kStSlot;
-    asm volatile("s_mov_b32 m0, %2\n s_nop 0\n global_load_lds_dwordx4 %0, %1" ::"v"(lane * 16), "s"(a_src + kb * 1024), "s"(to + w4 * 1024) : "memory");
+    const uint32_t to = to0 + (uint32_t) (s & (kStRing - 1)) * kSlot;
+    if (w4 < RT) {
+      asm volatile("s_mov_b32 m0, %2\n s_nop 0\n global_load_lds_dwordx4 %0, %1" ::"v"(lane * 16), "s"(a_src + kb * 1024), "s"(to + w4 * 1024) : "memory");
+    }
     if (w4 >= 2) {
-      asm volatile("s_mov_b32 m0, %2\n s_nop 0\n global_load_lds_dwordx4 %0, %1" ::"v"(lane * 16), "s"(b_src + kb * 1024), "s"(to + 5120 + (w4 - 2) * 1024) : "memory");
+      asm volatile("s_mov_b32 m0, %2\n s_nop 0\n global_load_lds_dwordx4 %0, %1" ::"v"(lane * 16), "s"(b_src + kb * 1024), "s"(to + kCols + (w4 - 2) * 1024) : "memory");
     } else if (w4 == 0) {
-      asm volatile("s_mov_b32 m0, %1\n s_nop 0\n global_load_lds_dwordx4 %0, off" ::"v"(as_src + kb * 256), "s"(to + 4096) : "memory");
+      asm volatile("s_mov_b32 m0, %1\n s_nop 0\n global_load_lds_dwordx4 %0, off" ::"v"(as_src + kb * 256), "s"(to + kScales) : "memory");
     } else {
-      asm volatile("s_mov_b32 m0, %1\n s_nop 0\n global_load_lds_dword %0, off" ::"v"(bs_src + kb * 128), "s"(to + 7168) : "memory");
+      asm volatile("s_mov_b32 m0, %1\n s_nop 0\n global_load_lds_dword %0, off" ::"v"(bs_src + kb * 128), "s"(to + kColScales) : "memory");
     }
   };
-  v16f acc[2];
+  v16f acc[WT];
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
+  for (int u = 0; u < WT; ++u) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       acc[u][r] = 0.0f;
@@ -798,7 +805,7 @@ __global__ __launch_bounds__(kStWaves *kWave, 4) void gemm_i8_fragments_staged_k
   const v16f zf = { 0 };
   const v16i zi = { 0 };
   // the column's scale; lanes 32 .. 63 read a zero, the upper half of the first row's activation scale
-  const uint32_t db_at = h == 0 ? 7168 + wn * 128 + c * 4 : 4096 + 128;
+  const uint32_t db_at = h == 0 ? kColScales + wn * 128 + c * 4 : kScales + 128;
 #pragma unroll
   for (int s = 0; s < kStRing - 1; ++s) {
     fetch(s);
@@ -806,23 +813,27 @@ __global__ __launch_bounds__(kStWaves *kWave, 4) void gemm_i8_fragments_staged_k
   for (int s = 0; s < steps; ++s) {
     // this wave's pieces of block s have landed (those of two more blocks may be on their way); behind the barrier everybody's
     // have, and nobody reads the slot of block s - 1 any more
-    asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+    if (w4 < RT) {  // (two requests a block)
+      asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+    } else {
+      asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+    }
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     fetch(s + kStRing - 1);
     if (s < mine) {
       const uint8_t *at = &lds[kh][s & (kStRing - 1)][0];
-      const v4i      b  = *reinterpret_cast<const v4i *>(at + 5120 + wn * 1024 + lane * 16);
+      const v4i      b  = *reinterpret_cast<const v4i *>(at + kCols + wn * 1024 + lane * 16);
       const uint2    db = make_uint2(*reinterpret_cast<const uint32_t *>(at + db_at), 0u);
-      v4i            a[2];
-      uint2          da[2];
+      v4i            a[WT];
+      uint2          da[WT];
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        a[u]  = *reinterpret_cast<const v4i *>(at + (2 * wm + u) * 1024 + lane * 16);
-        da[u] = make_uint2(*reinterpret_cast<const uint32_t *>(at + 4096 + (2 * wm + u) * 256 + lane * 4), 0u);
+      for (int u = 0; u < WT; ++u) {
+        a[u]  = *reinterpret_cast<const v4i *>(at + (WT * wm + u) * 1024 + lane * 16);
+        da[u] = make_uint2(*reinterpret_cast<const uint32_t *>(at + kScales + (WT * wm + u) * 256 + lane * 4), 0u);
       }
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
+      for (int u = 0; u < WT; ++u) {
         const v16i sum = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[u], b, zi, 0, 0, 0);
         const v16f scl = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(v4h, da[u]), __builtin_bit_cast(v4h, db), zf, 0, 0, 0);
 #pragma unroll
@@ -833,12 +844,12 @@ __global__ __launch_bounds__(kStWaves *kWave, 4) void gemm_i8_fragments_staged_k
     }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (pieces past the end have landed before the ring is used again)
-  float *xch = reinterpret_cast<float *>(&lds[0][0][0]) + (size_t) w4 * 2 * 16 * kWave + lane;
-  static_assert(4 * 2 * 16 * kWave * sizeof(float) <= sizeof(lds), "the sums of a half fit");
+  float *xch = reinterpret_cast<float *>(&lds[0][0][0]) + (size_t) w4 * WT * 16 * kWave + lane;
+  static_assert(4 * WT * 16 * kWave * sizeof(float) <= sizeof(lds), "the sums of a half fit");
   __syncthreads();
   if (kh == 1) {
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    for (int u = 0; u < WT; ++u) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         xch[(16 * u + r) * kWave] = acc[u][r];
@@ -851,10 +862,10 @@ __global__ __launch_bounds__(kStWaves *kWave, 4) void gemm_i8_fragments_staged_k
   }
   const int col = (nt0 + wn) * 32 + c;
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
+  for (int u = 0; u < WT; ++u) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const int   row = (mt0 + 2 * wm + u) * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
+      const int   row = (mt0 + WT * wm + u) * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
       const float v   = acc[u][r] + xch[(16 * u + r) * kWave];
       if (row < m && col < n) {
         mem.out[(size_t) row * n + col] = v;
@@ -902,7 +913,8 @@ hipError_t launch_weights_to_i8_fragments(hipStream_t stream, void *dst, const v
 
 namespace {
 
-constexpr int kStagedUnit = 3;  // gemm_i8_fragments_staged_kernel
+constexpr int kStagedUnit   = 3;    // gemm_i8_fragments_staged_kernel
+constexpr int kStagedMinWgs = 280;  // (measured at 256 and at 280)
 
 struct TileConfig {
   int unit, ksplit;
@@ -916,12 +928,13 @@ struct TileConfig {
 TileConfig tile_config(int m, int n, int k, int forced_unit) {
   const int m_tiles = (m + 31) / 32, n_tiles = (n + 31) / 32, nblk = k / 32;
   const int wave_tiles  = ((m_tiles + 1) / 2) * ((n_tiles + 1) / 2);
-  // Both operands through LDS where that gives every CU a workgroup of 128 x 64 and pads the rows by less than a seventh.
-  // Before / with it, Q8_0: seven projections at 256 rows, Llama-7B / Qwen2-1.5B, 238 / 82.7 and 197 / 61.8 us; layers of 512 rows 441 /
-  // 165 and 393 / 147. (From 128 workgroups on: the projections 161, but a layer of 200 rows, whose o has a launch of
-  // its own, 283 against 247; 300 rows, padded by a fifth, 315 and 325; one matrix of 344 workgroups 47.5 and 50.4.)
+  // Both operands through LDS where the matrix alone gives more workgroups of 128 x 64 than there are CUs and pads the rows by
+  // less than a seventh. Without / with it, Q8_0: seven projections at 256 rows, Llama-7B 239 / 208 us, gate and up of Llama-7B at
+  // 512 rows 195 / 149, of Qwen2-1.5B at 256 and 512 rows 46.6 / 36.7 and 71.9 / 55.3. A launch of one workgroup a CU loses, so a
+  // matrix of 256 stays out: 512 rows of 4096 x 4096 and 11008 x 4096 by themselves 33.8 / 41.7 and 70.7 / 88.3, three of the
+  // former in one launch 92.3 / 85.8. (300 rows, padded by a fifth, a layer: 315 and 325.)
   const int row_blocks = (m_tiles + 3) / 4;
-  if (forced_unit != 1 && forced_unit != 2 && 28 * row_blocks <= 8 * m_tiles && row_blocks * ((n_tiles + 1) / 2) >= 256) {
+  if (forced_unit != 1 && forced_unit != 2 && 28 * row_blocks <= 8 * m_tiles && row_blocks * ((n_tiles + 1) / 2) >= kStagedMinWgs) {
     return { kStagedUnit, 2 };
   }
   const int unit        = forced_unit == 1 || forced_unit == 2 ? forced_unit : (m_tiles == 1 || wave_tiles < 512 ? 1 : 2);
@@ -975,9 +988,14 @@ SmallTilePlan small_tile_plan(int m_tiles, int n_tiles, int nblk, TileConfig cfg
   return { staged && cfg.ksplit == 1 ? kShareActivations : kSharePlain, cfg.ksplit, 1 };
 }
 
-unsigned member_workgroups(int m_tiles, int n_tiles, TileConfig cfg, SmallTilePlan plan) {
+// workgroups of a member of a staged launch whose workgroups own `row_tiles` row tiles
+unsigned staged_workgroups(int m_tiles, int n_tiles, int row_tiles) {
+  return (unsigned) (((n_tiles + 1) / 2 + 7) / 8 * 8 * ((m_tiles + row_tiles - 1) / row_tiles));
+}
+
+unsigned member_workgroups(int m_tiles, int n_tiles, TileConfig cfg, SmallTilePlan plan, int staged_row_tiles) {
   if (cfg.unit == kStagedUnit) {
-    return (unsigned) (((n_tiles + 1) / 2 + 7) / 8 * 8 * ((m_tiles + 3) / 4));
+    return staged_workgroups(m_tiles, n_tiles, staged_row_tiles);
   }
   if (plan.share == kShareWeights) {
     return (unsigned) ((n_tiles + 7) / 8 * 8 * (m_tiles / kGiWaves) * plan.kparts);
@@ -1062,6 +1080,14 @@ hipError_t launch_members(hipStream_t stream, int count, float *const *outs, con
   }
   auto walk = [&](int i) { return ks[i] <= 0 || ns[i] <= 0 ? 0 : ks[i] / 32 / tile_config(m, ns[i], ks[i], forced_unit).ksplit; };
   std::stable_sort(order, order + count, [&](int a, int b) { return walk(a) > walk(b); });
+  // Staged tiles of 64 rows where those of 128 would not fill the device (512 workgroups, two a CU), Q8_0, 128 / 64 rows: 256
+  // rows, 4096 x 11008 (344 workgroups) 50.1 / 47.8 us; 384 rows, 1024 x 8192 (384) 20.3 / 19.4; 448 rows, 2048 x 4736 (296)
+  // 30.1 / 27.7; but 1024 rows, 4096 x 4096 (512) 58.2 / 68.6.
+  unsigned large = 0;
+  for (int i = 0; i < count; ++i) {
+    large += staged_workgroups(m_tiles, (ns[i] + 31) / 32, 4);
+  }
+  const int staged_row_tiles = large < 512 ? 2 : 4;
   for (int slot = 0; slot < count; ++slot) {
     const int i = order[slot];
     if (ks[i] <= 0 || ks[i] % 32 != 0 || ns[i] <= 0) {
@@ -1098,11 +1124,13 @@ hipError_t launch_members(hipStream_t stream, int count, float *const *outs, con
       grp.m[slot].tickets  = tickets + tickets_used;
       exchange_used += xbytes, tickets_used += xslots;
     }
-    total += member_workgroups(m_tiles, n_tiles, cfg, plan);
+    total += member_workgroups(m_tiles, n_tiles, cfg, plan, staged_row_tiles);
   }
   grp.count = count;
-  if (cfg.unit == kStagedUnit) {
-    hipLaunchKernelGGL(gemm_i8_fragments_staged_kernel, dim3(total), dim3(kStWaves * kWave), 0, stream, grp, m, m_tiles);
+  if (cfg.unit == kStagedUnit && staged_row_tiles == 2) {
+    hipLaunchKernelGGL(gemm_i8_fragments_staged_kernel<2>, dim3(total), dim3(kStWaves * kWave), 0, stream, grp, m, m_tiles);
+  } else if (cfg.unit == kStagedUnit) {
+    hipLaunchKernelGGL(gemm_i8_fragments_staged_kernel<4>, dim3(total), dim3(kStWaves * kWave), 0, stream, grp, m, m_tiles);
   } else if (cfg.unit == 1) {
     hipLaunchKernelGGL(gemm_i8_fragments_small_kernel, dim3(total), dim3(kGiThreads), 0, stream, grp, m, m_tiles);
   } else if (cfg.ksplit == 4) {

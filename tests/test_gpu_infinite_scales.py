@@ -20,7 +20,8 @@ def ctx():
 @pytest.mark.parametrize("wt", [wl.GGML_TYPE_Q4_0, wl.GGML_TYPE_Q8_0])
 @pytest.mark.parametrize("m,k,n", [
     (20, 8960, 70), (40, 1536, 100), (33, 256, 40), (17, 1568, 70),                              # K over waves and workgroups
-    (128, 1024, 96), (128, 8960, 64), (70, 1024, 8200), (128, 96, 16384), (600, 512, 1100)])     # operands shared, staged, 64 x 64 tiles
+    (128, 1024, 96), (128, 8960, 64), (70, 1024, 8200), (600, 512, 1100),                        # operands shared, 64 x 64 tiles
+    (128, 96, 17920), (128, 96, 32768)])                                                      # staged, tiles of 64 and of 128 rows
 def test_infinite_weight_scales(ctx, oracle, wt, m, k, n):
     rng = wl.rng_for(96, m + k + n + wt)
     w = np.ascontiguousarray(wl.make_weights(rng, n, k, wt)).view(np.uint8).reshape(n, k // 32, -1).copy()

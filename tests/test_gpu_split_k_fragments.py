@@ -43,11 +43,37 @@ def test_staged_operands_at_the_edges(ctx, oracle, wt, m, k, n):
     ctx.set_option("gemm_fp6", api.DEFAULT_OPTIONS["gemm_fp6"])
 
 
+@pytest.mark.parametrize("wt", [wl.GGML_TYPE_Q4_0, wl.GGML_TYPE_Q8_0])
+@pytest.mark.parametrize("m,k,n", [
+    (97, 32, 17920), (110, 96, 17921), (225, 320, 8961), (256, 1120, 8960),      # 280 to 511 workgroups of 128 rows: tiles of 64
+    (128, 64, 32768), (200, 96, 16384), (512, 1056, 8161), (110, 2080, 32770)])  # 512 and more: tiles of 128
+def test_staged_tiles_of_both_sizes(ctx, oracle, wt, m, k, n):
+    with ctx.option("gemm_fp6", 0):
+        check_mat_mul(ctx, oracle, wl.rng_for(59, m * 131 + k + n + wt), m, k, n, wt)
+
+
+def test_staged_tiles_of_both_sizes_give_the_same_bits(ctx, oracle):
+    # alone a matrix takes tiles of 64 rows, two of them in a message tiles of 128
+    m, n, k, wt = 256, 8960, 608, wl.GGML_TYPE_Q8_0
+    rng = wl.rng_for(61, 0)
+    ha = ctx.upload(oracle.quantize_q8_0(wl.make_activations(rng, m, k)))
+    ws = [ctx.upload(wl.make_weights(rng, n, k, wt)) for _ in range(2)]
+    outs = [ctx.alloc(m * n * 4) for _ in range(4)]
+    reqs = [(api.REQUEST_TYPE_OP_COMPUTE, api.op_compute_request(api.HTP_OPS_MAT_MUL_Q8_0_Q8_0, api.mat_mul_params(
+        (outs[j], 0), (ha, 0), (ws[j % 2], 0), m, k, n))) for j in range(4)]
+    for msg in (api.build_message(reqs[:2]), api.build_message(reqs[2:3]), api.build_message(reqs[3:])):
+        assert ctx.process_message(msg) == 0 and not any(api.message_request_states(msg)), ctx.last_error()
+    both = [ctx.read(h, np.uint32, m * n) for h in outs]
+    assert np.array_equal(both[0], both[2]) and np.array_equal(both[1], both[3]) and both[0].any()
+    for h in [ha] + ws + outs:
+        ctx.release(h)
+
+
 @pytest.mark.parametrize("m", [17, 50, 128])
 def test_grouped_split_k_equals_single_requests(ctx, oracle, m):
     rng = wl.rng_for(60, m)
     wt, op = wl.GGML_TYPE_Q8_0, api.HTP_OPS_MAT_MUL_Q8_0_Q8_0
-    shapes = [(96, 1536), (256, 1536), (64, 8960), (40, 256), (1000, 1536)] + ([(16384, 256)] if m == 128 else [])  # (the last: staged)
+    shapes = [(96, 1536), (256, 1536), (64, 8960), (40, 256), (1000, 1536)] + ([(17920, 256)] if m == 128 else [])  # (the last: staged)
     acts = {k: ctx.upload(oracle.quantize_q8_0(wl.make_activations(rng, m, k))) for k in (1536, 8960, 256)}
     ws = [ctx.upload(wl.make_weights(rng, n, k, wt)) for n, k in shapes]
     results = []
