@@ -1312,7 +1312,7 @@ struct PrefillPlan {
   unsigned x, q_blocks, splits;
   size_t   tiles;  // of 32 queries of one head
 };
-PrefillPlan prefill_plan(int dp, int qo_len, int kv_len, int n_heads, int n_kv_heads, int forced) {
+PrefillPlan prefill_plan(int dp, int qo_len, int kv_len, int n_heads, int n_kv_heads, bool mask, int forced) {
   const int group      = n_heads / n_kv_heads;
   const int gc         = group < 4 ? group : 4;
   const int qsub       = 4 / gc;
@@ -1322,10 +1322,13 @@ PrefillPlan prefill_plan(int dp, int qo_len, int kv_len, int n_heads, int n_kv_h
   p.q_blocks = (unsigned) ((qo_len + qsub * kBQ - 1) / (qsub * kBQ));
   p.tiles    = (size_t) ((qo_len + kBQ - 1) / kBQ) * n_heads;
   p.splits   = 1;
-  // Split the keys while that gives CUs without a workgroup one, down to two blocks per key group and workgroup (the merge
-  // is a second launch of about 4 us). Whole decoder layers on the 256-CU device, unsplit (with the mask loaded straight into
-  // registers) and split: 5 rows over 1029 keys, 12 / 2 heads of 128 (4 workgroups) 65.3 and 47.8 us; 128 rows over 1152
-  // (16 workgroups) 118.0 and 94.5 us; 512 rows over 2048 keys, 32 / 8 heads (128 workgroups) 372 and 338 us.
+  // Split the keys while that gives CUs without a workgroup one, down to two blocks per key group and workgroup, where the
+  // blocks that the longest workgroup is spared take longer than the parts and their merge: a turn of the key groups
+  // some 0.2 us and 0.96 us per 128 of the padded head dim, 0.35 us more with a mask; the merge 1 us and 0.3 us for every MB
+  // of parts. (526 shapes of
+  // 2 to 1000 rows over 100 to 6000 keys, 8 head layouts: within 4 % of the better one everywhere. 512 rows over 512 keys,
+  // causal, 32 / 8 heads of 128, unsplit / split 14.8 / 22.3 us, over 2012 keys 36.7 / 34.6, with a mask
+  // 46.1 / 36.6; 2 rows over 1502 keys 25.7 / 12.8.)
   const unsigned wgs = p.x * p.q_blocks;
   if (!forced && wgs <= kCus / 2) {
     const size_t share  = p.tiles * prefill_partial_floats(dp / 8) * sizeof(float);
@@ -1334,7 +1337,12 @@ PrefillPlan prefill_plan(int dp, int qo_len, int kv_len, int n_heads, int n_kv_h
     // (for few tiles down to one block, while one trip of the merge takes all shares: 5 rows over 1029 keys, 12 tiles, 14.4 ->
     // 12.6 us; but 128 rows over 1152, 48 tiles, 17.5 -> 17.8, and 500 rows over 500, 256 tiles, 18.7 -> 20.2)
     const size_t finer  = std::min({ (size_t) (kCus / wgs), blocks / groups, kAttnSharesBytes / share, (size_t) kPfMergeChunk });
-    p.splits            = most < 2 ? 1u : (unsigned) (p.tiles <= 32 ? std::max(most, finer) : most);
+    const size_t splits = most < 2 ? 1 : p.tiles <= 32 ? std::max(most, finer) : most;
+    const auto   turns  = [&](size_t n) { return (n + groups - 1) / groups; };
+    const size_t spared = turns(blocks) - turns((blocks + splits - 1) / splits);
+    if (spared * (200 + 15 * (size_t) dp / 2 + (mask ? 350 : 0)) > 1000 + splits * share * 3 / 10000) {  // (ns)
+      p.splits = (unsigned) splits;
+    }
   }
   return p;
 }
@@ -1343,7 +1351,7 @@ template <int DP, bool FULL, bool QO_F32>
 hipError_t launch_prefill(hipStream_t stream, void *o, const void *q, const void *k, const void *v, const void *mask,
                           int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim, bool causal, int forced,
                           bool mask_threshold, float *scratch) {
-  const PrefillPlan plan = prefill_plan(DP, qo_len, kv_len, n_heads, n_kv_heads, forced);
+  const PrefillPlan plan = prefill_plan(DP, qo_len, kv_len, n_heads, n_kv_heads, mask != nullptr, forced);
   if (plan.q_blocks > 65535u) {
     return hipErrorInvalidValue;
   }
@@ -1476,9 +1484,10 @@ bool takes_prefill(int qo_len, int head_dim) {
 
 }  // namespace
 
-bool flash_attn_splits_keys(int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim, int forced_key_groups) {
+bool flash_attn_splits_keys(int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim, bool mask,
+                            int forced_key_groups) {
   return takes_prefill(qo_len, head_dim) &&
-         prefill_plan((head_dim + 31) / 32 * 32, qo_len, kv_len, n_heads, n_kv_heads, forced_key_groups).splits > 1;
+         prefill_plan((head_dim + 31) / 32 * 32, qo_len, kv_len, n_heads, n_kv_heads, mask, forced_key_groups).splits > 1;
 }
 
 hipError_t launch_flash_attn_decode_part(hipStream_t stream, int part, void *o, const void *q, const void *k,

@@ -163,7 +163,8 @@ hipError_t launch_copy_results(hipStream_t stream, float *dst, const float *src,
 // workgroups that share a query block's keys leave their parts (used where flash_attn_splits_keys says so); nullptr: one
 // workgroup walks all of them, with the same results bit for bit.
 constexpr size_t kAttnSharesBytes = (size_t) 32 << 20;  // two shares of 512 queries of 32 heads of 128 take 17 MB
-bool       flash_attn_splits_keys(int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim, int forced_key_groups);
+bool       flash_attn_splits_keys(int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim, bool mask,
+                                  int forced_key_groups);
 size_t     flash_attn_workspace_bytes(int qo_len, int kv_len, int n_heads, int head_dim);
 hipError_t launch_flash_attn(hipStream_t stream, void *o, const void *q, const void *k, const void *v,
                              const void *mask, int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim,

@@ -505,7 +505,7 @@ int op_flash_attn(htpops_context *ctx, void *o, const void *q, const void *k, co
     note_device_write(ctx, q8_out, q8_0_bytes(1, (size_t) n_heads * head_dim));
   }
   void *shares = nullptr;
-  if (flash_attn_splits_keys(qo_len, kv_len, n_heads, n_kv_heads, head_dim, ctx->opt.attn_key_groups)) {
+  if (flash_attn_splits_keys(qo_len, kv_len, n_heads, n_kv_heads, head_dim, mask != nullptr, ctx->opt.attn_key_groups)) {
     shares = attention_shares(ctx);
   }
   HTPOPS_HIP(ctx, launch_flash_attn(ctx->stream, o, q, k, v, mask, qo_len, kv_len, n_heads, n_kv_heads, head_dim,
