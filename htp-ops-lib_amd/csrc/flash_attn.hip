@@ -105,9 +105,9 @@ __host__ __device__ constexpr size_t prefill_partial_floats(int units) {
   return (size_t) units * 4 * kWave + 2 * kWave;
 }
 
-// FULL: head_dim == DP (64 or 128); else head_dim is any multiple of 16 in (DP - 32, DP], and the probabilities keep
-// 22 bits (an fp16 pair, two matrix instructions per fragment of V): the plain kernel that these head dims took before
-// held them in fp32. GROUPS = 1 or 2 key groups per workgroup (4 waves each); with 2 they take alternate KV blocks of the
+// FULL: head_dim == DP (64 or 128); else head_dim is any multiple of 16 in (DP - 32, DP], and the probabilities are
+// fp16 pairs (two matrix instructions per fragment of V): the plain kernel that these head dims took before held them in
+// fp32. GROUPS = 1 or 2 key groups per workgroup (4 waves each); with 2 they take alternate KV blocks of the
 // same queries. MASK: there is one (a kernel of its own: the tests for it cost 2048 x 2048 without one 1 to 2 %). With
 // `shares` > 1 the blocks of a workgroup's queries are dealt to that many workgroups (gridDim.z), each of which leaves its
 // (max, sum, O) in `part` for flash_attn_prefill_merge_kernel. ALL: one workgroup walks all shares itself and folds them in
@@ -125,6 +125,7 @@ __global__ __launch_bounds__(kPfThreads *GROUPS, DP <= 128 ? 2 : 1) void flash_a
   __shared__ __align__(1024) Smem sm_all[GROUPS];
   constexpr int KSTEPS = DP / 16;  // MFMA k-steps over the head dimension
   constexpr int DT     = DP / 32;  // 32-row tiles of O^T
+  constexpr float kPScale = FULL ? 1.0f : 32768.0f;  // of the probabilities: O and l are both too large by it
   const int     D      = FULL ? DP : head_dim;
   // With GROUPS = 2, two groups of 4 waves work on the same queries and heads: group g takes KV blocks g, g + 2, ...
   // with its own K/V tiles in LDS and its own running (max, sum, O); the two states are merged through LDS at the
@@ -504,23 +505,29 @@ __global__ __launch_bounds__(kPfThreads *GROUPS, DP <= 128 ? 2 : 1) void flash_a
       }
       // the probabilities, rounded to fp16 in pairs as the matrix instruction takes them. FULL: the row sum adds up the
       // rounded values (v_dot2_f32_f16 with ones: two per instruction, fp32 sums), so O and l see the same numbers; else
-      // what the rounding left out goes into a second fp16 pair and the row sum adds up the fp32 values.
+      // they are at most 2^15 and cut off, what is cut off goes into a second fp16 pair, and the row sum adds up the fp32
+      // values. That holds 21 bits of each down to 2^-18 of the largest and 2^-39 of it below: behind a key that takes all but
+      // 2^-16 of the weight and has a value of zero the result is off by 7e-7, as with fp32 probabilities. (Unscaled pairs end
+      // at 2^-25 of the largest: 3e-5.) Where the first half is not zero neither is the second: times an infinite value it
+      // must not become not-a-number.
       uint32_t pk[2][8], pk_lo[FULL ? 1 : 2][FULL ? 1 : 8];
       float    psum[4] = { 0.0f, 0.0f, 0.0f, 0.0f };  // (four chains: an addition waits for the one before it in its chain)
       {
-        const v2h ones = { (_Float16) 1.0f, (_Float16) 1.0f };
+        const v2h ones = { (_Float16) 1.0f, (_Float16) 1.0f }, least = __builtin_bit_cast(v2h, 0x00010001u);  // (2^-24)
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt) {
 #pragma unroll
           for (int r = 0; r < 16; r += 2) {
-            const float p0 = fast_exp2(st[kt][r]), p1 = fast_exp2(st[kt][r + 1]);
-            const v2h   p2 = { (_Float16) p0, (_Float16) p1 };
-            pk[kt][r / 2]  = __builtin_bit_cast(uint32_t, p2);
+            const float p0 = fast_exp2(st[kt][r]) * kPScale, p1 = fast_exp2(st[kt][r + 1]) * kPScale;
             if constexpr (FULL) {
+              const v2h p2  = { (_Float16) p0, (_Float16) p1 };
+              pk[kt][r / 2] = __builtin_bit_cast(uint32_t, p2);
               psum[(r / 2) & 3] = __builtin_amdgcn_fdot2(p2, ones, psum[(r / 2) & 3], false);
             } else {
-              const v2h lo      = { (_Float16) (p0 - (float) p2[0]), (_Float16) (p1 - (float) p2[1]) };
-              pk_lo[kt][r / 2]  = __builtin_bit_cast(uint32_t, lo);
+              const v2h hi      = __builtin_bit_cast(v2h, __builtin_amdgcn_cvt_pkrtz(p0, p1));
+              const v2h lo      = { (_Float16) (p0 - (float) hi[0]), (_Float16) (p1 - (float) hi[1]) };
+              pk[kt][r / 2]     = __builtin_bit_cast(uint32_t, hi);
+              pk_lo[kt][r / 2]  = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(lo, __builtin_elementwise_min(hi, least)));
               psum[(r / 2) & 3] += p0 + p1;
             }
           }

@@ -155,3 +155,47 @@ def test_a_callers_graph_holds_nothing_of_the_context(ctx, name):
     assert hip.hipGraphExecDestroy(executable) == 0 and hip.hipGraphDestroy(graph) == 0 and hip.hipStreamDestroy(other) == 0
     for h in hs:
         ctx.release(h)
+
+
+def _exact(q, k, v, nh, nkv, d):
+    """Attention in 64 bits over the queries as the kernels round them: scaled in fp32, then fp16."""
+    scale = np.float32(1) / np.sqrt(np.float32(d)) * np.float32(1.4426950408889634)
+    qs = (q.astype(np.float32) * scale).astype(np.float16).astype(np.float64)
+    out = np.empty(q.shape, np.float64)
+    for h in range(nh):
+        s = qs[:, h] @ k[:, h // (nh // nkv)].astype(np.float64).T
+        p = np.exp2(s - s.max(axis=1, keepdims=True))
+        out[:, h] = p @ v[:, h // (nh // nkv)].astype(np.float64) / p.sum(axis=1, keepdims=True)
+    return out
+
+
+@pytest.mark.parametrize("qo,kv,nh,nkv,d", [(50, 500, 4, 2, 96), (1, 4096, 4, 2, 96), (7, 3000, 4, 2, 80), (64, 2000, 2, 1, 256), (33, 1000, 4, 4, 48),
+                                            (40, 70, 2, 2, 16), (3, 900, 2, 1, 160)])
+@pytest.mark.parametrize("weight", [0, 16, 26])
+def test_probabilities_of_padded_head_dims_keep_their_bits(ctx, qo, kv, nh, nkv, d, weight):
+    # `weight` > 0: one key takes all but some 2^-weight of the probability, and its value is zero, so the others decide. Bound:
+    # 21 bits of a probability (13 of one of 2^-26, over hundreds of keys), fp32 exponentials and sums: 1.5e-7 to 3e-6 measured
+    # (without the second pairs 2e-4, with pairs that end at 2^-25 of the largest 3e-5 and 4e-2).
+    rng = wl.rng_for(68, qo + kv + d + weight)
+    q, k, v = wl.make_attention_inputs(rng, qo, kv, nh, nkv, d)
+    q = q.astype(np.float32)
+    if weight:
+        q = np.abs(q) + 0.5
+        k[3] = weight * 0.6931 * d ** 0.5 / (d * 1.3)
+        v[3] = 0
+    print("attention bits", qo, kv, nh, nkv, d, weight, flush=True)
+    got = ctx.run_flash_attn(q, k, v, None, nh, nkv, d)
+    want = _exact(q, k, v, nh, nkv, d)
+    error = np.linalg.norm(got.astype(np.float64) - want) / np.linalg.norm(want)
+    print("relative error %.2e" % error, flush=True)
+    assert error <= 6e-6
+
+
+@pytest.mark.parametrize("qo,kv,d", [(1, 300, 96), (40, 700, 80), (130, 130, 256)])
+def test_an_infinite_value_gives_an_infinity_in_its_column_alone(ctx, qo, kv, d):
+    rng = wl.rng_for(69, qo + kv + d)
+    q, k, v = wl.make_attention_inputs(rng, qo, kv, 2, 1, d)
+    v[kv // 2, 0, 5], v[kv // 3, 0, d - 1] = np.inf, -np.inf
+    got = ctx.run_flash_attn(q.astype(np.float32), k, v, None, 2, 1, d)
+    assert np.isposinf(got[:, :, 5]).all() and np.isneginf(got[:, :, d - 1]).all()
+    assert np.isfinite(np.delete(got, (5, d - 1), axis=2)).all()
