@@ -220,6 +220,7 @@ const void *find_copy(htpops_context *ctx, const void *weight, int kind, int k, 
 int  new_copy(htpops_context *ctx, const void *weight, size_t src_bytes, int kind, int k, int n, size_t frag_bytes,
               void **out);
 void forget_copy(htpops_context *ctx, void *frag);
+bool copy_fits_cap(const htpops_context *ctx, size_t bytes);  // ... beside the copies that are there
 
 // ---- ops (ops.cc) ----
 constexpr int kSkinnyGroupMaxM = 8;   // rows of the K-sliced kernel's grouped launch

@@ -81,7 +81,7 @@ int run_fragment_group(htpops_context *ctx, GemvBatch &b) {
       return 1;  // (a converted copy went away since the member joined: the caller runs the members one by one)
     }
     if (int r = plan_weight_copy(ctx, plan, b.w[i], b.k[i], b.n[i], b.wt, &wf[i])) {
-      return r;
+      return b.m < kFp6MinM ? 1 : r;  // (no memory for a copy that only buys speed: the members see to it themselves)
     }
   }
   // distinct (activation, k) pairs and where their conversions go

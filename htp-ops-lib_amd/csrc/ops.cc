@@ -29,16 +29,15 @@ int op_rms_norm(htpops_context *ctx, float *dst, const float *src, const float *
 namespace {
 
 // where a quantizer of m rows of k leaves them in operand order as well (nullptr: nobody asked)
-int wanted_fragments(htpops_context *ctx, int m, int k, void **where) {
+void wanted_fragments(htpops_context *ctx, int m, int k, void **where) {
   *where = nullptr;
   if (ctx->next_fragments_ws == 0 || (long long) m * (k / 32) > 0x7fffffffLL) {
-    return HTPOPS_OK;
+    return;
   }
-  if (int r = ensure_workspace(ctx, ctx->next_fragments_ws)) {
-    return r;
+  // (no memory for what would only spare the matmul a launch: the rows are quantized without it)
+  if (ensure_workspace(ctx, ctx->next_fragments_ws) == HTPOPS_OK) {
+    *where = ctx->workspace;
   }
-  *where = ctx->workspace;
-  return HTPOPS_OK;
 }
 
 void note_fragments(htpops_context *ctx, const void *where, const void *rows, int m, int k) {
@@ -61,9 +60,7 @@ int op_quantize(htpops_context *ctx, void *dst, const float *src, int k, int m) 
     return r;
   }
   void *frags = nullptr;
-  if (int r = wanted_fragments(ctx, m, k, &frags)) {
-    return r;
-  }
+  wanted_fragments(ctx, m, k, &frags);
   note_device_write(ctx, dst, q8_0_bytes((size_t) m, (size_t) k));
   HTPOPS_HIP(ctx, launch_quantize_q8_0(ctx->stream, dst, src, k, m, frags));
   note_fragments(ctx, frags, dst, m, k);
@@ -83,9 +80,7 @@ int op_rms_norm_quantize(htpops_context *ctx, void *dst, const float *src, const
   }
   if (ne0 <= 16384) {
     void *frags = nullptr;
-    if (int r = wanted_fragments(ctx, ne1, ne0, &frags)) {
-      return r;
-    }
+    wanted_fragments(ctx, ne1, ne0, &frags);
     note_device_write(ctx, dst, q8_0_bytes((size_t) ne1, (size_t) ne0));
     HTPOPS_HIP(ctx, launch_rms_norm_quantize_q8_0(ctx->stream, dst, src, weight, eps, ne0, ne1, frags));
     note_fragments(ctx, frags, dst, ne1, ne0);
@@ -198,9 +193,11 @@ MatMulPlan plan_mat_mul(htpops_context *ctx, const void *weight, bool act_aligne
   // 17 to 32 rows, K-sliced kernel / here: seven projections of a Llama-7B / Qwen2-1.5B layer, Q8_0, 117 and 65 us in seven
   // launches / 47 and 19 us; one matrix over fp32 rows, k = 8960, n = 1537 13.2 / 11.9, k = 4096, n = 11008 27.5 / 17.0,
   // but k = 1024, n = 700 8.4 / 9.6.
+  // And only over one that needs no room another copy has (a cap on all of them): those kernels need none.
   if (m < kFp6MinM && !overwrites) {
     lookup_copy(kFragKindRowLayout + wt);
-    if (!p.cached && !p.cacheable) {
+    if (!p.cached && !(p.cacheable && copy_fits_cap(ctx, (gemm_i8_weight_fragment_bytes(k, n) + 255) & ~(size_t) 255))) {
+      p.cacheable = false;
       p.ws_bytes = mat_mul_workspace_bytes(m, k, n);
       return p;
     }
@@ -235,6 +232,17 @@ int plan_weight_copy(htpops_context *ctx, MatMulPlan &plan, const void *weight, 
 }
 
 namespace {
+
+// Up to 32 rows a copy only buys speed: where there is no memory for it, the matmul takes the kernels that read the weights
+// as they are.
+void settle_copy(htpops_context *ctx, MatMulPlan &plan, const void *weight, int m, int k, int n, int wt) {
+  const void *copy = nullptr;
+  if (plan.kind == kPlanFragments && m < kFp6MinM && plan.cacheable &&
+      plan_weight_copy(ctx, plan, weight, k, n, wt, &copy) != HTPOPS_OK) {
+    plan          = MatMulPlan();
+    plan.ws_bytes = mat_mul_workspace_bytes(m, k, n);
+  }
+}
 
 int run_few_rows(htpops_context *ctx, float *dst, const void *act, const void *weight, int m, int k, int n, int wt,
                  uint8_t *ws) {
@@ -342,6 +350,7 @@ int op_mat_mul_q8(htpops_context *ctx, float *dst, const void *act, const void *
   }
   note_device_write(ctx, dst, (size_t) m * n * 4);
   MatMulPlan plan = plan_mat_mul(ctx, weight, aligned(act, 4), m, k, n, weight_type, writes_weights(dst, weight, m, k, n, weight_type));
+  settle_copy(ctx, plan, weight, m, k, n, weight_type);
   if (int r = ensure_workspace(ctx, plan.ws_bytes, /*keep_act_fragments=*/true)) {
     return r;
   }
@@ -361,6 +370,7 @@ int op_mat_mul_f32(htpops_context *ctx, float *dst, const float *act, const void
   }
   note_device_write(ctx, dst, (size_t) m * n * 4);
   MatMulPlan plan = plan_mat_mul(ctx, weight, true, m, k, n, weight_type, writes_weights(dst, weight, m, k, n, weight_type));
+  settle_copy(ctx, plan, weight, m, k, n, weight_type);
   if (plan.kind == kPlanFragments && (long long) m * (k / 32) <= 0x7fffffffLL) {
     // the quantizer writes the operand order the matmul wants: the rows in block_q8_0 form would have one reader, another
     // launch that puts them into that order (33 rows, k = 8960, n = 1537: 3 of 18 us)

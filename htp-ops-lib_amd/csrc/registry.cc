@@ -190,6 +190,10 @@ int new_copy(htpops_context *ctx, const void *weight, size_t src_bytes, int kind
   return HTPOPS_OK;
 }
 
+bool copy_fits_cap(const htpops_context *ctx, size_t bytes) {
+  return ctx->opt.converted_cap_mib <= 0 || ctx->converted_bytes + bytes <= (size_t) ctx->opt.converted_cap_mib << 20;
+}
+
 void forget_copy(htpops_context *ctx, void *frag) {
   for (size_t i = 0; i < ctx->frag_cache.size(); ++i) {
     if (ctx->frag_cache[i].frag == frag) {
