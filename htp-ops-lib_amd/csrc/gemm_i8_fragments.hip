@@ -979,9 +979,10 @@ SmallTilePlan small_tile_plan(int m_tiles, int n_tiles, int nblk, TileConfig cfg
   // a wave at least / split: k = 8960, n = 1537, 33 rows 23.7 / 14.3 us; k = n = 4096, 33 rows 20.5 / 14.5. (16 waves of
   // one workgroup on a tile's K instead, no exchange: 27 rows, k = 8960, n = 1537 14.2 against 11.9 us.)
   // (short K with 128 tiles and more keeps the shared activations: seven projections of Qwen2 size at 70 rows 26.6 against
-  // 28.5 us)
+  // 28.5 us; one row tile, whose 128 column tiles would be 32 workgroups, does up to 255: 17 rows, k = 2048, n = 4096 14.3 /
+  // 11.1 us, but k = 512, n = 8960 8.0 / 9.5)
   const int wgs = m_tiles * ((n_tiles + kGiWaves / cfg.ksplit - 1) / (kGiWaves / cfg.ksplit));
-  if (split_k && wgs < kSmallWgs && nblk >= 2 * kGiWaves && (cfg.ksplit > 1 || m_tiles * n_tiles < kSmallWgs / 2)) {
+  if (split_k && wgs < kSmallWgs && nblk >= 2 * kGiWaves && (cfg.ksplit > 1 || m_tiles * n_tiles < (m_tiles == 1 ? kSmallWgs : kSmallWgs / 2))) {
     return { kSharePlain, kGiWaves, std::max(1, std::min({ kMaxParts, kSmallWgs / (m_tiles * n_tiles), nblk / (kGiWaves * 12) })) };
   }
   // (measured on the Qwen2 block at 128 rows: weights shared 39.6 us, activations shared 40.2 us, neither 43.9 us)

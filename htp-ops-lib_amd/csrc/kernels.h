@@ -55,11 +55,13 @@ hipError_t launch_gemv_rows_group_q8_0_act(hipStream_t stream, int count, float 
 size_t     matmul_skinny_workspace_bytes(int m, int k, int n);
 hipError_t launch_matmul_skinny(hipStream_t stream, float *out, const void *act, const void *weight, int m, int k,
                                 int n, WeightType wt, void *workspace, unsigned *tickets, int ticket_slots);
-// several weight matrices against the same 2 <= m <= 8 activation rows in one launch; hipErrorNotSupported when the
-// shapes do not fit the K-sliced kernel (the caller then launches them one by one)
-size_t     matmul_skinny_group_workspace_bytes(int count, const int *ns, int m, int k);
-hipError_t launch_matmul_skinny_group(hipStream_t stream, int count, float *const *outs, const void *act,
-                                      const void *const *weights, const int *ns, int m, int k, WeightType wt,
+// several weight matrices, each with its own 2 <= m <= 32 activation rows and k, in one launch; hipErrorNotSupported when the
+// shapes do not fit the K-sliced kernel (matmul_skinny_slices_fit, and tickets enough; the caller then launches them one by
+// one). A member's result is what its own launch gives.
+bool       matmul_skinny_slices_fit(const void *weight, int n, int k, WeightType wt);
+size_t     matmul_skinny_group_workspace_bytes(int count, const int *ns, int m, const int *ks);
+hipError_t launch_matmul_skinny_group(hipStream_t stream, int count, float *const *outs, const void *const *acts,
+                                      const void *const *weights, const int *ns, int m, const int *ks, WeightType wt,
                                       void *workspace, unsigned *tickets, int ticket_slots);
 // 2 <= m <= 16 rows against Q4_0 or Q8_0 weights repacked once (launch_weights_to_lane_order into
 // matmul_lane_order_weight_bytes, same size as the weights; the caller can cache the copy) into matrix-core operand

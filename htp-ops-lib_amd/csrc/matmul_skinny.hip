@@ -20,6 +20,8 @@
 #include "device_utils.h"
 #include "kernels.h"
 
+#include <algorithm>
+
 namespace htpops {
 
 namespace {
@@ -316,27 +318,34 @@ struct SliceGeom {
 typedef __attribute__((address_space(1))) const void *sk_gptr_t;
 typedef __attribute__((address_space(3))) void       *sk_lptr_t;
 
-// Several weight matrices that meet the same activation rows (the q/k/v or gate/up projections of a decoder layer)
-// share one launch: blockIdx.z picks the member, whose weight pointer, output pointer, row count and first tile
-// (for its partial tiles and ticket counters) come from the argument table.
+// Several weight matrices (the projections of a decoder layer) share one launch: blockIdx.z picks the member, whose weights,
+// activation rows, output, sizes, first tile (for its ticket counters) and first partial tile come from the argument table.
 struct SkinnyGroupArgs {
-  const uint8_t *w[kGemvGroupMax];
+  const uint8_t *w[kGemvGroupMax], *act[kGemvGroupMax];
   float         *out[kGemvGroupMax];
-  int            n[kGemvGroupMax];
-  int            tile0[kGemvGroupMax];
+  int            n[kGemvGroupMax], k[kGemvGroupMax];
+  int            tile0[kGemvGroupMax], partial0[kGemvGroupMax];
 };
+int tiles_of(int n) {
+  return (n + kSkRows - 1) / kSkRows;
+}
+int slices_of(int k) {
+  return (k / 64 + kSlPairs - 1) / kSlPairs;
+}
 
 template <WeightType WT, int MR>
-__global__ __launch_bounds__(kSlThreads) void matmul_skinny_slice_kernel(SkinnyGroupArgs grp,
-                                                                        const uint8_t *__restrict__ act, int m,
-                                                                        int k, float *__restrict__ partials,
+__global__ __launch_bounds__(kSlThreads) void matmul_skinny_slice_kernel(SkinnyGroupArgs grp, int m,
+                                                                        float *__restrict__ partials,
                                                                         unsigned *__restrict__ tickets) {
   typedef SliceGeom<WT> G;
   const int                     n      = grp.n[blockIdx.z];
   float *__restrict__           out    = grp.out[blockIdx.z];
   const uint8_t *__restrict__   weight = grp.w[blockIdx.z];
-  if ((int) (blockIdx.x * kSkRows) >= n) {
-    return;  // whole workgroup: this member has fewer rows than the widest one
+  const uint8_t *__restrict__   act    = grp.act[blockIdx.z];
+  const int                     k      = grp.k[blockIdx.z];
+  const int                     nslices = (k / 64 + kSlPairs - 1) / kSlPairs;
+  if ((int) (blockIdx.x * kSkRows) >= n || (int) blockIdx.y >= nslices) {
+    return;  // whole workgroup: this member has fewer rows or slices than the widest one
   }
   constexpr int MPAD     = 2 * MR;
   constexpr int WROW_BLK = WT == kQ4_0 ? 18 : 34;
@@ -351,8 +360,9 @@ __global__ __launch_bounds__(kSlThreads) void matmul_skinny_slice_kernel(SkinnyG
   const int lane = tid & 63, wave = tid >> 6;
   const int nl = lane & 31, half = lane >> 5;
   const int nblk    = k / 32;
-  const int tile    = blockIdx.x, slice = blockIdx.y, nslices = gridDim.y;
-  const int gtile   = grp.tile0[blockIdx.z] + tile;  // among all members: partial tiles and tickets
+  const int tile    = blockIdx.x, slice = blockIdx.y;
+  const int gtile   = grp.tile0[blockIdx.z] + tile;  // among all members (tickets)
+  float    *parts   = partials + ((size_t) grp.partial0[blockIdx.z] + (size_t) tile * nslices) * (MR * 64);
   const int n0      = tile * kSkRows;
   const int a_slot  = min(nl, MPAD - 1);
   const int pair0   = slice * kSlPairs;
@@ -421,7 +431,7 @@ __global__ __launch_bounds__(kSlThreads) void matmul_skinny_slice_kernel(SkinnyG
     // The partials travel as device-scope atomic stores and loads (written through to / read from the level all
     // XCDs share) and the ticket is taken only after the stores are acknowledged; a device-scope fence would do the
     // same job by writing back the whole L2, which costs tens of microseconds per workgroup.
-    float *mine = partials + ((size_t) gtile * nslices + slice) * (MR * 64);
+    float *mine = parts + (size_t) slice * (MR * 64);
 #pragma unroll
     for (int e = 0; e < EPT; ++e) {
       __hip_atomic_store(&mine[e * kSlThreads + tid], v[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -436,7 +446,7 @@ __global__ __launch_bounds__(kSlThreads) void matmul_skinny_slice_kernel(SkinnyG
       return;
     }
     __atomic_signal_fence(__ATOMIC_SEQ_CST);  // (compile time: the loads below stay behind the ticket; the barrier above orders them in hardware)
-    const float *all = partials + (size_t) gtile * nslices * (MR * 64);
+    const float *all = parts;
 #pragma unroll
     for (int e = 0; e < EPT; ++e) {
       v[e] = 0.0f;
@@ -490,36 +500,35 @@ hipError_t allow_big_lds(K kernel) {
 
 template <int MR>
 size_t slice_partial_bytes(int k, int n) {
-  const size_t tiles = ((size_t) n + kSkRows - 1) / kSkRows, nslices = ((size_t) k / 64 + kSlPairs - 1) / kSlPairs;
+  const size_t tiles = (size_t) tiles_of(n), nslices = (size_t) slices_of(k);
   return nslices > 1 ? tiles * nslices * MR * 64 * sizeof(float) : 0;
 }
 
 template <WeightType WT, int MR>
-hipError_t launch_skinny_slices(hipStream_t stream, const SkinnyGroupArgs &grp, int count, const void *act, int m, int k,
-                                void *workspace, unsigned *tickets) {
-  int n_max = 0;
+hipError_t launch_skinny_slices(hipStream_t stream, const SkinnyGroupArgs &grp, int count, int m, void *workspace,
+                                unsigned *tickets) {
+  int tiles = 0, nslices = 0;
   for (int i = 0; i < count; ++i) {
-    n_max = grp.n[i] > n_max ? grp.n[i] : n_max;
+    tiles = std::max(tiles, tiles_of(grp.n[i])), nslices = std::max(nslices, slices_of(grp.k[i]));
   }
-  const unsigned tiles = (unsigned) ((n_max + kSkRows - 1) / kSkRows), nslices = (unsigned) ((k / 64 + kSlPairs - 1) / kSlPairs);
-  hipLaunchKernelGGL((matmul_skinny_slice_kernel<WT, MR>), dim3(tiles, nslices, (unsigned) count), dim3(kSlThreads), 0, stream,
-                     grp, static_cast<const uint8_t *>(act), m, k, static_cast<float *>(workspace), tickets);
+  hipLaunchKernelGGL((matmul_skinny_slice_kernel<WT, MR>), dim3((unsigned) tiles, (unsigned) nslices, (unsigned) count),
+                     dim3(kSlThreads), 0, stream, grp, m, static_cast<float *>(workspace), tickets);
   return hipGetLastError();
 }
 
 // true when the K-sliced kernel can take these matrices in one launch
 template <WeightType WT>
-bool slices_fit(const SkinnyGroupArgs &grp, int count, int k, const void *workspace, const unsigned *tickets, int ticket_slots) {
-  const size_t row_bytes = (size_t) (k / 32) * (WT == kQ4_0 ? 18 : 34);
-  const bool   split     = k / 64 > kSlPairs;
-  int          tiles     = 0;
+bool slices_fit(const SkinnyGroupArgs &grp, int count, const void *workspace, const unsigned *tickets, int ticket_slots) {
+  bool split = false;
+  int  tiles = 0;
   for (int i = 0; i < count; ++i) {
-    if (reinterpret_cast<uintptr_t>(grp.w[i]) % 16 != 0 || (grp.n[i] + kSkRows - 1) / kSkRows > 65535) {
+    if (!matmul_skinny_slices_fit(grp.w[i], grp.n[i], grp.k[i], WT)) {
       return false;
     }
-    tiles += (grp.n[i] + kSkRows - 1) / kSkRows;
+    split = split || slices_of(grp.k[i]) > 1;
+    tiles += tiles_of(grp.n[i]);
   }
-  return row_bytes % 16 == 0 && (!split || (workspace && tickets && tiles <= ticket_slots));
+  return !split || (workspace && tickets && tiles <= ticket_slots);
 }
 
 template <WeightType WT, int MR>
@@ -527,9 +536,10 @@ hipError_t launch_skinny(hipStream_t stream, float *out, const void *act, const 
                          void *workspace, unsigned *tickets, int ticket_slots) {
   const int nblk = k / 32;
   SkinnyGroupArgs  one = {};
-  one.w[0] = static_cast<const uint8_t *>(weight), one.out[0] = out, one.n[0] = n, one.tile0[0] = 0;
-  if (slices_fit<WT>(one, 1, k, workspace, tickets, ticket_slots)) {
-    return launch_skinny_slices<WT, MR>(stream, one, 1, act, m, k, workspace, tickets);
+  one.w[0] = static_cast<const uint8_t *>(weight), one.act[0] = static_cast<const uint8_t *>(act), one.out[0] = out;
+  one.n[0] = n, one.k[0] = k;
+  if (slices_fit<WT>(one, 1, workspace, tickets, ticket_slots)) {
+    return launch_skinny_slices<WT, MR>(stream, one, 1, m, workspace, tickets);
   }
   constexpr int per_kb = ActChunk<MR>::PER_KB;
   const size_t  budget = 96 * 1024;
@@ -574,32 +584,44 @@ size_t matmul_skinny_workspace_bytes(int m, int k, int n) {
   return rows <= 8 ? slice_partial_bytes<4>(k, n) : rows <= 16 ? slice_partial_bytes<8>(k, n) : slice_partial_bytes<16>(k, n);
 }
 
-size_t matmul_skinny_group_workspace_bytes(int count, const int *ns, int m, int k) {
+bool matmul_skinny_slices_fit(const void *weight, int n, int k, WeightType wt) {
+  return k % 64 == 0 && (size_t) (k / 32) * (wt == kQ4_0 ? 18 : 34) % 16 == 0 && reinterpret_cast<uintptr_t>(weight) % 16 == 0 &&
+         tiles_of(n) <= 65535 && slices_of(k) <= 65535;
+}
+
+size_t matmul_skinny_group_workspace_bytes(int count, const int *ns, int m, const int *ks) {
   size_t total = 0;
   for (int i = 0; i < count; ++i) {
-    total += matmul_skinny_workspace_bytes(m, k, ns[i]);
+    total += matmul_skinny_workspace_bytes(m, ks[i], ns[i]);
   }
   return total;
 }
 
-hipError_t launch_matmul_skinny_group(hipStream_t stream, int count, float *const *outs, const void *act,
-                                      const void *const *weights, const int *ns, int m, int k, WeightType wt,
+hipError_t launch_matmul_skinny_group(hipStream_t stream, int count, float *const *outs, const void *const *acts,
+                                      const void *const *weights, const int *ns, int m, const int *ks, WeightType wt,
                                       void *workspace, unsigned *tickets, int ticket_slots) {
-  if (count < 1 || count > kGemvGroupMax || k % 64 != 0 || m < 2 || m > 8) {
+  if (count < 1 || count > kGemvGroupMax || m < 2 || m > 32) {
     return hipErrorNotSupported;
   }
   SkinnyGroupArgs grp = {};
   int             tile0 = 0;
+  long long       partial0 = 0;
   for (int i = 0; i < count; ++i) {
-    grp.w[i] = static_cast<const uint8_t *>(weights[i]), grp.out[i] = outs[i], grp.n[i] = ns[i], grp.tile0[i] = tile0;
-    tile0 += (ns[i] + kSkRows - 1) / kSkRows;
+    grp.w[i] = static_cast<const uint8_t *>(weights[i]), grp.act[i] = static_cast<const uint8_t *>(acts[i]), grp.out[i] = outs[i];
+    grp.n[i] = ns[i], grp.k[i] = ks[i], grp.tile0[i] = tile0, grp.partial0[i] = (int) partial0;
+    tile0 += tiles_of(ns[i]);
+    partial0 += slices_of(ks[i]) > 1 ? (long long) tiles_of(ns[i]) * slices_of(ks[i]) : 0;
   }
-  if (wt == kQ4_0) {
-    return slices_fit<kQ4_0>(grp, count, k, workspace, tickets, ticket_slots) ?
-             launch_skinny_slices<kQ4_0, 4>(stream, grp, count, act, m, k, workspace, tickets) : hipErrorNotSupported;
+  const bool fit = wt == kQ4_0 ? slices_fit<kQ4_0>(grp, count, workspace, tickets, ticket_slots) :
+                                 slices_fit<kQ8_0>(grp, count, workspace, tickets, ticket_slots);
+  if (!fit || partial0 > 0x7fffffffLL) {
+    return hipErrorNotSupported;
   }
-  return slices_fit<kQ8_0>(grp, count, k, workspace, tickets, ticket_slots) ?
-           launch_skinny_slices<kQ8_0, 4>(stream, grp, count, act, m, k, workspace, tickets) : hipErrorNotSupported;
+#define HTPOPS_SLICES(MR)                                                                              \
+  wt == kQ4_0 ? launch_skinny_slices<kQ4_0, MR>(stream, grp, count, m, workspace, tickets) :           \
+                launch_skinny_slices<kQ8_0, MR>(stream, grp, count, m, workspace, tickets)
+  return m <= 8 ? HTPOPS_SLICES(4) : m <= 16 ? HTPOPS_SLICES(8) : HTPOPS_SLICES(16);
+#undef HTPOPS_SLICES
 }
 
 hipError_t launch_matmul_skinny(hipStream_t stream, float *out, const void *act, const void *weight, int m, int k,

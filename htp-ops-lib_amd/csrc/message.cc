@@ -42,8 +42,9 @@ namespace {
 //    launch; where a real data dependency exists (o after attention after q/k/v) the run is split there;
 //  * 2..16 rows: members of the same k; those that take the repacked-weight kernel share its launch whatever rows
 //    they read, the others only with members that read the same rows (q/k/v or gate/up);
-//  * many rows (17 and more over converted weights): one launch per tile configuration for the products, one for the
-//    conversions of activations that their quantizers have not left in operand order already.
+//  * many rows (17 and more): over converted weights one launch per tile configuration for the products and one for the
+//    conversions of activations that their quantizers have not left in operand order already; one launch for members of up to
+//    32 rows that read the weights as they are.
 struct GemvBatch {
   int                   wt = 0, m = 0, count = 0;
   struct RequestHeader *hdr[kGemvGroupMax];
@@ -68,6 +69,12 @@ struct GemvBatch {
   bool fp6   = false;  // many-row members of the FP6-tile kernel (all over the same activation rows and k)
   bool pairs_fit = false;  // every member fits the two-blocks-per-instruction kernel (such members may differ in k)
 };
+
+// A matmul of 17 to 32 rows that by itself takes the K-sliced kernel (see plan_mat_mul)
+bool takes_slices(htpops_context *ctx, const void *w, int m, int k, int n, int wt) {
+  return m >= kManyRowsMinM && m < kFp6MinM && matmul_skinny_slices_fit(w, n, k, (WeightType) wt) &&
+         plan_mat_mul(ctx, w, true, m, k, n, wt).kind == kPlanFewRows;
+}
 
 // The many-row members of a batch: converted weights from the cache (made now where missing), the distinct activation
 // matrices converted side by side in the workspace by one launch, then one launch for all the products. Returns a
@@ -125,6 +132,36 @@ int run_fragment_group(htpops_context *ctx, GemvBatch &b) {
   }
   HTPOPS_HIP(ctx, launch_gemm_i8_fragments_group(ctx->stream, b.count, b.out, af, wf, b.n, b.k, b.m, ws + total, xbytes,
                                                  ctx->tickets, kTicketSlots, ctx->opt.gemm_tile_units));
+  return HTPOPS_OK;
+}
+
+// Members of 17 to 32 rows and of more that are not of the FP6-tile kernel: those that take the K-sliced kernel by themselves
+// share a launch of it, behind the others' (which may find their rows in the workspace already). Returns as above.
+int run_many_rows_group(htpops_context *ctx, GemvBatch &all) {
+  GemvBatch of[2];  // [1]: K-sliced
+  for (int i = 0; i < all.count; ++i) {
+    GemvBatch &b = of[takes_slices(ctx, all.w[i], all.m, all.k[i], all.n[i], all.wt) ? 1 : 0];
+    b.wt = all.wt, b.m = all.m, b.out[b.count] = all.out[i], b.w[b.count] = all.w[i], b.act[b.count] = all.act[i];
+    b.n[b.count] = all.n[i], b.k[b.count++] = all.k[i];
+  }
+  if (of[0].count > 0) {
+    if (int r = run_fragment_group(ctx, of[0])) {
+      return r;
+    }
+  }
+  const GemvBatch &b = of[1];
+  if (b.count > 0) {
+    if (int r = ensure_workspace(ctx, matmul_skinny_group_workspace_bytes(b.count, b.n, b.m, b.k))) {
+      return r;
+    }
+    const hipError_t e = launch_matmul_skinny_group(ctx->stream, b.count, b.out, b.act, b.w, b.n, b.m, b.k, (WeightType) b.wt,
+                                                    ctx->workspace, ctx->tickets, kTicketSlots);
+    if (e == hipErrorNotSupported) {
+      (void) hipGetLastError();
+      return 1;
+    }
+    HTPOPS_HIP(ctx, e);
+  }
   return HTPOPS_OK;
 }
 
@@ -212,7 +249,7 @@ void flush_batch(htpops_context *ctx, GemvBatch &b) {
     const int        k0 = b.k[0];
     hipError_t e;
     if (b.m > kBatchMaxM) {
-      ret = b.fp6 ? run_fp6_group(ctx, b) : run_fragment_group(ctx, b);
+      ret = b.fp6 ? run_fp6_group(ctx, b) : run_many_rows_group(ctx, b);
       e   = ret == 1 ? hipErrorNotSupported : hipSuccess;
       ret = ret == 1 ? HTPOPS_OK : ret;
     } else if (b.m == 1) {
@@ -277,19 +314,20 @@ void flush_batch(htpops_context *ctx, GemvBatch &b) {
           continue;
         }
         float      *out_b[kGemvGroupMax];
-        const void *w_b[kGemvGroupMax];
-        int         n_b[kGemvGroupMax], count_b = 0;
+        const void *w_b[kGemvGroupMax], *act_b[kGemvGroupMax];
+        int         n_b[kGemvGroupMax], k_b[kGemvGroupMax], count_b = 0;
         for (int i = first; i < b.count; ++i) {  // everybody left that reads the rows of `first`
           if (sliced[i] && b.act[i] == b.act[first] && b.k[i] == b.k[first]) {
-            out_b[count_b] = b.out[i], w_b[count_b] = b.w[i], n_b[count_b++] = b.n[i];
+            out_b[count_b] = b.out[i], w_b[count_b] = b.w[i], act_b[count_b] = b.act[i], k_b[count_b] = b.k[i];
+            n_b[count_b++] = b.n[i];
             sliced[i] = false;
           }
         }
-        const size_t ws = matmul_skinny_group_workspace_bytes(count_b, n_b, b.m, b.k[first]);
+        const size_t ws = matmul_skinny_group_workspace_bytes(count_b, n_b, b.m, k_b);
         if (int r = ensure_workspace(ctx, ws)) {
           ret = r;
         } else {
-          e = launch_matmul_skinny_group(ctx->stream, count_b, out_b, b.act[first], w_b, n_b, b.m, b.k[first],
+          e = launch_matmul_skinny_group(ctx->stream, count_b, out_b, act_b, w_b, n_b, b.m, k_b,
                                                  (WeightType) b.wt, ctx->workspace, ctx->tickets, kTicketSlots);
         }
       }
@@ -365,14 +403,13 @@ bool try_batch(htpops_context *ctx, const struct OpComputeRequest *req, struct R
   bool       fp6       = false;
   if (many_rows) {
     // only matmuls over a converted copy kept with the weight buffer that take the FP6-tile kernel (members of a launch
-    // read the same activation rows) or the fragment kernel in its small-tile configuration; everything else runs on
-    // its own
+    // read the same activation rows) or the fragment kernel in a configuration that takes members of any k, and those of up
+    // to 32 rows that take the K-sliced kernel; everything else runs on its own
     const MatMulPlan plan = plan_mat_mul(ctx, w, aligned(act, 4), p->m, p->k, p->n, wt);
-    if (!(plan.cached || plan.cacheable)) {
-      return false;
-    }
-    fp6 = plan.kind == kPlanLdsFp6;
-    if (!fp6 && !(plan.kind == kPlanFragments && gemm_i8_fragments_groupable(p->m, p->n, ctx->opt.gemm_tile_units))) {
+    fp6 = plan.kind == kPlanLdsFp6 && (plan.cached || plan.cacheable);
+    if (!fp6 && !(plan.kind == kPlanFragments && (plan.cached || plan.cacheable) &&
+                  gemm_i8_fragments_groupable(p->m, p->n, ctx->opt.gemm_tile_units)) &&
+        !(plan.kind == kPlanFewRows && p->m < kFp6MinM && matmul_skinny_slices_fit(w, p->n, p->k, (WeightType) wt))) {
       return false;
     }
   }

@@ -189,13 +189,19 @@ MatMulPlan plan_mat_mul(htpops_context *ctx, const void *weight, bool act_aligne
       return p;
     }
   }
-  // Up to 32 rows only over a copy that is kept: the kernels that read the weights as they are beat a conversion per call.
-  // 17 to 32 rows, K-sliced kernel / here: seven projections of a Llama-7B / Qwen2-1.5B layer, Q8_0, 117 and 65 us in seven
-  // launches / 47 and 19 us; one matrix over fp32 rows, k = 8960, n = 1537 13.2 / 11.9, k = 4096, n = 11008 27.5 / 17.0,
-  // but k = 1024, n = 700 8.4 / 9.6.
-  // And only over one that needs no room another copy has (a cap on all of them): those kernels need none.
+  // Up to 32 rows only over a copy that is kept: the kernels that read the weights as they are beat a conversion per call. And
+  // only over one that needs no room another copy has (a cap on all of them): those kernels need none. And only large matrices
+  // or long K (gemm_tile_units set: any). 17 rows of Q8_0 behind their quantizer, K-sliced kernel / here: k = 512 to 2048 and n
+  // up to 2048 6.8 - 10.1 / 8.8 - 11.0 us; k = 4096 and n up to 2048 10.0 - 10.9 / 10.2 - 10.7, and the rows of one layer's q, k
+  // and v should meet one kernel; k = 2048, n = 4096 10.5 / 11.2, k = 1536, n = 8960 14.8 / 12.4, k = n = 4096 13.6 / 11.2, k =
+  // 8960, n = 1536 13.7 / 11.6, k = n = 8960 39 / 31. Layers of hidden 512 / 1024 / 1536 / 2048 with the line there, against
+  // all matrices here, 41 / 46 / 57 / 56 and 48 / 51 / 59 / 59 us. What it costs: a message whose matrices are all ready and
+  // fall on both sides takes two launches (seven projections of hidden 1536 24.8 against 17.6 us; seven K-sliced ones 65).
   if (m < kFp6MinM && !overwrites) {
-    lookup_copy(kFragKindRowLayout + wt);
+    const bool large = k >= 4096 || (size_t) n * k > (size_t) 4 << 20 || ctx->opt.gemm_tile_units != 0;
+    if (large) {
+      lookup_copy(kFragKindRowLayout + wt);
+    }
     if (!p.cached && !(p.cacheable && copy_fits_cap(ctx, (gemm_i8_weight_fragment_bytes(k, n) + 255) & ~(size_t) 255))) {
       p.cacheable = false;
       p.ws_bytes = mat_mul_workspace_bytes(m, k, n);

@@ -36,9 +36,10 @@ def test_output_over_the_weights(oracle, wt, m, k, n, fp32_rows):
         want = run((ho, 0), hw)
         assert np.array_equal(want, run((ho, 0), hb)) and want.any()  # (a copy of the second buffer's weights is there now)
         got = run((hb, at), hb)
-        if m <= 40:
+        if m == 32 or m == 40:
             assert np.array_equal(want, got)
-        else:  # (without a copy that may be kept Q4_0 takes the int8 kernels: other fp32 sums over the same exact block sums)
+        else:  # (a converted copy in the workspace: not the kernels of few rows and small matrices or of FP6 tiles, but other fp32
+               # sums over the same exact block sums)
             assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max()
         # what lies there now, read as weights: the columns whose blocks were left alone are what they were
         left = at // (w.size // n)

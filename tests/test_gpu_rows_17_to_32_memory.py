@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("grouped", [False, True])
 def test_a_copy_that_does_not_fit_the_cap_is_not_made(oracle, grouped):
-    wt, m, k, n = wl.GGML_TYPE_Q8_0, 24, 2048, 2048
+    wt, m, k, n = wl.GGML_TYPE_Q8_0, 24, 4096, 1024
     rng = wl.rng_for(97, 0)
     ws = [wl.make_weights(rng, n, k, wt) for _ in range(3)]
     x = wl.make_activations(rng, m, k)

@@ -29,6 +29,9 @@ def test_split_k_at_the_edges(ctx, oracle, wt, m, k, n):
     first, x, w = check_mat_mul(ctx, oracle, rng, m, k, n, wt)
     again = ctx.run_mat_mul(oracle.quantize_q8_0(x), w, m, k, n, wt)
     assert np.array_equal(first, again)
+    if m <= 32:  # (small matrices of so few rows take another kernel on their own)
+        with ctx.option("gemm_tile_units", 1):
+            check_mat_mul(ctx, oracle, rng, m, k, n, wt)
 
 
 @pytest.mark.parametrize("wt", [wl.GGML_TYPE_Q4_0, wl.GGML_TYPE_Q8_0])
@@ -66,6 +69,42 @@ def test_staged_tiles_of_both_sizes_give_the_same_bits(ctx, oracle):
     both = [ctx.read(h, np.uint32, m * n) for h in outs]
     assert np.array_equal(both[0], both[2]) and np.array_equal(both[1], both[3]) and both[0].any()
     for h in [ha] + ws + outs:
+        ctx.release(h)
+
+
+@pytest.mark.parametrize("wt", [wl.GGML_TYPE_Q4_0, wl.GGML_TYPE_Q8_0])
+@pytest.mark.parametrize("m", [17, 32])
+def test_members_over_weights_as_they_are_and_over_copies_equal_single_requests(ctx, oracle, m, wt):
+    # small matrices (K-sliced kernel, one to three slices) and large ones (fragments) in one message behind their quantizers,
+    # in both orders; small ones over caller-owned memory; each output byte for byte what its own message gives
+    rng = wl.rng_for(62, m + wt)
+    op = api.HTP_OPS_MAT_MUL_Q4_0_Q8_0 if wt == wl.GGML_TYPE_Q4_0 else api.HTP_OPS_MAT_MUL_Q8_0_Q8_0
+    shapes = [(300, 256), (1000, 1536), (4096, 4096), (64, 4096), (40, 2560), (33, 256)]
+    xs = {k: ctx.upload(wl.make_activations(rng, m, k)) for k in (256, 1536, 2560, 4096)}
+    acts = {k: ctx.alloc(m * (k // 32) * 34) for k in xs}
+    quantize = {k: (api.REQUEST_TYPE_OP_COMPUTE, api.op_compute_request(api.HTP_OPS_QUANTIZE_Q8_0, api.rms_norm_params(
+        (acts[k], 0), (xs[k], 0), k, m))) for k in xs}
+    ws = [ctx.upload(wl.make_weights(rng, n, k, wt)) for n, k in shapes]
+    alias = ctx.register(ctx.device_ptr(ws[1]), ctx.size(ws[1]))
+    seen = [ws[0], alias] + ws[2:]
+    results = []
+    for order in ([0, 1, 2, 3, 4, 5], [2, 0, 5, 4, 3, 1], None):
+        outs = [ctx.upload(np.zeros(m * n, np.float32)) for n, _ in shapes]
+        req = lambda j: (api.REQUEST_TYPE_OP_COMPUTE, api.op_compute_request(op, api.mat_mul_params(
+            (outs[j], 0), (acts[shapes[j][1]], 0), (seen[j], 0), m, shapes[j][1], shapes[j][0])))
+        msgs = [[quantize[k] for k in (256, 1536, 2560, 4096)] + [req(j) for j in order]] if order else \
+            [[quantize[shapes[j][1]], req(j)] for j in range(len(shapes))]
+        for msg in msgs:
+            msg = api.build_message(msg)
+            assert ctx.process_message(msg) == 0 and not any(api.message_request_states(msg)), ctx.last_error()
+        if order:
+            assert ctx.last_message_submissions() == 4 + 1
+        results.append([ctx.read(h, np.uint8, ctx.size(h)) for h in outs])
+        for h in outs:
+            ctx.release(h)
+    for a, b, c in zip(*results):
+        assert np.array_equal(a, b) and np.array_equal(a, c) and a.any()
+    for h in list(xs.values()) + list(acts.values()) + ws + [alias]:
         ctx.release(h)
 
 
