@@ -611,12 +611,25 @@ size_t act_bytes(int m, int k) {
 
 }  // namespace
 
-size_t permuted_rows_workspace_bytes(const PermutedMatMul *members, int count, int m) {
+// copies of the activations in operand order, one for the members that read the same rows
+size_t permuted_gemm_workspace_bytes(const PermutedMatMul *members, int count, int m) {
   size_t bytes = 0;
-  for (int j = 0; j < count; ++j) {  // (members that read the same rows share a copy; counted once each, which is enough)
-    bytes += act_bytes(m, members[j].k);
+  for (int j = 0; j < count; ++j) {
+    bool first = true;
+    for (int i = 0; i < j; ++i) {
+      first = first && !(members[i].act == members[j].act && members[i].k == members[j].k);
+    }
+    bytes += first ? act_bytes(m, members[j].k) : 0;
   }
   return bytes;
+}
+
+size_t permuted_rows_workspace_bytes(const PermutedMatMul *members, int count, int m) {
+  bool act_lds = true;
+  for (int j = 0; j < count; ++j) {
+    act_lds = act_lds && act_in_lds(m, members[j].k);
+  }
+  return act_lds ? 0 : permuted_gemm_workspace_bytes(members, count, m);
 }
 
 hipError_t launch_permuted_rows_group(hipStream_t stream, const PermutedMatMul *members, int count, int m, int weight_kind,
@@ -694,10 +707,6 @@ hipError_t launch_permuted_rows_group(hipStream_t stream, const PermutedMatMul *
     default:
       return launch_kind<4>(stream, args, grid, lds, act_lds, wide);
   }
-}
-
-size_t permuted_gemm_workspace_bytes(const PermutedMatMul *members, int count, int m) {
-  return permuted_rows_workspace_bytes(members, count, m);
 }
 
 hipError_t launch_permuted_gemm_group(hipStream_t stream, const PermutedMatMul *members, int count, int m, int weight_kind,

@@ -410,8 +410,10 @@ int op_mat_mul_permuted_group(htpops_context *ctx, const PermutedMatMul *members
   const size_t   out_bytes = (size_t) m * aside.n * 4, w_bytes = permuted_weight_bytes((size_t) aside.n, (size_t) aside.k, kind);
   const bool     overlaps  = count == 1 && (ranges_overlap(where, out_bytes, aside.act, (size_t) m * aside.k * 4) ||
                                         ranges_overlap(where, out_bytes, aside.weight, w_bytes));
-  if (int r = ensure_workspace(ctx, bytes + (overlaps ? out_bytes : 0))) {
-    return r;
+  if (bytes > 0 || overlaps) {  // (rows that fit LDS need none, and leave what lies there alone)
+    if (int r = ensure_workspace(ctx, bytes + (overlaps ? out_bytes : 0))) {
+      return r;
+    }
   }
   if (overlaps) {
     aside.out = reinterpret_cast<float *>(static_cast<uint8_t *>(ctx->workspace) + bytes);

@@ -63,3 +63,22 @@ def test_grouped_requests_equal_their_own_launches(ctx, kind, m):
         assert np.array_equal(a, b) and a.any()
     for h in list(acts.values()) + ws + [w_last]:
         ctx.release(h)
+
+
+def test_rows_in_lds_take_no_workspace():
+    # one row of a decode step: nothing is allocated for it, and what an earlier request left in the workspace stays
+    rng = wl.rng_for(89, 0)
+    k, n = 2048, 256
+    with api.Context(device=0) as own:
+        x, (raw, _) = own.upload(wl.make_activations(rng, 1, k)), make_weights(rng, n, k, 2)
+        w, out = own.upload(np.ascontiguousarray(raw).view(np.uint8)), own.alloc(n * 4)
+        assert own.execute(OPS[2], api.mat_mul_params((out, 0), (x, 0), (w, 0), 1, k, n)) == 0, own.last_error()
+        own.synchronize()
+        assert own.workspace_bytes() == 0
+        # 32 rows in operand order: one copy for two members that read the same rows
+        xs, outs = own.upload(wl.make_activations(rng, 32, k)), [own.alloc(32 * n * 4) for _ in range(2)]
+        msg = api.build_message([(api.REQUEST_TYPE_OP_COMPUTE, api.op_compute_request(OPS[2], api.mat_mul_params(
+            (o, 0), (xs, 0), (w, 0), 32, k, n))) for o in outs])
+        assert own.process_message(msg) == 0 and not any(api.message_request_states(msg)), own.last_error()
+        assert own.workspace_bytes() == 1 << 20  # (128 KiB, rounded up)
+        assert np.array_equal(own.read(outs[0], np.uint8, 32 * n * 4), own.read(outs[1], np.uint8, 32 * n * 4))
