@@ -145,7 +145,8 @@ struct PermutedMatMul {
 // out fp32 [m][n] = fp16(act fp16 x W fp16), the weights read as they lie, nothing converted or kept: up to kPermutedGroupMax
 // matmuls of one row count and weight kind in one launch (plus one that puts the distinct activations into operand order
 // where they do not fit LDS). The caller guarantees that no member reads what one of them writes. A member's result does not
-// depend on the others. The first for up to kPermutedRowsMax rows, the second for more; `workspace`: theirs.
+// depend on the others. The first for up to kPermutedRowsMax rows, the second for more
+// (hipErrorNotSupported: a K beyond 2 GiB of weights per 32 columns); `workspace`: theirs.
 constexpr int kPermutedRowsMax = 32;
 size_t     permuted_rows_workspace_bytes(const PermutedMatMul *members, int count, int m);
 hipError_t launch_permuted_rows_group(hipStream_t stream, const PermutedMatMul *members, int count, int m, int weight_kind,

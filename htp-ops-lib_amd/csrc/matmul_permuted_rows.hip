@@ -193,7 +193,7 @@ __global__ __launch_bounds__(kRowsThreads) void permuted_rows_kernel(const RowsA
     const int kt = min(wave + step * kRowsWaves, k_tiles - 1);  // (branch-free: steps past the end repeat the last tile)
 #pragma unroll
     for (int c = 0; c < NT; ++c) {
-      load_step(raw[d][c], w[c] + (uint32_t) kt * (uint32_t) RawStep<KIND>::kTileBytes, g, i);
+      load_step(raw[d][c], w[c] + (size_t) kt * RawStep<KIND>::kTileBytes, g, i);
     }
     if constexpr (!ACT_LDS) {
 #pragma unroll
@@ -337,8 +337,8 @@ __global__ __launch_bounds__(256) void permuted_rows_act_kernel(const RowsActArg
     ++idx;
   }
   const int k = args.k[idx], k_tiles = k / 32;
-  const int t = ((int) blockIdx.x - args.first[idx]) * 256 + (int) threadIdx.x;
-  const int lane = t & 63, f = t >> 6, step = f % k_tiles, tile = f / k_tiles;
+  const unsigned t = (blockIdx.x - (unsigned) args.first[idx]) * 256u + threadIdx.x, f = t >> 6;  // (a grid is less than 2^32 threads)
+  const int lane = t & 63, step = (int) (f % (unsigned) k_tiles), tile = (int) (f / (unsigned) k_tiles);
   if (tile >= args.tiles) {
     return;
   }
@@ -715,9 +715,13 @@ hipError_t launch_permuted_gemm_group(hipStream_t stream, const PermutedMatMul *
     return hipErrorInvalidValue;
   }
   int order[kPermutedGroupMax];
+  const size_t tile_bytes = weight_kind == 1 ? 2048 : weight_kind == 3 ? 4 * 272 : 4 * 144;
   for (int j = 0; j < count; ++j) {
     if (members[j].k % 32 != 0 || members[j].n % 32 != 0 || members[j].k <= 0 || members[j].n <= 0) {
       return hipErrorInvalidValue;
+    }
+    if ((size_t) (members[j].k / 32) * tile_bytes > 0x7fffffffu) {
+      return hipErrorNotSupported;  // (the kernel's offsets within a column group are 32 bits)
     }
     order[j] = j;
   }

@@ -5,6 +5,8 @@
 // range checks the reference lacks, then its kernels are enqueued on the context's stream.
 #include "context.h"
 
+#include <algorithm>
+
 namespace htpops {
 namespace host {
 
@@ -419,8 +421,19 @@ int op_mat_mul_permuted_group(htpops_context *ctx, const PermutedMatMul *members
     aside.out = reinterpret_cast<float *>(static_cast<uint8_t *>(ctx->workspace) + bytes);
     members   = &aside;
   }
-  HTPOPS_HIP(ctx, few ? launch_permuted_rows_group(ctx->stream, members, count, m, kind, ctx->workspace) :
-                        launch_permuted_gemm_group(ctx->stream, members, count, m, kind, ctx->workspace));
+  hipError_t e = few ? hipErrorNotSupported : launch_permuted_gemm_group(ctx->stream, members, count, m, kind, ctx->workspace);
+  if (e == hipErrorNotSupported) {
+    e = hipSuccess;
+    for (int m0 = 0; m0 < m && e == hipSuccess; m0 += kPermutedRowsMax) {  // (once, but for a K that the other cannot address)
+      PermutedMatMul part[kPermutedGroupMax];
+      for (int i = 0; i < count; ++i) {
+        part[i] = members[i];
+        part[i].out += (size_t) m0 * part[i].n, part[i].act += (size_t) m0 * part[i].k;
+      }
+      e = launch_permuted_rows_group(ctx->stream, part, count, std::min(m - m0, kPermutedRowsMax), kind, ctx->workspace);
+    }
+  }
+  HTPOPS_HIP(ctx, e);
   if (overlaps) {
     HTPOPS_HIP(ctx, launch_copy_results(ctx->stream, where, aside.out, out_bytes));
   }

@@ -82,3 +82,27 @@ def test_rows_in_lds_take_no_workspace():
         assert own.process_message(msg) == 0 and not any(api.message_request_states(msg)), own.last_error()
         assert own.workspace_bytes() == 1 << 20  # (128 KiB, rounded up)
         assert np.array_equal(own.read(outs[0], np.uint8, 32 * n * 4), own.read(outs[1], np.uint8, 32 * n * 4))
+
+
+@pytest.mark.parametrize("m,k", [(1, (1 << 26) + 64), (33, (1 << 25) + 32)])
+def test_more_than_four_and_two_gib_of_weights_in_one_column_group(m, k):
+    # 32 columns of fp16 tiles: offsets that 32 and 31 bits do not hold. All zeros but for one weight here and there.
+    zeros = np.zeros(1 << 28, np.uint8)
+    with api.Context(device=0) as own:
+        def cleared(nbytes):
+            h = own.alloc(nbytes)
+            for at in range(0, nbytes, zeros.size):
+                own.write(h, zeros[:min(zeros.size, nbytes - at)], at)
+            return h
+        print("permuted matmul over %.1f GiB of weights" % (k * 64 / 2**30), flush=True)
+        act, weight, out = cleared(m * k * 4), cleared(k * 64), own.alloc(m * 32 * 4)
+        want = np.zeros((m, 32), np.float32)
+        places = [(0, 3), (k // 2 + 1, 5), (k - 1, 31), (k - 33, 0)]
+        for i, (kk, col) in enumerate(places):
+            own.write(weight, np.float16([1.5 + i]), (kk // 32 * 1024 + (kk % 32 & ~1) * 32 + col * 2 + (kk & 1)) * 2)
+            for row in {0, m - 1}:
+                own.write(act, np.float32([2.0 + row]), (row * k + kk) * 4)
+                want[row, col] = (1.5 + i) * (2.0 + row)
+        assert own.execute(OPS[1], api.mat_mul_params((out, 0), (act, 0), (weight, 0), m, k, 32)) == 0, own.last_error()
+        own.synchronize()
+        assert np.array_equal(own.read(out, np.float32, m * 32).reshape(m, 32), want)
