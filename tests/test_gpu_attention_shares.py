@@ -199,3 +199,25 @@ def test_an_infinite_value_gives_an_infinity_in_its_column_alone(ctx, qo, kv, d)
     got = ctx.run_flash_attn(q.astype(np.float32), k, v, None, 2, 1, d)
     assert np.isposinf(got[:, :, 5]).all() and np.isneginf(got[:, :, d - 1]).all()
     assert np.isfinite(np.delete(got, (5, d - 1), axis=2)).all()
+
+
+@pytest.mark.parametrize("qo,kv,nh,nkv,d", [(5, 1029, 12, 2, 128), (40, 640, 4, 4, 64), (70, 900, 2, 2, 112), (1, 500, 2, 1, 96)])
+@pytest.mark.parametrize("low", [-np.inf, -65504.0, -16.0])
+def test_masks_that_select_keys_over_hidden_and_untouched_blocks(ctx, oracle, qo, kv, nh, nkv, d, low):
+    # attn_mask_threshold: keys are kept where the mask exceeds -16, whatever its value. Whole blocks of zeros (and of -0.0), of
+    # biases that must not be added, and of values that hide (the type's lowest, -inf, and -16 itself).
+    rng = wl.rng_for(70, qo + kv + d)
+    q, k, v = wl.make_attention_inputs(rng, qo, kv, nh, nkv, d)
+    mask = np.full((qo, (kv + 63) // 64 * 64), low, np.float16)
+    mask[:, :128] = 0.0
+    mask[:, 64:70] = -0.0
+    mask[:, 128:192] = 5.0
+    mask[:, 256:330] = np.where(rng.random((qo, 74)) < 0.5, low, -15.9)
+    keep = np.where(mask > -16, np.float16(0), np.float16(-np.inf))
+    print("threshold mask", qo, kv, nh, nkv, d, low, flush=True)
+    with ctx.option("attn_mask_threshold", 1):
+        got = ctx.run_flash_attn(q, k, v, mask, nh, nkv, d)
+        same = ctx.run_flash_attn(q, k, v, keep, nh, nkv, d)
+    want = oracle.flash_attn(q, k, v, keep, nh, nkv, d, False)
+    assert np.array_equal(got.view(np.uint16), same.view(np.uint16))
+    assert np.abs(got.astype(np.float32) - want.astype(np.float32)).max() <= ATOL
