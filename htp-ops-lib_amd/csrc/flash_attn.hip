@@ -16,17 +16,17 @@
 //    the score registers straight into the MFMA B operand. Scores are accumulated on top of minus the running
 //    maximum, so most blocks need no rescaling. Under `causal`, KV blocks above the diagonal are skipped and the
 //    longest query blocks start first. Timing-only builds on the 256-CU device (2048 x 2048 causal, 32 / 8 heads of
-//    128: 59 us) put the kernel without any matrix instruction and without the exponentials at 39 us, without the DMA
-//    at 51 us: every wave reads the whole K and V tile out of LDS for its 32 queries (1 KiB per matrix instruction:
-//    LDS bandwidth would be exhausted at the matrix cores' full rate), and that traffic, not the arithmetic, sets the
-//    pace.
+//    128, ten calls behind idle: 59 us; 48 to 50 us sustained) put the kernel without any matrix instruction and without the
+//    exponentials at 39 us, without the DMA at 51 us. The matrix instructions alone take 16 us, the LDS reads (every wave reads
+//    the whole K and V tile for its 32 queries, 1 KiB per matrix instruction) about 14: the bound is that scores, softmax and
+//    P V of a block follow each other.
 //  * decode (qo_len == 1, head_dim 64 or 128): bandwidth bound. The KV range is split across workgroups (n_kv_heads
 //    alone would leave the GPU idle); both products run on the matrix cores with the heads of the GQA group as one
 //    operand, and a second tiny kernel merges the per-split (max, sum, O) partials in one trip to memory.
 //  * head dims that are other multiples of 16 up to 256 (the reference's flash_attn_sp_hdim.c domain): the prefill kernel
-//    with rows padded to a multiple of 32, for one query row too (its keys split over workgroups, like every grid that
-//    would leave CUs idle); the probabilities as fp16 pairs. 500 causal rows by mask, 16 / 4 heads of 96: 364 us in the
-//    plain kernel, 18.8 us here.
+//    with rows padded to a multiple of 32, for one query row too (keys split over workgroups as in every grid that
+//    would leave CUs idle, where it pays: see prefill_plan); the probabilities as fp16 pairs. 500 causal rows by mask, 16 / 4 heads of 96: 364 us in the
+//    plain kernel, 18.7 us here.
 //  * any other even head_dim up to 256: a plain kernel without MFMA.
 #include "device_utils.h"
 #include "kernels.h"
@@ -1369,8 +1369,8 @@ hipError_t launch_prefill(hipStream_t stream, void *o, const void *q, const void
   const dim3     grid(plan.x, plan.q_blocks, alone ? 1 : splits);
   // Two key groups per workgroup when the grid leaves CUs without a second workgroup, or (causal) when the workgroups
   // all fit at once and their uneven lengths would leave the long ones running alone. Measured on the 256-CU device,
-  // 32 query / 8 KV heads of 128: 2048 x 2048 causal 59 us against 65 us, 1024 x 1024 without `causal` 30 against
-  // 33 us; but 2048 x 2048 without `causal` 101 against 92 us. (A split grid never has more workgroups than CUs.)
+  // 32 query / 8 KV heads of 128, ten calls behind idle: 2048 x 2048 causal 59 us against 65 us, 1024 x 1024 without `causal` 30
+  // against 33 us; but 2048 x 2048 without `causal` 101 against 92 us. (A split grid never has more workgroups than CUs.)
   const unsigned all = plan.x * plan.q_blocks * splits;
   const bool     two = kMaxGroups == 2 && (forced ? forced == 2 : (all <= kCus || (causal && all <= 2 * kCus)));
   const int      flags = (causal ? 1 : 0) | (mask_threshold ? 2 : 0);

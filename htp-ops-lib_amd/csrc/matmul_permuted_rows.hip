@@ -104,7 +104,8 @@ __device__ __forceinline__ v2h biased_to_half(uint32_t x, _Float16 bias) {
 }
 
 // IQ4_NL code book (reference: src/dsp/ops/mat_mul.c:29-32), every value + 128: the four nibbles in the low halves of
-// x's bytes -> four bytes
+// x's bytes -> four bytes. (The usual way to look 16 bytes up with byte permutes: one for either half of the book by the low three
+// bits, one that picks by the fourth.)
 __device__ __forceinline__ uint32_t iq4_nl_bytes(uint32_t x) {
   const uint32_t low3 = x & 0x07070707u;
   const uint32_t a    = __builtin_amdgcn_perm(0x766a5d4fu, 0x3f2d1801u, low3);  // values 0 .. 7

@@ -103,7 +103,7 @@ int htpops_buffer_invalidate(htpops_context *ctx, int handle);
 
 /* Makes, now, the converted copy of the weight matrix [n][k/32] (weight_type GGML_TYPE_Q4_0 or GGML_TYPE_Q8_0) at
  * `offset` of the buffer that matmuls over `m_hint` activation rows will use (none at m_hint = 1; operand-order nibbles
- * for 2..16 rows; int8 fragments from 17 rows, or FP6 tiles from 33), so that the first matmul does not pay for the conversion
+ * for 2..16 rows; int8 fragments from 17 rows, up to 32 only where k >= 4096 or n * k > 4 Mi, or FP6 tiles from 33), so that the first matmul does not pay for the conversion
  * and its hipMalloc. The reference maps weights once and treats them as immutable (src/dsp/op_executor.cc:124-130);
  * this call states the same for the buffer: it is the opt-in that puts CALLER-REGISTERED memory under the contract of
  * the context's own buffers -- converted copies of its weights are kept from now on (also those that later matmuls at
@@ -146,8 +146,8 @@ int htpops_finish_message(htpops_context *ctx, struct MessageHeader *msg);
 /* How many separately submitted units the most recent walk of a message on this context issued: compute requests that
  * were grouped count once (diagnostic; the reference runs one op per request, src/dsp/commu.c:91-100). A group is one
  * kernel launch where all its members take the same kernel (the projections of a decoder layer do); a group of
- * many-row matmuls adds one launch that converts the activations, and a few-row group whose members take different
- * kernels (by shape and weight type) issues one launch per kernel. Grouping never changes a result: a request joins a group only if it neither reads nor
+ * many-row matmuls adds one launch that converts the activations, and a group whose members take different kernels (by
+ * shape and weight type, at 17 to 32 rows also by size) issues one launch per kernel. Grouping never changes a result: a request joins a group only if it neither reads nor
  * overwrites what an earlier member writes and writes nothing an earlier member reads. */
 int htpops_last_message_submissions(htpops_context *ctx);
 
@@ -228,7 +228,7 @@ int htpops_flash_attn_ptr(htpops_context *ctx, void *o, const void *q, const voi
  * device array inside the library instead of the context's grown-on-demand workspace, and the call performs no
  * hipMalloc / hipFree of any kind. Where several workgroups share the keys of other shapes, their parts go to a block that
  * the context holds from the start (32 MiB), from both entry points; calls that are being captured into a caller's graph
- * use no memory of the context's instead (one workgroup then takes all parts in turn: the same bits, in up to twice the
+ * use no memory of the context's instead (one workgroup then takes all parts in turn: the same bits, in about twice the
  * time that not sharing would take), so such a graph may be launched on any stream, and after htpops_close.
  * Limit (decode with head_dim 64 or 128 only): n_heads * ceil(kv_len / 64) * (head_dim + 2) * 4 bytes <= 8 MiB (e.g. 32
  * heads of 128 up to kv_len 32256); larger requests, and outputs that overlap weights the context holds a converted copy
