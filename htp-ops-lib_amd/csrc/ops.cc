@@ -296,6 +296,10 @@ int run_few_rows(htpops_context *ctx, float *dst, const void *act, const void *w
   return HTPOPS_OK;
 }
 
+bool writes_weights(const void *dst, const void *weight, int m, int k, int n, int wt) {
+  return ranges_overlap(dst, (size_t) m * n * 4, weight, weight_bytes((size_t) n, (size_t) k, wt));
+}
+
 // `ws` is this matmul's share of the workspace (plan.ws_bytes, already ensured by the caller, who has noted the write to `dst`
 // before planning: it drops copies). act = nullptr (int8 fragments only): the activations lie at its start in operand order
 // already.
@@ -303,7 +307,11 @@ int run_mat_mul(htpops_context *ctx, MatMulPlan &plan, float *dst, const void *a
                 int n, int wt, uint8_t *ws) {
   if (plan.kind == kPlanFewRows) {
     ctx->act_fragments.src = nullptr;  // these kernels put something else at the start of the workspace
-    return run_few_rows(ctx, dst, act, weight, m, k, n, wt, ws);
+    const int r = run_few_rows(ctx, dst, act, weight, m, k, n, wt, ws);
+    if (writes_weights(dst, weight, m, k, n, wt)) {  // a copy made just now is of weights that are gone
+      note_device_write(ctx, dst, (size_t) m * n * 4);
+    }
+    return r;
   }
   // the converted copy of the weights, for the kernels that want one: kept with the buffer, or (weights whose copies
   // may not be kept; int8 fragments only) made in the workspace for this call
@@ -340,10 +348,6 @@ int run_mat_mul(htpops_context *ctx, MatMulPlan &plan, float *dst, const void *a
     af.src = act, af.src_bytes = q8_0_bytes((size_t) m, (size_t) k), af.m = m, af.k = k, af.kind = (int) plan.kind;
   }
   return HTPOPS_OK;
-}
-
-bool writes_weights(const void *dst, const void *weight, int m, int k, int n, int wt) {
-  return ranges_overlap(dst, (size_t) m * n * 4, weight, weight_bytes((size_t) n, (size_t) k, wt));
 }
 
 }  // namespace

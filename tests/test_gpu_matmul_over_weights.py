@@ -46,3 +46,27 @@ def test_output_over_the_weights(oracle, wt, m, k, n, fp32_rows):
         assert np.array_equal(run((ho, 0), hb)[:, :left], want[:, :left])
         ctx.write(hb, image)
         assert np.array_equal(run((ho, 0), hb), want)
+
+
+@pytest.mark.parametrize("wt", [wl.GGML_TYPE_Q4_0, wl.GGML_TYPE_Q8_0])
+@pytest.mark.parametrize("m", [8, 12])  # (over copies in two operand orders, made by the request that overwrites the weights)
+@pytest.mark.parametrize("fp32_rows", [False, True])
+def test_few_rows_over_the_weights_leave_no_copy_of_them(oracle, wt, m, fp32_rows):
+    k, n = 1024, 2048
+    rng = wl.rng_for(96, m + wt)
+    w, x = np.ascontiguousarray(wl.make_weights(rng, n, k, wt)).view(np.uint8).reshape(-1), wl.make_activations(rng, m, k)
+    x = x if fp32_rows else oracle.quantize_q8_0(x)
+    print("few rows over the weights", wt, m, fp32_rows, flush=True)
+    with api.Context(device=0) as ctx:
+        hx, hw, hb, ho = ctx.upload(x), ctx.upload(w), ctx.upload(w), ctx.alloc(m * n * 4)
+
+        def run(out, weights):
+            assert ctx.execute(OPS[wt, fp32_rows], api.mat_mul_params(out, (hx, 0), (weights, 0), m, k, n)) == 0, ctx.last_error()
+            ctx.synchronize()
+            return ctx.read(out[0], np.uint8, m * n * 4, out[1])
+
+        want = run((ho, 0), hw)
+        assert np.array_equal(run((hb, w.size // 2 // 256 * 256), hb), want)
+        # what lies there now, against the same bytes in a buffer of their own
+        other = ctx.upload(ctx.read(hb, np.uint8, w.size))
+        assert np.array_equal(run((ho, 0), hb), run((ho, 0), other))
