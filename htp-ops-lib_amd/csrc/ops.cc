@@ -163,7 +163,8 @@ int lane_order_weights(htpops_context *ctx, const void *weight, const void *act,
 }
 
 // `act_aligned`: the Q8_0 activations start on a 4-byte boundary (the re-tiling pass of the FP6 kernel reads dwords)
-// `overwrites`: the output lies over the weights, so no copy of them is used or kept (one is made in the workspace, in order)
+// `overwrites`: the output lies over the weights (or, up to 32 rows, over the rows), so no copy of them is used or kept (one is
+// made in the workspace, in order)
 MatMulPlan plan_mat_mul(htpops_context *ctx, const void *weight, bool act_aligned, int m, int k, int n, int wt, bool overwrites) {
   MatMulPlan p;
   if (m < kManyRowsMinM || k % 32 != 0) {
@@ -361,7 +362,11 @@ int op_mat_mul_q8(htpops_context *ctx, float *dst, const void *act, const void *
     return r;
   }
   note_device_write(ctx, dst, (size_t) m * n * 4);
-  MatMulPlan plan = plan_mat_mul(ctx, weight, aligned(act, 4), m, k, n, weight_type, writes_weights(dst, weight, m, k, n, weight_type));
+  // (17 to 32 rows under the output are put into operand order first, like their weights: the K-sliced kernel reads rows while
+  // other workgroups store. More rows always are.)
+  const bool overwrites = writes_weights(dst, weight, m, k, n, weight_type) ||
+                          (m < kFp6MinM && ranges_overlap(dst, (size_t) m * n * 4, act, q8_0_bytes((size_t) m, (size_t) k)));
+  MatMulPlan plan = plan_mat_mul(ctx, weight, aligned(act, 4), m, k, n, weight_type, overwrites);
   settle_copy(ctx, plan, weight, m, k, n, weight_type);
   if (int r = ensure_workspace(ctx, plan.ws_bytes, /*keep_act_fragments=*/true)) {
     return r;

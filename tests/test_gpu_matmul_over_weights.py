@@ -70,3 +70,28 @@ def test_few_rows_over_the_weights_leave_no_copy_of_them(oracle, wt, m, fp32_row
         # what lies there now, against the same bytes in a buffer of their own
         other = ctx.upload(ctx.read(hb, np.uint8, w.size))
         assert np.array_equal(run((ho, 0), hb), run((ho, 0), other))
+
+
+@pytest.mark.parametrize("wt", [wl.GGML_TYPE_Q4_0, wl.GGML_TYPE_Q8_0])
+# (17 to 32 rows of small matrices take the K-sliced kernel otherwise; more column tiles than are resident; more rows)
+@pytest.mark.parametrize("m,k,n", [(17, 64, 32 * 1600), (24, 1024, 2048), (32, 512, 700), (32, 4096, 1024), (40, 512, 700)])
+@pytest.mark.parametrize("at_end", [False, True])
+def test_output_over_the_rows(oracle, wt, m, k, n, at_end):
+    rng = wl.rng_for(97, m + k + n + wt)
+    w, q = wl.make_weights(rng, n, k, wt), np.ascontiguousarray(oracle.quantize_q8_0(wl.make_activations(rng, m, k)))
+    q, out_bytes = q.view(np.uint8).reshape(-1), m * n * 4
+    at = (q.size - 1) // 16 * 16 if at_end else 0
+    image = np.zeros(max(q.size, at + out_bytes), np.uint8)
+    image[:q.size] = q
+    print("matmul over its rows", wt, m, k, n, at_end, flush=True)
+    with api.Context(device=0) as ctx:
+        op = OPS[wt, False]
+        hx, hw, hb, ho = ctx.upload(q), ctx.upload(w), ctx.upload(image), ctx.alloc(out_bytes)
+
+        def run(out, rows):
+            assert ctx.execute(op, api.mat_mul_params(out, (rows, 0), (hw, 0), m, k, n)) == 0, ctx.last_error()
+            ctx.synchronize()
+            return ctx.read(out[0], np.float32, m * n, out[1]).reshape(m, n)
+
+        want, got = run((ho, 0), hx), run((hb, at), hb)
+        assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max() and want.any()  # (other fp32 sums of the same exact block sums)
