@@ -146,14 +146,15 @@ struct PermutedMatMul {
 // matmuls of one row count and weight kind in one launch (plus one that puts the distinct activations into operand order
 // where they do not fit LDS). The caller guarantees that no member reads what one of them writes. A member's result does not
 // depend on the others. The first for up to kPermutedRowsMax rows, the second for more
-// (hipErrorNotSupported: a K beyond 2 GiB of weights per 32 columns); `workspace`: theirs.
+// (hipErrorNotSupported: a K beyond 2 GiB of weights per 32 columns); `workspace`: theirs; `tickets`: zeroed counters, 12288
+// at most, left zeroed.
 constexpr int kPermutedRowsMax = 32;
 size_t     permuted_rows_workspace_bytes(const PermutedMatMul *members, int count, int m);
 hipError_t launch_permuted_rows_group(hipStream_t stream, const PermutedMatMul *members, int count, int m, int weight_kind,
                                       void *workspace);
 size_t     permuted_gemm_workspace_bytes(const PermutedMatMul *members, int count, int m);
 hipError_t launch_permuted_gemm_group(hipStream_t stream, const PermutedMatMul *members, int count, int m, int weight_kind,
-                                      void *workspace);
+                                      void *workspace, unsigned *tickets);
 // Results made aside to where they belong; 16-byte aligned, a multiple of 16 bytes, no overlap.
 hipError_t launch_copy_results(hipStream_t stream, float *dst, const float *src, size_t bytes);
 

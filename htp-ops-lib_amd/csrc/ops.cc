@@ -430,7 +430,7 @@ int op_mat_mul_permuted_group(htpops_context *ctx, const PermutedMatMul *members
     aside.out = reinterpret_cast<float *>(static_cast<uint8_t *>(ctx->workspace) + bytes);
     members   = &aside;
   }
-  hipError_t e = few ? hipErrorNotSupported : launch_permuted_gemm_group(ctx->stream, members, count, m, kind, ctx->workspace);
+  hipError_t e = few ? hipErrorNotSupported : launch_permuted_gemm_group(ctx->stream, members, count, m, kind, ctx->workspace, ctx->tickets);
   if (e == hipErrorNotSupported) {
     e = hipSuccess;
     for (int m0 = 0; m0 < m && e == hipSuccess; m0 += kPermutedRowsMax) {  // (once, but for a K that the other cannot address)
