@@ -16,9 +16,11 @@
 // contiguous, so a workgroup reads one stream), and their sums meet in LDS in wave order: a result does not depend on
 // the launch it is part of. Several steps of every wave are in flight before the first use.
 // Measured on MI355X, a message with the seven projections of a Llama-7B layer over Q4_0 super-blocks, one token
-// (114 MB): 28.1 us = 4.1 TB/s, against 374 us for a launch per matrix over fp16 copies in operand order (7 x 41 us on 64
-// to 172 workgroups, each behind a 5 us conversion of the row). Vector-ALU work is about 30 instructions per step and wave,
-// 10 us of it; depth 8 instead of 4 for the 4-bit formats 28.9 us, 4 or 16 waves per workgroup 30.3 and 31.0 us.
+// (114 MB): 24.0 us = 4.75 TB/s; 29.0 with all 16 bytes of a super-block's scales loaded by every lane (the path into the
+// CU then carried 24 bytes a lane and step instead of 12, and registers kept a CU to fewer waves), 374 us for a launch
+// per matrix over fp16 copies in operand order (7 x 41 us on 64 to 172 workgroups, each behind a 5 us conversion of the
+// row). Vector-ALU work is about 30 instructions per step and wave, 10 us of it; 8 steps in flight instead of 4 for the 4-bit
+// formats 24.5 us, 4 or 16 waves per workgroup (before) 30.3 and 31.0 against 28.1.
 // The activations, rounded to fp16, are read from LDS where they fit (one or a few rows: every workgroup converts them
 // for itself), else from a copy in operand order that one small launch makes.
 #include "device_utils.h"
@@ -64,7 +66,7 @@ struct RawStep<1> {
 template <>
 struct RawStep<2> {
   static constexpr int kTileBytes = 4 * 144;
-  uint4                s;  // 8 scales of super-block g
+  uint32_t             s;  // two of the 8 scales of super-block g: those of place i % 4; the quad holds all
   uint2                q;  // 8 nibbles of column 2 i, 8 of column 2 i + 1
 };
 template <>
@@ -72,7 +74,7 @@ struct RawStep<4> : RawStep<2> {};
 template <>
 struct RawStep<3> {
   static constexpr int kTileBytes = 4 * 272;
-  uint4                s;
+  uint32_t             s;
   uint32_t             q[4];  // row pair v: two bytes of column 2 i, two of column 2 i + 1
 };
 
@@ -84,19 +86,29 @@ __device__ __forceinline__ void load_step(RawStep<KIND> &r, const uint8_t *__res
       r.q[v] = *reinterpret_cast<const uint2 *>(tile + (uint32_t) (4 * g * 128 + 8 * i) + 128 * v);
     }
   } else if constexpr (KIND == 3) {
-    r.s = *reinterpret_cast<const uint4 *>(tile + (uint32_t) (g * 272));
+    r.s = *reinterpret_cast<const uint32_t *>(tile + (uint32_t) (g * 272 + 4 * (i & 3)));
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       r.q[v] = *reinterpret_cast<const uint32_t *>(tile + (uint32_t) (g * 272 + 4 * i) + 16 + 64 * v);
     }
   } else {
-    r.s = *reinterpret_cast<const uint4 *>(tile + (uint32_t) (g * 144));
+    r.s = *reinterpret_cast<const uint32_t *>(tile + (uint32_t) (g * 144 + 4 * (i & 3)));
     r.q = *reinterpret_cast<const uint2 *>(tile + (uint32_t) (g * 144 + 8 * i) + 16);
   }
 }
 
 __device__ __forceinline__ v2h as_v2h(uint32_t x) {
   return __builtin_bit_cast(v2h, x);
+}
+// The four scales of a lane's columns, each in both halves of a dword, out of the dwords that the lanes of its quad loaded (one
+// load of 16 bytes per lane would ask for the same bytes sixteen times: 16 turns of the path into the CU instead of 4)
+__device__ __forceinline__ void scales_of_quad(uint32_t own, uint32_t half_sel, v2h (&sc)[4]) {
+  // (half_sel is the same throughout a quad)
+  const int x = (int) __builtin_amdgcn_perm(own, own, half_sel);
+  sc[0] = as_v2h((uint32_t) __builtin_amdgcn_mov_dpp(x, 0x00, 0xf, 0xf, true));
+  sc[1] = as_v2h((uint32_t) __builtin_amdgcn_mov_dpp(x, 0x55, 0xf, 0xf, true));
+  sc[2] = as_v2h((uint32_t) __builtin_amdgcn_mov_dpp(x, 0xaa, 0xf, 0xf, true));
+  sc[3] = as_v2h((uint32_t) __builtin_amdgcn_mov_dpp(x, 0xff, 0xf, 0xf, true));
 }
 // (a | b) of the masks below turns bytes into fp16 numbers 1024 + byte: 0x64xx
 __device__ __forceinline__ v2h biased_to_half(uint32_t x, _Float16 bias) {
@@ -170,7 +182,9 @@ __global__ __launch_bounds__(kRowsThreads) void permuted_rows_kernel(const RowsA
   const int   lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int   g = lane >> 4, i = lane & 15;
   const int   nt0 = ((int) blockIdx.x - mb.first) * NT, n_tiles = n / 32, k_tiles = k / 32;
-  constexpr int DEPTH = (KIND == 2 || KIND == 4 || NT == 2) ? 4 : 8;  // steps of a wave in flight
+  // Steps of a wave in flight. Eight of Q8_0 cost a workgroup per CU (hidden 2048, ffn 5632: one row 13.1 against 12.0 us, 20
+  // rows 20.0 / 16.3); 16 rows in operand order, which travel with the weights, gain (IQ4_NL, 2048, 8960: 17.8 against 20.5).
+  constexpr int DEPTH = KIND == 1 || ((KIND == 2 || KIND == 4) && MT == 1 && !ACT_LDS) ? 8 : 4;
   const uint8_t *w[NT];
 #pragma unroll
   for (int c = 0; c < NT; ++c) {
@@ -262,12 +276,7 @@ __global__ __launch_bounds__(kRowsThreads) void permuted_rows_kernel(const RowsA
       for (int c = 0; c < NT; ++c) {
         v2h sc[4];
         if constexpr (KIND != 1) {
-          const uint4    s     = raw[d][c].s;
-          const uint32_t s4[4] = { s.x, s.y, s.z, s.w };
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            sc[v] = as_v2h(__builtin_amdgcn_perm(s4[v], s4[v], half_sel));
-          }
+          scales_of_quad(raw[d][c].s, half_sel, sc);
         }
         const v8h b0 = dequant<KIND, 0>(raw[d][c], sc, vc), b1 = dequant<KIND, 1>(raw[d][c], sc, vc);
 #pragma unroll
@@ -365,9 +374,9 @@ __global__ __launch_bounds__(256) void permuted_rows_act_kernel(const RowsActArg
 // slots, three steps ahead, and are read as they are used. One barrier a step; two workgroups on a CU fill each
 // other's gaps. The matmuls of a message that nothing orders share a launch, longest walk first; a long K is dealt to
 // several workgroups (gemm_parts).
-// Seven projections, 300 rows (hidden 2048, ffn 5632, IQ4_NL), weights not in a cache: 52.5 us (590 TFLOP/s), 76.2 before long
+// Seven projections, 300 rows (hidden 2048, ffn 5632, IQ4_NL), weights not in a cache: 50.8 us (605 TFLOP/s), 76.2 before long
 // K was split and row tiles were chosen by the walks, 94.7 with fp16 copies of the weights staged through LDS like the rows
-// and 264.8 with a launch per matrix over such copies. Of the 52.5, 25 are the rows' conversion, the launches and the ends
+// and 264.8 with a launch per matrix over such copies. Of it, 25 are the rows' conversion, the launches and the ends
 // of the walks, 15 the matrix instructions (timing-only builds; they add up, two waves a SIMD cover little of each
 // other). Workgroups of eight waves over twice the columns, which halve the rows' traffic: 55.2.
 struct GemmMember {
@@ -397,13 +406,13 @@ __device__ __forceinline__ void load_step_counted(RawStep<KIND> &r, __amdgpu_buf
       r.q[v] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(tiles, 4 * g * 128 + 8 * i + 128 * v, at, 0));
     }
   } else if constexpr (KIND == 3) {
-    r.s.x = __builtin_amdgcn_raw_buffer_load_b32(tiles, g * 272 + 4 * (i & 3), at, 0);
+    r.s = __builtin_amdgcn_raw_buffer_load_b32(tiles, g * 272 + 4 * (i & 3), at, 0);
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       r.q[v] = __builtin_amdgcn_raw_buffer_load_b32(tiles, g * 272 + 4 * i + 16 + 64 * v, at, 0);
     }
   } else {
-    r.s.x = __builtin_amdgcn_raw_buffer_load_b32(tiles, g * 144 + 4 * (i & 3), at, 0);
+    r.s = __builtin_amdgcn_raw_buffer_load_b32(tiles, g * 144 + 4 * (i & 3), at, 0);
     r.q = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(tiles, g * 144 + 8 * i + 16, at, 0));
   }
 }
@@ -512,13 +521,7 @@ __global__ __launch_bounds__(256, 2) void permuted_gemm_kernel(const GemmArgs ar
       for (int c = 0; c < 2; ++c) {
         v2h sc[4];
         if constexpr (KIND != 1) {
-          const int      q     = (int) raw[d][c].s.x;
-          const uint32_t q4[4] = { (uint32_t) __builtin_amdgcn_mov_dpp(q, 0x00, 0xf, 0xf, true), (uint32_t) __builtin_amdgcn_mov_dpp(q, 0x55, 0xf, 0xf, true),
-                                   (uint32_t) __builtin_amdgcn_mov_dpp(q, 0xaa, 0xf, 0xf, true), (uint32_t) __builtin_amdgcn_mov_dpp(q, 0xff, 0xf, 0xf, true) };
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            sc[v] = as_v2h(__builtin_amdgcn_perm(q4[v], q4[v], half_sel));
-          }
+          scales_of_quad(raw[d][c].s, half_sel, sc);
         }
         b[c][0] = dequant<KIND, 0>(raw[d][c], sc, vc), b[c][1] = dequant<KIND, 1>(raw[d][c], sc, vc);
       }
