@@ -1105,13 +1105,15 @@ __global__ __launch_bounds__(D *MG) void flash_attn_decode_merge_kernel(void *__
     const float m_safe = (m_new == -INFINITY) ? 0.0f : m_new;
     const float keep   = fast_exp2(m_run - m_safe);  // 0 for the first chunk
     const float f      = fast_exp2(m_s - m_safe);    // 0 in lanes without a split
-    l_run              = l_run * keep + wave_sum(l_s * f);
+    float       lf     = l_s * f;
+    asm("" : "+v"(lf));  // (a product of its own: not fused into the sum's first addition)
+    l_run              = __builtin_fmaf(l_run, keep, wave_sum(lf));
     float v            = 0.0f;
 #pragma unroll
     for (int u = 0; u < kMergeChunk; ++u) {
-      v += x[u] * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), u));
+      v = __builtin_fmaf(x[u], __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), u)), v);
     }
-    v_run = v_run * keep + v;
+    v_run = __builtin_fmaf(v_run, keep, v);
     m_run = m_new;
   }
   if (MG > 1) {
@@ -1138,7 +1140,8 @@ __global__ __launch_bounds__(D *MG) void flash_attn_decode_merge_kernel(void *__
       v_run += grp_v[j * D + d] * f;
     }
   }
-  const float out = v_run * (1.0f / l_run);
+  float out = v_run * (1.0f / l_run);
+  asm("" : "+v"(out));  // (rounded here, not fused into the conversion)
   if (QO_F32) {
     reinterpret_cast<float *>(o_ptr)[(size_t) head * D + d] = out;
     if (q8_out != nullptr) {
@@ -1162,6 +1165,284 @@ __global__ __launch_bounds__(D *MG) void flash_attn_decode_merge_kernel(void *__
     }
   } else {
     reinterpret_cast<_Float16 *>(o_ptr)[(size_t) head * D + d] = (_Float16) out;
+  }
+}
+
+// ------------------------------------------------------------------------------------------------ a few rows
+
+// The same for a few query rows (several sequences' tokens, drafted tokens that are verified): the rows of a score tile are
+// the (query, head) pairs of a GQA group, query by query, 16 to a workgroup (blockIdx.z). Bound by latency: two short launches,
+// a wave has 32 keys and one trip to memory. The prefill kernel gives every head a tile of 32 queries of its own and walks
+// 64 keys at a time, a microsecond a turn: 5 rows over 1029 keys, 12 / 2 heads of 128, fp32 with a mask 12.5 us there, 8.5 here;
+// 4 rows over 3000, 32 / 8 heads 17.8 and 10.0 (see few_plan).
+// Keys that a row may not see score -inf whatever K holds, and a wave none of whose keys is seen by any row leaves its V alone,
+// as the prefill kernel passes over such blocks. fp32 queries count with 22 bits here, with 11 there.
+// ALL: one workgroup walks all splits of its rows, once for the maxima and sums and once more for O, with the arithmetic of
+// this kernel and of flash_attn_decode_merge_kernel (at most kMergeChunk splits): the same bits without memory between
+// workgroups, for launches that must not hold an address of the context's.
+constexpr int kFewRows = 16;
+
+template <int D, bool QO_F32, int SPLIT, bool ALL>
+__global__ __launch_bounds__(SPLIT / kDecWaveKeys * kWave) void flash_attn_few_rows_kernel(
+  void *__restrict__ out, const void *__restrict__ q_ptr, const _Float16 *__restrict__ k_ptr, const _Float16 *__restrict__ v_ptr,
+  const _Float16 *__restrict__ mask, int qo_len, int kv_len, int n_heads, int n_kv_heads, int n_splits, int flags) {
+  constexpr int WAVES   = SPLIT / kDecWaveKeys;
+  constexpr int THREADS = WAVES * kWave;
+  constexpr int KSTEPS  = D / 32;  // k steps of a score tile
+  constexpr int CT      = D / 16;  // 16-column tiles of O
+  constexpr int ROWB    = D * 2;   // bytes of a K or V row
+  constexpr int CHUNKS  = ROWB / 16;
+  constexpr int DMA_ROWS = 1024 / ROWB;
+  constexpr int DMAS    = kDecWaveKeys / DMA_ROWS;
+  constexpr int PAIRS   = kFewRows * D / 2 / THREADS;  // pairs of neighbouring columns that a thread puts together
+  typedef float v4f __attribute__((ext_vector_type(4)));
+  typedef short v4s __attribute__((ext_vector_type(4)));
+  // a wave's V rows and, when it is done with them, its O [16][D]: the same bytes
+  static_assert(kDecWaveKeys * ROWB == kFewRows * D * (int) sizeof(float), "O takes the place of V");
+  __shared__ __align__(1024) uint8_t v_sh[SPLIT * ROWB];
+  __shared__ float red_m[WAVES][kFewRows], red_l[WAVES][kFewRows];
+  __shared__ float tab_m[ALL ? kFewRows : 1][kMergeChunk], tab_l[ALL ? kFewRows : 1][kMergeChunk];
+
+  const bool causal = (flags & 1) != 0, mask_threshold = (flags & 2) != 0;
+  const int  group = n_heads / n_kv_heads, rows = qo_len * group;
+  const int  h_kv  = blockIdx.y, row0 = (int) blockIdx.z * kFewRows;
+  const int  lane  = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int  col   = lane & 15, kg = lane >> 4;
+  const float  scale     = (1.0f / sqrtf((float) D)) * kLog2e;
+  const size_t kv_stride = (size_t) n_kv_heads * D;
+  const size_t mask_ld   = ((size_t) kv_len + 63) / 64 * 64;
+  // this lane's row of the score tile (rows past the last one repeat it with queries of zero; nobody reads their results)
+  const int row = min(row0 + col, rows - 1), q_row = row / group, head = h_kv * group + row % group;
+  const int vis_last = causal ? q_row + kv_len - qo_len : kv_len - 1;
+
+  v8h qf[KSTEPS], qf_lo[KSTEPS];
+  {
+    const size_t base = ((size_t) q_row * n_heads + head) * D + 8 * kg;
+    const bool   q_on = row0 + col < rows;
+#pragma unroll
+    for (int s = 0; s < KSTEPS; ++s) {
+      if (QO_F32) {
+        const float4 *qp = reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(q_ptr) + base + 32 * s);
+        const float4  q0 = qp[0], q1 = qp[1];
+        const float   x[8] = { q0.x * scale, q0.y * scale, q0.z * scale, q0.w * scale, q1.x * scale, q1.y * scale, q1.z * scale, q1.w * scale };
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          qf[s][e]    = q_on ? (_Float16) x[e] : (_Float16) 0.0f;
+          qf_lo[s][e] = q_on ? (_Float16) (x[e] - (float) qf[s][e]) : (_Float16) 0.0f;
+        }
+      } else {
+        const v8h qv = *reinterpret_cast<const v8h *>(reinterpret_cast<const _Float16 *>(q_ptr) + base + 32 * s);
+        qf[s]        = q_on ? qv : (v8h){ 0, 0, 0, 0, 0, 0, 0, 0 };
+        qf_lo[s]     = (v8h){ 0, 0, 0, 0, 0, 0, 0, 0 };  // (not used)
+      }
+    }
+  }
+
+  uint8_t *v_wave = v_sh + wave * kDecWaveKeys * ROWB;
+  float   *o_wave = reinterpret_cast<float *>(v_wave);
+  // one split: maxima and sums, and O (`with_o`), of every wave in LDS, behind a barrier
+  auto walk = [&](int split, bool with_o) __attribute__((always_inline)) {
+    const int k_end  = min(kv_len, (split + 1) * SPLIT);
+    const int k_wave = split * SPLIT + wave * kDecWaveKeys;  // (keys from k_end on are read as key k_end - 1 and score -inf)
+    if (with_o) {
+      const uint32_t to = (uint32_t) (uintptr_t) v_wave;
+#pragma unroll
+      for (int i = 0; i < DMAS; ++i) {
+        const int r     = i * DMA_ROWS + lane / CHUNKS;
+        const int piece = (lane % CHUNKS) ^ (2 * (r & 3));
+        const int key   = min(k_wave + r, k_end - 1);
+        const _Float16 *src = v_ptr + (size_t) key * kv_stride + (size_t) h_kv * D + 8 * piece;
+        asm volatile("s_mov_b32 m0, %1\n s_nop 0\n global_load_lds_dwordx4 %0, off" ::"v"(src), "s"(to + (uint32_t) (i * 1024)) : "memory");
+      }
+    }
+    v8h kf[2][KSTEPS];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int    key = min(k_wave + 16 * t + col, k_end - 1);
+      const size_t off = (size_t) key * kv_stride + (size_t) h_kv * D + 8 * kg;
+#pragma unroll
+      for (int s = 0; s < KSTEPS; ++s) {
+        kf[t][s] = *reinterpret_cast<const v8h *>(k_ptr + off + 32 * s);
+      }
+    }
+    // this row's mask for keys 16 t + 4 kg .. + 3 (a wave behind the last key reads the last one's: a mask row is whole
+    // groups of 64)
+    v4h mv[2];
+    if (mask) {
+      const _Float16 *at = mask + (size_t) q_row * mask_ld + min(k_wave, (kv_len - 1) / kDecWaveKeys * kDecWaveKeys) + 4 * kg;
+      mv[0] = *reinterpret_cast<const v4h *>(at), mv[1] = *reinterpret_cast<const v4h *>(at + 16);
+    }
+    float sc[2][4], m_w = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      v4f acc = { 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+      for (int s = 0; s < KSTEPS; ++s) {
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[t][s], qf[s], acc, 0, 0, 0);
+        if (QO_F32) {
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[t][s], qf_lo[s], acc, 0, 0, 0);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int   key = k_wave + 16 * t + 4 * kg + i;
+        const float mk  = mask ? mask_term(mv[t][i], mask_threshold) : 0.0f;
+        const bool  see = key < k_end && key <= vis_last && mk != -INFINITY;
+        sc[t][i]        = see ? (QO_F32 ? acc[i] + mk : __builtin_fmaf(acc[i], scale, mk)) : -INFINITY;
+        m_w             = fmaxf(m_w, sc[t][i]);
+      }
+    }
+    m_w = fmaxf(m_w, __shfl_xor(m_w, 16, kWave));
+    m_w = fmaxf(m_w, __shfl_xor(m_w, 32, kWave));
+    const float m_safe = (m_w == -INFINITY) ? 0.0f : m_w;
+    float       l_w    = 0.0f;
+    v8h         pf;  // A operand of P V: k slot 8 kg + 4 t + i
+    bool        seen = false;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        seen          = seen || sc[t][i] != -INFINITY;
+        pf[4 * t + i] = (_Float16) fast_exp2(sc[t][i] - m_safe);
+        l_w += (float) pf[4 * t + i];  // (as the prefill kernel: O and l see the same numbers)
+      }
+    }
+    l_w += __shfl_xor(l_w, 16, kWave);
+    l_w += __shfl_xor(l_w, 32, kWave);
+    if (kg == 0) {
+      red_m[wave][col] = m_w, red_l[wave][col] = l_w;
+    }
+    if (with_o) {
+      const bool any = __builtin_amdgcn_ballot_w64(seen) != 0;
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      v4f       oacc[CT];
+      const int j = col >> 2, q = col & 3;
+#pragma unroll
+      for (int c = 0; c < CT; ++c) {
+        oacc[c] = (v4f){ 0.0f, 0.0f, 0.0f, 0.0f };
+        if (any) {
+          v4s b[2];
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const int r     = 16 * h + 4 * kg + j;
+            const int piece = (2 * c + (q >> 1)) ^ (2 * (r & 3));
+            const uint8_t *at = v_wave + r * ROWB + piece * 16 + 8 * (q & 1);
+            b[h] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((v4s __attribute__((address_space(3))) *) at);
+          }
+          const v8h bf = __builtin_bit_cast(v8h, (short __attribute__((ext_vector_type(8)))){ b[0][0], b[0][1], b[0][2], b[0][3],
+                                                                                               b[1][0], b[1][1], b[1][2], b[1][3] });
+          oacc[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pf, bf, oacc[c], 0, 0, 0);
+        }
+      }
+      // (every read of the wave's V rows has returned before the first of these stores)
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+          o_wave[(4 * kg + i) * D + 16 * c + col] = oacc[c][i];
+        }
+      }
+    }
+    __syncthreads();
+  };
+  // the waves of a split put together: row g, columns d and d + 1
+  auto together = [&](int g, int d, float &m_all, float &l, float &v0, float &v1) {
+    m_all = red_m[0][g];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) {
+      m_all = fmaxf(m_all, red_m[w][g]);
+    }
+    const float m_ref = (m_all == -INFINITY) ? 0.0f : m_all;
+    v0 = 0.0f, v1 = 0.0f, l = 0.0f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      const float  f = fast_exp2(red_m[w][g] - m_ref);
+      const float2 x = *reinterpret_cast<const float2 *>(v_sh + w * kDecWaveKeys * ROWB + (g * D + d) * 4);
+      l  = __builtin_fmaf(red_l[w][g], f, l);
+      v0 = __builtin_fmaf(x.x, f, v0), v1 = __builtin_fmaf(x.y, f, v1);
+    }
+  };
+  if constexpr (!ALL) {
+    const int split = blockIdx.x;
+    walk(split, true);
+#pragma unroll
+    for (int p = 0; p < PAIRS; ++p) {
+      const int i = 2 * ((int) threadIdx.x + p * THREADS), g = i / D, d = i % D, r = row0 + g;
+      if (r >= rows) {
+        continue;
+      }
+      float m_all, l, v0, v1;
+      together(g, d, m_all, l, v0, v1);
+      float *rec = static_cast<float *>(out) + (((size_t) (r / group) * n_heads + h_kv * group + r % group) * n_splits + split) * (D + 2);
+      *reinterpret_cast<float2 *>(rec + 2 + d) = make_float2(v0, v1);
+      if (d == 0) {
+        *reinterpret_cast<float2 *>(rec) = make_float2(m_all, l);
+      }
+    }
+    return;
+  }
+  if constexpr (ALL) {
+    for (int split = 0; split < n_splits; ++split) {
+      walk(split, false);
+      if (threadIdx.x < kFewRows) {
+        const int g = threadIdx.x;
+        float     m_all = red_m[0][g], l = 0.0f;
+        for (int w = 1; w < WAVES; ++w) {
+          m_all = fmaxf(m_all, red_m[w][g]);
+        }
+        const float m_ref = (m_all == -INFINITY) ? 0.0f : m_all;
+        for (int w = 0; w < WAVES; ++w) {
+          l = __builtin_fmaf(red_l[w][g], fast_exp2(red_m[w][g] - m_ref), l);
+        }
+        tab_m[g][split] = m_all, tab_l[g][split] = l;
+      }
+      __syncthreads();
+    }
+    // every split's factor takes its maximum's place, the row's sum that of split 0
+    for (int g = wave; g < kFewRows; g += WAVES) {
+      const float m_s = lane < n_splits ? tab_m[g][lane] : -INFINITY, l_s = lane < n_splits ? tab_l[g][lane] : 0.0f;
+      const float m_new = wave_max(m_s), m_safe = (m_new == -INFINITY) ? 0.0f : m_new, f = fast_exp2(m_s - m_safe);
+      float       lf = l_s * f;
+      asm("" : "+v"(lf));
+      const float l_all = wave_sum(lf);
+      tab_m[g][lane] = f;
+      if (lane == 0) {
+        tab_l[g][0] = l_all;
+      }
+    }
+    float t0[PAIRS], t1[PAIRS];
+#pragma unroll
+    for (int p = 0; p < PAIRS; ++p) {
+      t0[p] = t1[p] = 0.0f;
+    }
+    for (int split = 0; split < n_splits; ++split) {
+      __syncthreads();  // (the factors are there; nobody reads the split before any more)
+      walk(split, true);
+#pragma unroll
+      for (int p = 0; p < PAIRS; ++p) {
+        const int i = 2 * ((int) threadIdx.x + p * THREADS), g = i / D;
+        float     m_all, l, v0, v1;
+        together(g, i % D, m_all, l, v0, v1);
+        t0[p] = __builtin_fmaf(v0, tab_m[g][split], t0[p]), t1[p] = __builtin_fmaf(v1, tab_m[g][split], t1[p]);
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < PAIRS; ++p) {
+      const int i = 2 * ((int) threadIdx.x + p * THREADS), g = i / D, d = i % D, r = row0 + g;
+      if (r >= rows) {
+        continue;
+      }
+      const size_t at  = ((size_t) (r / group) * n_heads + h_kv * group + r % group) * D + d;
+      const float  inv = 1.0f / tab_l[g][0];
+      float        y0 = t0[p] * inv, y1 = t1[p] * inv;
+      asm("" : "+v"(y0), "+v"(y1));
+      if (QO_F32) {
+        *reinterpret_cast<float2 *>(static_cast<float *>(out) + at) = make_float2(y0, y1);
+      } else {
+        *reinterpret_cast<v2h *>(static_cast<_Float16 *>(out) + at) = (v2h){ (_Float16) y0, (_Float16) y1 };
+      }
+    }
   }
 }
 
@@ -1354,6 +1635,66 @@ PrefillPlan prefill_plan(int dp, int qo_len, int kv_len, int n_heads, int n_kv_h
   return p;
 }
 
+// A few rows: (query, head) pairs of a GQA group in tiles of 16
+struct FewPlan {
+  int split = 0, n_splits = 0;  // split = 0: not this way
+};
+FewPlan few_plan(int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim, bool mask, int forced) {
+  FewPlan    p;
+  // Two short launches against the one or two of the prefill kernel, 12 / 2, 32 / 8, 28 / 4 and 8 / 8 heads of 128 and 16 / 8 of
+  // 64, prefill / here: 2 to 16 rows over 1029 keys with a mask 9.8 - 14.8 / 6.9 - 11.9 us, over 200 7.2 - 12.1 / 6.9 - 8.7; 3 rows
+  // of 32 / 8 heads over 600 keys without one 10.6 / 8.1, but over 120 6.7 / 7.9: one prefill launch of few turns. Every row
+  // tile reads the keys again, so that many of them over many keys lose: 16 rows of 32 / 8 heads over 3000 keys (768
+  // workgroups) 18.7 / 16.0, over 6000 (1504) 19.8 / 23.1; and with more rows the prefill kernel's tiles of 32 are fuller: 48 rows of
+  // 28 / 4 over 600 (420) 14.3 / 12.2, 64 of 12 / 2 over 1500 (576) 13.1 / 13.8.
+  const long rows  = (long) qo_len * (n_heads / n_kv_heads);
+  const int  least = head_dim == 64 ? (mask ? 200 : 512) : (mask ? 128 : 384);
+  if (forced || qo_len < 2 || (head_dim != 64 && head_dim != 128) || kv_len < least || rows > 512 || n_kv_heads > 65535) {
+    return p;
+  }
+  const long tiles = (rows + kFewRows - 1) / kFewRows;
+  const bool small = (long) ((kv_len + kDecSplit - 1) / kDecSplit) * n_kv_heads * tiles < 128 && (kv_len + kDecSplitShort - 1) / kDecSplitShort <= kMergeChunk;
+  const int  split = small ? kDecSplitShort : kDecSplit;
+  const int  n     = (kv_len + split - 1) / split;
+  if (n <= kMergeChunk && n * n_kv_heads * tiles <= (qo_len > 16 ? 512 : 768) &&
+      (size_t) qo_len * n_heads * n * (head_dim + 2) * sizeof(float) <= kAttnSharesBytes) {
+    p.split = split, p.n_splits = n;
+  }
+  return p;
+}
+
+template <int D, bool QO_F32>
+hipError_t launch_few_rows(hipStream_t stream, FewPlan plan, void *o, const void *q, const void *k, const void *v, const void *mask,
+                           int qo_len, int kv_len, int n_heads, int n_kv_heads, bool causal, bool mask_threshold, float *scratch,
+                           void *q8_out) {
+  const unsigned tiles = (unsigned) ((qo_len * (n_heads / n_kv_heads) + kFewRows - 1) / kFewRows);
+  const dim3     grid(scratch ? (unsigned) plan.n_splits : 1u, (unsigned) n_kv_heads, tiles);
+  const int      flags = (causal ? 1 : 0) | (mask_threshold ? 2 : 0);
+  void          *out   = scratch ? scratch : o;
+#define HTPOPS_FEW(SPLIT, ALL)                                                                                        \
+  hipLaunchKernelGGL((flash_attn_few_rows_kernel<D, QO_F32, SPLIT, ALL>), grid, dim3(SPLIT / kDecWaveKeys * kWave), 0, stream, out, q, \
+                     (const _Float16 *) k, (const _Float16 *) v, (const _Float16 *) mask, qo_len, kv_len, n_heads, n_kv_heads,     \
+                     plan.n_splits, flags)
+  if (plan.split == kDecSplit) {
+    if (scratch) {
+      HTPOPS_FEW(kDecSplit, false);
+    } else {
+      HTPOPS_FEW(kDecSplit, true);
+    }
+  } else if (scratch) {
+    HTPOPS_FEW(kDecSplitShort, false);
+  } else {
+    HTPOPS_FEW(kDecSplitShort, true);
+  }
+#undef HTPOPS_FEW
+  if (hipError_t e = hipGetLastError(); e != hipSuccess || !scratch) {
+    return e;
+  }
+  hipLaunchKernelGGL((flash_attn_decode_merge_kernel<D, QO_F32, 1>), dim3((unsigned) (qo_len * n_heads)), dim3(D), 0, stream, o, scratch,
+                     plan.n_splits, QO_F32 ? static_cast<uint8_t *>(q8_out) : nullptr);
+  return hipGetLastError();
+}
+
 template <int DP, bool FULL, bool QO_F32>
 hipError_t launch_prefill(hipStream_t stream, void *o, const void *q, const void *k, const void *v, const void *mask,
                           int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim, bool causal, int forced,
@@ -1468,8 +1809,12 @@ hipError_t launch_decode(hipStream_t stream, void *o, const void *q, const void 
 
 }  // namespace
 
-bool flash_attn_writes_q8_0(int qo_len, int head_dim, bool qo_is_f32) {
-  return qo_len == 1 && qo_is_f32 && (head_dim == 64 || head_dim == 128);
+// (more rows than a few meet a matmul that wants them in operand order, which the quantizer leaves as well)
+constexpr int kFewQ8Rows = 16;
+bool flash_attn_writes_q8_0(int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim, bool qo_is_f32, bool mask,
+                            int forced_key_groups) {
+  return qo_is_f32 && ((qo_len == 1 && (head_dim == 64 || head_dim == 128)) ||
+                       (qo_len <= kFewQ8Rows && few_plan(qo_len, kv_len, n_heads, n_kv_heads, head_dim, mask, forced_key_groups).split != 0));
 }
 
 size_t flash_attn_workspace_bytes(int qo_len, int kv_len, int n_heads, int head_dim) {
@@ -1493,8 +1838,9 @@ bool takes_prefill(int qo_len, int head_dim) {
 
 bool flash_attn_splits_keys(int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim, bool mask,
                             int forced_key_groups) {
-  return takes_prefill(qo_len, head_dim) &&
-         prefill_plan((head_dim + 31) / 32 * 32, qo_len, kv_len, n_heads, n_kv_heads, mask, forced_key_groups).splits > 1;
+  return few_plan(qo_len, kv_len, n_heads, n_kv_heads, head_dim, mask, forced_key_groups).split != 0 ||
+         (takes_prefill(qo_len, head_dim) &&
+          prefill_plan((head_dim + 31) / 32 * 32, qo_len, kv_len, n_heads, n_kv_heads, mask, forced_key_groups).splits > 1);
 }
 
 hipError_t launch_flash_attn_decode_part(hipStream_t stream, int part, void *o, const void *q, const void *k,
@@ -1525,6 +1871,15 @@ hipError_t launch_flash_attn(hipStream_t stream, void *o, const void *q, const v
     }
     return qo_is_f32 ? launch_decode<64, true>(stream, o, q, k, v, mask, kv_len, n_heads, n_kv_heads, ws, q8_out, mask_threshold) :
                        launch_decode<64, false>(stream, o, q, k, v, mask, kv_len, n_heads, n_kv_heads, ws, q8_out, mask_threshold);
+  }
+  const FewPlan few = few_plan(qo_len, kv_len, n_heads, n_kv_heads, head_dim, mask != nullptr, forced_key_groups);
+  if (few.split != 0) {
+    float *sh = static_cast<float *>(shares);
+#define HTPOPS_FEW_ROWS(D, F32) \
+  launch_few_rows<D, F32>(stream, few, o, q, k, v, mask, qo_len, kv_len, n_heads, n_kv_heads, causal, mask_threshold, sh, q8_out)
+    return head_dim == 128 ? (qo_is_f32 ? HTPOPS_FEW_ROWS(128, true) : HTPOPS_FEW_ROWS(128, false)) :
+                             (qo_is_f32 ? HTPOPS_FEW_ROWS(64, true) : HTPOPS_FEW_ROWS(64, false));
+#undef HTPOPS_FEW_ROWS
   }
 #define HTPOPS_PREFILL(DP, FULL)                                                                                     \
   qo_is_f32 ? launch_prefill<DP, FULL, true>(stream, o, q, k, v, mask, qo_len, kv_len, n_heads, n_kv_heads, head_dim, \

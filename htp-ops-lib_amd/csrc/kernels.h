@@ -159,13 +159,13 @@ hipError_t launch_permuted_gemm_group(hipStream_t stream, const PermutedMatMul *
 hipError_t launch_copy_results(hipStream_t stream, float *dst, const float *src, size_t bytes);
 
 // attention; see htpops_flash_attn_ptr. `workspace` holds split-KV partials (decode), size from
-// flash_attn_workspace_bytes. `q8_out` (or nullptr; used only where flash_attn_writes_q8_0 says so: decode with
-// head_dim 64 / 128 and fp32 output): the output row is also written there as Q8_0 blocks, bit for bit what
-// launch_quantize_q8_0 makes of it. `forced_key_groups` 1 / 2 forces how many key groups a prefill workgroup holds
+// flash_attn_workspace_bytes. `q8_out` (or nullptr; used only where flash_attn_writes_q8_0 says so, one row or a few of head
+// dim 64 / 128 and fp32 output, the few only with `shares`): the output rows are also written there as Q8_0 blocks, bit for
+// bit what launch_quantize_q8_0 makes of them. `forced_key_groups` 1 / 2 forces how many key groups a prefill workgroup holds
 // (0: by grid size). `mask_threshold`: the mask selects keys (keep iff mask > -16, reference:
 // src/dsp/ops/flash_attn.c:448-460) instead of being added to the scores (:1505-1512). `shares`: kAttnSharesBytes, where the
-// workgroups that share a query block's keys leave their parts (used where flash_attn_splits_keys says so); nullptr: one
-// workgroup walks all of them, with the same results bit for bit.
+// workgroups that share a query block's or a few rows' keys leave their parts (used where flash_attn_splits_keys says so);
+// nullptr: one workgroup walks all of them, with the same results bit for bit.
 constexpr size_t kAttnSharesBytes = (size_t) 32 << 20;  // two shares of 512 queries of 32 heads of 128 take 17 MB
 bool       flash_attn_splits_keys(int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim, bool mask,
                                   int forced_key_groups);
@@ -179,7 +179,8 @@ hipError_t launch_flash_attn(hipStream_t stream, void *o, const void *q, const v
 hipError_t launch_flash_attn_decode_part(hipStream_t stream, int part, void *o, const void *q, const void *k,
                                          const void *v, int kv_len, int n_heads, int n_kv_heads, int head_dim,
                                          bool qo_is_f32, void *workspace);
-bool       flash_attn_writes_q8_0(int qo_len, int head_dim, bool qo_is_f32);
+bool       flash_attn_writes_q8_0(int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim, bool qo_is_f32,
+                                  bool mask, int forced_key_groups);
 
 // What the calling thread's most recent launch of the one-row matmul kernel was: kernel instance and geometry. The bench
 // harness compares it with the launch its hardware-counter figures were taken from.

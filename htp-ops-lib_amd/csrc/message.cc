@@ -540,8 +540,8 @@ size_t fragments_of_next(htpops_context *ctx, const struct OpComputeRequest *req
   return plan.kind == kPlanFragments ? plan.ws_bytes : 0;
 }
 
-// `next` behind a one-token fp32 attention request `req`: if it is the Q8_0 quantization of exactly that attention's
-// output row into a buffer that overlaps none of the attention's operands, notes where it wants the row
+// `next` behind an fp32 attention request `req` of one row or a few: if it is the Q8_0 quantization of exactly that
+// attention's output rows into a buffer that overlaps none of the attention's operands, notes where it wants the rows
 // (ctx->attn_q8_out) and returns it; nullptr otherwise.
 struct RequestHeader *attention_output_quantizer(htpops_context *ctx, const struct OpComputeRequest *req,
                                                  struct RequestHeader *next, size_t next_size) {
@@ -552,12 +552,14 @@ struct RequestHeader *attention_output_quantizer(htpops_context *ctx, const stru
   }
   const auto *nreq = reinterpret_cast<const struct OpComputeRequest *>(next->data);
   const auto *pq   = reinterpret_cast<const RmsNormF32Params *>(nreq->payload);
-  if (nreq->op != HTP_OPS_QUANTIZE_Q8_0 || p->qo_len != 1 || p->kv_len <= 0 || p->n_heads <= 0 || p->n_kv_heads <= 0 ||
-      p->head_dim <= 0 || p->n_heads > (1 << 20) || p->head_dim > 256 || pq->ne1 != 1 ||
-      pq->ne0 != p->n_heads * p->head_dim || !flash_attn_writes_q8_0(1, p->head_dim, true)) {
+  if (nreq->op != HTP_OPS_QUANTIZE_Q8_0 || p->qo_len <= 0 || p->kv_len <= 0 || p->n_heads <= 0 || p->n_kv_heads <= 0 ||
+      p->head_dim <= 0 || p->n_heads > (1 << 20) || p->head_dim > 256 || p->n_heads % p->n_kv_heads != 0 || pq->ne1 != p->qo_len ||
+      pq->ne0 != p->n_heads * p->head_dim ||
+      !flash_attn_writes_q8_0(p->qo_len, p->kv_len, p->n_heads, p->n_kv_heads, p->head_dim, true,
+                              p->mask.fd >= 0 && lookup(ctx, p->mask.fd), ctx->opt.attn_key_groups)) {
     return nullptr;
   }
-  const size_t row = (size_t) pq->ne0 * 4, q_bytes = q8_0_bytes(1, (size_t) pq->ne0);
+  const size_t row = (size_t) p->qo_len * pq->ne0 * 4, q_bytes = q8_0_bytes((size_t) p->qo_len, (size_t) pq->ne0);
   const size_t kv  = (size_t) p->kv_len * p->n_kv_heads * p->head_dim * 2;
   const void  *o = resolve(ctx, p->o, row), *src = resolve(ctx, pq->src, row);
   void        *dst = resolve(ctx, pq->dst, q_bytes);
@@ -567,7 +569,7 @@ struct RequestHeader *attention_output_quantizer(htpops_context *ctx, const stru
     return nullptr;
   }
   if (p->mask.fd >= 0 && lookup(ctx, p->mask.fd)) {
-    const size_t mask_bytes = ((size_t) p->kv_len + 63) / 64 * 64 * 2;
+    const size_t mask_bytes = (size_t) p->qo_len * (((size_t) p->kv_len + 63) / 64 * 64) * 2;
     const void  *mask       = resolve(ctx, p->mask, mask_bytes);
     if (mask && ranges_overlap(dst, q_bytes, mask, mask_bytes)) {
       return nullptr;
@@ -684,8 +686,8 @@ int enqueue_message(htpops_context *ctx, struct MessageHeader *msg, size_t msg_b
               !(matmul_payload && try_batch(ctx, req, hdr, batch))) {
             flush_batch(ctx, batch);
             ++ctx->message_submissions;
-            // one-token attention whose fp32 output the NEXT request quantizes to Q8_0 (on its way to the o projection):
-            // the launch that finishes the attention writes that row too, and the next request is done with it
+            // attention of one token or a few whose fp32 output the NEXT request quantizes to Q8_0 (on its way to the o
+            // projection): the launch that finishes the attention writes those rows too, and the next request is done with it
             struct RequestHeader *next = nullptr;
             if (req->op == HTP_OPS_FLASH_ATTN_QO_F32_KV_F16 && i + 1 < n_reqs &&
                 size >= sizeof(struct RequestHeader) + sizeof(struct OpComputeRequest) + sizeof(FlashAttnParams)) {
@@ -702,7 +704,7 @@ int enqueue_message(htpops_context *ctx, struct MessageHeader *msg, size_t msg_b
             ctx->next_fragments_ws = 0;
             if (next && ctx->attn_q8_done && hdr->state == HTPOPS_OK) {
               next->state = HTPOPS_OK;
-              ++i;  // (the row is written: that request needs no launch)
+              ++i;  // (the rows are written: that request needs no launch)
             }
           }
         }

@@ -539,14 +539,16 @@ int op_flash_attn(htpops_context *ctx, void *o, const void *q, const void *k, co
     note_device_write(ctx, o, o_bytes);
     ws = ctx->workspace;
   }
-  void *q8_out = nullptr;
-  if (ctx->attn_q8_out && flash_attn_writes_q8_0(qo_len, head_dim, qo_is_f32 != 0)) {
-    q8_out = ctx->attn_q8_out;
-    note_device_write(ctx, q8_out, q8_0_bytes(1, (size_t) n_heads * head_dim));
-  }
   void *shares = nullptr;
   if (flash_attn_splits_keys(qo_len, kv_len, n_heads, n_kv_heads, head_dim, mask != nullptr, ctx->opt.attn_key_groups)) {
     shares = attention_shares(ctx);
+  }
+  void *q8_out = nullptr;
+  if (ctx->attn_q8_out && (qo_len == 1 || shares) &&
+      flash_attn_writes_q8_0(qo_len, kv_len, n_heads, n_kv_heads, head_dim, qo_is_f32 != 0, mask != nullptr,
+                             ctx->opt.attn_key_groups)) {
+    q8_out = ctx->attn_q8_out;
+    note_device_write(ctx, q8_out, q8_0_bytes((size_t) qo_len, (size_t) n_heads * head_dim));
   }
   HTPOPS_HIP(ctx, launch_flash_attn(ctx->stream, o, q, k, v, mask, qo_len, kv_len, n_heads, n_kv_heads, head_dim,
                                     qo_is_f32 != 0, causal != 0, ws, q8_out, ctx->opt.attn_key_groups,
