@@ -1,4 +1,4 @@
-// Q4_0 x Q8_0 matmul for 2..8 activation rows, two blocks per matrix instruction:
+// Q4_0 (and, from k = 4096 on, Q8_0) x Q8_0 matmul for 2..8 activation rows, two blocks per matrix instruction:
 // out[m][n] = sum over 32-wide blocks of (int dot of the block) * d_act * d_weight (reference: src/dsp/ops/mat_mul.c:572-640,
 // block formats include/dsp/quants.h:8-14, ggml block_q4_0 / block_q8_0).
 //
@@ -17,6 +17,8 @@
 // 16-byte load per quad of blocks: for a tile of 16 rows and blocks 4 q .. 4 q + 3,
 //   1024 B: lane (n, g)'s 16 bytes = nibble bytes 8 (g & 1) .. + 7 of block 4 q + (g >> 1), then of block 4 q + 2 + (g >> 1)
 //    128 B: row n's 4 fp16 scales of those blocks
+// (Q8_0: 2 x 1024 B of operand bytes, elements 8 (g & 1) .. + 7 and 16 + 8 (g & 1) .. + 7 of those blocks, one KiB for either
+// pair; no "- 8" and no table for it.)
 // A workgroup works on one tile at a time over the whole of K (its 8 waves take every eighth quad and add up through
 // LDS): nothing is exchanged between workgroups. The activation rows come as they are (block_q8_0 rows) by
 // global_load_lds DMA, one row per wave, into a row-major LDS image (row starts 16 bytes past a multiple of 128 apart:
@@ -45,13 +47,18 @@ constexpr int kBpWaves     = 8;                      // waves of a workgroup
 constexpr int kBpThreads   = kBpWaves * kWave;
 constexpr int kBpRows      = 16;                     // weight rows per tile
 constexpr int kBpActRows   = 8;                      // activation rows of the image
-constexpr int kBpQuadBytes = 64 * 16 + kBpRows * 8;  // 1152 = 16 rows x 4 blocks x 18 B
+constexpr int bp_quad_bytes(int wt) {  // 16 rows x 4 blocks x 18 B (Q4_0) or 34 B (Q8_0)
+  return 64 * (wt == kQ4_0 ? 16 : 32) + kBpRows * 8;
+}
+constexpr int kBpLongQ8    = 4096;                   // Q8_0 rows from which this kernel is used
 constexpr int kBpZeroBytes = 64;                     // the zeroed corner (a lane reads up to 28 bytes of it)
 constexpr size_t kBpLdsLimit = 160 * 1024;
 
-// ---- repack: one thread per (tile, quad, lane) writes its 16 nibble bytes; lanes 0..15 also write the scales ----
-__global__ __launch_bounds__(256) void q4_0_to_block_pairs_kernel(uint8_t *__restrict__ dst, const uint8_t *__restrict__ src,
-                                                                 int nblk, int n) {
+// ---- repack: one thread per (tile, quad, lane) writes its 16 nibble or 32 operand bytes; lanes 0..15 also write the scales ----
+template <int WT>
+__global__ __launch_bounds__(256) void weights_to_block_pairs_kernel(uint8_t *__restrict__ dst, const uint8_t *__restrict__ src,
+                                                                    int nblk, int n) {
+  constexpr int kBlock = WT == kQ4_0 ? 18 : 34, kLane = WT == kQ4_0 ? 16 : 32;
   const int    nquads = nblk / 4;
   const size_t item   = (size_t) blockIdx.x * 256 + threadIdx.x;  // (tile * nquads + quad) * 64 + lane
   const size_t total  = (size_t) (n / kBpRows) * nquads * 64;
@@ -62,26 +69,33 @@ __global__ __launch_bounds__(256) void q4_0_to_block_pairs_kernel(uint8_t *__res
   const size_t tq   = item >> 6;
   const int    quad = (int) (tq % nquads);
   const size_t tile = tq / nquads;
-  const uint8_t *row = src + ((size_t) (tile * kBpRows + nl) * nblk + 4 * (size_t) quad) * 18;
-  uint8_t       *out = dst + tq * kBpQuadBytes;
-  uint32_t       w[4];
+  const uint8_t *row = src + ((size_t) (tile * kBpRows + nl) * nblk + 4 * (size_t) quad) * kBlock;
+  uint8_t       *out = dst + tq * bp_quad_bytes(WT);
+  auto           dword = [](const uint8_t *q) {
+    return (uint32_t) q[0] | ((uint32_t) q[1] << 8) | ((uint32_t) q[2] << 16) | ((uint32_t) q[3] << 24);
+  };
+  uint32_t w[kLane / 4];
 #pragma unroll
   for (int p = 0; p < 2; ++p) {
-    const uint8_t *q = row + (2 * p + (g >> 1)) * 18 + 2 + 8 * (g & 1);
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      w[2 * p + h] = (uint32_t) q[4 * h] | ((uint32_t) q[4 * h + 1] << 8) | ((uint32_t) q[4 * h + 2] << 16) |
-                     ((uint32_t) q[4 * h + 3] << 24);
+    const uint8_t *q = row + (2 * p + (g >> 1)) * kBlock + 2 + 8 * (g & 1);
+    if constexpr (WT == kQ4_0) {
+      w[2 * p] = dword(q), w[2 * p + 1] = dword(q + 4);
+    } else {
+      w[4 * p] = dword(q), w[4 * p + 1] = dword(q + 4), w[4 * p + 2] = dword(q + 16), w[4 * p + 3] = dword(q + 20);
     }
   }
-  *reinterpret_cast<uint4 *>(out + lane * 16) = make_uint4(w[0], w[1], w[2], w[3]);
+  // (Q8_0: the lanes' pieces of the first pair of blocks, then those of the second: a load instruction reads one KiB)
+#pragma unroll
+  for (int i = 0; i < kLane / 16; ++i) {
+    *reinterpret_cast<uint4 *>(out + i * 1024 + lane * 16) = make_uint4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
+  }
   if (g == 0) {
     uint16_t s[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      s[j] = (uint16_t) (row[j * 18] | (row[j * 18 + 1] << 8));
+      s[j] = (uint16_t) (row[j * kBlock] | (row[j * kBlock + 1] << 8));
     }
-    *reinterpret_cast<uint2 *>(out + 1024 + nl * 8) =
+    *reinterpret_cast<uint2 *>(out + 64 * kLane + nl * 8) =
       make_uint2((uint32_t) s[0] | ((uint32_t) s[1] << 16), (uint32_t) s[2] | ((uint32_t) s[3] << 16));
   }
 }
@@ -103,20 +117,20 @@ struct BlockPairsGroupArgs {
 struct BpLayout {
   int row_stride, image, sums, scales, red, total;
 };
-__host__ __device__ inline BpLayout bp_layout(int nblk) {
+__host__ __device__ inline BpLayout bp_layout(int nblk, int wt) {
   BpLayout l;
   // rows 16 bytes (4 banks) past a multiple of 128 bytes apart: the 8 rows a wave reads at one offset fall into
   // different banks (a row itself is a multiple of 16 bytes long)
   l.row_stride = (nblk * 34 + 127 - 16) / 128 * 128 + 16;
   l.image      = kBpZeroBytes;
   l.sums       = l.image + kBpActRows * l.row_stride;
-  l.scales     = l.sums + nblk * kBpActRows * 4;
+  l.scales     = l.sums + (wt == kQ4_0 ? nblk * kBpActRows * 4 : 0);
   l.red        = l.scales + (nblk / 2) * kBpActRows * 4;   // the waves' sums of a tile, two buffers
   l.total      = l.red + 2 * kBpWaves * 4 * 32 * 4;
   return l;
 }
 
-template <int DEPTH>  // steps whose weights are requested ahead
+template <int DEPTH, int WT>  // DEPTH: steps whose weights are requested ahead
 __global__ __launch_bounds__(kBpThreads) void matmul_block_pairs_kernel(BlockPairsGroupArgs grp, int m) {
   extern __shared__ __align__(16) uint8_t bp_lds[];
   int member = 0;
@@ -128,7 +142,7 @@ __global__ __launch_bounds__(kBpThreads) void matmul_block_pairs_kernel(BlockPai
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, g = lane >> 4;
   const int nblk = grp.k[member] / 32, nquads = nblk / 4;
-  const BpLayout L = bp_layout(nblk);
+  const BpLayout L = bp_layout(nblk, WT);
   const uint8_t *__restrict__ act = grp.act[member];
   float *__restrict__         out = grp.out[member];
 
@@ -154,7 +168,7 @@ __global__ __launch_bounds__(kBpThreads) void matmul_block_pairs_kernel(BlockPai
   }
   // this wave's quads wave, wave + 8, ...: two at a time, the next two in flight behind them
   struct Quad {
-    uint4 q;  // this lane's nibble bytes of the quad's two block pairs
+    uint4 q[WT == kQ4_0 ? 1 : 2];  // this lane's nibble bytes of the quad's two block pairs, or operand bytes of either
     uint2 d;  // the 4 fp16 scales of this lane's weight row
   };
   // A wave's work is a sequence of steps: (tile, h) = its quads wave + 16 h and wave + 16 h + 8 of that tile, tile after
@@ -163,13 +177,16 @@ __global__ __launch_bounds__(kBpThreads) void matmul_block_pairs_kernel(BlockPai
   const int steps = (nquads + 2 * kBpWaves - 1) / (2 * kBpWaves);  // per tile
   auto fetch = [&](Quad (&r)[2], int tile, int h) {
     // (a step past the workgroup's last tile re-reads its last tile, a quad past the end of K the last quad: never used)
-    const uint8_t *tw = grp.w[member] + (size_t) min(tile, n_tiles - 1) * nquads * kBpQuadBytes;
+    const uint8_t *tw = grp.w[member] + (size_t) min(tile, n_tiles - 1) * nquads * bp_quad_bytes(WT);
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
       const int      q = min(wave + (2 * h + c) * kBpWaves, nquads - 1);
-      const uint8_t *p = tw + (size_t) q * kBpQuadBytes;
-      r[c].q = *reinterpret_cast<const uint4 *>(p + lane * 16);
-      r[c].d = *reinterpret_cast<const uint2 *>(p + 1024 + r16 * 8);
+      const uint8_t *p = tw + (size_t) q * bp_quad_bytes(WT);
+#pragma unroll
+      for (int i = 0; i < (WT == kQ4_0 ? 1 : 2); ++i) {
+        r[c].q[i] = *reinterpret_cast<const uint4 *>(p + i * 1024 + lane * 16);
+      }
+      r[c].d = *reinterpret_cast<const uint2 *>(p + (WT == kQ4_0 ? 1024 : 2048) + r16 * 8);
       // keep the loads in program order everywhere: the compiler counts the loads that may still be in flight when a
       // register is used, and takes the worst order over all paths that reach the use
       __builtin_amdgcn_sched_barrier(0);
@@ -188,16 +205,17 @@ __global__ __launch_bounds__(kBpThreads) void matmul_block_pairs_kernel(BlockPai
     fetch(sets[d], tf, hf);
     next_step(tf, hf);
   }
-  // the DMA pieces of this wave have landed once only the 4 DEPTH weight loads issued after them are outstanding
+  // the DMA pieces of this wave have landed once only the weight loads issued after them are outstanding
   // (s_waitcnt operand: vmcnt in bits 3:0 and 15:14, expcnt (7 = no wait) in 6:4, lgkmcnt in 11:8)
-  static_assert(4 * DEPTH < 64, "vmcnt is a 6-bit counter");
-  __builtin_amdgcn_s_waitcnt(0x0070 | ((4 * DEPTH) & 15) | (((4 * DEPTH) >> 4) << 14));
+  constexpr int kLoads = (WT == kQ4_0 ? 4 : 6) * DEPTH;
+  static_assert(kLoads < 64, "vmcnt is a 6-bit counter");
+  __builtin_amdgcn_s_waitcnt(0x0070 | (kLoads & 15) | ((kLoads >> 4) << 14));
   __builtin_amdgcn_s_barrier();  // (bare barriers: __syncthreads would also wait for the weight loads)
 
   // ---- tables: -8 x block sum per (block, row) and the scale operand per (pair of blocks, result row) ----
   {
     int *sums = reinterpret_cast<int *>(bp_lds + L.sums);
-    for (int i = tid; i < nblk * kBpActRows; i += kBpThreads) {
+    for (int i = tid; WT == kQ4_0 && i < nblk * kBpActRows; i += kBpThreads) {
       const int      blk = i / kBpActRows, row = i % kBpActRows;
       const int      s   = blk * 34 + 2;  // the block's 32 int8 start here: 2 bytes off a dword in even blocks
       const uint8_t *p   = bp_lds + L.image + row * L.row_stride + (s & ~3);
@@ -242,7 +260,7 @@ __global__ __launch_bounds__(kBpThreads) void matmul_block_pairs_kernel(BlockPai
 
   const uint32_t a_at0 = a_at, c_at0 = c_at, s_at0 = s_at;
   v4f acc;
-  auto pair = [&](uint32_t w0, uint32_t w1, uint32_t dw) {
+  auto pair = [&](const uint4 (&q)[WT == kQ4_0 ? 1 : 2], int second, uint32_t dw) {
     // activations: bytes [x, x + 8) and [x + 16, x + 24) of the row, x = a_at + shift
     const uint32_t *ap = reinterpret_cast<const uint32_t *>(bp_lds + a_at);
     const uint32_t  t0 = ap[0], t1 = ap[1], t2 = ap[2], t4 = ap[4], t5 = ap[5], t6 = ap[6];
@@ -251,12 +269,20 @@ __global__ __launch_bounds__(kBpThreads) void matmul_block_pairs_kernel(BlockPai
     a[1] = (int) __builtin_amdgcn_alignbyte(t2, t1, shift);
     a[2] = (int) __builtin_amdgcn_alignbyte(t5, t4, shift);
     a[3] = (int) __builtin_amdgcn_alignbyte(t6, t5, shift);
-    const v4i c = *reinterpret_cast<const v4i *>(bp_lds + c_at);
+    v4i c = { 0, 0, 0, 0 };
     const uint32_t sa = *reinterpret_cast<const uint32_t *>(bp_lds + s_at) & s_mask;
     // weights: nibbles as they are (0..15), low nibbles = elements e .. e + 7, high nibbles = elements 16 + e ..
+    // (Q8_0: the operand as it lies)
     v4i b;
-    b[0] = (int) (w0 & 0x0f0f0f0fu), b[1] = (int) (w1 & 0x0f0f0f0fu);
-    b[2] = (int) ((w0 >> 4) & 0x0f0f0f0fu), b[3] = (int) ((w1 >> 4) & 0x0f0f0f0fu);
+    if constexpr (WT == kQ4_0) {
+      c = *reinterpret_cast<const v4i *>(bp_lds + c_at);
+      const uint32_t w0 = second ? q[0].z : q[0].x, w1 = second ? q[0].w : q[0].y;
+      b[0] = (int) (w0 & 0x0f0f0f0fu), b[1] = (int) (w1 & 0x0f0f0f0fu);
+      b[2] = (int) ((w0 >> 4) & 0x0f0f0f0fu), b[3] = (int) ((w1 >> 4) & 0x0f0f0f0fu);
+    } else {
+      const uint4 o = q[WT == kQ4_0 ? 0 : second];
+      b = (v4i){ (int) o.x, (int) o.y, (int) o.z, (int) o.w };
+    }
     const v4i sums = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
     const v4f zero = { 0.0f, 0.0f, 0.0f, 0.0f };
     const v4f prod = __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(v4h, make_uint2(sa, 0u)),
@@ -310,8 +336,8 @@ __global__ __launch_bounds__(kBpThreads) void matmul_block_pairs_kernel(BlockPai
 #pragma unroll
     for (int cidx = 0; cidx < 2; ++cidx) {
       if (wave + (2 * h + cidx) * kBpWaves < nquads && tile < n_tiles) {
-        pair(r[cidx].q.x, r[cidx].q.y, r[cidx].d.x);
-        pair(r[cidx].q.z, r[cidx].q.w, r[cidx].d.y);
+        pair(r[cidx].q, 0, r[cidx].d.x);
+        pair(r[cidx].q, 1, r[cidx].d.y);
         skip_to_next_quad();
       }
     }
@@ -340,37 +366,51 @@ __global__ __launch_bounds__(kBpThreads) void matmul_block_pairs_kernel(BlockPai
 // seven matrices of a Llama-7B layer in one launch (8 rows): depth 2 28.3 us, 3 27.2 us, 5 28.1 us, 6 29.5 us; 16 waves
 // per workgroup instead of 8 (each tile split 16 ways) 28.3 us.
 constexpr int kBpDepthShared = 2, kBpDepthAlone = 3;
-bool bp_alone(int nblk) {
-  return (size_t) bp_layout(nblk).total * 2 > kBpLdsLimit;
+bool bp_alone(int nblk, int wt) {
+  return (size_t) bp_layout(nblk, wt).total * 2 > kBpLdsLimit;
 }
+
+typedef void (*BpKernel)(BlockPairsGroupArgs, int);
+const BpKernel kBpKernels[2][2] = {
+  { matmul_block_pairs_kernel<kBpDepthShared, kQ4_0>, matmul_block_pairs_kernel<kBpDepthAlone, kQ4_0> },
+  { matmul_block_pairs_kernel<kBpDepthShared, kQ8_0>, matmul_block_pairs_kernel<kBpDepthAlone, kQ8_0> } };
 
 }  // namespace
 
 bool matmul_block_pairs_fits(int n, int m, int k, WeightType wt) {
   // k % 256: activation rows (34 B per 32 elements) are whole 16-byte pieces, weight rows whole quads of blocks
-  return wt == kQ4_0 && m >= 2 && m <= kBpActRows && k > 0 && k % 256 == 0 && n > 0 && n % kBpRows == 0 &&
-         (size_t) bp_layout(k / 32).total <= kBpLdsLimit;
+  // Q8_0 from k = 4096 on: seven projections of a Llama-7B layer, 4 / 8 rows, 40.9 / 42.0 us, in four launches of the
+  // lane-order kernel 45.8 / 48.7; 8960 x 1536 10.9 and 11.1 by itself. Short rows pay the tables more often than they gain: 1536
+  // x 8960 10.8 us here and 8.9 there, 512 x 512 7.6 and 6.8 (two tiles at a time with half of the waves each: 9.8, 7.6).
+  return (wt == kQ4_0 || (wt == kQ8_0 && k >= kBpLongQ8)) && m >= 2 && m <= kBpActRows && k > 0 && k % 256 == 0 && n > 0 && n % kBpRows == 0 &&
+         (size_t) bp_layout(k / 32, wt).total <= kBpLdsLimit;
 }
 
-hipError_t launch_weights_to_block_pairs(hipStream_t stream, void *dst, const void *weight, int k, int n) {
+hipError_t launch_weights_to_block_pairs(hipStream_t stream, void *dst, const void *weight, int k, int n, WeightType wt) {
   if (k % 128 != 0 || n % kBpRows != 0) {
     return hipErrorNotSupported;
   }
   const size_t items = (size_t) (n / kBpRows) * (size_t) (k / 128) * 64;
-  hipLaunchKernelGGL(q4_0_to_block_pairs_kernel, dim3((unsigned) ((items + 255) / 256)), dim3(256), 0, stream,
-                     static_cast<uint8_t *>(dst), static_cast<const uint8_t *>(weight), k / 32, n);
+  const dim3   grid((unsigned) ((items + 255) / 256));
+  if (wt == kQ4_0) {
+    hipLaunchKernelGGL(weights_to_block_pairs_kernel<kQ4_0>, grid, dim3(256), 0, stream, static_cast<uint8_t *>(dst),
+                       static_cast<const uint8_t *>(weight), k / 32, n);
+  } else {
+    hipLaunchKernelGGL(weights_to_block_pairs_kernel<kQ8_0>, grid, dim3(256), 0, stream, static_cast<uint8_t *>(dst),
+                       static_cast<const uint8_t *>(weight), k / 32, n);
+  }
   return hipGetLastError();
 }
 
 hipError_t launch_matmul_block_pairs_group(hipStream_t stream, int count, float *const *outs, const void *const *acts,
-                                           const void *const *pair_order_weights, const int *ns, int m, const int *ks) {
+                                           const void *const *pair_order_weights, const int *ns, int m, const int *ks, WeightType wt) {
   if (count < 1 || count > kGemvGroupMax) {
     return hipErrorNotSupported;
   }
   BlockPairsGroupArgs grp = {};
   int                 k_max = 0;
   for (int i = 0; i < count; ++i) {
-    if (!matmul_block_pairs_fits(ns[i], m, ks[i], kQ4_0) || (reinterpret_cast<uintptr_t>(pair_order_weights[i]) & 15) != 0 ||
+    if (!matmul_block_pairs_fits(ns[i], m, ks[i], wt) || (reinterpret_cast<uintptr_t>(pair_order_weights[i]) & 15) != 0 ||
         (reinterpret_cast<uintptr_t>(acts[i]) & 15) != 0) {
       return hipErrorNotSupported;
     }
@@ -382,17 +422,16 @@ hipError_t launch_matmul_block_pairs_group(hipStream_t stream, int count, float 
     k_max      = std::max(k_max, ks[i]);
   }
   // (the longest rows of the launch decide its LDS size and with it how many workgroups share a compute unit)
-  const bool   alone = bp_alone(k_max / 32);
-  const size_t lds   = (size_t) bp_layout(k_max / 32).total;
-  const void  *fn    = alone ? reinterpret_cast<const void *>(matmul_block_pairs_kernel<kBpDepthAlone>) :
-                               reinterpret_cast<const void *>(matmul_block_pairs_kernel<kBpDepthShared>);
-  static bool attr_set[2] = {};  // more than the default 64 KiB of dynamic LDS for long rows
-  if (!attr_set[alone]) {
-    const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int) kBpLdsLimit);
+  const bool     alone  = bp_alone(k_max / 32, wt);
+  const size_t   lds    = (size_t) bp_layout(k_max / 32, wt).total;
+  const BpKernel kernel = kBpKernels[wt == kQ8_0][alone];
+  static bool attr_set[2][2] = {};  // more than the default 64 KiB of dynamic LDS for long rows
+  if (!attr_set[wt == kQ8_0][alone]) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int) kBpLdsLimit);
     if (e != hipSuccess) {
       return e;
     }
-    attr_set[alone] = true;
+    attr_set[wt == kQ8_0][alone] = true;
   }
   // As many workgroups as the device holds at once (LDS decides: three of 43 KB for k = 4096, one of 113 KB for
   // k = 11008, on each of 256 compute units), shared out among the members by their weight bytes; a member's
@@ -451,11 +490,7 @@ hipError_t launch_matmul_block_pairs_group(hipStream_t stream, int count, float 
     grp.wg_begin[i + 1] = grp.wg_begin[i] + (int) wgs[i];
   }
   const dim3 grid((unsigned) grp.wg_begin[count]), block(kBpThreads);
-  if (alone) {
-    hipLaunchKernelGGL((matmul_block_pairs_kernel<kBpDepthAlone>), grid, block, lds, stream, grp, m);
-  } else {
-    hipLaunchKernelGGL((matmul_block_pairs_kernel<kBpDepthShared>), grid, block, lds, stream, grp, m);
-  }
+  hipLaunchKernelGGL(kernel, grid, block, lds, stream, grp, m);
   return hipGetLastError();
 }
 

@@ -299,7 +299,7 @@ void flush_batch(htpops_context *ctx, GemvBatch &b) {
       e = hipSuccess;
       if (pairs_g.count > 0) {
         e = launch_matmul_block_pairs_group(ctx->stream, pairs_g.count, pairs_g.out, pairs_g.act, pairs_g.w, pairs_g.n, b.m,
-                                            pairs_g.k);
+                                            pairs_g.k, (WeightType) b.wt);
       }
       if (e == hipSuccess && lane_g.count > 0) {
         e = launch_matmul_lane_order_group(ctx->stream, lane_g.count, lane_g.out, lane_g.act, lane_g.w, lane_g.n, b.m, k0,

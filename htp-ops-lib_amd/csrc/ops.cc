@@ -152,7 +152,7 @@ int lane_order_weights(htpops_context *ctx, const void *weight, const void *act,
   if (int r = new_copy(ctx, weight, w_bytes, kind, k, n, matmul_lane_order_weight_bytes(k, n, (WeightType) wt), &fresh)) {
     return r;
   }
-  const hipError_t e = *block_pairs ? launch_weights_to_block_pairs(ctx->stream, fresh, weight, k, n) :
+  const hipError_t e = *block_pairs ? launch_weights_to_block_pairs(ctx->stream, fresh, weight, k, n, (WeightType) wt) :
                                       launch_weights_to_lane_order(ctx->stream, fresh, weight, k, n, (WeightType) wt);
   if (e != hipSuccess) {
     forget_copy(ctx, fresh);
@@ -281,7 +281,7 @@ int run_few_rows(htpops_context *ctx, float *dst, const void *act, const void *w
     }
   }
   if (lw) {
-    const hipError_t e = pairs ? launch_matmul_block_pairs_group(ctx->stream, 1, &dst, &act, &lw, &n, m, &k) :
+    const hipError_t e = pairs ? launch_matmul_block_pairs_group(ctx->stream, 1, &dst, &act, &lw, &n, m, &k, (WeightType) wt) :
                                  launch_matmul_lane_order_group(ctx->stream, 1, &dst, &act, &lw, &n, m, k, (WeightType) wt,
                                                                 ctx->opt.lane_order);
     if (e == hipSuccess) {
