@@ -30,7 +30,8 @@ __global__ __launch_bounds__(kThreads) void quantize_q8_0_kernel(uint8_t *__rest
 
   const int       lane       = threadIdx.x & (kWave - 1);
   const int       wave       = threadIdx.x / kWave;
-  const long long wave_block = ((long long) blockIdx.x * (kThreads / kWave) + wave) * kBlocksPerWave;
+  const unsigned  group      = FRAGMENTS && fragments.m_tiles > 1 ? xcd_neighbours(blockIdx.x, gridDim.x) : blockIdx.x;
+  const long long wave_block = ((long long) group * (kThreads / kWave) + wave) * kBlocksPerWave;
   if (wave_block >= total_blocks) {
     return;
   }

@@ -137,7 +137,7 @@ __global__ __launch_bounds__(kThreads) void rms_norm_quantize_kernel(uint8_t *__
                                                                      const float *__restrict__ weight, float eps,
                                                                      int ne0, ActFragments fragments) {
   __shared__ float lds[kWaves];
-  const size_t row = blockIdx.x;
+  const size_t row = FRAGMENTS && fragments.m_tiles > 1 ? xcd_neighbours(blockIdx.x, gridDim.x) : blockIdx.x;
   const int    nb  = ne0 / kQK;
   const float *x   = src + row * ne0;
   uint8_t     *out = dst + row * (size_t) nb * 34;
