@@ -88,6 +88,43 @@ __device__ __forceinline__ unsigned xcd_neighbours(unsigned b, unsigned n) {
   return xcd * (n >> 3) + min(xcd, n & 7u) + (b >> 3);
 }
 
+// Rows that a launch of other work quantizes to Q8_0 beside it (see QuantizeJob): its workgroups `first` and on do that, THREADS
+// / 4 blocks each, with the arithmetic of quantize_q8_0_kernel (four lanes a block). No other launch has to be paid for a few
+// KB of rows, nor waited for.
+struct QuantizeBeside {
+  const float *src   = nullptr;
+  uint8_t     *dst   = nullptr;
+  unsigned     blocks = 0;
+  int          first  = 0x7fffffff;
+};
+__device__ __forceinline__ void quantize_beside(const QuantizeBeside &job, int workgroup, int threads) {
+  const unsigned block = (unsigned) workgroup * (unsigned) (threads / 4) + threadIdx.x / 4, part = threadIdx.x & 3u;
+  const bool     live  = block < job.blocks;
+  float          x[8], amax = 0.0f;
+  const float4  *p  = reinterpret_cast<const float4 *>(job.src + (size_t) (live ? block : 0u) * kQK + part * 8);
+  const float4   v0 = p[0], v1 = p[1];
+  x[0] = v0.x, x[1] = v0.y, x[2] = v0.z, x[3] = v0.w, x[4] = v1.x, x[5] = v1.y, x[6] = v1.z, x[7] = v1.w;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    amax = fmaxf(amax, fabsf(x[i]));
+  }
+  amax = quad_max(amax);
+  const float d  = amax / 127.0f;
+  const float id = (d != 0.0f) ? 1.0f / d : 0.0f;
+  if (!live) {
+    return;
+  }
+  uint16_t *to = reinterpret_cast<uint16_t *>(job.dst + (size_t) block * 34);
+  if (part == 0) {
+    to[0] = __half_as_ushort(__float2half_rn(d));
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int q0 = (int) roundf(x[2 * i] * id), q1 = (int) roundf(x[2 * i + 1] * id);
+    to[1 + part * 4 + i] = (uint16_t) ((q0 & 0xff) | ((q1 & 0xff) << 8));
+  }
+}
+
 // Activations in the operand order of the int8 matmul, [32-row tile][block][64 lanes] of 16 bytes: lane (c = row % 32, h)
 // holds elements 16 h .. 16 h + 15 of its row's block. The scale array behind them holds a dword (fp16 scale, 0) per row and
 // block, [tile][block][64] with zeros in the upper 32, and ends in one row of 64 zeros.

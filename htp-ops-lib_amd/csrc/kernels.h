@@ -31,8 +31,17 @@ hipError_t launch_gemv_q8_0_act(hipStream_t stream, float *out, const void *act,
 // member does not fit the fast kernel (k % 64, k <= 12288, 4-byte aligned buffers): the caller then launches them one
 // by one.
 constexpr int kGemvGroupMax = 8;
+// fp32 rows of `blocks` 32-value blocks in all that a launch of other work quantizes to Q8_0 beside it (the bytes of
+// launch_quantize_q8_0; src 16-byte, dst 4-byte aligned, both apart from everything the other work reads or writes)
+struct QuantizeJob {
+  const float *src;
+  void        *dst;
+  unsigned     blocks;
+};
+// (`beside`: or nullptr, here and below; it is always taken along)
 hipError_t launch_gemv_group_q8_0_act(hipStream_t stream, int count, float *const *outs, const void *const *acts,
-                                      const void *const *weights, const int *ns, const int *ks, WeightType wt);
+                                      const void *const *weights, const int *ns, const int *ks, WeightType wt,
+                                      const QuantizeJob *beside = nullptr);
 // The same launch with the activation row made inside it: RMSNorm(src [* norm_weight], eps) quantized to Q8_0 is what
 // every member multiplies by (all of one k), and it is also written to `q_out`, bit for bit what
 // launch_rms_norm_quantize_q8_0 writes (`normalize` false: src quantized as it is, the bytes of launch_quantize_q8_0). hipErrorNotSupported (nothing launched; the caller runs the two steps) unless
@@ -40,7 +49,8 @@ hipError_t launch_gemv_group_q8_0_act(hipStream_t stream, int count, float *cons
 // workgroup makes the row for itself, which beats a launch of its own up to about a thousand workgroups of 16 rows.
 hipError_t launch_gemv_group_rms_norm_q8_0_act(hipStream_t stream, int count, float *const *outs, const void *const *weights,
                                                const int *ns, int k, WeightType wt, const float *src,
-                                               const float *norm_weight, float eps, void *q_out, bool normalize);
+                                               const float *norm_weight, float eps, void *q_out, bool normalize,
+                                               const QuantizeJob *beside = nullptr);
 // 2 <= m <= 4 activation rows against several weight matrices in one launch: the decode kernel's stream over the
 // weights with the rows held in registers; member i reads the rows acts[i] of length ks[i] (k % 64 == 0, k <= 12288,
 // 4-byte aligned buffers; else hipErrorNotSupported)
@@ -71,10 +81,12 @@ hipError_t launch_matmul_skinny_group(hipStream_t stream, int count, float *cons
 bool       matmul_lane_order_fits(int n, int m, int k, WeightType wt);
 size_t     matmul_lane_order_weight_bytes(int k, int n, WeightType wt);
 hipError_t launch_weights_to_lane_order(hipStream_t stream, void *dst, const void *weight, int k, int n, WeightType wt);
-// (one launch for `count` matmuls of the same m, k and weight type; member i reads the activation rows acts[i])
+// (one launch for `count` matmuls of the same m, k and weight type; member i reads the activation rows acts[i]; *taken: whether
+// `beside` ran in it)
 hipError_t launch_matmul_lane_order_group(hipStream_t stream, int count, float *const *outs, const void *const *acts,
                                           const void *const *lane_order_weights, const int *ns, int m, int k,
-                                          WeightType wt, int forced_tiles);  // forced_tiles 2 / 3: one / two tiles per workgroup
+                                          WeightType wt, int forced_tiles,   // forced_tiles 2 / 3: one / two tiles per workgroup
+                                          const QuantizeJob *beside = nullptr, bool *taken = nullptr);
 // 2 <= m <= 8 rows against weights repacked once into another operand order (launch_weights_to_block_pairs, the
 // same size again): two blocks per matrix instruction, the second one in the result rows that 8 activation rows leave
 // unused. A workgroup keeps its member's activation rows in LDS and streams tiles of 16 weight rows over the whole of
@@ -83,7 +95,7 @@ bool       matmul_block_pairs_fits(int n, int m, int k, WeightType wt);
 hipError_t launch_weights_to_block_pairs(hipStream_t stream, void *dst, const void *weight, int k, int n, WeightType wt);
 hipError_t launch_matmul_block_pairs_group(hipStream_t stream, int count, float *const *outs, const void *const *acts,
                                            const void *const *pair_order_weights, const int *ns, int m, const int *ks,
-                                           WeightType wt);
+                                           WeightType wt, const QuantizeJob *beside = nullptr, bool *taken = nullptr);
 // many-row path for Q4_0 weights, k % 64 == 0: FP6 scaled MFMA (exact: int8 = 16 hi + lo, all parts |t| <= 15) over operand
 // tiles staged in LDS by DMA. The weight tiles (gemm_fp6_lds_weight_tile_bytes, 1 byte per weight) are converted once
 // (launch_q4_0_to_fp6_tiles) and can be cached by the caller; the activation tiles (gemm_fp6_lds_act_tile_bytes) are

@@ -108,6 +108,7 @@ struct BlockPairsGroupArgs {
   int            k[kGemvGroupMax];
   int            wg_begin[kGemvGroupMax + 1];  // member i owns workgroups wg_begin[i] .. wg_begin[i + 1] - 1
   int            count;
+  QuantizeBeside beside;                       // by the workgroups behind the members'
 };
 
 // LDS of a workgroup, in bytes from its start: the zeroed corner, the row image, the table of -8 x (block sums) as the
@@ -133,6 +134,10 @@ __host__ __device__ inline BpLayout bp_layout(int nblk, int wt) {
 template <int DEPTH, int WT>  // DEPTH: steps whose weights are requested ahead
 __global__ __launch_bounds__(kBpThreads) void matmul_block_pairs_kernel(BlockPairsGroupArgs grp, int m) {
   extern __shared__ __align__(16) uint8_t bp_lds[];
+  if ((int) blockIdx.x >= grp.beside.first) {
+    quantize_beside(grp.beside, (int) blockIdx.x - grp.beside.first, kBpThreads);
+    return;
+  }
   int member = 0;
   while (member + 1 < grp.count && (int) blockIdx.x >= grp.wg_begin[member + 1]) {
     ++member;
@@ -403,7 +408,8 @@ hipError_t launch_weights_to_block_pairs(hipStream_t stream, void *dst, const vo
 }
 
 hipError_t launch_matmul_block_pairs_group(hipStream_t stream, int count, float *const *outs, const void *const *acts,
-                                           const void *const *pair_order_weights, const int *ns, int m, const int *ks, WeightType wt) {
+                                           const void *const *pair_order_weights, const int *ns, int m, const int *ks, WeightType wt,
+                                           const QuantizeJob *beside, bool *taken) {
   if (count < 1 || count > kGemvGroupMax) {
     return hipErrorNotSupported;
   }
@@ -437,7 +443,10 @@ hipError_t launch_matmul_block_pairs_group(hipStream_t stream, int count, float 
   // k = 11008, on each of 256 compute units), shared out among the members by their weight bytes; a member's
   // workgroups take its tiles in turn.
   const int  per_cu   = alone ? 1 : (int) std::min<size_t>(3, kBpLdsLimit / lds);
-  const long resident = 256L * per_cu;
+  // (rows to be quantized beside take a few of those places while the members' workgroups walk)
+  const unsigned more = beside ? (beside->blocks + kBpThreads / 4 - 1) / (kBpThreads / 4) : 0;
+  const bool     take = more > 0 && more <= 16;
+  const long resident = 256L * per_cu - (take ? more : 0);
   long       tiles    = 0;
   for (int i = 0; i < count; ++i) {
     tiles += ns[i] / kBpRows;
@@ -489,7 +498,13 @@ hipError_t launch_matmul_block_pairs_group(hipStream_t stream, int count, float 
   for (int i = 0; i < count; ++i) {
     grp.wg_begin[i + 1] = grp.wg_begin[i] + (int) wgs[i];
   }
-  const dim3 grid((unsigned) grp.wg_begin[count]), block(kBpThreads);
+  dim3 grid((unsigned) grp.wg_begin[count]), block(kBpThreads);
+  if (take) {
+    grp.beside.src = beside->src, grp.beside.dst = static_cast<uint8_t *>(beside->dst), grp.beside.blocks = beside->blocks;
+    grp.beside.first = grp.wg_begin[count];
+    grid.x += more;
+    *taken = true;
+  }
   hipLaunchKernelGGL(kernel, grid, block, lds, stream, grp, m);
   return hipGetLastError();
 }

@@ -117,6 +117,8 @@ struct LaneOrderGroupArgs {
   const uint8_t *act[kGemvGroupMax];  // Q8_0 activation rows of each member (members may share them)
   float         *out[kGemvGroupMax];
   int            n[kGemvGroupMax];
+  int            count;
+  QuantizeBeside beside;  // by the workgroups of a grid row behind the members'
 };
 
 template <int WT>
@@ -138,6 +140,12 @@ __global__ __launch_bounds__(kLoThreads) void matmul_lane_order_kernel(LaneOrder
   constexpr int kLoActRows  = ROWS;
   constexpr int kLoScaleBlk = ROWS * 4;  // bytes of the scale table per block (one float per row)
   extern __shared__ __align__(16) uint8_t lo_lds[];  // activation panel, later the waves' sums
+  if ((int) blockIdx.y == grp.count) {
+    if (blockIdx.x * (kLoThreads / 4) < grp.beside.blocks) {
+      quantize_beside(grp.beside, (int) blockIdx.x, kLoThreads);
+    }
+    return;
+  }
   const int n = grp.n[blockIdx.y];
   if ((int) (blockIdx.x * kLoRows * TPW) >= n) {
     return;  // whole workgroup: this member has fewer rows than the widest one
@@ -340,7 +348,7 @@ hipError_t launch_weights_to_lane_order(hipStream_t stream, void *dst, const voi
 
 hipError_t launch_matmul_lane_order_group(hipStream_t stream, int count, float *const *outs, const void *const *acts,
                                           const void *const *lane_order_weights, const int *ns, int m, int k,
-                                          WeightType wt, int forced_tiles) {
+                                          WeightType wt, int forced_tiles, const QuantizeJob *beside, bool *taken) {
   if (count < 1 || count > kGemvGroupMax) {
     return hipErrorNotSupported;
   }
@@ -381,7 +389,13 @@ hipError_t launch_matmul_lane_order_group(hipStream_t stream, int count, float *
     pairs += (ns[i] / kLoRows + 1) / 2;
   }
   const int    tpw    = forced_tiles == 2 || forced_tiles == 3 ? forced_tiles - 1 : (pairs >= 512 ? 2 : 1);
-  const dim3   grid((unsigned) ((n_max / kLoRows + tpw - 1) / tpw), (unsigned) count);
+  dim3         grid((unsigned) ((n_max / kLoRows + tpw - 1) / tpw), (unsigned) count);
+  grp.count = count;
+  if (beside && (beside->blocks + kLoThreads / 4 - 1) / (kLoThreads / 4) <= grid.x) {
+    grp.beside.src = beside->src, grp.beside.dst = static_cast<uint8_t *>(beside->dst), grp.beside.blocks = beside->blocks;
+    ++grid.y;
+    *taken = true;
+  }
   const int    rows = panel_rows(m);
   const size_t lds  = panel_bytes(k, rows);
   hipLaunchKernelGGL(kernels[wt == kQ8_0][rows == 16][tpw - 1], grid, dim3(kLoThreads), lds, stream, grp, m, k);

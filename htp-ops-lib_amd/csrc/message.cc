@@ -66,6 +66,15 @@ struct GemvBatch {
     int                   ne0 = 0;
   } norm;
   bool fused = false;  // the members read norm.dst and run in the launch that makes it
+  // A Q8_0 quantization behind the members that nothing of theirs orders (the gated rows behind gate and up): it runs in their
+  // launch, on workgroups of its own, where that kernel takes it along, else behind it. The batch takes no more members then.
+  struct {
+    bool                  on = false;
+    struct RequestHeader *hdr = nullptr;
+    void                 *dst = nullptr;
+    const float          *src = nullptr;
+    int                   k = 0, m = 0;
+  } beside;
   bool fp6   = false;  // many-row members of the FP6-tile kernel (all over the same activation rows and k)
   bool pairs_fit = false;  // every member fits the two-blocks-per-instruction kernel (such members may differ in k)
 };
@@ -203,7 +212,7 @@ int run_fp6_group(htpops_context *ctx, GemvBatch &b) {
   return HTPOPS_OK;
 }
 
-void flush_batch(htpops_context *ctx, GemvBatch &b) {
+void flush_members(htpops_context *ctx, GemvBatch &b, const QuantizeJob *beside, bool *taken) {
   if (b.norm.waiting) {
     b.norm.waiting = false;
     const size_t q_bytes = q8_0_bytes(1, (size_t) b.norm.ne0);
@@ -216,8 +225,9 @@ void flush_batch(htpops_context *ctx, GemvBatch &b) {
       const hipError_t e = launch_gemv_group_rms_norm_q8_0_act(ctx->stream, b.count, b.out, b.w, b.n, b.norm.ne0,
                                                                        (WeightType) b.wt, b.norm.src,
                                                                        b.norm.weight, b.norm.eps, b.norm.dst,
-                                                                       b.norm.normalize);
+                                                                       b.norm.normalize, beside);
       if (e != hipErrorNotSupported) {
+        *taken = e == hipSuccess;
         ++ctx->message_submissions;
         if (e != hipSuccess) {
           const int ret = fail(ctx, HTPOPS_ERR_HIP, "rms_norm + mat_mul launch: %s", hipGetErrorString(e));
@@ -242,7 +252,7 @@ void flush_batch(htpops_context *ctx, GemvBatch &b) {
   }
   ++ctx->message_submissions;
   int ret = HTPOPS_OK;
-  if (b.count > 1) {
+  if (b.count > 1 || (beside && b.m == 1)) {
     for (int i = 0; i < b.count; ++i) {
       note_device_write(ctx, b.out[i], (size_t) b.m * b.n[i] * 4);
     }
@@ -253,7 +263,8 @@ void flush_batch(htpops_context *ctx, GemvBatch &b) {
       e   = ret == 1 ? hipErrorNotSupported : hipSuccess;
       ret = ret == 1 ? HTPOPS_OK : ret;
     } else if (b.m == 1) {
-      e = launch_gemv_group_q8_0_act(ctx->stream, b.count, b.out, b.act, b.w, b.n, b.k, (WeightType) b.wt);
+      e      = launch_gemv_group_q8_0_act(ctx->stream, b.count, b.out, b.act, b.w, b.n, b.k, (WeightType) b.wt, beside);
+      *taken = e == hipSuccess;
     } else {
       // 2..16 rows. Which kernel a matrix gets depends on that matrix alone, in the order of the single request
       // (run_few_rows): two and three rows of Q4_0 that fit the two-blocks-per-instruction kernel and have, or get, their
@@ -299,11 +310,11 @@ void flush_batch(htpops_context *ctx, GemvBatch &b) {
       e = hipSuccess;
       if (pairs_g.count > 0) {
         e = launch_matmul_block_pairs_group(ctx->stream, pairs_g.count, pairs_g.out, pairs_g.act, pairs_g.w, pairs_g.n, b.m,
-                                            pairs_g.k, (WeightType) b.wt);
+                                            pairs_g.k, (WeightType) b.wt, *taken ? nullptr : beside, taken);
       }
       if (e == hipSuccess && lane_g.count > 0) {
         e = launch_matmul_lane_order_group(ctx->stream, lane_g.count, lane_g.out, lane_g.act, lane_g.w, lane_g.n, b.m, k0,
-                                           (WeightType) b.wt, ctx->opt.lane_order);
+                                           (WeightType) b.wt, ctx->opt.lane_order, *taken ? nullptr : beside, taken);
       }
       if (e == hipSuccess && rows_g.count > 0) {
         e = launch_gemv_rows_group_q8_0_act(ctx->stream, rows_g.count, rows_g.out, rows_g.act, rows_g.w, rows_g.n, b.m,
@@ -349,6 +360,58 @@ void flush_batch(htpops_context *ctx, GemvBatch &b) {
     }
   }
   b.count = 0;
+}
+
+void flush_batch(htpops_context *ctx, GemvBatch &b) {
+  if (!b.beside.on) {
+    bool taken = false;
+    flush_members(ctx, b, nullptr, &taken);
+    return;
+  }
+  const auto        job = b.beside;
+  const QuantizeJob beside = { job.src, job.dst, (unsigned) ((size_t) job.m * (job.k / 32)) };
+  bool              taken = false;
+  b.beside.on = false;
+  note_device_write(ctx, job.dst, q8_0_bytes((size_t) job.m, (size_t) job.k));
+  flush_members(ctx, b, &beside, &taken);
+  ++ctx->message_submissions;  // (a unit of its own, in whichever launch)
+  if (!taken) {
+    job.hdr->state = op_quantize(ctx, job.dst, job.src, job.k, job.m);
+  }
+}
+
+// true: the Q8_0 quantization (op 14) `req` now runs beside the members of the open batch (or behind them)
+bool try_beside(htpops_context *ctx, const struct OpComputeRequest *req, struct RequestHeader *hdr, GemvBatch &b) {
+  const auto *p = reinterpret_cast<const RmsNormF32Params *>(req->payload);
+  // (a row that its own matmuls can make in their launch stays with those; many rows want the operand order as well)
+  if (!ctx->has_device || b.count == 0 || b.beside.on || b.m > kBatchMaxM || p->ne0 <= 0 || p->ne1 <= 0 || p->ne0 % 32 != 0 ||
+      p->ne1 > kBatchMaxM || p->ne0 > (1 << 20) || (p->ne1 == 1 && p->ne0 <= 4096)) {
+    return false;
+  }
+  const size_t src_bytes = (size_t) p->ne1 * p->ne0 * 4, q_bytes = q8_0_bytes((size_t) p->ne1, (size_t) p->ne0);
+  const float *src = (const float *) resolve(ctx, p->src, src_bytes);
+  void        *dst = resolve(ctx, p->dst, q_bytes);
+  if (!src || !dst || !aligned(src, 16) || !aligned(dst, 4) || ranges_overlap(dst, q_bytes, src, src_bytes)) {
+    return false;  // the ordinary path reports what is wrong
+  }
+  for (int i = 0; i < b.count; ++i) {
+    const size_t oi = (size_t) b.m * b.n[i] * 4;
+    if (ranges_overlap(dst, q_bytes, b.out[i], oi) || ranges_overlap(src, src_bytes, b.out[i], oi) ||
+        ranges_overlap(dst, q_bytes, b.w[i], weight_bytes((size_t) b.n[i], (size_t) b.k[i], b.wt)) ||
+        ranges_overlap(dst, q_bytes, b.act[i], q8_0_bytes((size_t) b.m, (size_t) b.k[i]))) {
+      return false;
+    }
+  }
+  if (b.norm.waiting) {
+    const size_t row = (size_t) b.norm.ne0 * 4, made = q8_0_bytes(1, (size_t) b.norm.ne0);
+    if (ranges_overlap(dst, q_bytes, b.norm.dst, made) || ranges_overlap(src, src_bytes, b.norm.dst, made) ||
+        ranges_overlap(dst, q_bytes, b.norm.src, row) || (b.norm.weight && ranges_overlap(dst, q_bytes, b.norm.weight, row))) {
+      return false;
+    }
+  }
+  b.beside.on = true, b.beside.hdr = hdr, b.beside.dst = dst, b.beside.src = src, b.beside.k = p->ne0, b.beside.m = p->ne1;
+  hdr->state = HTPOPS_OK;
+  return true;
 }
 
 // true: the one-row RMSNorm + Q8_0 (op 13) or Q8_0 quantization (op 14) request now waits in the (empty) batch for the
@@ -426,7 +489,7 @@ bool try_batch(htpops_context *ctx, const struct OpComputeRequest *req, struct R
       flush_batch(ctx, b);  // runs the waiting request by itself
     }
   }
-  bool join = b.count > 0 && b.count < kGemvGroupMax && b.wt == wt && b.m == p->m && (!b.fused || reads_norm) &&
+  bool join = b.count > 0 && b.count < kGemvGroupMax && !b.beside.on && b.wt == wt && b.m == p->m && (!b.fused || reads_norm) &&
               b.fp6 == fp6 && (!fp6 || (b.act[0] == act && b.k[0] == p->k)) &&
               (p->m == 1 || many_rows || b.k[0] == p->k ||
                (ctx->opt.gemv_rows_kernel != 0 && gemv_rows_fits(p->m, p->k, (WeightType) wt) &&
@@ -680,6 +743,9 @@ int enqueue_message(htpops_context *ctx, struct MessageHeader *msg, size_t msg_b
             (req->op == HTP_OPS_QUANTIZE_Q8_0 &&
              size >= sizeof(struct RequestHeader) + sizeof(struct OpComputeRequest) + sizeof(RmsNormF32Params));
           if (norm_payload) {
+            if (req->op == HTP_OPS_QUANTIZE_Q8_0 && try_beside(ctx, req, hdr, batch)) {
+              break;
+            }
             flush_batch(ctx, batch);
           }
           if (!(norm_payload && try_defer_norm(ctx, req, hdr, batch)) &&

@@ -147,7 +147,8 @@ int htpops_finish_message(htpops_context *ctx, struct MessageHeader *msg);
  * were grouped count once (diagnostic; the reference runs one op per request, src/dsp/commu.c:91-100). A group is one
  * kernel launch where all its members take the same kernel (the projections of a decoder layer do); a group of
  * many-row matmuls adds one launch that converts the activations, and a group whose members take different kernels (by
- * shape and weight type, at 17 to 32 rows also by size) issues one launch per kernel. Grouping never changes a result: a request joins a group only if it neither reads nor
+ * shape and weight type, at 17 to 32 rows also by size) issues one launch per kernel. A
+ * quantization that runs beside a group, in its launch, counts as a unit of its own. Grouping never changes a result: a request joins a group only if it neither reads nor
  * overwrites what an earlier member writes and writes nothing an earlier member reads. */
 int htpops_last_message_submissions(htpops_context *ctx);
 
