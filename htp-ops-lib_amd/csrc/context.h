@@ -127,9 +127,10 @@ struct htpops_context {
     int         kind = 0;  // which kernel family's layout (PlanKind)
   } act_fragments;
   // Workspace that the next request of the message needs for the matmul it makes of the rows the current one quantizes, when
-  // that takes the int8 fragment kernels (0: it is something else): the quantizer then leaves the rows there in operand order
-  // too, and notes them in `act_fragments`.
-  size_t next_fragments_ws = 0;
+  // that takes the int8 fragment kernels or the FP6-tile kernel, `next_fragments_kind` (0: it is something else): the quantizer
+  // then leaves the rows there in that operand order too, and notes them in `act_fragments`.
+  size_t next_fragments_ws   = 0;
+  int    next_fragments_kind = 0;
   bool in_message = false;
   // how many separately launched units (grouped launches and single ops) the most recent message walk issued
   int  message_submissions = 0;

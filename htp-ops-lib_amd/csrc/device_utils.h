@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "kernels.h"
+
 namespace htpops {
 
 constexpr int kWave = 64;
@@ -79,10 +81,10 @@ __device__ __forceinline__ float quad_max(float v) {
 #undef HTPOPS_DPP_STEP
 
 // Workgroups are handed to the 8 XCDs round robin: the index of workgroup b of n when each XCD is to have neighbouring indices.
-// The quantizers that write operand order go by it: the 16-byte pieces of eight rows are one cache line, which would
-// otherwise lie partly written in eight L2 caches (layers of 128 / 256 / 400 rows of Q8_0, hidden 1536 / 1536 / 2048, 85.5 -> 84.3,
-// 113.5 -> 110.7, 162.7 -> 160.3 us; 100 fp32 rows of 8960 against 1537 22.4 -> 21.6; a single row tile, whose few rows all go
-// everywhere, 12.7 -> 13.2, stays as it comes).
+// RMSNorm + Q8_0 that writes operand order goes by it, a workgroup to a row: the 16-byte pieces of eight rows are one cache line,
+// which would otherwise lie partly written in eight L2 caches (layers of 128 / 256 / 400 rows of Q8_0, hidden 1536 / 1536 /
+// 2048, 85.5 -> 84.3, 113.5 -> 110.7, 162.7 -> 160.3 us, with the plain quantizer, whose waves held one row then, doing so
+// too; a single row tile, whose few rows all go everywhere, 12.7 -> 13.2, stays as it comes).
 __device__ __forceinline__ unsigned xcd_neighbours(unsigned b, unsigned n) {
   const unsigned xcd = b & 7u;
   return xcd * (n >> 3) + min(xcd, n & 7u) + (b >> 3);
@@ -128,17 +130,23 @@ __device__ __forceinline__ void quantize_beside(const QuantizeBeside &job, int w
 // Activations in the operand order of the int8 matmul, [32-row tile][block][64 lanes] of 16 bytes: lane (c = row % 32, h)
 // holds elements 16 h .. 16 h + 15 of its row's block. The scale array behind them holds a dword (fp16 scale, 0) per row and
 // block, [tile][block][64] with zeros in the upper 32, and ends in one row of 64 zeros.
+// In the operand order of the FP6 matmul (k % 64 == 0): [32-row tile][step of two blocks] of kFp6ActTile bytes, each quant split
+// as 16 hi + lo into two E2M3 planes (see the head of gemm_fp6_lds.hip, and its converter of stored rows, whose bytes these are);
+// the scales behind, [kFp6RowBlock rows][step][row] of (fp16, fp16, 0).
+constexpr int kFp6ActTile = 3 * 1024, kFp6RowBlock = 128;
 struct ActFragments {
   uint2    *frag   = nullptr;
   uint32_t *scales = nullptr;
   int       m_tiles = 0, nblk = 0;
 };
-inline ActFragments act_fragments_at(void *base, int m, int k) {
+inline ActFragments act_fragments_at(void *base, int m, int k, ActOrder order) {
   ActFragments f;
   if (base) {
     f.m_tiles = (m + 31) / 32, f.nblk = k / kQK;
     f.frag   = static_cast<uint2 *>(base);
-    f.scales = reinterpret_cast<uint32_t *>(static_cast<uint8_t *>(base) + (((size_t) f.m_tiles * f.nblk * 1024 + 255) & ~(size_t) 255));
+    const size_t operand = order == kActFp6 ? (size_t) f.m_tiles * (f.nblk / 2) * kFp6ActTile :
+                                              ((size_t) f.m_tiles * f.nblk * 1024 + 255) & ~(size_t) 255;
+    f.scales = reinterpret_cast<uint32_t *>(static_cast<uint8_t *>(base) + operand);
   }
   return f;
 }
@@ -148,6 +156,50 @@ __device__ __forceinline__ void store_act_fragment(const ActFragments &f, int ro
   f.frag[(at + 32 * (part >> 1)) * 2 + (part & 1)] = quants;
   if (part < 2) {
     f.scales[at + 32 * part] = part == 0 ? scale : 0u;
+  }
+}
+// The codes of four quants as E2M3, 24 bits: low nibbles (0..15) and high ones (two's complement) as sign and magnitude, times 1/8.
+__device__ __forceinline__ uint32_t fp6_pack(uint32_t c) {
+  return (c & 0x3fu) | ((c >> 2) & 0xfc0u) | ((c >> 4) & 0x3f000u) | ((c >> 6) & 0xfc0000u);
+}
+__device__ __forceinline__ uint32_t fp6_low_codes(uint32_t q) {
+  return fp6_pack(q & 0x0f0f0f0fu);
+}
+__device__ __forceinline__ uint32_t fp6_high_codes(uint32_t q) {
+  const uint32_t h = (q >> 4) & 0x0f0f0f0fu, neg = (h >> 3) & 0x01010101u;
+  return fp6_pack(((h ^ (neg * 15u)) + neg) | (neg << 5));  // |hi| <= 8 per byte, no carry between bytes
+}
+template <int PERM>
+__device__ __forceinline__ uint32_t quad_move(uint32_t v) {
+  return (uint32_t) __builtin_amdgcn_mov_dpp((int) v, PERM, 0xf, 0xf, true);
+}
+// The same for the FP6 order, by the whole quad that holds the block. A lane's eight quants are six bytes of either plane; lanes
+// 0 and 2 gather the first 16 of the 24 bytes of the high and of the low plane, lanes 1 and 3 the other 8, and store them whole.
+__device__ __forceinline__ void store_act_fp6(const ActFragments &f, int row, int kb, int part, uint2 quants, uint16_t scale) {
+  const uint32_t h0 = fp6_high_codes(quants.x), h1 = fp6_high_codes(quants.y);
+  const uint32_t l0 = fp6_low_codes(quants.x), l1 = fp6_low_codes(quants.y);
+  const uint32_t hx = h0 | (h1 << 24), hy = h1 >> 8, lx = l0 | (l1 << 24), ly = l1 >> 8;
+  const bool     low = part >= 2;
+  const uint32_t x03h = quad_move<0xcc>(hx), x03l = quad_move<0xcc>(lx);  // of lane 0 for the heads, of lane 3 for the tails
+  const uint32_t y03h = quad_move<0xcc>(hy), y03l = quad_move<0xcc>(ly);
+  const uint32_t x1h = quad_move<0x55>(hx), x1l = quad_move<0x55>(lx);
+  const uint32_t y12h = quad_move<0x99>(hy), y12l = quad_move<0x99>(ly);  // of lane 1 for the heads, of lane 2 for the tails
+  const uint32_t x2h = quad_move<0xaa>(hx), x2l = quad_move<0xaa>(lx);
+  const uint32_t x03 = low ? x03l : x03h, y03 = low ? y03l : y03h, x1 = low ? x1l : x1h, y12 = low ? y12l : y12h,
+                 x2 = low ? x2l : x2h;
+  const size_t step = (size_t) (row / 32) * (f.nblk / 2) + kb / 2;
+  const int    b = kb & 1, lane = (row & 31) + (low ? 32 : 0);
+  uint8_t     *tile = reinterpret_cast<uint8_t *>(f.frag) + step * kFp6ActTile;
+  uint32_t    *sc   = f.scales + (((size_t) (row / kFp6RowBlock) * (f.nblk / 2) + kb / 2) * kFp6RowBlock + row % kFp6RowBlock) * 2;
+  if ((part & 1) == 0) {
+    reinterpret_cast<uint4 *>(tile + 2048 * b)[lane] = make_uint4(x03, y03 | (x1 << 16), (x1 >> 16) | (y12 << 16), x2);
+  } else {
+    reinterpret_cast<uint2 *>(tile + 1024 + 512 * b)[lane] = make_uint2(y12 | (x03 << 16), (x03 >> 16) | (y03 << 16));
+  }
+  if (part == 0) {
+    reinterpret_cast<uint16_t *>(sc)[b] = scale;
+  } else if (part == 1 && b == 0) {
+    sc[1] = 0u;
   }
 }
 // the row of zeros, from 64 threads of the grid

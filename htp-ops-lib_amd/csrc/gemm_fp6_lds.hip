@@ -43,7 +43,7 @@ typedef int      v8i __attribute__((ext_vector_type(8)));
 typedef float    v16f __attribute__((ext_vector_type(16)));
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 
-constexpr int kBM = 128;        // output rows per workgroup; its columns: 32 NT, NT = 2 or 3
+constexpr int kBM = kFp6RowBlock;        // output rows per workgroup; its columns: 32 NT, NT = 2 or 3
 constexpr int kMinTiles = 192;  // 128 x 64 output tiles from which the kernel is used
 
 // ---- tiles ----------------------------------------------------------------------------------------------------------
@@ -59,7 +59,7 @@ constexpr int kMinTiles = 192;  // 128 x 64 output tiles from which the kernel i
 //                                    then the scales as operand dwords of the scale product: [block][64 lanes], lane
 //                                    l < 32: the column's fp16 scale in the half-word of its block (K slot 0 or 1),
 //                                    lanes 32..63: 0.
-constexpr int kATile  = 3 * 1024;
+constexpr int kATile  = kFp6ActTile;
 constexpr int kWTile  = 2 * 1024;
 constexpr int kSaTile = 1024;
 constexpr int kOffA   = 0;
@@ -178,16 +178,7 @@ __global__ __launch_bounds__(256) void q8_0_to_fp6_tiles_kernel(uint8_t *__restr
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const uint32_t q = b == 0 ? __builtin_amdgcn_alignbyte(a[i + 1], a[i], 2) : a[i + 1];
-    uint32_t       code;
-    if (lo) {
-      code = q & 0x0f0f0f0fu;
-    } else {
-      const uint32_t h   = (q >> 4) & 0x0f0f0f0fu;         // high nibbles: 4-bit two's complement
-      const uint32_t neg = (h >> 3) & 0x01010101u;
-      const uint32_t mag = (h ^ (neg * 15u)) + neg;        // |hi| <= 8 per byte, no carry between bytes
-      code               = mag | (neg << 5);
-    }
-    g[i] = (code & 0x3fu) | ((code >> 2) & 0xfc0u) | ((code >> 4) & 0x3f000u) | ((code >> 6) & 0xfc0000u);
+    g[i]             = lo ? fp6_low_codes(q) : fp6_high_codes(q);
   }
   const uint4 head = make_uint4(g[0] | (g[1] << 24), (g[1] >> 8) | (g[2] << 16), (g[2] >> 16) | (g[3] << 8), g[4] | (g[5] << 24));
   const uint2 tail = make_uint2((g[5] >> 8) | (g[6] << 16), (g[6] >> 16) | (g[7] << 8));

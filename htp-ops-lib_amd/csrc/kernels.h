@@ -10,17 +10,21 @@ namespace htpops {
 
 enum WeightType { kQ4_0 = 2, kQ8_0 = 8 };  // enum ggml_type values (reference: include/dsp/quants.h:33-74)
 
+// The operand order of the matmul that follows a quantizer: of the int8 fragments, or of the FP6 tiles (k % 64 == 0)
+enum ActOrder { kActI8, kActFp6 };
 // fp32 [m][k] -> block_q8_0 [m][k/32]. `act_fragments` (or nullptr; gemm_i8_act_fragment_bytes, 256-byte aligned): the rows
-// are also written there in the operand order of the int8 matmul, what launch_act_to_i8_fragments_group makes of them (rows
-// past the last are left as they are: nothing depends on them); `dst` may then be nullptr.
-hipError_t launch_quantize_q8_0(hipStream_t stream, void *dst, const float *src, int k, int m, void *act_fragments = nullptr);
+// are also written there in the operand order `order` (kActFp6: gemm_fp6_lds_act_tile_bytes), what the matmul's own conversion
+// makes of them (rows past the last are left as they are: nothing depends on them); `dst` may then be nullptr.
+hipError_t launch_quantize_q8_0(hipStream_t stream, void *dst, const float *src, int k, int m, void *act_fragments = nullptr,
+                                ActOrder order = kActI8);
 
 // y = x * rsqrt(mean(x^2) + eps) * w; w may be null
 hipError_t launch_rms_norm_f32(hipStream_t stream, float *dst, const float *src, const float *weight, float eps,
                                int ne0, int ne1);
 // same, result quantized to block_q8_0 [ne1][ne0/32]; ne0 % 32 == 0
 hipError_t launch_rms_norm_quantize_q8_0(hipStream_t stream, void *dst, const float *src, const float *weight,
-                                         float eps, int ne0, int ne1, void *act_fragments = nullptr);
+                                         float eps, int ne0, int ne1, void *act_fragments = nullptr,
+                                         ActOrder order = kActI8);
 
 // out fp32 [m][n] = act block_q8_0 [m][k/32] x weight [n][k/32]
 // decode path: one pass over the weight bytes per activation row

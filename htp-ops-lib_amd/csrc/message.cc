@@ -574,7 +574,8 @@ bool try_batch_permuted(htpops_context *ctx, const struct OpComputeRequest *req,
 }
 
 // What `next` behind a quantizing request `req` (op 13 or 14) needs of the workspace if it is a matmul over exactly the rows
-// that one writes and takes the int8 fragment kernels (see htpops_context::next_fragments_ws); else 0.
+// that one writes and takes the int8 fragment kernels or the FP6-tile kernel (see htpops_context::next_fragments_ws, whose kind
+// it sets); else 0.
 size_t fragments_of_next(htpops_context *ctx, const struct OpComputeRequest *req, const struct RequestHeader *next, size_t size) {
   if (next->type != REQUEST_TYPE_OP_COMPUTE ||
       size < sizeof(struct RequestHeader) + sizeof(struct OpComputeRequest) + sizeof(MatMulParams)) {
@@ -600,7 +601,8 @@ size_t fragments_of_next(htpops_context *ctx, const struct OpComputeRequest *req
     return 0;
   }
   const MatMulPlan plan = plan_mat_mul(ctx, w, aligned(act, 4), p->m, p->k, p->n, wt);
-  return plan.kind == kPlanFragments ? plan.ws_bytes : 0;
+  ctx->next_fragments_kind = (int) plan.kind;
+  return plan.kind == kPlanFragments || plan.kind == kPlanLdsFp6 ? plan.ws_bytes : 0;
 }
 
 // `next` behind an fp32 attention request `req` of one row or a few: if it is the Q8_0 quantization of exactly that

@@ -42,10 +42,14 @@ void wanted_fragments(htpops_context *ctx, int m, int k, void **where) {
   }
 }
 
+ActOrder next_order(const htpops_context *ctx) {
+  return ctx->next_fragments_kind == (int) kPlanLdsFp6 ? kActFp6 : kActI8;
+}
+
 void note_fragments(htpops_context *ctx, const void *where, const void *rows, int m, int k) {
   if (where) {
     auto &af = ctx->act_fragments;
-    af.src = rows, af.src_bytes = q8_0_bytes((size_t) m, (size_t) k), af.m = m, af.k = k, af.kind = (int) kPlanFragments;
+    af.src = rows, af.src_bytes = q8_0_bytes((size_t) m, (size_t) k), af.m = m, af.k = k, af.kind = ctx->next_fragments_kind;
   }
 }
 
@@ -64,7 +68,7 @@ int op_quantize(htpops_context *ctx, void *dst, const float *src, int k, int m) 
   void *frags = nullptr;
   wanted_fragments(ctx, m, k, &frags);
   note_device_write(ctx, dst, q8_0_bytes((size_t) m, (size_t) k));
-  HTPOPS_HIP(ctx, launch_quantize_q8_0(ctx->stream, dst, src, k, m, frags));
+  HTPOPS_HIP(ctx, launch_quantize_q8_0(ctx->stream, dst, src, k, m, frags, next_order(ctx)));
   note_fragments(ctx, frags, dst, m, k);
   return HTPOPS_OK;
 }
@@ -84,7 +88,7 @@ int op_rms_norm_quantize(htpops_context *ctx, void *dst, const float *src, const
     void *frags = nullptr;
     wanted_fragments(ctx, ne1, ne0, &frags);
     note_device_write(ctx, dst, q8_0_bytes((size_t) ne1, (size_t) ne0));
-    HTPOPS_HIP(ctx, launch_rms_norm_quantize_q8_0(ctx->stream, dst, src, weight, eps, ne0, ne1, frags));
+    HTPOPS_HIP(ctx, launch_rms_norm_quantize_q8_0(ctx->stream, dst, src, weight, eps, ne0, ne1, frags, next_order(ctx)));
     note_fragments(ctx, frags, dst, ne1, ne0);
     return HTPOPS_OK;
   }
@@ -388,13 +392,15 @@ int op_mat_mul_f32(htpops_context *ctx, float *dst, const float *act, const void
   note_device_write(ctx, dst, (size_t) m * n * 4);
   MatMulPlan plan = plan_mat_mul(ctx, weight, true, m, k, n, weight_type, writes_weights(dst, weight, m, k, n, weight_type));
   settle_copy(ctx, plan, weight, m, k, n, weight_type);
-  if (plan.kind == kPlanFragments && (long long) m * (k / 32) <= 0x7fffffffLL) {
+  if ((plan.kind == kPlanFragments || plan.kind == kPlanLdsFp6) && (long long) m * (k / 32) <= 0x7fffffffLL) {
     // the quantizer writes the operand order the matmul wants: the rows in block_q8_0 form would have one reader, another
-    // launch that puts them into that order (33 rows, k = 8960, n = 1537: 3 of 18 us)
+    // launch that puts them into that order (33 rows, k = 8960, n = 1537: 3 of 18 us; 512 rows,
+    // Q4_0, 4096 x 4096: 31.4 -> 29.1 us)
     if (int r = ensure_workspace(ctx, plan.ws_bytes)) {
       return r;
     }
-    HTPOPS_HIP(ctx, launch_quantize_q8_0(ctx->stream, nullptr, act, k, m, ctx->workspace));
+    HTPOPS_HIP(ctx, launch_quantize_q8_0(ctx->stream, nullptr, act, k, m, ctx->workspace,
+                                         plan.kind == kPlanLdsFp6 ? kActFp6 : kActI8));
     return run_mat_mul(ctx, plan, dst, nullptr, weight, m, k, n, weight_type, static_cast<uint8_t *>(ctx->workspace));
   }
   // workspace: [quantized activations][what the matmul itself needs]

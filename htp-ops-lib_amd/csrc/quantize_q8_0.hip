@@ -20,39 +20,8 @@ constexpr int kBlocksPerGroup = kBlocksPerWave * (kThreads / kWave);
 constexpr int kWaveOutBytes   = kBlocksPerWave * 34;       // 544
 constexpr int kWaveOutDwords  = kWaveOutBytes / 4;         // 136
 
-// total_blocks = m * k / 32; blocks are contiguous in both src (128 B each) and dst (34 B each).
-// FRAGMENTS: the quants also go to `fragments` (see ActFragments), and dst may be nullptr.
-template <bool FRAGMENTS>
-__global__ __launch_bounds__(kThreads) void quantize_q8_0_kernel(uint8_t *__restrict__ dst,
-                                                                  const float *__restrict__ src,
-                                                                  long long total_blocks, ActFragments fragments) {
-  __shared__ __attribute__((aligned(16))) uint16_t stage[kThreads / kWave][kWaveOutBytes / 2];
-
-  const int       lane       = threadIdx.x & (kWave - 1);
-  const int       wave       = threadIdx.x / kWave;
-  const unsigned  group      = FRAGMENTS && fragments.m_tiles > 1 ? xcd_neighbours(blockIdx.x, gridDim.x) : blockIdx.x;
-  const long long wave_block = ((long long) group * (kThreads / kWave) + wave) * kBlocksPerWave;
-  if (wave_block >= total_blocks) {
-    return;
-  }
-  const long long block = wave_block + (lane >> 2);
-  const int       part  = lane & 3;  // which 8 of the block's 32 values
-  const bool      live  = block < total_blocks;
-
-  float x[8];
-  if (live) {
-    const float4 *p  = reinterpret_cast<const float4 *>(src + block * kQK + part * 8);
-    const float4  v0 = p[0];
-    const float4  v1 = p[1];
-    x[0] = v0.x, x[1] = v0.y, x[2] = v0.z, x[3] = v0.w;
-    x[4] = v1.x, x[5] = v1.y, x[6] = v1.z, x[7] = v1.w;
-  } else {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      x[i] = 0.0f;
-    }
-  }
-
+// The eight values of a lane and its quad's block: quants (two dwords) and fp16 scale
+__device__ __forceinline__ uint2 quantize_eight(const float x[8], uint16_t *scale) {
   float amax = 0.0f;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
@@ -68,36 +37,66 @@ __global__ __launch_bounds__(kThreads) void quantize_q8_0_kernel(uint8_t *__rest
   for (int i = 0; i < 8; ++i) {
     q[i] = (int) roundf(x[i] * id);
   }
+  *scale = __half_as_ushort(__float2half_rn(d));
+  return { (uint32_t) ((q[0] & 0xff) | ((q[1] & 0xff) << 8) | ((q[2] & 0xff) << 16) | ((uint32_t) q[3] << 24)),
+           (uint32_t) ((q[4] & 0xff) | ((q[5] & 0xff) << 8) | ((q[6] & 0xff) << 16) | ((uint32_t) q[7] << 24)) };
+}
 
-  if constexpr (FRAGMENTS) {
-    if (live) {
-      const unsigned b = (unsigned) block, nblk = (unsigned) fragments.nblk;  // (the launcher sees to the range)
-      const uint2    packed = { (uint32_t) ((q[0] & 0xff) | ((q[1] & 0xff) << 8) | ((q[2] & 0xff) << 16) | ((uint32_t) q[3] << 24)),
-                                (uint32_t) ((q[4] & 0xff) | ((q[5] & 0xff) << 8) | ((q[6] & 0xff) << 16) | ((uint32_t) q[7] << 24)) };
-      store_act_fragment(fragments, (int) (b / nblk), (int) (b % nblk), part, packed, __half_as_ushort(__float2half_rn(d)));
-    }
-    if (blockIdx.x == 0 && threadIdx.x < kWave) {
-      end_act_fragments(fragments, threadIdx.x);
-    }
-    if (dst == nullptr) {
-      return;
+__device__ __forceinline__ void load_eight(float x[8], const float *src, bool live) {
+  if (live) {
+    const float4 *p  = reinterpret_cast<const float4 *>(src);
+    const float4  v0 = p[0];
+    const float4  v1 = p[1];
+    x[0] = v0.x, x[1] = v0.y, x[2] = v0.z, x[3] = v0.w;
+    x[4] = v1.x, x[5] = v1.y, x[6] = v1.z, x[7] = v1.w;
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      x[i] = 0.0f;
     }
   }
+}
 
-  // LDS image of this wave's 16 blocks: block b at byte 34 b; its quants start at 34 b + 2 + 8 part.
-  uint16_t *img  = stage[wave];
-  const int base = ((lane >> 2) * 34 + 2 + part * 8) / 2;  // in uint16 units
-  img[base + 0]  = (uint16_t) ((q[0] & 0xff) | ((q[1] & 0xff) << 8));
-  img[base + 1]  = (uint16_t) ((q[2] & 0xff) | ((q[3] & 0xff) << 8));
-  img[base + 2]  = (uint16_t) ((q[4] & 0xff) | ((q[5] & 0xff) << 8));
-  img[base + 3]  = (uint16_t) ((q[6] & 0xff) | ((q[7] & 0xff) << 8));
+// A block's 34 bytes in the image of its wave, from the four lanes that hold it
+__device__ __forceinline__ void stage_block(uint16_t *block, int part, uint2 quants, uint16_t scale) {
+  uint16_t *to = block + 1 + part * 4;
+  to[0]        = (uint16_t) quants.x;
+  to[1]        = (uint16_t) (quants.x >> 16);
+  to[2]        = (uint16_t) quants.y;
+  to[3]        = (uint16_t) (quants.y >> 16);
   if (part == 0) {
-    img[(lane >> 2) * 17] = __half_as_ushort(__float2half_rn(d));
+    block[0] = scale;
   }
-  // the image is private to this wave: a wavefront-scope release/acquire pair orders the LDS traffic
+}
+
+// the image is private to its wave: a wavefront-scope release/acquire pair orders the LDS traffic
+__device__ __forceinline__ void image_complete() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// total_blocks = m * k / 32; blocks are contiguous in both src (128 B each) and dst (34 B each).
+__global__ __launch_bounds__(kThreads) void quantize_q8_0_kernel(uint8_t *__restrict__ dst, const float *__restrict__ src,
+                                                                  long long total_blocks) {
+  __shared__ __attribute__((aligned(16))) uint16_t stage[kThreads / kWave][kWaveOutBytes / 2];
+
+  const int       lane       = threadIdx.x & (kWave - 1);
+  const int       wave       = threadIdx.x / kWave;
+  const long long wave_block = ((long long) blockIdx.x * (kThreads / kWave) + wave) * kBlocksPerWave;
+  if (wave_block >= total_blocks) {
+    return;
+  }
+  const long long block = wave_block + (lane >> 2);
+  const int       part  = lane & 3;  // which 8 of the block's 32 values
+  float           x[8];
+  uint16_t        scale;
+  load_eight(x, src + block * kQK + part * 8, block < total_blocks);
+  const uint2 quants = quantize_eight(x, &scale);
+
+  uint16_t *img = stage[wave];
+  stage_block(img + (lane >> 2) * 17, part, quants, scale);
+  image_complete();
 
   // 16 blocks start at a multiple of 16 blocks = 544 bytes, so the image is dword aligned in dst.
   long long remaining = total_blocks - wave_block;
@@ -114,20 +113,90 @@ __global__ __launch_bounds__(kThreads) void quantize_q8_0_kernel(uint8_t *__rest
   }
 }
 
+// The same rows, also in the operand order ORDER of the matmul behind (see ActFragments); dst may be nullptr. There the 16 bytes
+// of neighbouring rows lie side by side, so a wave's sixteen blocks are two blocks of eight rows: its stores of the operand
+// are whole lines of 128 bytes, and its pieces of the rows in block_q8_0 form 68 bytes, continued by its neighbours. (With
+// sixteen blocks of one row a store instruction went to 32 lines, an eighth of each: int8 order of 128 rows of 1536 / 8960
+// 4.0 -> 3.1 / 5.6 -> 4.4 us, of 27 rows of 8960 5.1 -> 3.0, FP6 order of 512 rows of 4096 / 11008 6.0 -> 5.9 / 13.8 -> 12.1; the
+// rows alone 5.4 / 8.2 and the launch that put them into FP6 order 5.5 / 6.3. Neighbouring groups on one XCD: the same,
+// but 64 rows of 1056 12.7 -> 13.1 with their matmul.)
+constexpr int kRowsPerWave = 8;
+template <int ORDER>
+__global__ __launch_bounds__(kThreads) void quantize_operand_kernel(uint8_t *__restrict__ dst, const float *__restrict__ src, int m,
+                                                                     unsigned groups_per_row, ActFragments fragments) {
+  __shared__ __attribute__((aligned(16))) uint16_t stage[kThreads / kWave][kWaveOutBytes / 2];
+
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = threadIdx.x / kWave;
+  if (ORDER == kActI8 && blockIdx.x == 0 && threadIdx.x < kWave) {
+    end_act_fragments(fragments, threadIdx.x);
+  }
+  const unsigned group = blockIdx.x;
+  const int      row0 = (int) (group / groups_per_row) * kRowsPerWave, nblk = fragments.nblk;
+  const int      kb0 = ((int) (group % groups_per_row) * (kThreads / kWave) + wave) * 2;
+  if (kb0 >= nblk) {
+    return;
+  }
+  const int  part = lane & 3, r = (lane >> 2) & 7, b = lane >> 5;
+  const int  row = row0 + r, kb = kb0 + b;
+  const bool live = row < m && kb < nblk;
+  float      x[8];
+  uint16_t   scale;
+  load_eight(x, src + ((size_t) row * nblk + kb) * kQK + part * 8, live);
+  const uint2 quants = quantize_eight(x, &scale);
+  if (live) {
+    if constexpr (ORDER == kActFp6) {
+      store_act_fp6(fragments, row, kb, part, quants, scale);
+    } else {
+      store_act_fragment(fragments, row, kb, part, quants, scale);
+    }
+  }
+  if (dst == nullptr) {
+    return;
+  }
+
+  // LDS image of this wave's pieces of eight rows, 68 bytes each
+  uint16_t *img = stage[wave];
+  stage_block(img + r * 34 + b * 17, part, quants, scale);
+  image_complete();
+  uint8_t *out = dst + ((size_t) row0 * nblk + kb0) * 34;
+  if (nblk % 2 == 0) {  // pieces of whole dwords
+    for (int i = lane; i < kRowsPerWave * 17; i += kWave) {
+      const int to = i / 17;
+      if (row0 + to < m) {
+        reinterpret_cast<uint32_t *>(out + (size_t) to * nblk * 34)[i % 17] = reinterpret_cast<const uint32_t *>(img)[i];
+      }
+    }
+  } else {
+    for (int i = lane; i < kRowsPerWave * 34; i += kWave) {
+      const int to = i / 34, at = i % 34;
+      if (row0 + to < m && (at < 17 || kb0 + 1 < nblk)) {
+        reinterpret_cast<uint16_t *>(out + (size_t) to * nblk * 34)[at] = img[i];
+      }
+    }
+  }
+}
+
 }  // namespace
 
-hipError_t launch_quantize_q8_0(hipStream_t stream, void *dst, const float *src, int k, int m, void *act_fragments) {
+hipError_t launch_quantize_q8_0(hipStream_t stream, void *dst, const float *src, int k, int m, void *act_fragments,
+                                ActOrder order) {
   const long long total_blocks = (long long) m * (k / kQK);
   const long long groups       = (total_blocks + kBlocksPerGroup - 1) / kBlocksPerGroup;
   if (act_fragments) {
     if (total_blocks > 0x7fffffffLL) {
       return hipErrorInvalidValue;
     }
-    hipLaunchKernelGGL(quantize_q8_0_kernel<true>, dim3((unsigned) groups), dim3(kThreads), 0, stream, (uint8_t *) dst, src,
-                       total_blocks, act_fragments_at(act_fragments, m, k));
+    const unsigned per_row = (unsigned) ((k / kQK + 2 * (kThreads / kWave) - 1) / (2 * (kThreads / kWave)));
+    const unsigned rows    = (unsigned) ((m + kRowsPerWave - 1) / kRowsPerWave);
+    if ((unsigned long long) per_row * rows > 0x7fffffffULL) {
+      return hipErrorInvalidValue;
+    }
+    hipLaunchKernelGGL(order == kActFp6 ? quantize_operand_kernel<kActFp6> : quantize_operand_kernel<kActI8>, dim3(per_row * rows),
+                       dim3(kThreads), 0, stream, (uint8_t *) dst, src, m, per_row, act_fragments_at(act_fragments, m, k, order));
   } else {
-    hipLaunchKernelGGL(quantize_q8_0_kernel<false>, dim3((unsigned) groups), dim3(kThreads), 0, stream, (uint8_t *) dst, src,
-                       total_blocks, ActFragments());
+    hipLaunchKernelGGL(quantize_q8_0_kernel, dim3((unsigned) groups), dim3(kThreads), 0, stream, (uint8_t *) dst, src,
+                       total_blocks);
   }
   return hipGetLastError();
 }
