@@ -90,6 +90,40 @@ __device__ __forceinline__ unsigned xcd_neighbours(unsigned b, unsigned n) {
   return xcd * (n >> 3) + min(xcd, n & 7u) + (b >> 3);
 }
 
+// The eight values of a lane and its quad's block: quants (two dwords) and fp16 scale
+__device__ __forceinline__ uint2 quantize_eight(const float x[8], uint16_t *scale) {
+  float amax = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    amax = fmaxf(amax, fabsf(x[i]));
+  }
+  amax = quad_max(amax);
+
+  const float d  = amax / 127.0f;
+  const float id = (d != 0.0f) ? 1.0f / d : 0.0f;
+
+  int q[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    q[i] = (int) roundf(x[i] * id);
+  }
+  *scale = __half_as_ushort(__float2half_rn(d));
+  return { (uint32_t) ((q[0] & 0xff) | ((q[1] & 0xff) << 8) | ((q[2] & 0xff) << 16) | ((uint32_t) q[3] << 24)),
+           (uint32_t) ((q[4] & 0xff) | ((q[5] & 0xff) << 8) | ((q[6] & 0xff) << 16) | ((uint32_t) q[7] << 24)) };
+}
+
+// A block's 34 bytes from the four lanes that hold it, to 2-byte aligned memory or LDS
+__device__ __forceinline__ void store_q8_0_block(uint16_t *block, int part, uint2 quants, uint16_t scale) {
+  uint16_t *to = block + 1 + part * 4;
+  to[0]        = (uint16_t) quants.x;
+  to[1]        = (uint16_t) (quants.x >> 16);
+  to[2]        = (uint16_t) quants.y;
+  to[3]        = (uint16_t) (quants.y >> 16);
+  if (part == 0) {
+    block[0] = scale;
+  }
+}
+
 // Rows that a launch of other work quantizes to Q8_0 beside it (see QuantizeJob): its workgroups `first` and on do that, THREADS
 // / 4 blocks each, with the arithmetic of quantize_q8_0_kernel (four lanes a block). No other launch has to be paid for a few
 // KB of rows, nor waited for.
@@ -102,28 +136,14 @@ struct QuantizeBeside {
 __device__ __forceinline__ void quantize_beside(const QuantizeBeside &job, int workgroup, int threads) {
   const unsigned block = (unsigned) workgroup * (unsigned) (threads / 4) + threadIdx.x / 4, part = threadIdx.x & 3u;
   const bool     live  = block < job.blocks;
-  float          x[8], amax = 0.0f;
+  float          x[8];
   const float4  *p  = reinterpret_cast<const float4 *>(job.src + (size_t) (live ? block : 0u) * kQK + part * 8);
   const float4   v0 = p[0], v1 = p[1];
   x[0] = v0.x, x[1] = v0.y, x[2] = v0.z, x[3] = v0.w, x[4] = v1.x, x[5] = v1.y, x[6] = v1.z, x[7] = v1.w;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    amax = fmaxf(amax, fabsf(x[i]));
-  }
-  amax = quad_max(amax);
-  const float d  = amax / 127.0f;
-  const float id = (d != 0.0f) ? 1.0f / d : 0.0f;
-  if (!live) {
-    return;
-  }
-  uint16_t *to = reinterpret_cast<uint16_t *>(job.dst + (size_t) block * 34);
-  if (part == 0) {
-    to[0] = __half_as_ushort(__float2half_rn(d));
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int q0 = (int) roundf(x[2 * i] * id), q1 = (int) roundf(x[2 * i + 1] * id);
-    to[1 + part * 4 + i] = (uint16_t) ((q0 & 0xff) | ((q1 & 0xff) << 8));
+  uint16_t    scale;
+  const uint2 quants = quantize_eight(x, &scale);
+  if (live) {
+    store_q8_0_block(reinterpret_cast<uint16_t *>(job.dst + (size_t) block * 34), (int) part, quants, scale);
   }
 }
 

@@ -759,11 +759,16 @@ __global__ __launch_bounds__(kPfThreads *GROUPS, DP <= 128 ? 2 : 1) void flash_a
 // (`units` of them), lane for lane as the prefill kernel left them. Each takes every G-th run of kPfMergeChunk shares, all
 // loads of a run requested before the first use, folded one by one into a running (max, sum, O); with G = 4 (more
 // shares than a run holds) the four states meet in LDS (one row, 16384 keys, 16 / 4 heads of 96, 64 shares: 23.0 -> 19.2 us).
-template <bool QO_F32, int G>
+// Q8 (QO_F32, G = 1, D = 8 units, a multiple of 32): the four waves of a workgroup hold one block of 32 output columns of 32 rows,
+// which are also stored as Q8_0 in `q8_out` and (1 + ActOrder) in that operand order, whose lines they fill (12 heads of 128,
+// 128 rows into int8 order: 3.9 -> 4.3 us for the launch of 3.1 behind it; 32 heads, 512 rows into FP6 order 8.1 -> 12.2 for one
+// of 5.9).
+template <bool QO_F32, int G, int Q8>
 __global__ __launch_bounds__(256) void flash_attn_prefill_merge_kernel(void *__restrict__ o_ptr,
                                                                        const float *__restrict__ part, int n_splits,
                                                                        int n_tiles, int units, int qo_len, int n_heads,
-                                                                       int D) {
+                                                                       int D, uint8_t *__restrict__ q8_out, ActFragments fragments) {
+  static_assert(Q8 < 0 || (QO_F32 && G == 1), "quantized rows come from one trip over fp32 rows");
   __shared__ float states[G == 1 ? 1 : G][6][G == 1 ? 1 : kWave];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6);
   const int id   = G == 1 ? (int) blockIdx.x * 4 + wave : (int) blockIdx.x;
@@ -828,6 +833,36 @@ __global__ __launch_bounds__(256) void flash_attn_prefill_merge_kernel(void *__r
     } else {
       v4h hv = { (_Float16) (v[0] * inv), (_Float16) (v[1] * inv), (_Float16) (v[2] * inv), (_Float16) (v[3] * inv) };
       *reinterpret_cast<v4h *>(reinterpret_cast<_Float16 *>(o_ptr) + at) = hv;
+    }
+  }
+  if constexpr (Q8 >= 0) {
+    __shared__ float rows[kBQ][kQK + 1];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      rows[lane & 31][8 * wave + 4 * (lane >> 5) + e] = v[e] * inv;
+    }
+    if (Q8 == 1 + kActI8 && blockIdx.x == 0) {
+      end_act_fragments(fragments, threadIdx.x);
+    }
+    __syncthreads();
+    const int row = tile / n_heads * kBQ + ((int) threadIdx.x >> 2), qpart = (int) threadIdx.x & 3;
+    if (threadIdx.x >= 4 * kBQ || row >= qo_len) {  // (a quad of lanes has one row)
+      return;
+    }
+    float x[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      x[i] = rows[threadIdx.x >> 2][8 * qpart + i];
+    }
+    uint16_t     scale;
+    const uint2  quants = quantize_eight(x, &scale);
+    const int    kb     = (head * units + unit) / 4;
+    const size_t nblk   = (size_t) n_heads * units / 4;
+    store_q8_0_block(reinterpret_cast<uint16_t *>(q8_out + ((size_t) row * nblk + kb) * 34), qpart, quants, scale);
+    if constexpr (Q8 == 1 + kActFp6) {
+      store_act_fp6(fragments, row, kb, qpart, quants, scale);
+    } else if constexpr (Q8 == 1 + kActI8) {
+      store_act_fragment(fragments, row, kb, qpart, quants, scale);
     }
   }
 }
@@ -1698,7 +1733,7 @@ hipError_t launch_few_rows(hipStream_t stream, FewPlan plan, void *o, const void
 template <int DP, bool FULL, bool QO_F32>
 hipError_t launch_prefill(hipStream_t stream, void *o, const void *q, const void *k, const void *v, const void *mask,
                           int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim, bool causal, int forced,
-                          bool mask_threshold, float *scratch) {
+                          bool mask_threshold, float *scratch, void *q8_out, void *act_fragments, ActOrder order) {
   const PrefillPlan plan = prefill_plan(DP, qo_len, kv_len, n_heads, n_kv_heads, mask != nullptr, forced);
   if (plan.q_blocks > 65535u) {
     return hipErrorInvalidValue;
@@ -1735,13 +1770,29 @@ hipError_t launch_prefill(hipStream_t stream, void *o, const void *q, const void
     return e;
   }
   constexpr int kUnits = DP / 8;
+  const ActFragments fragments = act_fragments_at(act_fragments, qo_len, n_heads * head_dim, order);
+#define HTPOPS_MERGE(G, Q8, WORKGROUPS)                                                                               \
+  hipLaunchKernelGGL((flash_attn_prefill_merge_kernel<QO_F32, G, Q8>), dim3((unsigned) (WORKGROUPS)), dim3(256), 0, stream, o, \
+                     scratch, (int) splits, (int) tiles, kUnits, qo_len, n_heads, head_dim, static_cast<uint8_t *>(q8_out), \
+                     fragments)
   if (splits > (unsigned) kPfMergeChunk) {
-    hipLaunchKernelGGL((flash_attn_prefill_merge_kernel<QO_F32, 4>), dim3((unsigned) (tiles * kUnits)), dim3(256), 0, stream, o,
-                       scratch, (int) splits, (int) tiles, kUnits, qo_len, n_heads, head_dim);
-  } else {
-    hipLaunchKernelGGL((flash_attn_prefill_merge_kernel<QO_F32, 1>), dim3((unsigned) ((tiles * kUnits + 3) / 4)), dim3(256), 0,
-                       stream, o, scratch, (int) splits, (int) tiles, kUnits, qo_len, n_heads, head_dim);
+    HTPOPS_MERGE(4, -1, tiles * kUnits);
+    return hipGetLastError();
   }
+  if constexpr (QO_F32) {
+    if (q8_out) {
+      if (!act_fragments) {
+        HTPOPS_MERGE(1, 0, tiles * kUnits / 4);
+      } else if (order == kActFp6) {
+        HTPOPS_MERGE(1, 1 + kActFp6, tiles * kUnits / 4);
+      } else {
+        HTPOPS_MERGE(1, 1 + kActI8, tiles * kUnits / 4);
+      }
+      return hipGetLastError();
+    }
+  }
+  HTPOPS_MERGE(1, -1, (tiles * kUnits + 3) / 4);
+#undef HTPOPS_MERGE
   return hipGetLastError();
 }
 
@@ -1811,19 +1862,6 @@ hipError_t launch_decode(hipStream_t stream, void *o, const void *q, const void 
 
 // (more rows than a few meet a matmul that wants them in operand order, which the quantizer leaves as well)
 constexpr int kFewQ8Rows = 16;
-bool flash_attn_writes_q8_0(int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim, bool qo_is_f32, bool mask,
-                            int forced_key_groups) {
-  return qo_is_f32 && ((qo_len == 1 && (head_dim == 64 || head_dim == 128)) ||
-                       (qo_len <= kFewQ8Rows && few_plan(qo_len, kv_len, n_heads, n_kv_heads, head_dim, mask, forced_key_groups).split != 0));
-}
-
-size_t flash_attn_workspace_bytes(int qo_len, int kv_len, int n_heads, int head_dim) {
-  if (qo_len != 1 || (head_dim != 64 && head_dim != 128)) {
-    return 0;
-  }
-  const size_t n_splits = ((size_t) kv_len + kDecSplitShort - 1) / kDecSplitShort;  // the most there can be
-  return (size_t) n_heads * n_splits * ((size_t) head_dim + 2) * sizeof(float);
-}
 
 namespace {
 
@@ -1835,6 +1873,30 @@ bool takes_prefill(int qo_len, int head_dim) {
 }
 
 }  // namespace
+
+bool flash_attn_writes_q8_0(int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim, bool qo_is_f32, bool mask,
+                            int forced_key_groups) {
+  if (!qo_is_f32 || (qo_len == 1 && (head_dim == 64 || head_dim == 128))) {
+    return qo_is_f32;
+  }
+  if (few_plan(qo_len, kv_len, n_heads, n_kv_heads, head_dim, mask, forced_key_groups).split != 0) {
+    return qo_len <= kFewQ8Rows;
+  }
+  // a prefill whose shares are put together in one trip, whole blocks of a head to a workgroup
+  if (!takes_prefill(qo_len, head_dim) || head_dim % 32 != 0) {
+    return false;
+  }
+  const unsigned splits = prefill_plan(head_dim, qo_len, kv_len, n_heads, n_kv_heads, mask, forced_key_groups).splits;
+  return splits > 1 && splits <= (unsigned) kPfMergeChunk;
+}
+
+size_t flash_attn_workspace_bytes(int qo_len, int kv_len, int n_heads, int head_dim) {
+  if (qo_len != 1 || (head_dim != 64 && head_dim != 128)) {
+    return 0;
+  }
+  const size_t n_splits = ((size_t) kv_len + kDecSplitShort - 1) / kDecSplitShort;  // the most there can be
+  return (size_t) n_heads * n_splits * ((size_t) head_dim + 2) * sizeof(float);
+}
 
 bool flash_attn_splits_keys(int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim, bool mask,
                             int forced_key_groups) {
@@ -1861,7 +1923,7 @@ hipError_t launch_flash_attn_decode_part(hipStream_t stream, int part, void *o, 
 hipError_t launch_flash_attn(hipStream_t stream, void *o, const void *q, const void *k, const void *v,
                              const void *mask, int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim,
                              bool qo_is_f32, bool causal, void *workspace, void *q8_out, int forced_key_groups,
-                             bool mask_threshold, void *shares) {
+                             bool mask_threshold, void *shares, void *act_fragments, ActOrder order) {
   // with a single query row the causal rule (key j visible iff j <= kv_len - 1) hides nothing
   if (qo_len == 1 && (head_dim == 64 || head_dim == 128)) {
     float *ws = static_cast<float *>(workspace);
@@ -1883,9 +1945,11 @@ hipError_t launch_flash_attn(hipStream_t stream, void *o, const void *q, const v
   }
 #define HTPOPS_PREFILL(DP, FULL)                                                                                     \
   qo_is_f32 ? launch_prefill<DP, FULL, true>(stream, o, q, k, v, mask, qo_len, kv_len, n_heads, n_kv_heads, head_dim, \
-                                             causal, forced_key_groups, mask_threshold, static_cast<float *>(shares)) : \
+                                             causal, forced_key_groups, mask_threshold, static_cast<float *>(shares), q8_out, \
+                                             act_fragments, order) :                                                  \
               launch_prefill<DP, FULL, false>(stream, o, q, k, v, mask, qo_len, kv_len, n_heads, n_kv_heads, head_dim, \
-                                              causal, forced_key_groups, mask_threshold, static_cast<float *>(shares))
+                                              causal, forced_key_groups, mask_threshold, static_cast<float *>(shares), q8_out, \
+                                              act_fragments, order)
   if (head_dim == 128) {
     return HTPOPS_PREFILL(128, true);
   }

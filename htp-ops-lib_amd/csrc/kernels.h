@@ -182,7 +182,8 @@ hipError_t launch_copy_results(hipStream_t stream, float *dst, const float *src,
 // (0: by grid size). `mask_threshold`: the mask selects keys (keep iff mask > -16, reference:
 // src/dsp/ops/flash_attn.c:448-460) instead of being added to the scores (:1505-1512). `shares`: kAttnSharesBytes, where the
 // workgroups that share a query block's or a few rows' keys leave their parts (used where flash_attn_splits_keys says so);
-// nullptr: one workgroup walks all of them, with the same results bit for bit.
+// nullptr: one workgroup walks all of them, with the same results bit for bit. `act_fragments` (or nullptr): the rows of
+// `q8_out` in operand order as well, as the quantizers write them; only of a prefill.
 constexpr size_t kAttnSharesBytes = (size_t) 32 << 20;  // two shares of 512 queries of 32 heads of 128 take 17 MB
 bool       flash_attn_splits_keys(int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim, bool mask,
                                   int forced_key_groups);
@@ -190,7 +191,8 @@ size_t     flash_attn_workspace_bytes(int qo_len, int kv_len, int n_heads, int h
 hipError_t launch_flash_attn(hipStream_t stream, void *o, const void *q, const void *k, const void *v,
                              const void *mask, int qo_len, int kv_len, int n_heads, int n_kv_heads, int head_dim,
                              bool qo_is_f32, bool causal, void *workspace, void *q8_out, int forced_key_groups,
-                             bool mask_threshold, void *shares);
+                             bool mask_threshold, void *shares, void *act_fragments = nullptr,
+                             ActOrder order = kActI8);
 // One of the two launches of one-token attention by itself, for timing: part 1 = the split-KV launch (writes the
 // partial records into `workspace`), part 2 = the merge launch (reads them). Same arguments as above otherwise.
 hipError_t launch_flash_attn_decode_part(hipStream_t stream, int part, void *o, const void *q, const void *k,

@@ -605,9 +605,9 @@ size_t fragments_of_next(htpops_context *ctx, const struct OpComputeRequest *req
   return plan.kind == kPlanFragments || plan.kind == kPlanLdsFp6 ? plan.ws_bytes : 0;
 }
 
-// `next` behind an fp32 attention request `req` of one row or a few: if it is the Q8_0 quantization of exactly that
-// attention's output rows into a buffer that overlaps none of the attention's operands, notes where it wants the rows
-// (ctx->attn_q8_out) and returns it; nullptr otherwise.
+// `next` behind an fp32 attention request `req`: if it is the Q8_0 quantization of exactly that attention's output rows into a
+// buffer that overlaps none of the attention's operands, notes where it wants the rows (ctx->attn_q8_out) and returns it;
+// nullptr otherwise.
 struct RequestHeader *attention_output_quantizer(htpops_context *ctx, const struct OpComputeRequest *req,
                                                  struct RequestHeader *next, size_t next_size) {
   const auto *p = reinterpret_cast<const FlashAttnParams *>(req->payload);
@@ -619,9 +619,7 @@ struct RequestHeader *attention_output_quantizer(htpops_context *ctx, const stru
   const auto *pq   = reinterpret_cast<const RmsNormF32Params *>(nreq->payload);
   if (nreq->op != HTP_OPS_QUANTIZE_Q8_0 || p->qo_len <= 0 || p->kv_len <= 0 || p->n_heads <= 0 || p->n_kv_heads <= 0 ||
       p->head_dim <= 0 || p->n_heads > (1 << 20) || p->head_dim > 256 || p->n_heads % p->n_kv_heads != 0 || pq->ne1 != p->qo_len ||
-      pq->ne0 != p->n_heads * p->head_dim ||
-      !flash_attn_writes_q8_0(p->qo_len, p->kv_len, p->n_heads, p->n_kv_heads, p->head_dim, true,
-                              p->mask.fd >= 0 && lookup(ctx, p->mask.fd), ctx->opt.attn_key_groups)) {
+      pq->ne0 != p->n_heads * p->head_dim) {
     return nullptr;
   }
   const size_t row = (size_t) p->qo_len * pq->ne0 * 4, q_bytes = q8_0_bytes((size_t) p->qo_len, (size_t) pq->ne0);
@@ -629,7 +627,10 @@ struct RequestHeader *attention_output_quantizer(htpops_context *ctx, const stru
   const void  *o = resolve(ctx, p->o, row), *src = resolve(ctx, pq->src, row);
   void        *dst = resolve(ctx, pq->dst, q_bytes);
   const void  *q = resolve(ctx, p->q, row), *k = resolve(ctx, p->k, kv), *v = resolve(ctx, p->v, kv);
-  if (!o || o != src || !dst || !q || !k || !v || !aligned(dst, 4) || ranges_overlap(dst, q_bytes, o, row) ||
+  // (the plan is asked for sizes that the buffers have)
+  if (!o || o != src || !dst || !q || !k || !v || !aligned(dst, 4) ||
+      !flash_attn_writes_q8_0(p->qo_len, p->kv_len, p->n_heads, p->n_kv_heads, p->head_dim, true,
+                              p->mask.fd >= 0 && lookup(ctx, p->mask.fd), ctx->opt.attn_key_groups) || ranges_overlap(dst, q_bytes, o, row) ||
       ranges_overlap(dst, q_bytes, q, row) || ranges_overlap(dst, q_bytes, k, kv) || ranges_overlap(dst, q_bytes, v, kv)) {
     return nullptr;
   }
@@ -754,13 +755,18 @@ int enqueue_message(htpops_context *ctx, struct MessageHeader *msg, size_t msg_b
               !(matmul_payload && try_batch(ctx, req, hdr, batch))) {
             flush_batch(ctx, batch);
             ++ctx->message_submissions;
-            // attention of one token or a few whose fp32 output the NEXT request quantizes to Q8_0 (on its way to the o
-            // projection): the launch that finishes the attention writes those rows too, and the next request is done with it
+            // attention whose fp32 output the NEXT request quantizes to Q8_0 (on its way to the o projection; one token, a
+            // few, or a prompt's rows whose keys are split): the launch that finishes the attention writes those rows too, and the next request is done with it
             struct RequestHeader *next = nullptr;
             if (req->op == HTP_OPS_FLASH_ATTN_QO_F32_KV_F16 && i + 1 < n_reqs &&
                 size >= sizeof(struct RequestHeader) + sizeof(struct OpComputeRequest) + sizeof(FlashAttnParams)) {
               next = attention_output_quantizer(ctx, req, message_header_get_request_ptr(msg, i + 1),
                                                 message_header_get_request_size(msg, i + 1));
+              if (next && i + 2 < n_reqs) {  // (in operand order as well for the matmul behind)
+                ctx->next_fragments_ws = fragments_of_next(ctx, reinterpret_cast<const struct OpComputeRequest *>(next->data),
+                                                           message_header_get_request_ptr(msg, i + 2),
+                                                           message_header_get_request_size(msg, i + 2));
+              }
             }
             if (norm_payload && i + 1 < n_reqs) {
               ctx->next_fragments_ws = fragments_of_next(ctx, req, message_header_get_request_ptr(msg, i + 1),

@@ -556,9 +556,15 @@ int op_flash_attn(htpops_context *ctx, void *o, const void *q, const void *k, co
     q8_out = ctx->attn_q8_out;
     note_device_write(ctx, q8_out, q8_0_bytes((size_t) qo_len, (size_t) n_heads * head_dim));
   }
+  // (17 rows and more, whose kernel needs no workspace of its own)
+  void *frags = nullptr;
+  if (q8_out && !ws_bytes) {
+    wanted_fragments(ctx, qo_len, n_heads * head_dim, &frags);
+  }
   HTPOPS_HIP(ctx, launch_flash_attn(ctx->stream, o, q, k, v, mask, qo_len, kv_len, n_heads, n_kv_heads, head_dim,
                                     qo_is_f32 != 0, causal != 0, ws, q8_out, ctx->opt.attn_key_groups,
-                                    ctx->opt.attn_mask_threshold != 0, shares));
+                                    ctx->opt.attn_mask_threshold != 0, shares, frags, next_order(ctx)));
+  note_fragments(ctx, frags, q8_out, qo_len, n_heads * head_dim);
   ctx->attn_q8_done = q8_out != nullptr;
   return HTPOPS_OK;
 }

@@ -20,28 +20,6 @@ constexpr int kBlocksPerGroup = kBlocksPerWave * (kThreads / kWave);
 constexpr int kWaveOutBytes   = kBlocksPerWave * 34;       // 544
 constexpr int kWaveOutDwords  = kWaveOutBytes / 4;         // 136
 
-// The eight values of a lane and its quad's block: quants (two dwords) and fp16 scale
-__device__ __forceinline__ uint2 quantize_eight(const float x[8], uint16_t *scale) {
-  float amax = 0.0f;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    amax = fmaxf(amax, fabsf(x[i]));
-  }
-  amax = quad_max(amax);
-
-  const float d  = amax / 127.0f;
-  const float id = (d != 0.0f) ? 1.0f / d : 0.0f;
-
-  int q[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    q[i] = (int) roundf(x[i] * id);
-  }
-  *scale = __half_as_ushort(__float2half_rn(d));
-  return { (uint32_t) ((q[0] & 0xff) | ((q[1] & 0xff) << 8) | ((q[2] & 0xff) << 16) | ((uint32_t) q[3] << 24)),
-           (uint32_t) ((q[4] & 0xff) | ((q[5] & 0xff) << 8) | ((q[6] & 0xff) << 16) | ((uint32_t) q[7] << 24)) };
-}
-
 __device__ __forceinline__ void load_eight(float x[8], const float *src, bool live) {
   if (live) {
     const float4 *p  = reinterpret_cast<const float4 *>(src);
@@ -54,18 +32,6 @@ __device__ __forceinline__ void load_eight(float x[8], const float *src, bool li
     for (int i = 0; i < 8; ++i) {
       x[i] = 0.0f;
     }
-  }
-}
-
-// A block's 34 bytes in the image of its wave, from the four lanes that hold it
-__device__ __forceinline__ void stage_block(uint16_t *block, int part, uint2 quants, uint16_t scale) {
-  uint16_t *to = block + 1 + part * 4;
-  to[0]        = (uint16_t) quants.x;
-  to[1]        = (uint16_t) (quants.x >> 16);
-  to[2]        = (uint16_t) quants.y;
-  to[3]        = (uint16_t) (quants.y >> 16);
-  if (part == 0) {
-    block[0] = scale;
   }
 }
 
@@ -95,7 +61,7 @@ __global__ __launch_bounds__(kThreads) void quantize_q8_0_kernel(uint8_t *__rest
   const uint2 quants = quantize_eight(x, &scale);
 
   uint16_t *img = stage[wave];
-  stage_block(img + (lane >> 2) * 17, part, quants, scale);
+  store_q8_0_block(img + (lane >> 2) * 17, part, quants, scale);
   image_complete();
 
   // 16 blocks start at a multiple of 16 blocks = 544 bytes, so the image is dword aligned in dst.
@@ -157,7 +123,7 @@ __global__ __launch_bounds__(kThreads) void quantize_operand_kernel(uint8_t *__r
 
   // LDS image of this wave's pieces of eight rows, 68 bytes each
   uint16_t *img = stage[wave];
-  stage_block(img + r * 34 + b * 17, part, quants, scale);
+  store_q8_0_block(img + r * 34 + b * 17, part, quants, scale);
   image_complete();
   uint8_t *out = dst + ((size_t) row0 * nblk + kb0) * 34;
   if (nblk % 2 == 0) {  // pieces of whole dwords
