@@ -1657,8 +1657,8 @@ PrefillPlan prefill_plan(int dp, int qo_len, int kv_len, int n_heads, int n_kv_h
     const size_t share  = p.tiles * prefill_partial_floats(dp / 8) * sizeof(float);
     const size_t blocks = ((size_t) kv_len + kBK - 1) / kBK, groups = (size_t) prefill_key_groups(dp);
     const size_t most   = std::min({ (size_t) (kCus / wgs), blocks / (2 * groups), kAttnSharesBytes / share });
-    // (for few tiles down to one block, while one trip of the merge takes all shares: 5 rows over 1029 keys, 12 tiles, 14.4 ->
-    // 12.6 us; but 128 rows over 1152, 48 tiles, 17.5 -> 17.8, and 500 rows over 500, 256 tiles, 18.7 -> 20.2)
+    // (for few tiles down to one block, while one trip of the merge takes all shares: 5 rows over 1029 keys, 12 tiles, of a head
+    // dim of 128, which few_plan takes now, 14.4 -> 12.6 us; but 128 rows over 1152, 48 tiles, 17.5 -> 17.8, and 500 rows over 500, 256 tiles, 18.7 -> 20.2)
     const size_t finer  = std::min({ (size_t) (kCus / wgs), blocks / groups, kAttnSharesBytes / share, (size_t) kPfMergeChunk });
     const size_t splits = most < 2 ? 1 : p.tiles <= 32 ? std::max(most, finer) : most;
     const auto   turns  = [&](size_t n) { return (n + groups - 1) / groups; };

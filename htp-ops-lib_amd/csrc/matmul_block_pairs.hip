@@ -131,10 +131,12 @@ __host__ __device__ inline BpLayout bp_layout(int nblk, int wt) {
   return l;
 }
 
-template <int DEPTH, int WT>  // DEPTH: steps whose weights are requested ahead
+// DEPTH: steps whose weights are requested ahead; BESIDE: the workgroups behind the members' quantize rows (an instance of its
+// own, so that launches without such rows have nothing to test)
+template <int DEPTH, int WT, bool BESIDE>
 __global__ __launch_bounds__(kBpThreads) void matmul_block_pairs_kernel(BlockPairsGroupArgs grp, int m) {
   extern __shared__ __align__(16) uint8_t bp_lds[];
-  if ((int) blockIdx.x >= grp.beside.first) {
+  if (BESIDE && (int) blockIdx.x >= grp.beside.first) {
     quantize_beside(grp.beside, (int) blockIdx.x - grp.beside.first, kBpThreads);
     return;
   }
@@ -274,13 +276,16 @@ __global__ __launch_bounds__(kBpThreads) void matmul_block_pairs_kernel(BlockPai
     a[1] = (int) __builtin_amdgcn_alignbyte(t2, t1, shift);
     a[2] = (int) __builtin_amdgcn_alignbyte(t5, t4, shift);
     a[3] = (int) __builtin_amdgcn_alignbyte(t6, t5, shift);
+    // (requested ahead of the scales: behind them the loop had 16 more waits, seven projections of 8 rows 25.1 -> 25.35 us)
     v4i c = { 0, 0, 0, 0 };
+    if constexpr (WT == kQ4_0) {
+      c = *reinterpret_cast<const v4i *>(bp_lds + c_at);
+    }
     const uint32_t sa = *reinterpret_cast<const uint32_t *>(bp_lds + s_at) & s_mask;
     // weights: nibbles as they are (0..15), low nibbles = elements e .. e + 7, high nibbles = elements 16 + e ..
     // (Q8_0: the operand as it lies)
     v4i b;
     if constexpr (WT == kQ4_0) {
-      c = *reinterpret_cast<const v4i *>(bp_lds + c_at);
       const uint32_t w0 = second ? q[0].z : q[0].x, w1 = second ? q[0].w : q[0].y;
       b[0] = (int) (w0 & 0x0f0f0f0fu), b[1] = (int) (w1 & 0x0f0f0f0fu);
       b[2] = (int) ((w0 >> 4) & 0x0f0f0f0fu), b[3] = (int) ((w1 >> 4) & 0x0f0f0f0fu);
@@ -376,9 +381,11 @@ bool bp_alone(int nblk, int wt) {
 }
 
 typedef void (*BpKernel)(BlockPairsGroupArgs, int);
-const BpKernel kBpKernels[2][2] = {
-  { matmul_block_pairs_kernel<kBpDepthShared, kQ4_0>, matmul_block_pairs_kernel<kBpDepthAlone, kQ4_0> },
-  { matmul_block_pairs_kernel<kBpDepthShared, kQ8_0>, matmul_block_pairs_kernel<kBpDepthAlone, kQ8_0> } };
+const BpKernel kBpKernels[2][2][2] = {
+  { { matmul_block_pairs_kernel<kBpDepthShared, kQ4_0, false>, matmul_block_pairs_kernel<kBpDepthAlone, kQ4_0, false> },
+    { matmul_block_pairs_kernel<kBpDepthShared, kQ8_0, false>, matmul_block_pairs_kernel<kBpDepthAlone, kQ8_0, false> } },
+  { { matmul_block_pairs_kernel<kBpDepthShared, kQ4_0, true>, matmul_block_pairs_kernel<kBpDepthAlone, kQ4_0, true> },
+    { matmul_block_pairs_kernel<kBpDepthShared, kQ8_0, true>, matmul_block_pairs_kernel<kBpDepthAlone, kQ8_0, true> } } };
 
 }  // namespace
 
@@ -430,22 +437,22 @@ hipError_t launch_matmul_block_pairs_group(hipStream_t stream, int count, float 
   // (the longest rows of the launch decide its LDS size and with it how many workgroups share a compute unit)
   const bool     alone  = bp_alone(k_max / 32, wt);
   const size_t   lds    = (size_t) bp_layout(k_max / 32, wt).total;
-  const BpKernel kernel = kBpKernels[wt == kQ8_0][alone];
-  static bool attr_set[2][2] = {};  // more than the default 64 KiB of dynamic LDS for long rows
-  if (!attr_set[wt == kQ8_0][alone]) {
+  // (rows to be quantized beside take a few of the resident places while the members' workgroups walk)
+  const unsigned more   = beside ? (beside->blocks + kBpThreads / 4 - 1) / (kBpThreads / 4) : 0;
+  const bool     take   = more > 0 && more <= 16;
+  const BpKernel kernel = kBpKernels[take][wt == kQ8_0][alone];
+  static bool attr_set[2][2][2] = {};  // more than the default 64 KiB of dynamic LDS for long rows
+  if (!attr_set[take][wt == kQ8_0][alone]) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int) kBpLdsLimit);
     if (e != hipSuccess) {
       return e;
     }
-    attr_set[wt == kQ8_0][alone] = true;
+    attr_set[take][wt == kQ8_0][alone] = true;
   }
   // As many workgroups as the device holds at once (LDS decides: three of 43 KB for k = 4096, one of 113 KB for
   // k = 11008, on each of 256 compute units), shared out among the members by their weight bytes; a member's
   // workgroups take its tiles in turn.
   const int  per_cu   = alone ? 1 : (int) std::min<size_t>(3, kBpLdsLimit / lds);
-  // (rows to be quantized beside take a few of those places while the members' workgroups walk)
-  const unsigned more = beside ? (beside->blocks + kBpThreads / 4 - 1) / (kBpThreads / 4) : 0;
-  const bool     take = more > 0 && more <= 16;
   const long resident = 256L * per_cu - (take ? more : 0);
   long       tiles    = 0;
   for (int i = 0; i < count; ++i) {

@@ -116,7 +116,7 @@ struct LaneOrderGroupArgs {
   const uint8_t *w[kGemvGroupMax];    // repacked weights
   const uint8_t *act[kGemvGroupMax];  // Q8_0 activation rows of each member (members may share them)
   float         *out[kGemvGroupMax];
-  int            n[kGemvGroupMax];
+  int            n[kGemvGroupMax + 1];  // (0 behind the last member)
   int            count;
   QuantizeBeside beside;  // by the workgroups of a grid row behind the members'
 };
@@ -140,14 +140,11 @@ __global__ __launch_bounds__(kLoThreads) void matmul_lane_order_kernel(LaneOrder
   constexpr int kLoActRows  = ROWS;
   constexpr int kLoScaleBlk = ROWS * 4;  // bytes of the scale table per block (one float per row)
   extern __shared__ __align__(16) uint8_t lo_lds[];  // activation panel, later the waves' sums
-  if ((int) blockIdx.y == grp.count) {
-    if (blockIdx.x * (kLoThreads / 4) < grp.beside.blocks) {
-      quantize_beside(grp.beside, (int) blockIdx.x, kLoThreads);
-    }
-    return;
-  }
   const int n = grp.n[blockIdx.y];
   if ((int) (blockIdx.x * kLoRows * TPW) >= n) {
+    if ((int) blockIdx.y == grp.count && blockIdx.x * (kLoThreads / 4) < grp.beside.blocks) {
+      quantize_beside(grp.beside, (int) blockIdx.x, kLoThreads);
+    }
     return;  // whole workgroup: this member has fewer rows than the widest one
   }
   constexpr int WQ = kLoWaves / TPW;  // waves that share a tile

@@ -269,7 +269,7 @@ void flush_members(htpops_context *ctx, GemvBatch &b, const QuantizeJob *beside,
       // 2..16 rows. Which kernel a matrix gets depends on that matrix alone, in the order of the single request
       // (run_few_rows): two and three rows of Q4_0 that fit the two-blocks-per-instruction kernel and have, or get, their
       // repacked copy go there; other two- and three-row members to the weight stream that keeps the rows in
-      // registers; the others to the kernel that streams their repacked copy (lane order), and what has no copy to
+      // registers; the others to the kernel that streams their repacked copy (block pairs or lane order), and what has no copy to
       // the K-sliced kernel. Every kind is one launch for all its members, each with its own activation rows (and
       // its own k, except in the lane-order kernel: a batch holds members of different k only where each of them fits
       // the two- and three-row kernel or the two-blocks-per-instruction kernel); the K-sliced kernel stages one set
